@@ -60,17 +60,7 @@ struct codag_ctx {
   uint32_t cu_count = 0;
   char name[256] = {0};
   codag_tune_params tune[4];
-  // cached hipGraph of the last batch launch
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t graph_exec = nullptr;
-  const void *g_descs = nullptr;
-  uint64_t g_n = 0;
-  const void *g_results = nullptr;
-  uint32_t g_flags = 0, g_groups = 0;
-  bool g_two_wave = false;
   uint32_t chunks_two_wave = 0;
-  hipStream_t g_stream = nullptr;
-  int g_slot = -1;
   uint32_t poll_shift = 0;  // RLE v2 queue kernel: nonzero = waits without polls (tests)
 };
 
@@ -122,7 +112,8 @@ void default_tune(codag_ctx *c) {
   // autotuner can pick per column
   c->tune[CODAG_RLEV1] = {512, 2048, 0, 4};
   c->tune[CODAG_RLEV2] = {128, 4096, 0, 2};
-  // two-wave batch workgroups, 12 per CU (the one-wave shape allows up to 32)
+  // batches by eight waves or one wave per stream, as their sizes have it, up
+  // to 12 workgroups per CU
   c->tune[CODAG_DEFLATE] = {128, 0, 12, 1};
   c->tune[0] = {0, 0, 0, 0};
 }
@@ -206,8 +197,6 @@ codag_status codag_ctx_destroy(codag_ctx *c) {
   if (!c) return CODAG_OK;
   DeviceGuard g(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
-  if (c->graph) (void)hipGraphDestroy(c->graph);
   for (auto &sl : c->slots)
     if (sl.done) {
       if (sl.used) (void)hipEventSynchronize(sl.done);
@@ -289,14 +278,12 @@ codag_status codag_inflate_chunks(codag_ctx *ctx, const uint8_t *d_comp, uint64_
   if (chunk_bytes == 0) return fail(CODAG_ERR_INVALID, "inflate_chunks: chunk_bytes is 0");
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "inflate_chunks: too many chunks");
   DeviceGuard g(ctx->device);
-  // Two-wave workgroups (a decoding and a writing wave per chunk) shorten
-  // each chunk's decode but hold fewer chunks in flight than one-wave
-  // workgroups (32 per CU): measured on 128 KiB chunks, they pay up to about
-  // 12 chunks per CU.
-  bool two_wave = n_chunks <= (uint64_t)ctx->cu_count * 12;
-  if (ctx->chunks_two_wave) two_wave = ctx->chunks_two_wave == 1;
+  // Eight waves per chunk while there are few chunks, else one wave per chunk
+  // (the line is drawn where launch_inflate_chunks gives both sides' times).
+  bool many = n_chunks <= (uint64_t)ctx->cu_count * 5;
+  if (ctx->chunks_two_wave) many = ctx->chunks_two_wave == 1;
   HIP_TRY(launch_inflate_chunks(d_comp, comp_bytes, d_offsets, n_chunks, chunk_bytes, d_out,
-                                d_out_len, d_status, flags, pick(ctx, stream), two_wave));
+                                d_out_len, d_status, flags, pick(ctx, stream), many));
   return CODAG_OK;
 }
 
@@ -337,8 +324,7 @@ codag_status codag_lzss_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t c
 }
 
 // The counter slot of stream s: the slot s already owns, else a free one,
-// else the least recently used, after waiting for its last launch (and
-// dropping the cached graph, which refers to the slot's counter).
+// else the least recently used, after waiting for its last launch.
 static codag_status counter_slot(codag_ctx *ctx, hipStream_t s, int *out) {
   int pick_i = -1;
   for (int i = 0; i < kCounterSlots; i++)
@@ -352,13 +338,6 @@ static codag_status counter_slot(codag_ctx *ctx, hipStream_t s, int *out) {
     for (int i = 1; i < kCounterSlots; i++)
       if (ctx->slots[i].last_use < ctx->slots[pick_i].last_use) pick_i = i;
     HIP_TRY(hipEventSynchronize(ctx->slots[pick_i].done));
-    if (ctx->g_slot == pick_i) {
-      if (ctx->graph_exec) (void)hipGraphExecDestroy(ctx->graph_exec);
-      if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-      ctx->graph_exec = nullptr;
-      ctx->graph = nullptr;
-      ctx->g_slot = -1;
-    }
   }
   auto &sl = ctx->slots[pick_i];
   sl.stream = s;
@@ -376,58 +355,12 @@ codag_status codag_inflate_batch(codag_ctx *ctx, const codag_stream_desc *d_desc
   if (n >= 0xffffffffull) return fail(CODAG_ERR_INVALID, "inflate_batch: too many streams");
   DeviceGuard g(ctx->device);
   hipStream_t s = pick(ctx, stream);
-  const uint32_t per_cu = std::max(1u, ctx->tune[CODAG_DEFLATE].groups_per_cu);
-  const bool two_wave = ctx->tune[CODAG_DEFLATE].threads_per_group == 128;
-  uint32_t groups = ctx->cu_count * per_cu;
-  if (n && groups > n) groups = (uint32_t)n;
-  if (groups == 0) groups = 1;
+  const codag_tune_params &t = ctx->tune[CODAG_DEFLATE];
   int slot = -1;
   if (codag_status st = counter_slot(ctx, s, &slot)) return st;
   uint32_t *counter = ctx->d_counter + slot * (kCounterStride / sizeof(uint32_t));
-  // Replay the captured graph when the same batch is launched again.
-  if (ctx->graph_exec && ctx->g_descs == d_descs && ctx->g_n == n &&
-      ctx->g_results == d_results && ctx->g_flags == flags && ctx->g_groups == groups &&
-      ctx->g_two_wave == two_wave && ctx->g_stream == s && ctx->g_slot == slot) {
-    HIP_TRY(hipGraphLaunch(ctx->graph_exec, s));
-    HIP_TRY(hipEventRecord(ctx->slots[slot].done, s));
-    return CODAG_OK;
-  }
-  if (ctx->graph_exec) {
-    (void)hipGraphExecDestroy(ctx->graph_exec);
-    ctx->graph_exec = nullptr;
-  }
-  if (ctx->graph) {
-    (void)hipGraphDestroy(ctx->graph);
-    ctx->graph = nullptr;
-  }
-  ctx->g_slot = -1;
-  // Capture counter reset + persistent kernel into a graph on this stream.
-  hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-  if (e == hipSuccess) {
-    hipError_t le = launch_inflate_batch(d_descs, n, d_results, flags, counter, groups, s, two_wave);
-    e = hipStreamEndCapture(s, &ctx->graph);
-    if (le != hipSuccess) e = le;
-  }
-  if (e == hipSuccess) e = hipGraphInstantiate(&ctx->graph_exec, ctx->graph, nullptr, nullptr, 0);
-  if (e == hipSuccess) {
-    ctx->g_descs = d_descs;
-    ctx->g_n = n;
-    ctx->g_results = d_results;
-    ctx->g_flags = flags;
-    ctx->g_groups = groups;
-    ctx->g_two_wave = two_wave;
-    ctx->g_stream = s;
-    ctx->g_slot = slot;
-    HIP_TRY(hipGraphLaunch(ctx->graph_exec, s));
-    HIP_TRY(hipEventRecord(ctx->slots[slot].done, s));
-    return CODAG_OK;
-  }
-  // Capture unavailable: launch directly.
-  (void)hipGetLastError();
-  if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-  ctx->graph = nullptr;
-  ctx->graph_exec = nullptr;
-  HIP_TRY(launch_inflate_batch(d_descs, n, d_results, flags, counter, groups, s, two_wave));
+  HIP_TRY(launch_inflate_batch(d_descs, n, d_results, flags, counter, ctx->cu_count,
+                               std::max(1u, t.groups_per_cu), s, t.threads_per_group == 128));
   HIP_TRY(hipEventRecord(ctx->slots[slot].done, s));
   return CODAG_OK;
 }
@@ -449,12 +382,8 @@ codag_status codag_inflate_batch_noalloc(const codag_stream_desc *d_descs, uint6
   HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   uint32_t *counter = nullptr;
   HIP_TRY(inflate_scratch_ptr(&counter));
-  const uint64_t per_cu = groups_per_cu ? groups_per_cu : 28;
-  uint64_t groups = (uint64_t)(cus > 0 ? cus : 256) * per_cu;
-  if (n && groups > n) groups = n;
-  if (groups == 0) groups = 1;
-  HIP_TRY(launch_inflate_batch(d_descs, n, d_results, flags, counter, (uint32_t)groups,
-                               static_cast<hipStream_t>(stream)));
+  HIP_TRY(launch_inflate_batch(d_descs, n, d_results, flags, counter, (uint32_t)(cus > 0 ? cus : 256),
+                               groups_per_cu ? groups_per_cu : 28, static_cast<hipStream_t>(stream), true));
   return CODAG_OK;
 }
 
@@ -775,18 +704,18 @@ codag_status codag_lzss_decode_host(codag_ctx *ctx, const uint8_t *c, uint64_t c
 
 // ------------------------------------------------------------------ tuning
 
-// Test hook, not in the public header (no counterpart in the reference):
-// `shift` nonzero switches the RLE v2 walker + expander kernel to its
-// variant without polls in its bounded waits (0 restores the normal one), so
-// a test can drive the waits' error path.
 // Test hook, not in the public header: codag_inflate_chunks' workgroups --
-// 0 chosen by chunk count, 1 two waves per chunk, 2 one wave per chunk.
+// 0 chosen by chunk count, 1 eight waves per chunk, 2 one wave per chunk.
 codag_status codag_test_chunks_two_wave(codag_ctx *ctx, uint32_t on) {
   if (!ctx) return fail(CODAG_ERR_INVALID, "test_chunks_two_wave: null ctx");
   ctx->chunks_two_wave = on;
   return CODAG_OK;
 }
 
+// Test hook, not in the public header (no counterpart in the reference):
+// `shift` nonzero switches the RLE v2 walker + expander kernel to its
+// variant without polls in its bounded waits (0 restores the normal one), so
+// a test can drive the waits' error path.
 codag_status codag_test_poll_shift(codag_ctx *ctx, uint32_t shift) {
   if (!ctx) return fail(CODAG_ERR_INVALID, "test_poll_shift: null ctx");
   ctx->poll_shift = shift;
@@ -832,7 +761,7 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
   std::vector<codag_tune_params> cands;
   if (codec == CODAG_DEFLATE) {
     for (uint32_t per : {8u, 16u, 20u, 24u, 28u}) cands.push_back({64, 0, per, 1});
-    for (uint32_t per : {8u, 12u, 14u}) cands.push_back({128, 0, per, 1});  // two-wave
+    for (uint32_t per : {8u, 12u, 14u}) cands.push_back({128, 0, per, 1});  // by size
   } else {
     if (codec == CODAG_RLEV1) cands.push_back({512, 2048, 0, 4});  // pipelined walker + helpers
     cands.push_back({256, 4096, 0, 2});  // walker + expander shapes
@@ -983,20 +912,12 @@ codag_status codag_stream_destroy(codag_ctx *ctx, codag_stream_t stream) {
   DeviceGuard g(ctx->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
   HIP_TRY(hipStreamSynchronize(s));
-  // a counter slot or cached graph bound to this stream is released with it
+  // a counter slot bound to this stream is released with it
   for (auto &sl : ctx->slots)
     if (sl.used && sl.stream == s) {
       sl.used = false;
       sl.stream = nullptr;
     }
-  if (ctx->g_stream == s) {
-    if (ctx->graph_exec) (void)hipGraphExecDestroy(ctx->graph_exec);
-    if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-    ctx->graph_exec = nullptr;
-    ctx->graph = nullptr;
-    ctx->g_stream = nullptr;
-    ctx->g_slot = -1;
-  }
   HIP_TRY(hipStreamDestroy(s));
   return CODAG_OK;
 }

@@ -1,46 +1,44 @@
-// inflate.hip -- gfx950 zlib/Deflate (RFC 1950/1951) decoder, one wave64 per stream.
+// inflate.hip -- gfx950 zlib/Deflate (RFC 1950/1951) decoder, a group of waves per stream.
 //
-// Mapping onto CDNA:
-//  * Bit reader: wave-uniform (SGPR) 64-bit bit buffer. The compressed input
-//    is held in two VGPR windows -- lane i holds dword i of a 256-byte window
-//    -- and refilled into the bit buffer with v_readlane, so a refill costs no
-//    memory round trip; the next window is prefetched with one coalesced load.
-//  * Huffman tables: per-wave LDS lookup tables built per block by all 64
-//    lanes (literal/length table of 10 bits in the one-wave kernels and 11
-//    in the decoding wave of a two-wave group, 8-bit distance table,
-//    canonical count/symbol arrays for the rare longer codes). Table entries carry the
-//    RFC 1951 length/distance base and extra-bit count directly; a literal's
-//    entry has bit 15 set so the symbol loop tests it with one scalar compare.
-//  * Two phases per batch of up to 64 symbols:
-//      1. decode only. The window decoder (vector unit) has lane j decode the
-//         token that would start at bit P + j of a 64-bit window, and a
-//         scalar readlane chain through the token lengths keeps the real
-//         token starts; the scalar symbol loop decodes the symbols that stop
-//         the chain (codes longer than the LUT, end-of-block, invalid codes)
-//         and the batches near the stream end. Token j of the batch is parked
-//         in lane j of a VGPR;
-//      2. the writer (this wave, or the second wave of a two-wave group)
-//         materialises the batch in ring-sized pieces: a wave prefix sum
-//         gives each token its output offset, literals go to an LDS ring in
-//         one store, matches whose source has left the ring are gathered from
-//         HBM (eight per memory round trip), short matches whose source
-//         precedes the piece are copied together (one lane each), and the
-//         remaining matches are copied ring -> ring in token order, 64 bytes
-//         per step.
-//    Decoding never depends on output bytes, so it runs without waiting on
-//    memory beyond its own table reads and stream loads.
-//  * The ring is written to HBM with 16-byte stores after each piece that
-//    leaves at least kFlush unwritten bytes; Adler-32 partial sums (sum b,
-//    sum pos*b) are accumulated on the way, so the trailer is verified without
-//    a second pass over the output.
-//  * Occupancy: a one-wave kernel uses a 1 KiB ring and 4736 B of LDS (32
-//    waves per CU); a two-wave group gives its writer a 2 KiB ring.
+// Mapping onto CDNA. A stream is decoded by a group of one wave (many streams:
+// throughput) or several waves (few streams: latency), in spans:
+//  * Span decode. The next 64 x waves x S bits of a block are staged in LDS and
+//    every lane decodes the subsequence of S bits that begins at its own bit.
+//    Only lane 0's start is known to be the start of a token; Huffman codes
+//    synchronise by themselves (a decoder started at a wrong bit meets the true
+//    token starts after about 90 bits at the median, 430 at the 95th
+//    percentile), so a lane's exit is mostly right although its entry was not.
+//    Each pass hands the exits on as the next lanes' entries and decodes the
+//    lanes whose entry changed, until no entry changes up to the first stop
+//    (end of block, invalid code, stream end). A lane does one table lookup a
+//    step: a literal takes one, a match two (length code, distance code), a
+//    code longer than the root table one more.
+//  * Output. The verified lanes know their byte counts; a prefix sum gives each
+//    its output position. They decode once more and write a 16-bit mark at each
+//    token's first byte into an LDS window (literal byte, or distance). The
+//    window is then resolved in rows of 64 bytes, one byte a lane: a DPP max
+//    scan hands every byte its token's mark, sources before the window are
+//    gathered from HBM (four rows in flight), sources inside it are followed by
+//    pointer doubling; the bytes are stored and summed for the Adler-32.
+//  * The scalar symbol loop decodes the symbol a span stopped at (end of block,
+//    or the error), so statuses are exactly the serial decoder's.
+// What bounds it: vector issue and its latency, not memory (without the far
+// gathers and the stores the launches take the same time). 128 KiB zlib level-6
+// chunks, before (one token chain per stream: 64 bit positions decoded to keep
+// about seven tokens, the chain scalar) and now: 4096 chunks 9.1 and 3.2 ms, 256
+// chunks 4.0 and 0.46 ms, 3 chunks 3.7 and 0.43 ms; 300 mixed streams of 4 KiB
+// to 4 MiB 119 and 15 ms. A chunk takes 0.27 M vector instructions (0.69 M
+// before): half of them passes, headers and tables, a fifth marks, a third the
+// resolving. Data that compress below 5% are slower than the copy loop of the
+// serial decoder where there are many chunks (4096 chunks of zeros 1.1 and 2.7
+// ms): a window byte costs the same whatever token it is in.
 //
 // Reference counterpart: include/zlib/zlib.h:807-866 (full_warp_shared_lut),
 // 531-707 (dynamic header / table build), 712-805 (symbol loop), 188-347
 // (warp copy). Differences: stored blocks are decoded (the reference's branch
 // is empty, zlib.h:840-842), BTYPE 11 is rejected (zlib.h:843 treats it as
 // dynamic), the zlib header and Adler-32 trailer are checked as zlib does.
+#include <algorithm>
 #include <cstddef>
 #include <mutex>
 
@@ -52,30 +50,12 @@ namespace inflate {
 
 using namespace codag::dev;
 
-// literal/length LUT bits: 10 for the one-wave kernels (32 waves fit a CU),
-// 11 for the decoding wave of a two-wave group (fewer codes leave the
-// window decoder for the symbol loop)
-constexpr uint32_t kLitBitsOne = 10;
-constexpr uint32_t kLitBitsPair = 11;
-constexpr uint32_t kDistBits = 8;
 constexpr uint32_t kCodeBits = 7;
-constexpr uint32_t kDistMask = (1u << kDistBits) - 1;
 
 enum : int32_t { kOk = 0, kTrunc = 1, kOverflow = 2, kCorrupt = 3 };
-constexpr int32_t kEob = 16;  // symbol loop stop: end of block (not a status)
-enum : uint32_t { kKindLit = 0, kKindLen = 1, kKindEob = 2, kKindBad = 3 };
+constexpr int32_t kEob = 16;   // end of block (not a status)
+constexpr int32_t kMore = 17;  // symbol loop: one symbol decoded (not a status)
 enum : uint32_t { kTabLit = 0, kTabDist = 1, kTabCodes = 2 };
-
-// 16-bit LUT entries (bits 3:0 always hold the code length; 0 = not in LUT):
-//   literal      : bit 15 set, byte in bits 11:4
-//   length code c: extra-bit count in bits 6:4 (0..5), base-3 in bits 14:7;
-//                  bits 6:4 = 7 marks end-of-block, 6 an invalid symbol
-//   distance d   : extra-bit count in bits 7:4, m in bits 9:8 with
-//                  base = (m << extra) + 1; bit 13 = invalid (d >= 30)
-//   code-length  : symbol in bits 12:8
-constexpr uint32_t kLitFlag = 0x8000u;
-constexpr uint32_t kDistBad = 0x2000u;
-constexpr uint32_t kXEob = 7, kXBad = 6;
 
 // RFC 1951 section 3.2.5 length and distance codes (the tables of
 // include/zlib/zlib.h:35-51) in closed form: length code c (0..28) has
@@ -101,419 +81,170 @@ template <int NSYM> struct Huff {
   uint16_t sym[NSYM];
 };
 
-// Output ring and piece limits. The writer materialises a batch (at most 64
-// tokens) in pieces: a piece ends at the first token at which its bytes
-// reach kBatch = R / 4, so it produces T < kBatch + 258 bytes, and the ring
-// is flushed to HBM once kFlush = R / 8 bytes are pending, so fewer than
-// kFlush bytes are unwritten at a piece start. Then (a) a piece never
-// overwrites a ring byte that is not yet in HBM and (b) a match whose source
-// lies before the ring's oldest intact byte reads only bytes that are
-// already in HBM, when R >= T + 258 + kFlush. One-wave kernels use a 1 KiB
-// ring, which leaves a wave under 5 KiB of LDS (32 waves per CU); the
-// writing wave of a two-wave group has a 2 KiB ring (fewer far gathers).
-template <uint32_t R> struct RingGeo {
-  static constexpr uint32_t kRing = R, kMask = R - 1, kBatch = R / 4, kFlush = R / 8;
-  static_assert((R & (R - 1)) == 0 && R >= kBatch + 258 + 258 + kFlush, "ring too small");
-};
-constexpr uint32_t kRingOne = 1024;
-constexpr uint32_t kRingPair = 2048;
-// A symbol reads at most 15 + 5 + 15 + 13 bits: a full batch (64 symbols)
-// that starts this far from the stream end cannot read past it, and the
-// 96-bit field the window decoder loads from the dword of any of its symbols
-// lies inside the stream's dwords.
-constexpr uint32_t kCarefulBits = 64 * 48 + 96;
-constexpr uint32_t kGather = 8;  // far-match pieces in flight per memory round trip
-// A wave's serial decode is latency-bound, so throughput grows with the waves
-// resident per SIMD: a one-wave kernel's LDS (4736 B, ten 512-byte allocation
-// blocks) allows 32 per CU, and its register budget is held to eight per SIMD
-// (64 VGPRs), so a 1 GiB container of 128 KiB chunks is decoded in one round.
-// Two-wave groups hold seven per SIMD.
-constexpr int kWavesOne = 8;
-constexpr int kWavesPair = 7;
+// 32-bit table entries:
+//   bits 4:0   bits this lookup consumes (code and extra bits); 0 = a stop: end
+//              of block, invalid symbol or no such code
+//   bits 8:5   extra-bit count
+//   bits 12:9  code bits this lookup consumes (the extra bits follow them)
+//   bit  13    literal
+//   bits 29:14 value: literal byte, length base, distance base, or, for a code
+//              longer than the root table, the sub-table's descriptor
+//   bits 31:30 0 the token is complete (literal, distance), 1 a length code
+//              (a distance code follows), 2 a sub-table lookup follows
+// A table descriptor is the table's index bits (bits 4:0, where a bit field
+// extract takes its width from) and its first entry (bits 15:5).
+constexpr uint32_t kLitFlag = 1u << 13;
+constexpr uint32_t kLenType = 1u << 30;
+constexpr uint32_t kSubType = 2u << 30;
 
-template <uint32_t LB> struct LdsT {
-  static constexpr uint32_t kLitBits = LB, kLitMask = (1u << LB) - 1;
-  alignas(16) uint8_t ring[kRingOne];
-  uint16_t lit[1u << LB];
-  uint16_t dist[1u << kDistBits];
+// One shape of the decoder: NW waves per stream, SD dwords of the stream per
+// lane in a span, each lane's part cut into SUB pieces for the output phase (a
+// wave writes its span in SUB groups, so that a group's bytes fit the window),
+// SEG window bytes per wave, root tables of LB and DB bits with room for LS and
+// DS sub-table entries. 340 / 272 entries hold every sub-table of a complete
+// 286 / 30 symbol code behind 9 / 7 root bits, 308 / 144 behind 10 / 8; a
+// sub-table that finds no room becomes a stop, which the symbol loop decodes.
+template <int NW_, int SD_, int SUB_, uint32_t SEG_, uint32_t LB_, uint32_t DB_, uint32_t LS_, uint32_t DS_>
+struct Cfg {
+  static constexpr int kNW = NW_, kSub = SUB_;
+  static constexpr uint32_t kThreads = NW_ * 64, kSD = SD_, kSpanBits = SD_ * 32;
+  static constexpr uint32_t kSeg = SEG_, kWin = NW_ * SEG_;
+  static constexpr uint32_t kLB = LB_, kDB = DB_, kLS = LS_, kDS = DS_;
+  static constexpr uint32_t kDistAt = (1u << LB_) + LS_, kTab = kDistAt + (1u << DB_) + DS_;
+  static constexpr uint32_t kLitDesc = LB_, kDistDesc = kDistAt << 5 | DB_;
+  static constexpr uint32_t kStage = kThreads * SD_ + 5;
+  static_assert(kTab <= 2048, "sub-table descriptors hold 11-bit positions");
+  static_assert(SEG_ % 512 == 0 && SEG_ <= 16384, "a segment is whole pairs of row groups, tracked in one 64-bit mask");
+  static_assert(NW_ * SEG_ <= 32768, "distances inside the window stay below the literal flag");
+  static_assert(NW_ == 1 || SUB_ == 1, "pieces are exchanged inside one wave");
+};
+// Odd SD: the lanes' first reads fall on different LDS banks.
+using One = Cfg<1, 13, 2, 4096, 9, 7, 340, 272>;
+using Many = Cfg<8, 9, 1, 2560, 10, 8, 308, 144>;
+
+template <class C> struct Sh {
+  alignas(16) uint32_t stage[C::kStage];  // the span's stream dwords
+  alignas(16) uint32_t tab[C::kTab];      // literal/length root, its sub-tables, distance root, its sub-tables
+  alignas(16) uint16_t win[C::kWin];      // marks of the window being written; CRC-32 slice tables
   Huff<288> hl;
   Huff<32> hd;
   alignas(4) uint8_t lens[320];
+  uint32_t err;                       // first output error of a window: position << 2 | status
+  // groups of several waves
+  uint32_t ex[C::kNW > 1 ? C::kThreads : 1];  // lanes' exits, bit 31 = stopped
+  uint32_t mis[C::kNW], stp[C::kNW];          // per wave: first lane with a changed entry / that stopped
+  uint32_t part[2][C::kNW];                   // per-wave partial sums
+  uint32_t end;                               // stage bit after the span's last token
+  // what the serial decoder found next (serial_step)
+  uint32_t op, P, ln, val, dist, pos;
+  int32_t st;
+  uint32_t last;
+  uint32_t stream;                            // the group's current stream
 };
-using Lds = LdsT<kLitBitsOne>;
-using LdsPair = LdsT<kLitBitsPair>;
-static_assert(sizeof(Lds::lens) >= 4 * (kWave + 16), "lens doubles as the token slots");
-// The first 4 KiB (ring, lit, dist and the start of hl) hold the CRC-32 slice
-// tables while no block is being decoded (gzip header and trailer)
-static_assert(sizeof(Lds) >= 4096, "CRC tables need 4 KiB");
+
+// LDS seen through a pointer of its own address space: functions that are not
+// inlined would else reach it by flat accesses.
+template <class T> using lds = __attribute__((address_space(3))) T;
 
 __device__ __forceinline__ uint32_t rdlane(uint32_t v, uint32_t j) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)j);
 }
 
-// Orders this wave's LDS accesses around a point where lanes exchange data
-// through LDS. The decoder's tables, slots and ring are written and read by
-// one wave, so fences (no workgroup barrier) are enough, and a second wave
-// of the workgroup (the writing wave of the two-wave batch kernel) is never
-// waited for.
+// Orders this wave's LDS accesses around a point where its lanes exchange data
+// through LDS.
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// ------------------------------------------------------------- bit reader
-
-struct Bits {
-  const uint32_t *w;  // 4-aligned address at or below the stream start
-  uint32_t limit;     // bit index (from w) one past the stream's last bit
-  uint32_t nw;        // dwords that hold stream bytes
-  uint32_t next;      // next dword to append to buf
-  uint64_t buf;
-  uint32_t cnt;
-  uint32_t wbase;     // first dword of the current 64-dword block (a multiple of 64)
-  // Blocks of 64 dwords, lane i holding dword i: the block at dword 64*m lives
-  // in w0 for even m and in w1 for odd m. The current block and the next one
-  // are resident; a register is reloaded only when its block is used up, so
-  // the windows never move between registers.
-  uint32_t w0, w1;
-};
-
-__device__ __forceinline__ uint32_t bits_block(const Bits &b, uint32_t first) {
-  const uint32_t i = first + lane_id();
-  return i < b.nw ? b.w[i] : 0u;
+// Keeps the compiler from moving LDS accesses across it; a wave's LDS
+// instructions are executed in order, so no wait is needed.
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ void bits_windows(Bits &b) {
-  const uint32_t cur = bits_block(b, b.wbase), nxt = bits_block(b, b.wbase + kWave);
-  const bool odd = (b.wbase / kWave) & 1;
-  b.w0 = odd ? nxt : cur;
-  b.w1 = odd ? cur : nxt;
+// The same for the whole group.
+template <class C> __device__ __forceinline__ void group_sync() {
+  if constexpr (C::kNW > 1) __syncthreads();
+  else wave_sync();
 }
 
-__device__ __forceinline__ void bits_refill(Bits &b) {
-  if (b.cnt <= 32) {
-    uint32_t k = b.next - b.wbase;
-    if (k >= (uint32_t)kWave) {
-      // the used-up block's register takes the block after the next one
-      if ((b.wbase / kWave) & 1) b.w1 = bits_block(b, b.wbase + 2 * kWave);
-      else b.w0 = bits_block(b, b.wbase + 2 * kWave);
-      b.wbase += kWave;
-      k -= kWave;
-    }
-    const uint32_t d = ((b.wbase / kWave) & 1) ? rdlane(b.w1, k) : rdlane(b.w0, k);
-    b.buf |= (uint64_t)d << b.cnt;
-    b.cnt += 32;
-    b.next++;
-  }
-}
-
-__device__ __forceinline__ void bits_drop(Bits &b, uint32_t n) {
-  b.buf >>= n;
-  b.cnt -= n;
-}
-
-// Moves the reader forward to bit P (P >= its position).
-__device__ __forceinline__ void bits_set(Bits &b, uint32_t P) {
-  const uint32_t nx = P >> 5;
-  if (nx - b.wbase >= 2u * kWave) {  // past both resident blocks
-    b.wbase = nx & ~(uint32_t)(kWave - 1);
-    bits_windows(b);
-  }
-  b.next = nx;
-  b.buf = 0;
-  b.cnt = 0;
-  bits_refill(b);
-  bits_drop(b, P & 31);
-}
-
-__device__ __forceinline__ uint32_t bits_pos(const Bits &b) { return b.next * 32 - b.cnt; }
-
-__device__ __forceinline__ bool bits_past_end(const Bits &b) { return bits_pos(b) > b.limit; }
-
-// Positions the reader at stream byte `at` (byte granular).
-__device__ __forceinline__ void bits_seek(Bits &b, uint64_t lead_plus_at) {
-  const uint64_t bit = lead_plus_at * 8;
-  b.next = (uint32_t)(bit >> 5);
-  b.wbase = b.next & ~(uint32_t)(kWave - 1);
-  bits_windows(b);
-  b.buf = 0;
-  b.cnt = 0;
-  bits_refill(b);
-  bits_drop(b, (uint32_t)(bit & 31));
-  bits_refill(b);
+// Inclusive wave64 prefix maximum with DPP row shifts and row broadcasts.
+__device__ __forceinline__ uint32_t wave_max_dpp(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));  // row_shr:2
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));  // row_shr:4
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));  // row_shr:8
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+  return v;
 }
 
 // ------------------------------------------------------------- output side
 
-// The most recent R output bytes live in an LDS ring. Byte x of the
-// stream sits at ring[(x + mis) & (R - 1)], where mis = dst & 15, so a
-// 16-byte aligned output address is also 16-byte aligned in the ring.
-// Positions are 32-bit (outputs below 2^31 bytes) so the wave-uniform state
-// stays in scalar registers.
-template <uint32_t R> struct Out : RingGeo<R> {
-  uint8_t *dst;      // global output
-  uint8_t *ring;     // LDS ring
+// Output state, the same in every wave of the group except the per-lane
+// Adler-32 partial sums: s1 = sum b, s2 = sum pos*b (mod 65521), both reduced
+// after every window. Positions are 32-bit (outputs below 2^31 bytes).
+struct Out {
+  uint8_t *dst;
   uint32_t cap;
-  uint32_t pos;      // bytes produced
-  uint32_t flushed;  // bytes [0, flushed) have been stored to dst
-  uint32_t mis;      // dst & 15
-  // Per-lane Adler-32 partial sums: s1 = sum b, s2 = sum pos*b (mod 65521),
-  // both reduced after every store. One store adds at most ~8e8 to s2 (at
-  // most 15 single bytes and two 16-byte groups per lane), so 32 bits hold.
+  uint32_t pos;  // bytes produced; all of them are stored
   uint32_t s1, s2;
 };
 
-template <class O> __device__ __forceinline__ uint32_t ridx(const O &o, uint32_t x) {
-  return (x + o.mis) & O::kMask;
-}
-
-template <class O> __device__ __forceinline__ void adler_add(O &o, uint32_t at, uint32_t b) {
+__device__ __forceinline__ void adler_add(Out &o, uint32_t at, uint32_t b) {
   o.s1 += b;
-  o.s2 += (at % 65521u) * b;
+  o.s2 = (o.s2 + (at % 65521u) * b) % 65521u;
 }
 
-// Stores ring bytes [flushed, end) to HBM; `last` also writes a partial
-// 16-byte tail.
-template <class O> __device__ __forceinline__ void out_store(O &o, uint32_t lane, uint32_t end, bool last) {
-  uint32_t x = o.flushed;
-  // head bytes up to a 16-byte aligned output address
-  uint32_t head = (16 - ((o.mis + x) & 15)) & 15;
-  if (head > end - x) head = end - x;
-  if (head) {
-    if (lane < head) {
-      const uint32_t b = o.ring[ridx(o, x + lane)];
-      o.dst[x + lane] = (uint8_t)b;
-      adler_add(o, x + lane, b);
-    }
-    x += head;
+// One token by one wave, straight in HBM (the symbol loop's tokens).
+__device__ __forceinline__ int32_t out_token(Out &o, uint32_t lane, bool lit, uint32_t val, uint32_t dist) {
+  const uint32_t n = lit ? 1u : val;
+  if (o.pos + n > o.cap) return kOverflow;
+  if (!lit && dist > o.pos) return kCorrupt;  // zlib: "invalid distance too far back"
+  for (uint32_t i = lane; i < n; i += kWave) {
+    const uint32_t b = lit ? val : o.dst[o.pos - dist + i % dist];
+    o.dst[o.pos + i] = (uint8_t)b;
+    adler_add(o, o.pos + i, b);
   }
-  const uint32_t nvec = (end - x) / 16;
-  for (uint32_t k = lane; k < nvec; k += kWave) {
-    const uint32_t at = x + 16 * k;
-    const uint4 q = *reinterpret_cast<const uint4 *>(o.ring + ridx(o, at));
-    *reinterpret_cast<uint4 *>(o.dst + at) = q;
-    // sum b and sum i*b over the 16 bytes (v_dot4_u32_u8 against the byte
-    // weights), then s2 += at*sum + sum(i*b)
-    const uint32_t sum = __builtin_amdgcn_udot4(
-        q.x, 0x01010101u,
-        __builtin_amdgcn_udot4(q.y, 0x01010101u,
-                               __builtin_amdgcn_udot4(q.z, 0x01010101u,
-                                                      __builtin_amdgcn_udot4(q.w, 0x01010101u, 0u, false),
-                                                      false),
-                               false),
-        false);
-    const uint32_t wsum = __builtin_amdgcn_udot4(
-        q.x, 0x03020100u,
-        __builtin_amdgcn_udot4(q.y, 0x07060504u,
-                               __builtin_amdgcn_udot4(q.z, 0x0b0a0908u,
-                                                      __builtin_amdgcn_udot4(q.w, 0x0f0e0d0cu, 0u, false),
-                                                      false),
-                               false),
-        false);
-    o.s1 += sum;
-    o.s2 += (at % 65521u) * sum + wsum;
-  }
-  x += nvec * 16;
-  if (last && x < end) {
-    const uint32_t tail = end - x;
-    if (lane < tail) {
-      const uint32_t b = o.ring[ridx(o, x + lane)];
-      o.dst[x + lane] = (uint8_t)b;
-      adler_add(o, x + lane, b);
-    }
-    x = end;
-  }
-  o.flushed = x;
   o.s1 %= 65521u;
-  o.s2 %= 65521u;
-}
-
-// Copies far matches (lanes in fm) from HBM into the ring. The first 64 bytes
-// of kGather matches are loaded before any is written, so a group costs one
-// memory round trip; the rest of the (rare) longer far matches follows.
-template <class O>
-__device__ __forceinline__ void gather_far(O &o, uint32_t lane, uint64_t fm, uint32_t x,
-                                           uint32_t dist, uint32_t mlen) {
-  uint64_t g = fm;
-  while (g) {
-    uint32_t v[kGather];
-    uint64_t h = g;
-#pragma unroll
-    for (uint32_t k = 0; k < kGather; k++) {
-      v[k] = 0;
-      if (h) {
-        const uint32_t j = (uint32_t)__builtin_ctzll(h);
-        h &= h - 1;
-        const uint32_t sj = rdlane(x, j) - rdlane(dist, j), lj = rdlane(mlen, j);
-        if (lane < lj) v[k] = o.dst[sj + lane];
-      }
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < kGather; k++) {
-      if (g) {
-        const uint32_t j = (uint32_t)__builtin_ctzll(g);
-        g &= g - 1;
-        const uint32_t xj = rdlane(x, j), lj = rdlane(mlen, j);
-        if (lane < lj) o.ring[ridx(o, xj + lane)] = (uint8_t)v[k];
-      }
-    }
-  }
-  uint64_t lm = fm & __ballot(mlen > (uint32_t)kWave);
-  while (lm) {
-    const uint32_t j = (uint32_t)__builtin_ctzll(lm);
-    lm &= lm - 1;
-    const uint32_t xj = rdlane(x, j), dj = rdlane(dist, j), lj = rdlane(mlen, j);
-#pragma clang loop vectorize(disable) interleave(disable) unroll(disable)
-    for (uint32_t i = kWave + lane; i < lj; i += kWave) o.ring[ridx(o, xj + i)] = o.dst[xj - dj + i];
-  }
-}
-
-// floor(2^16 / d) + 1 for d = 1..63: (i * m[d]) >> 16 == i / d for every
-// i < 512. The product overshoots i / d by i * (m[d] - 2^16 / d) / 2^16 <
-// 512 / 2^16 = 1/128, while the fractional part of i / d is at most
-// 1 - 1/d <= 1 - 1/63, so the overshoot never carries into the next integer.
-struct Recip16 {
-  uint32_t m[64];
-  constexpr Recip16() : m() {
-    for (uint32_t d = 1; d < 64; d++) m[d] = 0x10000u / d + 1;
-  }
-};
-__constant__ Recip16 kRecip16 = Recip16();
-
-// Materialises the tokens of lanes [a, b) of a batch as one piece: rel is
-// the token's inclusive byte count from the piece start, tl its byte count.
-// Errors are reported for the first offending token, in stream order:
-// output past cap (overflow) or a distance beyond the bytes produced so far.
-// The tokens before it are still written, so the bytes written before an
-// error do not depend on where batches and pieces end.
-template <class O>
-__device__ __forceinline__ int32_t out_piece(O &o, uint32_t lane, uint32_t tok, bool isl, uint32_t mlen,
-                                             uint32_t dist, uint32_t tl, uint32_t rel, uint32_t a,
-                                             uint32_t b) {
-  const uint32_t x = o.pos + rel - tl;  // output position of this token
-  const bool inp = lane >= a && lane < b;
-  uint32_t err = 0;
-  if (inp && x + tl > o.cap) err = kOverflow;
-  else if (inp && !isl && dist > x) err = kCorrupt;  // zlib: "invalid distance too far back"
-  const uint64_t em = __ballot(err != 0);
-  int32_t st = kOk;
-  if (em) {
-    const uint32_t k = (uint32_t)__builtin_ctzll(em);
-    st = (int32_t)rdlane(err, k);
-    b = k;
-    if (b == a) return st;
-  }
-  const bool act = lane >= a && lane < b;
-  const bool lit = act && isl;
-  const bool mat = act && !isl;
-  const uint32_t pend = o.pos + rdlane(rel, b - 1);
-
-  if (lit) o.ring[ridx(o, x)] = (uint8_t)(tok >> 4);
-  // a source byte y is intact in the ring iff y >= pend - R
-  const bool far = mat && (x - dist) + O::kRing < pend;
-  const uint64_t fm = __ballot(far);
-  if (fm) gather_far(o, lane, fm, x, dist, mlen);
-  // A near match whose source ends before the piece's first byte reads only
-  // bytes that were in the ring before the piece, and writes bytes that no
-  // earlier token of the piece reads: such matches of up to 16 bytes are
-  // copied together, each lane its own, 4 bytes per step (bytes past the
-  // match's end repeat its last byte's copy). The other near matches follow
-  // in token order.
-  const bool ind = mat && !far && mlen <= 16u && (x - dist) + mlen <= o.pos;
-  if (__ballot(ind)) {
-    const uint32_t src = x - dist, last = mlen - 1;
-#pragma unroll
-    for (uint32_t i = 0; i < 16u; i += 4) {
-      if (!__ballot(ind && i < mlen)) break;
-      if (ind && i < mlen) {
-        const uint32_t k1 = min(i + 1, last), k2 = min(i + 2, last), k3 = min(i + 3, last);
-        const uint8_t b0 = o.ring[ridx(o, src + i)], b1 = o.ring[ridx(o, src + k1)];
-        const uint8_t b2 = o.ring[ridx(o, src + k2)], b3 = o.ring[ridx(o, src + k3)];
-        o.ring[ridx(o, x + i)] = b0;
-        o.ring[ridx(o, x + k1)] = b1;
-        o.ring[ridx(o, x + k2)] = b2;
-        o.ring[ridx(o, x + k3)] = b3;
-      }
-    }
-  }
-  uint64_t nm = __ballot(mat && !far && !ind);
-  while (nm) {  // in token order: a match may read bytes of earlier tokens
-    const uint32_t j = (uint32_t)__builtin_ctzll(nm);
-    nm &= nm - 1;
-    const uint32_t xj = rdlane(x, j), dj = rdlane(dist, j), lj = rdlane(mlen, j);
-    const uint32_t sj = xj - dj;
-    if (dj >= (uint32_t)kWave || lj <= dj) {
-      // byte i reads source byte sj + i: either the source ends before the
-      // match (lj <= dj) or, for i >= dj, it repeats byte i - dj, written one
-      // 64-byte step earlier. Most matches take the single first step.
-      if (lane < lj) o.ring[ridx(o, xj + lane)] = o.ring[ridx(o, sj + lane)];
-#pragma clang loop vectorize(disable) interleave(disable) unroll(disable)
-      for (uint32_t i = kWave + lane; i < lj; i += kWave)
-        o.ring[ridx(o, xj + i)] = o.ring[ridx(o, sj + i)];
-    } else {
-      // periodic copy: byte i = source byte i mod dj, the quotient by an
-      // integer reciprocal multiply (exact for i < 512, dj < 64)
-      const uint32_t rm = kRecip16.m[dj];
-#pragma clang loop vectorize(disable) interleave(disable) unroll(disable)
-      for (uint32_t i = lane; i < lj; i += kWave) {
-        const uint32_t m = i - ((i * rm) >> 16) * dj;
-        o.ring[ridx(o, xj + i)] = o.ring[ridx(o, sj + m)];
-      }
-    }
-  }
-  o.pos = pend;
-  if (pend - o.flushed >= O::kFlush) out_store(o, lane, pend, false);
-  return st;
-}
-
-// Materialises a batch of nt tokens (lane j holds token j):
-//   literal: its LUT entry (bit 15 set, byte in bits 11:4);
-//   match: length in bits 8:0 (bit 15 clear), distance in bits 31:16.
-// A batch of up to 64 tokens can produce up to 64 x 258 bytes, more than the
-// ring holds, so it is written in pieces: a piece ends at the first token at
-// which its bytes reach O::kBatch, so a piece produces T < kBatch + 258
-// bytes. The decoder only limits batches to 64 tokens.
-template <class O>
-__device__ __forceinline__ int32_t out_tokens(O &o, uint32_t lane, uint32_t tok, uint32_t nt) {
-  if (nt == 0) return kOk;
-  const bool isl = (tok & kLitFlag) != 0;
-  const uint32_t mlen = tok & 0x1ff;
-  const uint32_t dist = tok >> 16;
-  const uint32_t tl = lane < nt ? (isl ? 1u : mlen) : 0u;
-  const uint32_t incl = wave_scan_dpp(tl);
-  uint32_t a = 0, base = 0;  // the piece's first lane; bytes of the tokens before it
-  for (;;) {
-    const uint64_t over = __ballot(lane >= a && lane < nt && incl - base >= O::kBatch);
-    const uint32_t b = over ? (uint32_t)__builtin_ctzll(over) + 1 : nt;
-    const int32_t st = out_piece(o, lane, tok, isl, mlen, dist, tl, incl - base, a, b);
-    if (st != kOk || b == nt) return st;
-    base = rdlane(incl, b - 1);
-    a = b;
-  }
-}
-
-// Copies ln stored-block bytes from src + at through the ring (RFC 1951
-// 3.2.4), 256 bytes per step.
-template <class O>
-__device__ __forceinline__ int32_t store_copy(O &o, const uint8_t *src, uint64_t at, uint32_t ln,
-                                              uint32_t lane) {
-  if (o.pos + ln > o.cap) return kOverflow;
-  for (uint32_t done = 0; done < ln;) {
-    const uint32_t step = (ln - done) < 256u ? (ln - done) : 256u;
-#pragma clang loop vectorize(disable) interleave(disable) unroll(disable)
-    for (uint32_t i = lane; i < step; i += kWave) o.ring[ridx(o, o.pos + i)] = src[at + done + i];
-    o.pos += step;
-    done += step;
-    if (o.pos - o.flushed >= O::kFlush) out_store(o, lane, o.pos, false);
-  }
+  o.pos += n;
   return kOk;
 }
 
-// The last partial flush, then the Adler-32 of the bytes written (a wave
-// reduction of the per-lane partial sums, each already < 65521).
-template <class O> __device__ __forceinline__ uint32_t out_finish(O &o, uint32_t lane) {
-  out_store(o, lane, o.pos, true);
+// Copies ln stored-block bytes from src (RFC 1951 3.2.4); thread t of T copies
+// aligned output dwords, the few bytes before and after them singly.
+__device__ __forceinline__ int32_t store_copy(Out &o, const uint8_t *src, uint32_t ln, uint32_t t, uint32_t T) {
+  if (o.pos + ln > o.cap) return kOverflow;
+  uint8_t *d = o.dst + o.pos;
+  const uint32_t head = min((uint32_t)(-reinterpret_cast<uintptr_t>(d) & 3), ln);
+  const uint32_t nd = (ln - head) / 4, tail = head + 4 * nd;
+  if (t < head) {
+    d[t] = src[t];
+    adler_add(o, o.pos + t, src[t]);
+  }
+  if (t < ln - tail) {
+    d[tail + t] = src[tail + t];
+    adler_add(o, o.pos + tail + t, src[tail + t]);
+  }
+  for (uint32_t k = t; k < nd; k += T) {
+    uint32_t v;
+    __builtin_memcpy(&v, src + head + 4 * k, 4);
+    *reinterpret_cast<uint32_t *>(d + head + 4 * k) = v;
+    const uint32_t sum = __builtin_amdgcn_udot4(v, 0x01010101u, 0u, false);
+    o.s1 += sum;
+    o.s2 = (o.s2 + ((o.pos + head + 4 * k) % 65521u) * sum + __builtin_amdgcn_udot4(v, 0x03020100u, 0u, false)) % 65521u;
+  }
+  o.s1 %= 65521u;
+  o.pos += ln;
+  return kOk;
+}
+
+// The Adler-32 of the bytes written: the lanes' partial sums (each < 65521)
+// over the waves of the group.
+template <class C> __device__ __forceinline__ uint32_t out_adler(Out &o, Sh<C> &S, uint32_t wave) {
   uint32_t s1r = o.s1, s2r = o.s2;
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) {
@@ -521,6 +252,16 @@ template <class O> __device__ __forceinline__ uint32_t out_finish(O &o, uint32_t
     s2r += __shfl_xor(s2r, d, kWave);
   }
   uint64_t s1 = s1r, s2 = s2r;
+  if constexpr (C::kNW > 1) {
+    S.part[0][wave] = s1r;
+    S.part[1][wave] = s2r;
+    group_sync<C>();
+    s1 = s2 = 0;
+    for (int i = 0; i < C::kNW; i++) {
+      s1 += S.part[0][i];
+      s2 += S.part[1][i];
+    }
+  }
   s1 %= 65521u;
   s2 %= 65521u;
   const uint64_t n = o.pos % 65521u;
@@ -531,111 +272,159 @@ template <class O> __device__ __forceinline__ uint32_t out_finish(O &o, uint32_t
 
 // ------------------------------------------------------------- table build
 
-__device__ __forceinline__ uint32_t make_entry(uint32_t tab, uint32_t sym, uint32_t len) {
-  if (tab == kTabCodes) return len | (sym << 8);
+// cl: the code bits the lookup consumes (the code's length, less the root bits
+// in a sub-table).
+__device__ __forceinline__ uint32_t make_entry(uint32_t tab, uint32_t sym, uint32_t cl) {
+  if (tab == kTabCodes) return cl | (sym << 14);
   if (tab == kTabDist) {
-    if (sym >= 30) return len | kDistBad;
-    const uint32_t m = sym < 4 ? sym : 2 + (sym & 1);  // dist_base == (m << extra) + 1
-    return len | (dist_extra(sym) << 4) | (m << 8);
+    if (sym >= 30) return 0;
+    const uint32_t x = dist_extra(sym);
+    return (cl + x) | (x << 5) | (cl << 9) | (dist_base(sym, x) << 14);
   }
-  if (sym < 256) return len | (sym << 4) | kLitFlag;
-  if (sym == 256) return len | (kXEob << 4);
-  if (sym <= 285) {
-    const uint32_t c = sym - 257, x = len_extra(c);
-    return len | (x << 4) | ((len_base(c, x) - 3) << 7);
-  }
-  return len | (kXBad << 4);
+  if (sym < 256) return cl | (cl << 9) | kLitFlag | (sym << 14);
+  if (sym == 256 || sym > 285) return 0;
+  const uint32_t c = sym - 257, x = len_extra(c);
+  return (cl + x) | (x << 5) | (cl << 9) | (len_base(c, x) << 14) | kLenType;
 }
 
-// Builds the canonical tables for n code lengths in lens[] and the LUT of
-// 2^bits entries. Applies zlib's acceptance rules (inftrees.c): an
-// over-subscribed set is rejected; an incomplete set is rejected unless it
-// has a single code of length 1 (literal/distance tables) or no codes at all.
-// Out of line: it runs once per block, and keeping its unrolled code out of
-// the symbol loop leaves that loop's uniform state in scalar registers.
+// Builds the canonical tables for n code lengths in lens[], the root table of
+// 2^bits entries at tab + at and up to `room` sub-table entries behind it.
+// Applies zlib's acceptance rules (inftrees.c): an over-subscribed set is
+// rejected; an incomplete set is rejected unless it has a single code of
+// length 1 (literal/distance tables) or no codes at all.
+// The tables are filled per entry: with the codes left-justified to 15 bits,
+// lim[L] is the first value above the codes of up to L bits, so a value's code
+// length is one more than the number of limits it reaches (no loop over the
+// 2^(bits - L) copies of a short code, which one lane would write alone). Codes
+// longer than the root share their first `bits` bits p with a range of values
+// that ends below (p + 1) << (15 - bits); the longest of them is the last, so
+// its length sizes p's sub-table.
+// Out of line: it runs once per block.
 template <int NSYM>
-__device__ __noinline__ int32_t build_table(const uint8_t *lens, uint32_t n, uint32_t tab, Huff<NSYM> &h,
-                               uint16_t *lut, uint32_t bits) {
+__device__ __noinline__ int32_t build_table(const lds<uint8_t> *lens, uint32_t n, uint32_t kind,
+                                            lds<Huff<NSYM>> *h, lds<uint32_t> *tab, uint32_t at, uint32_t bits,
+                                            uint32_t room) {
   const uint32_t lane = lane_id();
-  if (lane < 16) h.count[lane] = 0;
-  for (uint32_t i = lane; i < (1u << bits); i += kWave) lut[i] = 0;
-  wave_sync();
-  for (uint32_t s = lane; s < n; s += kWave) {
-    const uint32_t L = lens[s];
-    if (L) atomicAdd(reinterpret_cast<uint32_t *>(&h.count[0]) + (L >> 1), 1u << (16 * (L & 1)));
+  lds<uint32_t> *root = tab + at;
+  // lane L: the number of codes of length L
+  uint32_t mycount = 0;
+  for (uint32_t base = 0; base < n; base += kWave) {
+    const uint32_t L = base + lane < n ? lens[base + lane] : 0u;
+    const uint64_t b0 = __ballot(L & 1), b1 = __ballot(L & 2), b2 = __ballot(L & 4), b3 = __ballot(L & 8);
+    const uint64_t m = (lane & 1 ? b0 : ~b0) & (lane & 2 ? b1 : ~b1) & (lane & 4 ? b2 : ~b2) & (lane & 8 ? b3 : ~b3);
+    mycount += (uint32_t)__builtin_popcountll(m);
   }
-  wave_sync();
-  // counts are packed two per dword above; all lanes walk them uniformly
   int32_t left = 1;
   uint32_t maxlen = 0, code = 0, idx = 0;
   uint32_t first_l = 0, index_l = 0;
-  const uint32_t myL = lane < 16 ? lane : 0;
+  uint32_t lim[16];
+#pragma unroll
   for (uint32_t L = 1; L < 16; L++) {
-    const uint32_t c = uni(h.count[L]);
+    const uint32_t c = rdlane(mycount, L);
     left = 2 * left - (int32_t)c;
     if (c) maxlen = L;
-    if (L == myL) {
+    if (L == lane) {
       first_l = code;
       index_l = idx;
     }
+    lim[L] = (code + c) << (15 - L);
     code = (code + c) << 1;
     idx += c;
   }
   if (left < 0) return kCorrupt;
   if (left > 0) {
-    if (tab == kTabCodes) return kCorrupt;
+    if (kind == kTabCodes) return kCorrupt;
     if (maxlen > 1) return kCorrupt;
   }
-  wave_sync();
   if (lane >= 1 && lane < 16) {
-    h.first[lane] = (uint16_t)first_l;
-    h.index[lane] = (uint16_t)index_l;
+    h->count[lane] = (uint16_t)mycount;
+    h->first[lane] = (uint16_t)first_l;
+    h->index[lane] = (uint16_t)index_l;
   }
-  wave_sync();
-  uint32_t run[16];
-#pragma unroll
-  for (int L = 0; L < 16; L++) run[L] = 0;
+  // the symbols in code order: by length, then by value
+  uint32_t run = index_l;  // lane L: the next place of a code of length L
   for (uint32_t base = 0; base < n; base += kWave) {
-    const uint32_t s = base + lane;
-    const uint32_t L = s < n ? lens[s] : 0;
-    uint32_t r = 0;
-#pragma unroll
-    for (int q = 1; q < 16; q++) {
-      const uint64_t m = __ballot(L == (uint32_t)q);
-      if (L == (uint32_t)q) r = run[q] + __popcll(m & ((1ull << lane) - 1));
-      run[q] += __popcll(m);
-    }
-    if (L) {
-      h.sym[h.index[L] + r] = (uint16_t)s;
-      if (L <= bits) {
-        const uint32_t c = h.first[L] + r;
-        const uint32_t rev = __builtin_bitreverse32(c) >> (32 - L);
-        const uint32_t e = make_entry(tab, s, L);
-        for (uint32_t k = 0; k < (1u << (bits - L)); k++) lut[rev | (k << L)] = e;
-      }
-    }
+    const uint32_t L = base + lane < n ? lens[base + lane] : 0u;
+    const uint64_t b0 = __ballot(L & 1), b1 = __ballot(L & 2), b2 = __ballot(L & 4), b3 = __ballot(L & 8);
+    const uint64_t same = (L & 1 ? b0 : ~b0) & (L & 2 ? b1 : ~b1) & (L & 4 ? b2 : ~b2) & (L & 8 ? b3 : ~b3);
+    const uint64_t mine =
+        (lane & 1 ? b0 : ~b0) & (lane & 2 ? b1 : ~b1) & (lane & 4 ? b2 : ~b2) & (lane & 8 ? b3 : ~b3);
+    const uint32_t place = __shfl(run, L, kWave) + (uint32_t)__builtin_popcountll(same & ((1ull << lane) - 1));
+    if (L) h->sym[place] = (uint16_t)(base + lane);
+    run += (uint32_t)__builtin_popcountll(mine);
   }
-  wave_sync();
+  lds_order();
+  uint32_t limr = 0;                                   // lim[bits]
+#pragma unroll
+  for (uint32_t L = 1; L < 16; L++)
+    if (L == bits) limr = lim[L];
+  for (uint32_t k = lane; k < (1u << bits); k += kWave) {
+    const uint32_t v = (__builtin_bitreverse32(k) >> (32 - bits)) << (15 - bits);
+    uint32_t e = 0;
+    if (v < limr) {  // else a longer code, or none
+      uint32_t L = 1;
+#pragma unroll
+      for (uint32_t q = 1; q < 11; q++) L += v >= lim[q] ? 1u : 0u;  // bits <= 10: no longer code here
+      const uint32_t c = v >> (15 - L);
+      e = make_entry(kind, h->sym[h->index[L] + c - h->first[L]], L);
+    }
+    root[k] = e;
+  }
+  lds_order();
+  if (maxlen <= bits) return kOk;
+  // sub-tables of the prefixes from limr on, in order
+  const uint32_t p0 = limr >> (15 - bits), p1 = 1u << bits;
+  uint32_t used = 0;
+  for (uint32_t base = p0; base < p1; base += kWave) {
+    const uint32_t p = base + lane;
+    uint32_t sb = 0;
+    if (p < p1) {
+      const uint32_t v = ((p + 1) << (15 - bits)) - 1;
+      uint32_t L = 1;
+#pragma unroll
+      for (uint32_t q = 1; q < 15; q++) L += v >= lim[q] ? 1u : 0u;
+      sb = L - bits;
+    }
+    const uint32_t size = sb ? 1u << sb : 0u;
+    const uint32_t incl = wave_scan_dpp(size);
+    const uint32_t to = used + incl - size;
+    if (p < p1)
+      root[__builtin_bitreverse32(p) >> (32 - bits)] =
+          to + size <= room ? bits | (sb << 14) | ((at + (1u << bits) + to) << 19) | kSubType : 0u;
+    used += rdlane(incl, kWave - 1);
+  }
+  lds_order();
+  for (uint32_t i = rdlane(index_l, bits) + rdlane(mycount, bits) + lane; i < idx; i += kWave) {
+    uint32_t L = bits + 1;  // the length of the i-th code
+    for (uint32_t q = bits + 1; q < 15; q++) L += i >= h->index[q] + h->count[q] ? 1u : 0u;
+    const uint32_t c = h->first[L] + (i - h->index[L]);
+    const uint32_t sl = L - bits;  // code bits in the sub-table
+    const uint32_t d = root[__builtin_bitreverse32(c >> sl) >> (32 - bits)];
+    if (d == 0) continue;
+    const uint32_t sb = (d >> 14) & 31, rev = __builtin_bitreverse32(c) >> (32 - L) >> bits;
+    const uint32_t e = make_entry(kind, h->sym[i], sl);
+    for (uint32_t k = rev; k < (1u << sb); k += 1u << sl) tab[((d >> 19) & 0x7ff) + k] = e;
+  }
+  lds_order();
   return kOk;
 }
 
-// Canonical decode of codes longer than the LUT (or invalid ones), RFC 1951
-// 3.2.2: the code of length L is the first L stream bits read MSB-first, and
+// Canonical decode of one code, RFC 1951 3.2.2: the code of length L is the first L stream bits read MSB-first, and
 // it is valid when it lies in [first[L], first[L] + count[L]). Lane L (1..15)
 // tests length L, so the tables are read once instead of once per length; the
 // shortest length that hits is the code (canonical codes are prefix-free).
 // Called by the whole wave. Returns the symbol or -1; *len gets the length.
 template <int NSYM>
-__device__ __forceinline__ int32_t slow_decode(const Huff<NSYM> &h, uint64_t buf, uint32_t *len) {
+__device__ __forceinline__ int32_t slow_decode(const lds<Huff<NSYM>> *h, uint32_t buf, uint32_t *len) {
   const uint32_t lane = lane_id();
   const uint32_t L = lane & 15u;
-  const uint32_t c = h.count[L], f = h.first[L], ix = h.index[L];
-  const uint32_t code = __builtin_bitreverse32((uint32_t)buf) >> ((32u - L) & 31u);  // L = 0: unused
+  const uint32_t c = L ? h->count[L] : 0u, f = h->first[L], ix = h->index[L];
+  const uint32_t code = __builtin_bitreverse32(buf) >> ((32u - L) & 31u);  // L = 0: unused
   const uint64_t m = __ballot(lane >= 1u && lane < 16u && code - f < c);
   if (m == 0) return -1;
   const uint32_t hit = (uint32_t)__builtin_ctzll(m);
   *len = hit;
-  return (int32_t)uni(h.sym[rdlane(ix + code - f, hit)]);
+  return (int32_t)uni(h->sym[rdlane(ix + code - f, hit)]);
 }
 
 // ------------------------------------------------------------- stream decode
@@ -649,169 +438,47 @@ __device__ __forceinline__ int32_t status_code(int32_t st, uint32_t flags) {
   return st == kOverflow ? 1 : (st == kTrunc ? 2 : -1);
 }
 
-template <class LD>
-__device__ __forceinline__ int32_t read_dynamic(Bits &b, LD &S, uint32_t *nlen_out) {
+// 32 stream bits from stage bit q on.
+__device__ __forceinline__ uint32_t stage_bits(const lds<uint32_t> *stage, uint32_t q) {
+  return __builtin_amdgcn_alignbit(stage[(q >> 5) + 1], stage[q >> 5], q);
+}
+
+// Reads a dynamic block's code lengths (RFC 1951 3.2.7) from stage bit *q on
+// and builds its tables; `limit` is the stage bit after the stream's last.
+// The run-length coded lengths are decoded 64 bits at a time: lane j decodes
+// the code that would start at bit q + j, a scalar chain through their lengths
+// marks the true starts, a prefix sum of the repeat counts gives the positions
+// and a prefix maximum the last length before each repeat. (A scalar loop, one
+// code after the other, took 85 K cycles a block.)
+template <class C>
+__device__ __forceinline__ int32_t read_dynamic(lds<Sh<C>> *S, uint32_t *qp, uint32_t limit) {
   const uint32_t lane = lane_id();
-  bits_refill(b);
-  const uint32_t nlen = (uint32_t)(b.buf & 31) + 257;
-  const uint32_t ndist = (uint32_t)((b.buf >> 5) & 31) + 1;
-  const uint32_t ncode = (uint32_t)((b.buf >> 10) & 15) + 4;
-  bits_drop(b, 14);
+  uint32_t q = *qp;
+  const uint32_t h = uni(stage_bits(S->stage, q));
+  const uint32_t nlen = (h & 31) + 257, ndist = ((h >> 5) & 31) + 1, ncode = ((h >> 10) & 15) + 4;
   if (nlen > 286 || ndist > 30) return kCorrupt;  // zlib: "too many length or distance symbols"
-  // code-length code lengths, 3 bits each, in permuted order (<= 57 bits)
-  bits_refill(b);
-  const uint32_t n1 = ncode < 10 ? ncode : 10;
-  const uint64_t c1 = b.buf;
-  bits_drop(b, 3 * n1);
-  bits_refill(b);
-  const uint32_t n2 = ncode - n1;
-  const uint64_t c2 = b.buf;
-  bits_drop(b, 3 * n2);
-  if (lane < 19) {
-    uint32_t v = 0;
-    if (lane < n1) v = (uint32_t)((c1 >> (3 * lane)) & 7);
-    else if (lane < ncode) v = (uint32_t)((c2 >> (3 * (lane - n1))) & 7);
-    S.lens[kClOrder[lane]] = (uint8_t)v;
-  }
-  wave_sync();
-  int32_t st = (int32_t)uni((uint32_t)build_table(S.lens, 19, kTabCodes, S.hl, S.lit, kCodeBits));
+  q += 14;
+  if (lane < 19)  // code-length code lengths, 3 bits each, in permuted order
+    S->lens[kClOrder[lane]] = lane < ncode ? (uint8_t)(stage_bits(S->stage, q + 3 * lane) & 7) : (uint8_t)0;
+  q += 3 * ncode;
+  lds_order();
+  int32_t st = (int32_t)uni((uint32_t)build_table(S->lens, 19, kTabCodes, &S->hl, S->tab, 0, kCodeBits, 0));
   if (st != kOk) return st;
-  // literal/length + distance code lengths with repeat codes 16/17/18
   const uint32_t total = nlen + ndist;
-  uint32_t i = 0;
+  for (uint32_t k = lane; k < sizeof(S->lens) / 4; k += kWave) reinterpret_cast<lds<uint32_t> *>(S->lens)[k] = 0;
+  lds_order();
+  uint32_t i = 0, prev = 0;
   while (i < total) {
-    bits_refill(b);
-    const uint32_t e = uni(S.lit[b.buf & ((1u << kCodeBits) - 1)]);
-    const uint32_t L = e & 15;
-    if (L == 0) return bits_past_end(b) ? kTrunc : kCorrupt;
-    bits_drop(b, L);
-    const uint32_t sym = e >> 8;
-    if (sym < 16) {
-      if (lane == 0) S.lens[i] = (uint8_t)sym;
-      i++;
-      continue;
-    }
-    uint32_t rep, val = 0;
-    if (sym == 16) {
-      if (i == 0) return kCorrupt;  // zlib: "invalid bit length repeat"
-      wave_sync();
-      val = uni(S.lens[i - 1]);
-      rep = 3 + (uint32_t)(b.buf & 3);
-      bits_drop(b, 2);
-    } else if (sym == 17) {
-      rep = 3 + (uint32_t)(b.buf & 7);
-      bits_drop(b, 3);
-    } else {
-      rep = 11 + (uint32_t)(b.buf & 127);
-      bits_drop(b, 7);
-    }
-    if (i + rep > total) return kCorrupt;
-    if (lane < rep) S.lens[i + lane] = (uint8_t)val;  // rep <= 138: two passes at most
-    if (lane + kWave < rep) S.lens[i + kWave + lane] = (uint8_t)val;
-    if (lane + 2 * kWave < rep) S.lens[i + 2 * kWave + lane] = (uint8_t)val;
-    i += rep;
-  }
-  if (bits_past_end(b)) return kTrunc;
-  wave_sync();
-  if (uni(S.lens[256]) == 0) return kCorrupt;  // zlib: "missing end-of-block"
-  st = (int32_t)uni((uint32_t)build_table(S.lens, nlen, kTabLit, S.hl, S.lit, LD::kLitBits));
-  if (st != kOk) return st;
-  st = (int32_t)uni((uint32_t)build_table(S.lens + nlen, ndist, kTabDist, S.hd, S.dist, kDistBits));
-  *nlen_out = nlen;
-  return st;
-}
-
-template <class LD> __device__ __forceinline__ void load_fixed(LD &S) {
-  const uint32_t lane = lane_id();
-  for (uint32_t s = lane; s < 288; s += kWave)
-    S.lens[s] = (uint8_t)(s < 144 ? 8 : (s < 256 ? 9 : (s < 280 ? 7 : 8)));
-  wave_sync();
-  build_table(S.lens, 288, kTabLit, S.hl, S.lit, LD::kLitBits);
-  for (uint32_t s = lane; s < 32; s += kWave) S.lens[s] = 5;
-  wave_sync();
-  build_table(S.lens, 32, kTabDist, S.hd, S.dist, kDistBits);
-}
-
-// The three stream dwords that hold the 64 bits from stream bit `at` (the
-// window decoder's per-lane input): one load, its first dword clamped to
-// nw - 3. The window decoder runs only for full batches, which start at
-// least kCarefulBits before the stream end, so at every position that starts
-// a symbol of the batch the three dwords are inside the stream and the clamp
-// changes only lanes no symbol of the batch starts at. The bits are taken
-// apart where they are used, so the load stays in flight until then.
-struct Field {
-  uint32_t d0, d1, d2;
-};
-
-__device__ __forceinline__ Field load_field(const Bits &b, uint32_t at) {
-  typedef __attribute__((address_space(1))) const uint32_t gdword;
-  const gdword *w = (const gdword *)b.w + min(at >> 5, b.nw - 3);
-  Field f;
-  f.d0 = w[0];
-  f.d1 = w[1];
-  f.d2 = w[2];
-  return f;
-}
-
-// v_alignbit_b32 shifts by its third operand's low five bits.
-__device__ __forceinline__ uint64_t field_bits(const Field &f, uint32_t at) {
-  const uint32_t xl = __builtin_amdgcn_alignbit(f.d1, f.d0, at);
-  const uint32_t xh = __builtin_amdgcn_alignbit(f.d2, f.d1, at);
-  return ((uint64_t)xh << 32) | xl;
-}
-
-// Window decode on the vector unit. Lane j decodes the token (a literal, or a
-// length code with its distance and extra bits) that would start at bit P + j
-// of the stream, from its own three stream dwords and the same LUT entries as
-// the symbol loop; a scalar chain through the token lengths then keeps the
-// real token starts. A token whose code is not in the LUT, an end-of-block
-// and an invalid code stop the chain (token length 128); the symbol loop
-// decodes that symbol. A batch ends at its 64th token (the writer cuts it
-// into pieces that fit its ring). Token k of the batch goes to slot[k] in
-// LDS (the caller moves the slots into tok once per batch); slots 64..79
-// take the writes of the lanes that start no token. The next window's loads
-// are issued as soon as the chain has placed it, ahead of the slot work.
-// Returns true when the batch is full, false at a symbol for the loop.
-template <class LD>
-__device__ __forceinline__ bool decode_window(Bits &b, const LD &S, uint32_t *slot, uint32_t lane,
-                                              uint32_t &nt) {
-  const uint32_t P0 = bits_pos(b);
-  uint32_t P = P0;
-  bool full;
-  Field f = load_field(b, P + lane);
-  for (;;) {
-    const uint64_t x = field_bits(f, P + lane);
-    const uint32_t xl = (uint32_t)x;
-    const uint32_t e = S.lit[xl & LD::kLitMask];
-    const uint32_t L = e & 15, lx = (e >> 4) & 7;
-    // a length code's extra bits, its distance code and that code's extra
-    // bits lie within the 32 bits from bit L + lx (< 32) on
-    const uint32_t y = __builtin_amdgcn_alignbit((uint32_t)(x >> 32), xl, L + lx);
-    const uint32_t d = S.dist[y & kDistMask];
-    const uint32_t dl = d & 15, dx = (d >> 4) & 15;
-    const uint32_t mlen = ((e >> 7) & 255) + 3 + __builtin_amdgcn_ubfe(xl, L, lx);
-    const uint32_t dist = (((d >> 8) & 3) << dx) + 1 + __builtin_amdgcn_ubfe(y, dl, dx);
-    const uint64_t litm = __ballot(e >= kLitFlag);
-    const bool lit = __builtin_amdgcn_inverse_ballot_w64(litm);
-    // a length code stops the chain if it or its distance code is not in the
-    // LUT, if it is end-of-block or invalid (extra field 6, 7), or if the
-    // distance code is 30 or 31
-    const uint32_t bad = (((L - 1u) | (dl - 1u)) >> 31) | ((lx + 2u) >> 3) | ((d & kDistBad) >> 13);
-    uint32_t tlm = bad ? 128u : L + lx + dl + dx;
-    asm("" : "+v"(tlm));  // every lane computes it: no branch around the literal lanes
-    const uint32_t tl = lit ? L : tlm;
-    const uint32_t tk = lit ? e : (mlen | (dist << 16));
-    // chain: token starts from window bit 0 while they lie in the window; a
-    // stop lane (length 128) ends it at j >= 128
-    // M |= 1 << j, then tl of lane j, while j < 64. Written out eight links
-    // at a time with a fall-through test per link: a taken branch per link
-    // (the loop's back edge) costs a lone wave about as much as the link
-    // itself. j is kept as j - 64, so the add's carry is the test, and the
-    // bitset and the lane select use only its low six bits. The scalar
-    // bitset also gives the wait state a v_readlane needs after the vector
-    // write of tl.
+    const uint32_t x = stage_bits(S->stage, q + lane);
+    const uint32_t e = S->tab[x & ((1u << kCodeBits) - 1)];
+    const uint32_t L = e & 31, sym = e >> 14;
+    const uint32_t xb = sym < 16 ? 0u : (sym == 16 ? 2u : (sym == 17 ? 3u : 7u));
+    const uint32_t rep = (sym < 16 ? 1u : (sym == 18 ? 11u : 3u)) + __builtin_amdgcn_ubfe(x, L, xb);
+    const uint32_t tl = L ? L + xb : 128u;  // no such code: stops the chain
+    // M gets the starts. Eight links written out with a fall-through test each:
+    // j is kept as j - 64, so the add's carry is the test.
     uint64_t M = 0;
-    uint32_t j = 0u - (uint32_t)kWave;  // j - 64 (mod 2^32): the add carries once j >= 64
+    uint32_t j = 0u - (uint32_t)kWave;
     {
       uint32_t t;
       asm("1:\n"
@@ -828,186 +495,622 @@ __device__ __forceinline__ bool decode_window(Bits &b, const LD &S, uint32_t *sl
           : "scc");
     }
     j += (uint32_t)kWave;
-    const bool stop = j >= 128u;
-    uint32_t adv = j & 127u;  // bits used by the tokens before the stop / window end
-    // the next window, unless this one stops or ends the batch
-    f = load_field(b, P + adv + lane);
-    // The batch's 64th token ends it (nt < 64 here). The token starts are
-    // kept as wave masks in scalar registers; inverse ballots hand them to
-    // the vector unit as conditions. The two exits and the common path each
-    // store their own slots, so no flag has to live across a join.
-    const uint64_t mkm = M & ~__ballot(tl >= 128u);  // a stop lane starts no token
-    const uint32_t rank = lanes_below(mkm);
-    const uint32_t cnt = (uint32_t)__builtin_popcountll(mkm);
-    if (nt + cnt >= (uint32_t)kWave) {  // the batch ends at token lastc
-      const uint64_t cm = mkm & __ballot(rank >= (uint32_t)kWave - 1 - nt);
-      const uint32_t lastc = (uint32_t)__builtin_ctzll(cm);
-      const uint64_t keepm = mkm & ((2ull << lastc) - 1);
-      slot[__builtin_amdgcn_inverse_ballot_w64(keepm) ? nt + rank : kWave + (lane & 15)] = tk;
-      nt += (uint32_t)__builtin_popcountll(keepm);
-      P += lastc + rdlane(tl, lastc);
-      full = true;
-      break;
-    }
-    slot[__builtin_amdgcn_inverse_ballot_w64(mkm) ? nt + rank : kWave + (lane & 15)] = tk;
-    nt += cnt;
-    P += adv;
-    if (stop) {
-      full = false;
-      break;
+    const bool start = (M >> lane) & 1 && L;
+    const uint32_t incl = wave_scan_dpp(start ? rep : 0u);
+    const uint32_t off = i + incl - rep;
+    const bool take = start && off < total;
+    // a repeat with no length before it, or past the last length
+    if (__ballot(take && ((sym == 16 && off == 0) || off + rep > total))) return kCorrupt;
+    const uint32_t key = wave_max_dpp(start && sym != 16 ? ((lane + 1) << 8) | (sym < 16 ? sym : 0u) : 0u);
+    const uint32_t val = key ? key & 0xff : prev;
+    if (take && val)  // at most six copies of a length that is not 0
+      for (uint32_t r = 0; r < rep; r++) S->lens[off + r] = (uint8_t)val;
+    const uint64_t tm = __ballot(take);
+    const uint32_t lastl = tm ? 63u - (uint32_t)__builtin_clzll(tm) : 0u;
+    if (tm) i = rdlane(off + rep, lastl);
+    prev = rdlane(val, kWave - 1);
+    if (i >= total) {
+      q += lastl + rdlane(tl, lastl);
+    } else if (j >= 128u) {  // no such code at bit q + j - 128
+      return q + (j - 128u) > limit ? kTrunc : kCorrupt;
+    } else {
+      q += j;
     }
   }
-  if (P != P0) bits_set(b, P);
-  return full;
+  if (q > limit) return kTrunc;
+  lds_order();
+  if (uni(S->lens[256]) == 0) return kCorrupt;  // zlib: "missing end-of-block"
+  st = (int32_t)uni((uint32_t)build_table(S->lens, nlen, kTabLit, &S->hl, S->tab, 0, C::kLB, C::kLS));
+  if (st != kOk) return st;
+  *qp = q;
+  return (int32_t)uni((uint32_t)build_table(S->lens + nlen, ndist, kTabDist, &S->hd, S->tab, C::kDistAt, C::kDB, C::kDS));
 }
 
-// Symbol loop: decodes up to `limit` (<= 64) symbols of the current block
-// into tok (lane j <- token j, nt tokens); every token passes through its
-// LDS slot, written by lane 0 here and by decode_window. Returns kOk when
-// the batch is full (`limit` tokens), kEob at end-of-block, or the status
-// of an invalid symbol. The tokens decoded before
-// an invalid symbol are valid and still have to be written. All stops leave
-// through one exit so the loop's uniform state stays in scalar registers.
-// A full batch (limit 64) is decoded by decode_window, and the loop takes
-// only the symbols that stop it.
-template <class LD>
-__device__ __forceinline__ int32_t decode_tokens(Bits &b, const LD &S, uint32_t *slot, uint32_t lane,
-                                                 uint32_t &tok, uint32_t &nt, uint32_t limit) {
+template <class C> __device__ __forceinline__ void load_fixed(lds<Sh<C>> *S) {
+  const uint32_t lane = lane_id();
+  for (uint32_t s = lane; s < 288; s += kWave)
+    S->lens[s] = (uint8_t)(s < 144 ? 8 : (s < 256 ? 9 : (s < 280 ? 7 : 8)));
+  lds_order();
+  build_table(S->lens, 288, kTabLit, &S->hl, S->tab, 0, C::kLB, C::kLS);
+  for (uint32_t s = lane; s < 32; s += kWave) S->lens[s] = 5;
+  lds_order();
+  build_table(S->lens, 32, kTabDist, &S->hd, S->tab, C::kDistAt, C::kDB, C::kDS);
+}
+
+// Decodes the one symbol at stage bit *q with zlib's rules: kMore and the token
+// (literal: its byte, *dist = 0; else length and distance), kEob, or the status
+// of an invalid symbol.
+template <class C>
+__device__ __forceinline__ int32_t one_symbol(const lds<Sh<C>> *S, uint32_t *q, uint32_t limit, uint32_t *len,
+                                              uint32_t *dist) {
+  uint32_t L = 0;
+  const int32_t sym = slow_decode(&S->hl, uni(stage_bits(S->stage, *q)), &L);
+  if (sym < 0) return *q > limit ? kTrunc : kCorrupt;
+  *q += L;
+  if (sym == 256) return kEob;
+  if (sym > 285) return kCorrupt;
+  *len = (uint32_t)sym;
+  *dist = 0;
+  if (sym < 256) return kMore;
+  const uint32_t c = (uint32_t)sym - 257, lx = len_extra(c);
+  *len = len_base(c, lx) + __builtin_amdgcn_ubfe(uni(stage_bits(S->stage, *q)), 0, lx);
+  *q += lx;
+  const int32_t ds = slow_decode(&S->hd, uni(stage_bits(S->stage, *q)), &L);
+  if (ds < 0) return *q > limit ? kTrunc : kCorrupt;
+  if (ds >= 30) return kCorrupt;
+  *q += L;
+  const uint32_t dx = dist_extra((uint32_t)ds);
+  *dist = dist_base((uint32_t)ds, dx) + __builtin_amdgcn_ubfe(uni(stage_bits(S->stage, *q)), 0, dx);
+  *q += dx;
+  return kMore;
+}
+
+enum : uint32_t { kOpEnd = 0, kOpSpan = 1, kOpStored = 2, kOpToken = 3 };
+
+// The serial part of the decode, by one wave: with `symbol`, decodes the symbol
+// at bit P that a span stopped at; outside a block, reads the next block header
+// and builds its tables. *S gets what comes next: the operation (a span from
+// bit P on; a stored block of ln bytes at bit P; one token; the end), its
+// status and whether the block is the stream's last. Out of line, with its
+// results in LDS, so that its scalars do not crowd the span decoder's.
+// At most 4096 bits from P on are read: a dynamic header has less than 105 +
+// 316 * 7 + 14 (each length costs at most 7 bits, a repeat of at least three 14).
+template <class C>
+__device__ __noinline__ void serial_step(const uint32_t *w, uint32_t nw, uint32_t limit_bits,
+                                         uint32_t P, bool symbol, bool last, lds<Sh<C>> *S) {
+  const uint32_t lane = lane_id();
+  const uint32_t d0 = P >> 5;
+  static_assert(C::kStage >= 130, "stage holds a block header");
+  for (uint32_t k = lane; k < 130; k += kWave) S->stage[k] = d0 + k < nw ? w[d0 + k] : 0u;
+  lds_order();
+  const uint32_t limit = limit_bits - d0 * 32;
+  uint32_t q = P & 31, op = kOpEnd, ln = 0, val = 0, dist = 0;
   int32_t st = kOk;
-  for (;;) {
-    if (limit == (uint32_t)kWave && decode_window(b, S, slot, lane, nt)) break;
-    bits_refill(b);  // >= 33 bits
-    uint32_t e = uni(S.lit[(uint32_t)b.buf & LD::kLitMask]);
-    if (e & kLitFlag) {  // literal: the token is the table entry
-      bits_drop(b, e & 15);
-      if (lane == 0) slot[nt] = e;
-      if (++nt == limit) break;
-      // >= 18 bits are left: enough for the next code without a refill
-      e = uni(S.lit[(uint32_t)b.buf & LD::kLitMask]);
-      if (e & kLitFlag) {
-        bits_drop(b, e & 15);
-        if (lane == 0) slot[nt] = e;
-        if (++nt == limit) break;
-        continue;
-      }
+  bool inside = symbol;
+  if (symbol) {
+    st = one_symbol<C>(S, &q, limit, &val, &dist);
+    if (q > limit) st = kTrunc;
+    if (st == kMore) {
+      st = kOk;
+      op = kOpToken;
+    } else if (st == kEob) {
+      st = kOk;
+      inside = false;
     }
-    // a length / end-of-block / invalid code, or one longer than the LUT;
-    // the buffer holds >= 18 bits
-    uint32_t L = e & 15;
-    if (L == 0) {  // code longer than the LUT, or no such code
-      const int32_t sym = slow_decode(S.hl, b.buf, &L);
-      if (sym < 0) {
-        st = bits_past_end(b) ? kTrunc : kCorrupt;
-        break;
-      }
-      e = make_entry(kTabLit, (uint32_t)sym, L);
-    }
-    bits_drop(b, L);
-    if (e & kLitFlag) {
-      if (lane == 0) slot[nt] = e;
-      if (++nt == limit) break;
-      continue;
-    }
-    const uint32_t lx = (e >> 4) & 7;
-    if (lx >= kXBad) {
-      st = lx == kXEob ? kEob : kCorrupt;
-      break;
-    }
-    // >= 33 bits after the refill: length extra (<= 5), distance code (<= 15)
-    // and distance extra (<= 13)
-    bits_refill(b);
-    const uint32_t len = ((e >> 7) & 255) + 3 + ((uint32_t)b.buf & ((1u << lx) - 1));
-    bits_drop(b, lx);
-    uint32_t d = uni(S.dist[(uint32_t)b.buf & kDistMask]);
-    uint32_t dl = d & 15;
-    if (dl == 0) {
-      const int32_t sym = slow_decode(S.hd, b.buf, &dl);
-      if (sym < 0) {
-        st = bits_past_end(b) ? kTrunc : kCorrupt;
-        break;
-      }
-      d = make_entry(kTabDist, (uint32_t)sym, dl);
-    }
-    if (d & kDistBad) {  // distance codes 30 and 31
-      st = kCorrupt;
-      break;
-    }
-    bits_drop(b, dl);
-    const uint32_t dx = (d >> 4) & 15;
-    const uint32_t dist = (((d >> 8) & 3) << dx) + 1 + ((uint32_t)b.buf & ((1u << dx) - 1));
-    bits_drop(b, dx);
-    if (lane == 0) slot[nt] = len | (dist << 16);
-    if (++nt == limit) break;
   }
-  if (nt) {
-    wave_sync();
-    tok = slot[lane];
+  if (st == kOk && !inside && !last) {
+    const uint32_t h = uni(stage_bits(S->stage, q));
+    q += 3;
+    last = h & 1;
+    const uint32_t type = (h >> 1) & 3;
+    if (q > limit) {
+      st = kTrunc;
+    } else if (type == 0) {  // stored (RFC 1951 3.2.4)
+      q = (q + 7) & ~7u;
+      const uint32_t lw = uni(stage_bits(S->stage, q));
+      q += 32;
+      ln = lw & 0xffff;
+      if (q > limit) st = kTrunc;
+      else if (ln != (~lw >> 16)) st = kCorrupt;
+      else if (q + ln * 8 > limit) st = kTrunc;
+      else op = kOpStored;
+    } else if (type == 1) {  // fixed Huffman
+      load_fixed<C>(S);
+      op = kOpSpan;
+    } else if (type == 2) {  // dynamic Huffman
+      st = read_dynamic<C>(S, &q, limit);
+      if (st == kOk) op = kOpSpan;
+    } else {
+      st = kCorrupt;  // zlib: "invalid block type"
+    }
   }
+  if (lane == 0) {
+    S->op = st == kOk ? op : (uint32_t)kOpEnd;
+    S->P = d0 * 32 + q;
+    S->ln = ln;
+    S->val = val;
+    S->dist = dist;
+    S->st = st;
+    S->last = last;
+  }
+  lds_order();
+}
+
+// ------------------------------------------------------------- span decode
+
+// A lane's place in the staged stream: the two dwords at its bit and the one
+// after them, which is read a lookup ahead, so that a lookup waits for one LDS
+// read (its table) and not for two.
+struct Place {
+  uint32_t at, w0, w1, w2;
+};
+
+__device__ __forceinline__ Place place_at(const uint32_t *stage, uint32_t q) {
+  const uint32_t *s = stage + (q >> 5);
+  return Place{q, s[0], s[1], s[2]};
+}
+
+// The 32 stream bits from the place on.
+__device__ __forceinline__ uint32_t place_bits(const Place &p) { return __builtin_amdgcn_alignbit(p.w1, p.w0, p.at); }
+
+// Moves the place on by n <= 31 bits.
+__device__ __forceinline__ void place_move(Place &p, const uint32_t *stage, uint32_t n) {
+  const uint32_t to = p.at + n;
+  const bool cross = to > (p.at | 31);
+  p.w0 = cross ? p.w1 : p.w0;
+  p.w1 = cross ? p.w2 : p.w1;
+  p.w2 = stage[(to >> 5) + 2];
+  p.at = to;
+}
+
+// The entry of bits x in the table of descriptor d.
+__device__ __forceinline__ uint32_t look(const uint32_t *tab, uint32_t x, uint32_t d) {
+  return tab[(d >> 5) + __builtin_amdgcn_ubfe(x, 0, d)];  // the field's width is d's low five bits
+}
+
+// The value of a length or distance code: its base and extra bits.
+__device__ __forceinline__ uint32_t entry_value(uint32_t e, uint32_t x) {
+  return __builtin_amdgcn_ubfe(e, 14, 16) + __builtin_amdgcn_ubfe(x, __builtin_amdgcn_ubfe(e, 9, 4), __builtin_amdgcn_ubfe(e, 5, 4));
+}
+
+template <class C> __device__ __forceinline__ uint32_t next_table(uint32_t e) {
+  const uint32_t sub = __builtin_amdgcn_ubfe(e, 14, 16), root = e >= kLenType ? C::kDistDesc : C::kLitDesc;
+  return e >= kSubType ? sub : root;
+}
+
+// Decodes tokens from bit q on until one starts at or after `bound`: q becomes
+// that start (on a stop, the start of the token that stops). A token that ends
+// past `limit` stops. With Count, n gets the bytes the tokens produce. One
+// lookup a step in straight-line code: one LDS latency and about 30 vector
+// instructions; a branch per kind of entry doubled that in scalar mask
+// work.
+template <class C, bool Count>
+__device__ __forceinline__ bool run_tokens(const Sh<C> &S, uint32_t &q, uint32_t bound, uint32_t limit, uint32_t &n) {
+  uint32_t d = C::kLitDesc, pend = 1, end = bound;
+  Place p = place_at(S.stage, q);
+  while (q < end) {
+    const uint32_t x = place_bits(p), e = look(S.tab, x, d);
+    place_move(p, S.stage, e & 31);
+    const bool good = (e & 31) != 0 && p.at <= limit;
+    const bool whole = good && e < kLenType;
+    if (Count) {
+      uint32_t v = entry_value(e, x);
+      asm("" : "+v"(v));  // every lane computes it: no branch
+      n += whole ? pend : 0u;
+      v = e < kLenType ? 1u : v;
+      pend = e < kSubType ? v : pend;
+    }
+    q = whole ? p.at : q;
+    end = good ? end : 0u;
+    d = next_table<C>(e);
+  }
+  return end != bound;
+}
+
+// Buffer loads: a lane whose offset is not below the size takes no part in the
+// load and gets 0, so no branch stands around it and the loads of several rows
+// stay in flight together.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
+}
+
+// The bytes [0, wn) of the window at output position w0 are marked; resolves
+// them, stores them and adds them to the Adler-32 sums. A byte without a mark
+// continues the token of the byte before it; a token also has a mark where it
+// crosses into another wave's segment.
+// Each wave resolves its segment in groups of four rows of 64 bytes; the far
+// sources of the next group are loaded while this one's near sources are
+// followed. Nothing is stored before the segment is done: a wait for loads
+// would also wait for the stores before them.
+// A group's bytes first get 0x8000 | byte where the byte is known (literals,
+// far sources) and else the window index of their source; a byte then takes
+// what its source holds, byte or index, until it is a byte (pointer doubling).
+template <class C>
+__device__ __forceinline__ void resolve_window(Out &o, Sh<C> &S, uint32_t w0, uint32_t wn, uint32_t wave, uint32_t lane) {
+  constexpr uint32_t R = 4, G = R * kWave;
+  const uint32_t s0 = wave * C::kSeg, s1 = min(s0 + C::kSeg, wn);
+  uint32_t carry = 0x8000u;
+  uint64_t late = 0;  // groups with bytes whose source lies in another wave's segment
+  const __amdgpu_buffer_rsrc_t rsrc = buffer_of(o.dst, 0x80000000u);
+  // reads the marks of a group and loads its far sources
+  auto open = [&](uint32_t row, uint32_t *c, uint32_t *f) __attribute__((always_inline)) {
+    uint32_t k[R];
+#pragma unroll
+    for (uint32_t r = 0; r < R; r++) {
+      const uint32_t m = S.win[row + r * kWave + lane];
+      k[r] = m == 0xffffu ? 0u : ((lane + 1) << 16) | m;
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < R; r++) {
+      k[r] = wave_max_dpp(k[r]);
+      c[r] = k[r] ? k[r] & 0xffff : carry;
+      carry = rdlane(c[r], kWave - 1);
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < R; r++) {
+      const uint32_t i = row + r * kWave + lane;
+      // a distance beyond the window; past the stored bytes it may be anything,
+      // and an offset below 0 lies outside the buffer
+      const bool isfar = c[r] >= i && c[r] < 0x8000u;
+      f[r] = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rsrc, isfar ? w0 + (i - 1 - c[r]) : ~0u, 0, 0);
+    }
+  };
+  auto close = [&](uint32_t row, const uint32_t *c, const uint32_t *f) __attribute__((always_inline)) {
+    uint32_t v[R];
+#pragma unroll
+    for (uint32_t r = 0; r < R; r++) {
+      const uint32_t i = row + r * kWave + lane;
+      v[r] = c[r] < i ? i - 1 - c[r] : (c[r] >= 0x8000u ? c[r] : 0x8000u | f[r]);
+      S.win[i] = (uint16_t)v[r];
+    }
+    // an index in another wave's segment waits for the second pass
+    for (;;) {
+      bool go[R], more = false;
+#pragma unroll
+      for (uint32_t r = 0; r < R; r++) {
+        go[r] = C::kNW == 1 ? v[r] < 0x8000u : v[r] - s0 < 0x8000u - s0;
+        more |= go[r];
+      }
+      if (!__ballot(more)) break;
+      lds_order();
+      uint32_t t[R];
+#pragma unroll
+      for (uint32_t r = 0; r < R; r++) t[r] = S.win[v[r] & 0x7fff];
+#pragma unroll
+      for (uint32_t r = 0; r < R; r++) {
+        v[r] = go[r] ? t[r] : v[r];
+        S.win[row + r * kWave + lane] = (uint16_t)v[r];
+      }
+    }
+    if constexpr (C::kNW > 1) {
+      uint32_t low = v[0];
+#pragma unroll
+      for (uint32_t r = 1; r < R; r++) low = min(low, v[r]);
+      if (__ballot(low < 0x8000u)) late |= 1ull << ((row - s0) / G);
+    }
+  };
+  // two sets of registers in turn: a copy from one to the other would wait for
+  // the loads (rows from s1 to the next pair of groups are literals)
+  uint32_t ca[R], fa[R], cb[R], fb[R];
+  if (s0 < s1) open(s0, ca, fa);
+  for (uint32_t row = s0; row < s1; row += 2 * G) {
+    open(row + G, cb, fb);
+    close(row, ca, fa);
+    open(min(row + 2 * G, s0 + C::kSeg - G), ca, fa);
+    close(row + G, cb, fb);
+  }
+  if constexpr (C::kNW > 1) {
+    // every byte now is resolved or holds an index; the chains end at resolved
+    // bytes, so no wave waits for another
+    __syncthreads();
+    while (late) {
+      const uint32_t row = s0 + (uint32_t)__builtin_ctzll(late) * G;
+      late &= late - 1;
+      uint32_t v[R];
+#pragma unroll
+      for (uint32_t r = 0; r < R; r++) v[r] = S.win[row + r * kWave + lane];
+      for (;;) {
+        uint32_t low = v[0];
+#pragma unroll
+        for (uint32_t r = 1; r < R; r++) low = min(low, v[r]);
+        if (!__ballot(low < 0x8000u)) break;
+        lds_order();
+        uint32_t t[R];
+#pragma unroll
+        for (uint32_t r = 0; r < R; r++) t[r] = S.win[v[r] & 0x7fff];
+#pragma unroll
+        for (uint32_t r = 0; r < R; r++) {
+          v[r] = v[r] < 0x8000u ? t[r] : v[r];
+          S.win[row + r * kWave + lane] = (uint16_t)v[r];
+        }
+      }
+    }
+  }
+  lds_order();
+  // the segment to HBM, four bytes a lane
+  uint32_t a1 = 0, a2 = 0;
+  const uint32_t len = s1 > s0 ? s1 - s0 : 0u;
+  for (uint32_t k = 4 * lane; k < len; k += 4 * kWave) {
+    const uint2 w = *reinterpret_cast<const uint2 *>(S.win + s0 + k);
+    uint32_t b = __builtin_amdgcn_perm(w.y, w.x, 0x06040200u);
+    uint8_t *d = o.dst + (w0 + s0 + k);
+    if (k + 4 <= len) {
+      __builtin_memcpy(d, &b, 4);
+    } else {
+      b &= (1u << 8 * (len - k)) - 1;
+      for (uint32_t j = 0; j < len - k; j++) d[j] = (uint8_t)(b >> 8 * j);
+    }
+    const uint32_t sum = __builtin_amdgcn_udot4(b, 0x01010101u, 0u, false);
+    a1 += sum;
+    a2 += k * sum + __builtin_amdgcn_udot4(b, 0x03020100u, 0u, false);
+  }
+  // a1 = sum b <= 16320, a2 = sum of (position - w0 - s0) * b < 2^27
+  o.s1 = (o.s1 + a1) % 65521u;
+  o.s2 = (o.s2 + ((w0 + s0) % 65521u) * a1 + a2) % 65521u;
+}
+
+// Writes the tokens of the group's lanes, in lane order: this lane's begin at
+// stage bit q and produce n bytes. The lanes mark the bytes of one window after
+// the other. The first output error in stream order ends it: the tokens before
+// it are written.
+template <class C>
+__device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n, uint32_t wave, uint32_t lane) {
+  const uint32_t tid = wave * kWave + lane;
+  const uint32_t incl = wave_scan_dpp(n);
+  uint32_t x = incl - n, total = rdlane(incl, kWave - 1);
+  if constexpr (C::kNW > 1) {
+    if (lane == 0) S.part[0][wave] = total;
+    __syncthreads();
+    total = 0;
+    for (uint32_t k = 0; k < (uint32_t)C::kNW; k++) {
+      const uint32_t p = uni(S.part[0][k]);
+      if (k < wave) x += p;
+      total += p;
+    }
+  }
+  const uint32_t end = x + n;  // this lane's bytes: [x, end) from o.pos on
+  const bool check = o.pos < 32768u || o.pos + total > o.cap;
+  uint32_t lastx = ~0u, lastm = 0;  // this lane's last token
+  Place p = place_at(S.stage, q);
+  uint32_t done = 0;
+  int32_t st = kOk;
+  while (done < total) {
+    uint32_t wn = min(C::kWin, total - done);
+    for (uint32_t k = tid; k < (wn + 511) / 512 * 64; k += C::kThreads)
+      reinterpret_cast<uint4 *>(S.win)[k] = uint4{~0u, ~0u, ~0u, ~0u};
+    if (check && tid == 0) S.err = ~0u;
+    group_sync<C>();
+    // the bytes behind the last one count as literals
+    if (tid == 0 && wn < C::kWin) S.win[wn] = 0x8000u;
+    if (x > done && lastx < done) S.win[0] = (uint16_t)lastm;  // a token that began before this window
+    const uint32_t stopx = min(end, done + wn);
+    uint32_t d = C::kLitDesc, mlen = 0;
+    while (x < stopx) {
+      const uint32_t bits = place_bits(p), e = look(S.tab, bits, d);
+      if ((e & 31) == 0) break;  // not in a counted range
+      place_move(p, S.stage, e & 31);
+      d = next_table<C>(e);
+      const uint32_t v = entry_value(e, bits);
+      mlen = (e >> 30) == 1 ? v : mlen;
+      if (e >= kLenType) continue;
+      const bool lit = e & kLitFlag;
+      const uint32_t tl = lit ? 1u : mlen;
+      const uint32_t m = lit ? 0x8000u | v : v - 1;
+      if (check) {
+        const uint32_t at = o.pos + x;
+        if (at + tl > o.cap) atomicMin(&S.err, x << 2 | (uint32_t)kOverflow);
+        else if (!lit && v > at) atomicMin(&S.err, x << 2 | (uint32_t)kCorrupt);  // "invalid distance too far back"
+      }
+      S.win[x - done] = (uint16_t)m;
+      if constexpr (C::kNW > 1) {  // a mark for the next segment's wave, too
+        const uint32_t b = (x - done + tl - 1) / C::kSeg * C::kSeg;
+        if (b > x - done && b < C::kWin) S.win[b] = (uint16_t)m;
+      }
+      lastx = x;
+      lastm = m;
+      x += tl;
+    }
+    group_sync<C>();
+    if (check) {
+      const uint32_t e = uni(S.err);
+      if (e != ~0u) {
+        wn = (e >> 2) - done;
+        st = (int32_t)(e & 3);
+      }
+    }
+    resolve_window<C>(o, S, o.pos + done, wn, wave, lane);
+    group_sync<C>();
+    done += wn;
+    if (st != kOk) break;
+  }
+  o.pos += done;
   return st;
 }
 
-// Decodes symbols until end-of-block. Returns a status. The sink takes each
-// batch (SinkOne writes it on this wave, SinkQueue hands it to the writing
-// wave) and returns the first output error seen so far.
-template <class Sink, class LD>
-__device__ __forceinline__ int32_t decode_block(Bits &b, Sink &out, const LD &S, uint32_t *slot,
-                                                uint32_t lane) {
-  for (;;) {
-    // A symbol reads at most 48 bits, so a batch of floor(left / 48) symbols
-    // cannot pass the stream end; near the end batches shrink to one symbol,
-    // and reading past the end is caught at the symbol that does it.
-    // (left * 1365) >> 16 is at most left / 48 for left below 2^16.
-    const uint32_t pos = bits_pos(b);
-    const uint32_t left = pos < b.limit ? b.limit - pos : 0u;
-    uint32_t limit = (uint32_t)kWave;
-    if (left < kCarefulBits) {
-      const uint32_t safe = (left * 1365u) >> 16;
-      limit = safe == 0 ? 1u : (safe < (uint32_t)kWave ? safe : (uint32_t)kWave - 1);
-    }
-    uint32_t tok = 0, nt = 0;
-    const int32_t sa = decode_tokens(b, S, slot, lane, tok, nt, limit);
-    if (bits_past_end(b)) return kTrunc;
-    const int32_t sb = out.tokens(lane, tok, nt);
-    if (sb != kOk) return sb;
-    if (sa == kEob) return kOk;
-    if (sa != kOk) return sa;
+constexpr uint32_t kHardYes = 3, kHardNo = 4;
+
+// Where a span's lanes do not find each other's token starts (codes of nearly one
+// length keep a wrong phase: 128 equally frequent bytes, say), lane j decodes its
+// part from each of the 16 bits at which the token before it may end, and a chain
+// through these exits gives every lane its entry. Returns the lanes that have
+// one; the first that stops, or whose successor begins further behind, is the
+// last. 128 KiB chunks of 7-bit literals, by passes (one or two lanes verified a
+// pass) and by candidates: 16 chunks 20.0 and 2.2 ms, 4096 chunks by one wave
+// each 30.8 and 17.5 ms.
+template <class C>
+__device__ __forceinline__ uint32_t chain_entries(Sh<C> &S, uint32_t lo, uint32_t bound, uint32_t limit, uint32_t wave,
+                                                  uint32_t lane, uint32_t &entry) {
+  uint32_t exits[4] = {0, 0, 0, 0};  // byte c: the exit behind `bound` of entry lo + c, 255 = stop
+#pragma unroll 1
+  for (uint32_t c = 0; c < 16; c++) {
+    uint32_t q = lo + c, n = 0;
+    const uint32_t x = run_tokens<C, false>(S, q, bound, limit, n) ? 255u : q - bound;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) exits[k] |= c / 4 == k ? x << 8 * (c & 3) : 0u;
   }
+  uint32_t off = 0, have = 0;
+  for (uint32_t w = 0; w < (uint32_t)C::kNW; w++) {
+    if (w == wave) {
+      for (; have < (uint32_t)kWave && off < 16; have++) {
+        if (lane == have) entry = lo + off;
+        const uint32_t k = off / 4;
+        const uint32_t m = k == 0 ? exits[0] : k == 1 ? exits[1] : k == 2 ? exits[2] : exits[3];
+        off = (rdlane(m, have) >> 8 * (off & 3)) & 255;
+      }
+    }
+    if constexpr (C::kNW > 1) {
+      if (w == wave && lane == 0) {
+        S.mis[w] = have;
+        S.stp[w] = off;
+      }
+      __syncthreads();
+      have = uni(S.mis[w]);
+      off = uni(S.stp[w]);
+      if (have < (uint32_t)kWave || off >= 16) return w * kWave + have;
+      have = 0;
+    }
+  }
+  return C::kNW > 1 ? C::kThreads : have;
+}
+
+// Decodes and writes the tokens of one span from stream bit P on; P becomes the
+// bit after the last token written. *stopped: a symbol there needs the symbol
+// loop. Returns the first output error.
+template <class C>
+__device__ __forceinline__ int32_t span(const uint32_t *w, uint32_t nw, uint32_t limit_bits, uint32_t &P, bool &stopped,
+                                        uint32_t &hard, Out &o, Sh<C> &S, uint32_t wave, uint32_t lane) {
+  const uint32_t max_pass = hard == kHardYes ? 2 : 8;  // pass k verifies at least k lanes
+  const uint32_t tid = wave * kWave + lane;
+  const uint32_t d0 = P >> 5, off0 = P & 31;
+  {
+    constexpr uint32_t N = (C::kStage + C::kThreads - 1) / C::kThreads;
+    const __amdgpu_buffer_rsrc_t rsrc = buffer_of(w, nw * 4);
+    uint32_t v[N];
+#pragma unroll
+    for (uint32_t k = 0; k < N; k++)
+      v[k] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (d0 + k * C::kThreads + tid) * 4, 0, 0);
+#pragma unroll
+    for (uint32_t k = 0; k < N; k++)
+      if (k * C::kThreads + tid < C::kStage) S.stage[k * C::kThreads + tid] = v[k];
+  }
+  const uint32_t limit = limit_bits - d0 * 32;
+  group_sync<C>();
+  const uint32_t lo = off0 + tid * C::kSpanBits, bound = lo + C::kSpanBits;
+  uint32_t entry = lo, q = lo, n = 0;
+  uint32_t sq[C::kSub], sn[C::kSub];
+#pragma unroll
+  for (int k = 0; k < C::kSub; k++) sq[k] = sn[k] = 0;
+  bool stop = run_tokens<C, false>(S, q, bound, limit, n);
+  uint32_t valid;  // lanes verified
+  for (uint32_t pass = 2;; pass++) {
+    const uint32_t mine = q | (stop ? 0x80000000u : 0u);
+    uint32_t up = __shfl_up(mine, 1, kWave);
+    if constexpr (C::kNW > 1) {
+      if (lane == kWave - 1) S.ex[wave] = mine;
+      __syncthreads();
+      if (lane == 0 && wave) up = S.ex[wave - 1];
+    }
+    const uint32_t next = tid == 0 ? off0 : (up >> 31 ? entry : up);
+    const uint64_t mm = __ballot(next != entry), sm = __ballot(stop);
+    uint32_t fm = mm ? wave * kWave + (uint32_t)__builtin_ctzll(mm) : C::kThreads;
+    uint32_t fs = sm ? wave * kWave + (uint32_t)__builtin_ctzll(sm) : C::kThreads;
+    if constexpr (C::kNW > 1) {
+      if (lane == 0) {
+        S.mis[wave] = fm;
+        S.stp[wave] = fs;
+      }
+      __syncthreads();
+      for (uint32_t k = 0; k < (uint32_t)C::kNW; k++) {
+        fm = min(fm, uni(S.mis[k]));
+        fs = min(fs, uni(S.stp[k]));
+      }
+    }
+    if (pass > 2 && (fm > fs || fm == C::kThreads)) {
+      valid = min(fs + 1, C::kThreads);
+      break;
+    }
+    if (pass > max_pass) {
+      // the verified lanes make the span; a block in which they are few three
+      // times goes on with chain_entries, unless that finds few as well
+      valid = fm;
+      if (hard != kHardYes) {
+        if (hard < kHardYes && valid < max(C::kThreads / 8, 16u)) hard++;
+        break;
+      }
+      valid = chain_entries<C>(S, lo, bound, limit, wave, lane, entry);
+      if (valid < C::kThreads / 4) hard = kHardNo;
+      q = entry;
+      stop = false;
+#pragma unroll
+      for (int k = 0; k < C::kSub; k++) {
+        sq[k] = q;
+        n = 0;
+        if (!stop) stop = run_tokens<C, true>(S, q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
+        sn[k] = n;
+      }
+      break;
+    }
+    // every lane counts its bytes in pass 2; later only lanes with a new entry
+    // (those behind a stop, too: most stops before the last pass are not real)
+    if (pass == 2 || next != entry) {
+      const uint32_t q0 = q;
+      const bool stop0 = stop;
+      bool met = false;  // back on the tokens of the pass before
+      entry = q = next;
+      stop = false;
+#pragma unroll
+      for (int k = 0; k < C::kSub; k++) {
+        if (k && pass > 2 && q == sq[k]) met = true;
+        if (!met) {
+          sq[k] = q;
+          n = 0;
+          if (!stop) stop = run_tokens<C, true>(S, q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
+          sn[k] = n;
+        }
+      }
+      if (met) {
+        q = q0;
+        stop = stop0;
+      }
+    }
+  }
+  if (tid >= valid) {
+#pragma unroll
+    for (int k = 0; k < C::kSub; k++) sn[k] = 0;
+  }
+  // the exit of the last verified lane, and whether it stopped there
+  uint32_t endq = rdlane(q | (stop ? 0x80000000u : 0u), (valid - 1) & (kWave - 1));
+  if constexpr (C::kNW > 1) {
+    if (wave == (valid - 1) / kWave && lane == 0) S.end = endq;  // read after emit's barriers
+  }
+  int32_t st = kOk;
+#pragma unroll 1
+  for (int g = 0; g < C::kSub && st == kOk; g++) {
+    uint32_t eq = sq[0], en = sn[0];
+    if constexpr (C::kSub > 1) {
+      const uint32_t l = g * (kWave / C::kSub) + lane / C::kSub;
+      eq = en = 0;
+#pragma unroll
+      for (int k = 0; k < C::kSub; k++) {
+        const uint32_t a = __shfl(sq[k], l, kWave), b = __shfl(sn[k], l, kWave);
+        if ((int)(lane % C::kSub) == k) {
+          eq = a;
+          en = b;
+        }
+      }
+    }
+    st = emit<C>(o, S, eq, en, wave, lane);
+  }
+  if constexpr (C::kNW > 1) endq = uni(S.end);
+  stopped = endq >> 31;
+  P = d0 * 32 + (endq & 0x7fffffffu);
+  return st;
 }
 
 struct Result {
   int32_t status;
   uint64_t bytes;
   uint32_t adler;
-};
-
-// Output of a stream decoded by one wave: the wave writes its own batches
-// through an LDS ring of R bytes.
-template <uint32_t R> struct SinkOne {
-  Out<R> o;
-  __device__ __forceinline__ void init(uint8_t *dst, uint8_t *ring, uint64_t cap) {
-    o.dst = dst;
-    o.ring = ring;
-    o.cap = (uint32_t)cap;
-    o.pos = 0;
-    o.flushed = 0;
-    o.mis = (uint32_t)(reinterpret_cast<uintptr_t>(dst) & 15);
-    o.s1 = 0;
-    o.s2 = 0;
-  }
-  __device__ __forceinline__ int32_t tokens(uint32_t lane, uint32_t tok, uint32_t nt) {
-    return out_tokens(o, lane, tok, nt);
-  }
-  // stored block data: ln bytes from src + at (RFC 1951 3.2.4)
-  __device__ __forceinline__ int32_t stored(const uint8_t *src, uint64_t at, uint32_t ln,
-                                            uint32_t lane) {
-    return store_copy(o, src, at, ln, lane);
-  }
-  // the final flush; status st of the decode; fills bytes and Adler-32
-  __device__ __forceinline__ int32_t finish(uint32_t lane, int32_t st, Result &res) {
-    res.adler = out_finish(o, lane);
-    res.bytes = o.pos;
-    return st;
-  }
 };
 
 // ------------------------------------------------------------- CRC-32 (gzip)
@@ -1148,17 +1251,17 @@ __device__ __forceinline__ int64_t gzip_header(const uint8_t *src, uint64_t len,
   return (int64_t)at;
 }
 
-// Decodes one zlib / raw / gzip stream; `out` takes the decoded batches
-// (SinkOne: this wave writes them; SinkQueue: a second wave does).
-template <class Sink, class LD>
-__device__ __forceinline__ Result inflate_stream_t(const uint8_t *src, uint64_t len, uint8_t *dst,
-                                                   uint64_t cap, uint32_t flags, LD &S, Sink &out) {
+// ------------------------------------------------------------- streams
+
+// Decodes one zlib / raw / gzip stream by the whole group. Wave 0 reads the
+// headers, builds the tables and decodes the symbols that stop a span; spans
+// and stored blocks are done by all waves. The result is wave 0's.
+template <class C>
+__device__ __forceinline__ Result inflate_group(const uint8_t *src, uint64_t len, uint8_t *dst, uint64_t cap,
+                                                uint32_t flags, Sh<C> &S) {
   const uint32_t lane = lane_id();
-  // the code lengths are dead while a block's symbols are decoded: their
-  // bytes hold the window decoder's 64 token slots
-  uint32_t *slot = reinterpret_cast<uint32_t *>(S.lens);
+  const uint32_t wave = C::kNW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x) / kWave : 0u;
   Result res{kOk, 0, 1};
-  Bits b;
   // 32-bit bit positions bound the stream to < 2^28 bytes; outputs are
   // capped below 2^31 bytes.
   if (len >= (1ull << 28)) {
@@ -1168,83 +1271,99 @@ __device__ __forceinline__ Result inflate_stream_t(const uint8_t *src, uint64_t 
   if (cap > 0x7fffffffull) cap = 0x7fffffffull;
   const uintptr_t a = reinterpret_cast<uintptr_t>(src);
   const uint32_t lead = (uint32_t)(a & 3);
-  b.w = reinterpret_cast<const uint32_t *>(a - lead);
-  b.limit = (uint32_t)((lead + len) * 8);
-  b.nw = (uint32_t)((lead + len + 3) / 4);
+  const uint32_t *w = reinterpret_cast<const uint32_t *>(a - lead);  // bit positions count from here
+  const uint32_t limit = (uint32_t)((lead + len) * 8);               // one past the stream's last bit
+  const uint32_t nw = (uint32_t)((lead + len + 3) / 4);
+  Out o;
+  o.dst = dst;
+  o.cap = (uint32_t)cap;
+  o.pos = 0;
+  o.s1 = 0;
+  o.s2 = 0;
   const bool gzip = flags & CODAG_INFLATE_GZIP;
   const bool raw = (flags & CODAG_INFLATE_RAW) && !gzip;
-  uint64_t start = 0;
-  if (gzip) {
-    const int64_t h = gzip_header(src, len, reinterpret_cast<uint32_t *>(S.ring));
-    if (h < 0) {
-      res.status = (int32_t)(-h);
-      return res;
-    }
-    start = (uint64_t)h;
-  } else if (!raw) {
-    if (len < 2) {
-      res.status = kTrunc;
-      return res;
-    }
-    const uint32_t cmf = uni(src[0]), flg = uni(src[1]);
-    // zlib inflate.c: method 8, window <= 32K, header check, no preset dictionary
-    if ((cmf & 15) != 8 || (cmf >> 4) > 7 || ((cmf << 8) | flg) % 31 != 0 || (flg & 0x20)) {
-      res.status = kCorrupt;
-      return res;
-    }
-    start = 2;
-  }
-  bits_seek(b, lead + start);
-
+  uint32_t *crc_tab = reinterpret_cast<uint32_t *>(S.win);
   int32_t st = kOk;
-  bool last = false;
-  uint32_t tables = 0;  // 1 = fixed tables loaded
-  while (!last && st == kOk) {
-    bits_refill(b);
-    const uint32_t h = (uint32_t)(b.buf & 7);
-    bits_drop(b, 3);
-    if (bits_past_end(b)) { st = kTrunc; break; }
-    last = h & 1;
-    const uint32_t type = h >> 1;
-    if (type == 0) {  // stored (RFC 1951 3.2.4)
-      bits_drop(b, (uint32_t)((8 - (bits_pos(b) & 7)) & 7));
-      bits_refill(b);
-      const uint32_t ln = (uint32_t)(b.buf & 0xffff);
-      const uint32_t nln = (uint32_t)((b.buf >> 16) & 0xffff);
-      bits_drop(b, 32);
-      if (bits_past_end(b)) { st = kTrunc; break; }
-      if (ln != (~nln & 0xffff)) { st = kCorrupt; break; }
-      const uint64_t at = bits_pos(b) / 8 - lead;  // stream byte offset of the data
-      if (at + ln > len) { st = kTrunc; break; }
-      st = out.stored(src, at, ln, lane);
-      if (st != kOk) break;
-      bits_seek(b, lead + at + ln);
-    } else if (type == 1) {  // fixed Huffman
-      if (tables != 1) {
-        load_fixed(S);
-        tables = 1;
+  uint64_t start = 0;
+  if (wave == 0) {
+    if (gzip) {
+      const int64_t h = gzip_header(src, len, crc_tab);
+      if (h < 0) st = (int32_t)(-h);
+      else start = (uint64_t)h;
+    } else if (!raw) {
+      if (len < 2) {
+        st = kTrunc;
+      } else {
+        const uint32_t cmf = uni(src[0]), flg = uni(src[1]);
+        // zlib inflate.c: method 8, window <= 32K, header check, no preset dictionary
+        if ((cmf & 15) != 8 || (cmf >> 4) > 7 || ((cmf << 8) | flg) % 31 != 0 || (flg & 0x20)) st = kCorrupt;
+        start = 2;
       }
-      st = decode_block(b, out, S, slot, lane);
-    } else if (type == 2) {  // dynamic Huffman
-      uint32_t nlen = 0;
-      tables = 0;
-      st = read_dynamic(b, S, &nlen);
-      if (st == kOk) st = decode_block(b, out, S, slot, lane);
-    } else {
-      st = kCorrupt;  // zlib: "invalid block type"
     }
   }
-  // the last flush, the bytes written and their Adler-32; the status becomes
-  // the first error in stream order of the decode and the output
-  st = out.finish(lane, st, res);
+  const bool headed = st == kOk;  // the stream's header is accepted
+  uint32_t P = (uint32_t)((lead + start) * 8);
+  bool last = false, inside = false, stopped = false;
+  uint32_t hard = 0;  // the block's spans that were cut short, or kHardYes / kHardNo
+  for (;;) {
+    uint32_t op = kOpEnd;
+    if (wave == 0 && st == kOk) {
+      if (inside && !stopped) {
+        op = kOpSpan;
+      } else if (inside || !last) {
+        serial_step<C>(w, nw, limit, P, inside, last, (lds<Sh<C>> *)&S);
+        op = uni(S.op);
+        P = uni(S.P);
+        st = (int32_t)uni((uint32_t)S.st);
+        last = uni(S.last);
+        if (op == kOpToken) {
+          const uint32_t val = uni(S.val), dist = uni(S.dist);
+          st = out_token(o, lane, dist == 0, val, dist);
+          op = st == kOk ? kOpSpan : kOpEnd;
+        }
+        inside = op == kOpSpan;
+      }
+    }
+    if constexpr (C::kNW > 1) {
+      if (threadIdx.x == 0) {
+        S.op = op;
+        S.P = P;
+        S.pos = o.pos;
+      }
+      __syncthreads();
+      op = uni(S.op);
+      P = uni(S.P);
+      o.pos = uni(S.pos);
+    }
+    if (op == kOpEnd) break;
+    if (op == kOpSpan) {
+      const int32_t e = span<C>(w, nw, limit, P, stopped, hard, o, S, wave, lane);
+      hard = stopped ? 0u : hard;
+      if (wave == 0) st = e;
+    } else {
+      const uint32_t ln = uni(S.ln);
+      const int32_t e = store_copy(o, reinterpret_cast<const uint8_t *>(w) + P / 8, ln, wave * kWave + lane, C::kThreads);
+      if (wave == 0) st = e;
+      P += 8 * ln;
+      group_sync<C>();  // the command is read by all
+    }
+  }
+  if (gzip) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // wave 0 reads the output back
+  const uint32_t adler = out_adler<C>(o, S, wave);
+  if (wave != 0) return res;
+  if (!headed) {
+    res.status = st;
+    return res;
+  }
+  res.adler = adler;
+  res.bytes = o.pos;
   if (gzip) {
     // RFC 1952 trailer on the next byte boundary: CRC-32 and ISIZE, both
     // little-endian; zlib checks the CRC first ("incorrect data check"),
     // then the length ("incorrect length check")
-    res.adler = wave_crc32(dst, (uint32_t)res.bytes, reinterpret_cast<uint32_t *>(S.ring));
+    res.adler = wave_crc32(dst, (uint32_t)res.bytes, crc_tab);
     if (st == kOk) {
-      bits_drop(b, (uint32_t)((8 - (bits_pos(b) & 7)) & 7));
-      const uint64_t at = bits_pos(b) / 8 - lead;
+      const uint64_t at = (P + 7) / 8 - lead;
       if (at + 8 > len) {
         st = kTrunc;
       } else {
@@ -1258,8 +1377,7 @@ __device__ __forceinline__ Result inflate_stream_t(const uint8_t *src, uint64_t 
     }
   } else if (st == kOk && !raw) {
     // RFC 1950 trailer: Adler-32, big-endian, on the next byte boundary
-    bits_drop(b, (uint32_t)((8 - (bits_pos(b) & 7)) & 7));
-    const uint64_t at = bits_pos(b) / 8 - lead;
+    const uint64_t at = (P + 7) / 8 - lead;
     if (at + 4 > len) {
       st = kTrunc;
     } else if (!(flags & CODAG_INFLATE_SKIP_ADLER)) {
@@ -1272,321 +1390,141 @@ __device__ __forceinline__ Result inflate_stream_t(const uint8_t *src, uint64_t 
   return res;
 }
 
-__device__ __forceinline__ Result inflate_stream(const uint8_t *src, uint64_t len, uint8_t *dst,
-                                                 uint64_t cap, uint32_t flags, Lds &S) {
-  SinkOne<kRingOne> out;
-  out.init(dst, S.ring, cap > 0x7fffffffull ? 0x7fffffffull : cap);
-  return inflate_stream_t(src, len, dst, cap, flags, S, out);
-}
-
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kWavesOne)))
-inflate_chunks_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
-                      const uint64_t *__restrict__ off, uint64_t n, uint64_t chunk_bytes, uint8_t *__restrict__ out,
-                      uint64_t *__restrict__ out_len, int32_t *__restrict__ status, uint32_t flags) {
-  __shared__ Lds S;
+// Decodes and writes chunk c of a container; the group's result goes to its
+// length and status words.
+template <class C>
+__device__ __forceinline__ void inflate_chunk(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *off,
+                                              uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len, int32_t *status,
+                                              uint32_t flags, Sh<C> &S) {
   const uint64_t c = blockIdx.x;
   const uint64_t o0 = off[c], o1 = off[c + 1];
-  Result r;
-  if (o1 < o0 || o1 > comp_bytes) {
-    r = Result{kCorrupt, 0, 0};
-  } else {
-    r = inflate_stream(comp + o0, o1 - o0, out + c * chunk_bytes, chunk_bytes, flags, S);
-  }
-  if (lane_id() == 0) {
+  Result r{kCorrupt, 0, 0};
+  if (o1 >= o0 && o1 <= comp_bytes)
+    r = inflate_group<C>(comp + o0, o1 - o0, out + c * chunk_bytes, chunk_bytes, flags, S);
+  if (threadIdx.x == 0) {
     if (status) status[c] = status_code(r.status, flags);
     if (out_len) out_len[c] = r.bytes;
   }
 }
 
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kWavesOne)))
-inflate_batch_kernel(const codag_stream_desc *__restrict__ descs, uint64_t n,
-                     codag_stream_result *__restrict__ results, uint32_t flags,
-                     uint32_t *__restrict__ counter) {
-  __shared__ Lds S;
+__global__ void __launch_bounds__(One::kThreads) __attribute__((amdgpu_waves_per_eu(3)))
+inflate_chunks_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
+                      const uint64_t *__restrict__ off, uint64_t chunk_bytes, uint8_t *out,
+                      uint64_t *__restrict__ out_len, int32_t *__restrict__ status, uint32_t flags) {
+  __shared__ Sh<One> S;
+  inflate_chunk<One>(comp, comp_bytes, off, chunk_bytes, out, out_len, status, flags, S);
+}
+
+__global__ void __launch_bounds__(Many::kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+inflate_chunks_many_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
+                           const uint64_t *__restrict__ off, uint64_t chunk_bytes, uint8_t *out,
+                           uint64_t *__restrict__ out_len, int32_t *__restrict__ status, uint32_t flags) {
+  __shared__ Sh<Many> S;
+  inflate_chunk<Many>(comp, comp_bytes, off, chunk_bytes, out, out_len, status, flags, S);
+}
+
+// The queue of a batch, in device memory: its next stream and whether groups of
+// eight waves or of one decode it.
+//  * One wave takes about 20 ns per compressed byte of its stream and the GPU's
+//    one-wave groups together 1/85 ns; eight-wave groups take about 150 ns per
+//    stream and 1/78 ns per compressed byte over all. So eight waves win until
+//    there are many streams of about one size. Mixed zlib streams from 4 KiB on
+//    (one wave / eight waves, ms): 700 of up to 64 KiB 0.77 / 0.37, 3000 of up
+//    to 64 KiB 0.86 / 0.90, of up to 1 MiB 11.2 / 4.5, 6000 of up to 16 KiB
+//    0.49 / 1.08, of up to 256 KiB 3.19 / 3.39. (The large streams by eight
+//    waves and then the small ones by one wave each was never the faster.)
+struct BatchQueue {
+  uint32_t next;
+  uint32_t many;
+};
+constexpr uint32_t kPlanThreads = 1024, kPlanSample = 1u << 16;
+
+// Resets the queue and chooses the groups by the streams' sizes (of evenly
+// spaced streams, where there are more than kPlanSample). `shape`: 0 chosen
+// here, 1 one wave, 2 eight waves.
+__global__ void __launch_bounds__(kPlanThreads)
+plan_batch_kernel(const codag_stream_desc *__restrict__ descs, uint64_t n, BatchQueue *q, uint32_t shape) {
+  __shared__ uint64_t sums[kPlanThreads / kWave], tops[kPlanThreads / kWave];
+  const uint64_t m = min(n, (uint64_t)kPlanSample);
+  uint64_t sum = 0, top = 0;
+  if (shape == 0)
+    for (uint64_t k = threadIdx.x; k < m; k += blockDim.x) {
+      const uint64_t b = min(descs[k * n / m].src_bytes, (uint64_t)1 << 28);
+      sum += b;
+      top = max(top, b);
+    }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    sum += __shfl_xor(sum, d, kWave);
+    top = max(top, __shfl_xor(top, d, kWave));
+  }
+  if (lane_id() == 0) {
+    sums[threadIdx.x / kWave] = sum;
+    tops[threadIdx.x / kWave] = top;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  sum = top = 0;
+  for (uint32_t i = 0; i < blockDim.x / kWave; i++) {
+    sum += sums[i];
+    top = max(top, tops[i]);
+  }
+  if (m) sum = sum / m * n;
+  const uint64_t one = max(200000 + 20 * top, sum / 85), many = 150 * n + sum / 78;  // ns
+  q->next = 0;
+  q->many = shape == 0 ? many <= one : shape == 2;
+}
+
+// Persistent loop over a batch: each group takes the next stream from the queue
+// until none is left.
+template <class C>
+__device__ __forceinline__ void inflate_batch(const codag_stream_desc *descs, uint64_t n, codag_stream_result *results,
+                                              uint32_t flags, BatchQueue *q, Sh<C> &S) {
+  if (q->many != (C::kNW > 1)) return;
   for (;;) {
-    uint32_t i = 0;
-    if (lane_id() == 0) i = atomicAdd(counter, 1u);
-    i = __builtin_amdgcn_readfirstlane(__shfl(i, 0, kWave));
+    group_sync<C>();
+    if (threadIdx.x == 0) S.stream = atomicAdd(&q->next, 1u);
+    group_sync<C>();
+    const uint32_t i = uni(S.stream);
     if ((uint64_t)i >= n) break;
     const codag_stream_desc d = descs[i];
-    // A stream decodes serially on one wave, and the waves of a CU share its
-    // scalar pipe: in an uneven batch the largest streams set the finish
-    // time. Their waves issue first (wave priority by output size), the
-    // small streams fill the remaining issue slots.
+    // In an uneven batch the largest streams set the finish time: their waves
+    // issue first (wave priority by output size), the small streams fill the
+    // remaining issue slots.
     const uint64_t big = d.dst_cap;
     if (big >= (2u << 20)) __builtin_amdgcn_s_setprio(3);
     else if (big >= (1u << 20)) __builtin_amdgcn_s_setprio(2);
     else if (big >= (512u << 10)) __builtin_amdgcn_s_setprio(1);
     else __builtin_amdgcn_s_setprio(0);
-    const Result r = inflate_stream(d.src, d.src_bytes, d.dst, d.dst_cap, flags, S);
-    if (lane_id() == 0) {
+    const Result r = inflate_group<C>(d.src, d.src_bytes, d.dst, d.dst_cap, flags, S);
+    if (threadIdx.x == 0) {
       results[i].bytes_written = r.bytes;
       results[i].status = status_code(r.status, flags);
       results[i].adler32 = r.adler;
     }
-    __syncthreads();
   }
 }
 
-// ------------------------------------------------------ two-wave batch
-
-// A workgroup of two waves decodes one stream at a time: wave 0 decodes
-// (header, tables, symbols) and hands each batch of tokens, each stored
-// block and the end of the stream to wave 1 through a four-deep LDS queue;
-// wave 1 writes the output (ring copies, far gathers, flush, Adler-32). The
-// decoding wave's serial chain no longer waits for the output phase, which
-// bounds a large stream's time in an uneven batch. The two waves meet only
-// through the queue's head / tail / done words (release / acquire on LDS)
-// and at the top of each stream; every wait is bounded (kSpinLimit sleeps,
-// between half a second and two), and one that runs out ends the stream as
-// CORRUPT.
-constexpr uint32_t kQueue = 4;
-constexpr uint32_t kSpinLimit = 1u << 24;
-enum : uint32_t { kMsgTokens = 0, kMsgStored = 1, kMsgEnd = 2 };
-
-struct Msg {
-  uint32_t kind, nt, ln, pad;
-  uint64_t at;
-};
-
-struct Queue {
-  uint32_t tok[kQueue][kWave];
-  Msg msg[kQueue];
-  uint32_t head;    // messages published by the decoding wave
-  uint32_t tail;    // messages the writing wave has finished with
-  int32_t wstat;    // the writing wave's first error
-  uint32_t done;    // the writing wave has flushed the stream
-  uint32_t bytes, adler;
-  uint32_t stream;  // the workgroup's current stream index
-};
-
-__device__ __forceinline__ uint32_t lds_acquire(uint32_t *p) {
-  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void lds_release(uint32_t *p, uint32_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+__global__ void __launch_bounds__(One::kThreads) __attribute__((amdgpu_waves_per_eu(3)))
+inflate_batch_kernel(const codag_stream_desc *__restrict__ descs, uint64_t n,
+                     codag_stream_result *__restrict__ results, uint32_t flags, BatchQueue *q) {
+  __shared__ Sh<One> S;
+  inflate_batch<One>(descs, n, results, flags, q, S);
 }
 
-// The decoding wave's side: batches go into the queue.
-struct SinkQueue {
-  Queue *q;
-  uint32_t head;
-  uint32_t tail;  // the writer's last tail this wave read: slots below it are free
-  bool ended, stuck;
-  // Hands a message to the writer. The writer's tail is read again only when
-  // the last one read leaves no free slot, and the writer's status is not
-  // polled per batch (finish() returns the writer's first error before any
-  // later decode error), so a batch costs one LDS round trip, the release.
-  __device__ __forceinline__ int32_t push(uint32_t lane, uint32_t kind, uint32_t tok, uint32_t nt,
-                                          uint64_t at, uint32_t ln) {
-    for (uint32_t k = 0;; k++) {  // a free slot
-      if (head - tail < kQueue) break;
-      tail = uni(lds_acquire(&q->tail));
-      if (head - tail < kQueue) break;
-      if (k >= kSpinLimit) {
-        stuck = true;
-        return kCorrupt;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-    const uint32_t sl = head % kQueue;
-    q->tok[sl][lane] = tok;
-    if (lane == 0) {
-      q->msg[sl].kind = kind;
-      q->msg[sl].nt = nt;
-      q->msg[sl].ln = ln;
-      q->msg[sl].at = at;
-    }
-    head++;
-    lds_release(&q->head, head);
-    return kOk;
-  }
-  __device__ __forceinline__ int32_t tokens(uint32_t lane, uint32_t tok, uint32_t nt) {
-    if (nt == 0) return (int32_t)uni(lds_acquire(reinterpret_cast<uint32_t *>(&q->wstat)));
-    return push(lane, kMsgTokens, tok, nt, 0, 0);
-  }
-  __device__ __forceinline__ int32_t stored(const uint8_t *, uint64_t at, uint32_t ln, uint32_t lane) {
-    return push(lane, kMsgStored, 0, 0, at, ln);
-  }
-  // hands over the end of the stream and waits for the writing wave; the
-  // writer's first error precedes any later error of the decode
-  __device__ __forceinline__ int32_t finish(uint32_t lane, int32_t st, Result &res) {
-    ended = true;
-    res.bytes = 0;
-    res.adler = 1;
-    if (!stuck && push(lane, kMsgEnd, 0, 0, 0, 0) == kCorrupt && stuck) return kCorrupt;
-    if (stuck) return kCorrupt;
-    for (uint32_t k = 0;; k++) {
-      if (uni(lds_acquire(&q->done))) break;
-      if (k >= kSpinLimit) return kCorrupt;
-      __builtin_amdgcn_s_sleep(1);
-    }
-    res.bytes = uni(q->bytes);
-    res.adler = uni(q->adler);
-    const int32_t ws = (int32_t)uni((uint32_t)q->wstat);
-    return ws != kOk ? ws : st;
-  }
-};
-
-// The writing wave's side: takes messages in order until the end of the
-// stream, then publishes the bytes written, their Adler-32 and its first
-// error. After an error it only drains the queue.
-__device__ __forceinline__ void inflate_write(Queue &q, uint8_t *ring, uint8_t *dst, uint64_t cap,
-                                              const uint8_t *src) {
-  const uint32_t lane = lane_id();
-  SinkOne<kRingPair> w;
-  w.init(dst, ring, cap > 0x7fffffffull ? 0x7fffffffull : cap);
-  int32_t wst = kOk;
-  for (uint32_t t = 0;; t++) {
-    bool ready = false;
-    for (uint32_t k = 0; k < kSpinLimit; k++) {
-      if (uni(lds_acquire(&q.head)) > t) {
-        ready = true;
-        break;
-      }
-      // an idle writer polls every ~200 cycles: a batch takes the decoder
-      // thousands, and fewer polls leave the CU's issue slots to decoders
-      __builtin_amdgcn_s_sleep(3);
-    }
-    if (!ready) {
-      if (wst == kOk) wst = kCorrupt;
-      break;
-    }
-    const uint32_t sl = t % kQueue;
-    const uint32_t kind = uni(q.msg[sl].kind);
-    if (kind == kMsgEnd) break;
-    if (wst == kOk) {
-      int32_t e;
-      if (kind == kMsgTokens) e = w.tokens(lane, q.tok[sl][lane], uni(q.msg[sl].nt));
-      else e = w.stored(src, q.msg[sl].at, uni(q.msg[sl].ln), lane);
-      if (e != kOk) {
-        wst = e;
-        lds_release(reinterpret_cast<uint32_t *>(&q.wstat), (uint32_t)e);
-      }
-    }
-    lds_release(&q.tail, t + 1);
-  }
-  Result r;
-  w.finish(lane, kOk, r);
-  q.bytes = (uint32_t)r.bytes;
-  q.adler = r.adler;
-  q.wstat = wst;
-  // the output is in memory before the decoding wave reads it back (gzip
-  // CRC-32)
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  lds_release(&q.done, 1u);
+__global__ void __launch_bounds__(Many::kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+inflate_batch_many_kernel(const codag_stream_desc *__restrict__ descs, uint64_t n,
+                          codag_stream_result *__restrict__ results, uint32_t flags, BatchQueue *q) {
+  __shared__ Sh<Many> S;
+  inflate_batch<Many>(descs, n, results, flags, q, S);
 }
 
-struct Lds2 {
-  LdsPair dec;                   // the decoding wave's tables, slots and CRC space
-  alignas(16) uint8_t ring[kRingPair];  // the writing wave's output ring
-  Queue q;
-};
-
-__global__ void __launch_bounds__(2 * kWave) __attribute__((amdgpu_waves_per_eu(kWavesPair)))
-inflate_batch2_kernel(const codag_stream_desc *__restrict__ descs, uint64_t n,
-                      codag_stream_result *__restrict__ results, uint32_t flags,
-                      uint32_t *__restrict__ counter) {
-  __shared__ Lds2 S;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x) / kWave;
-  const uint32_t lane = lane_id();
-  for (;;) {
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      S.q.stream = atomicAdd(counter, 1u);
-      S.q.head = 0;
-      S.q.tail = 0;
-      S.q.wstat = kOk;
-      S.q.done = 0;
-    }
-    __syncthreads();
-    const uint32_t i = uni(S.q.stream);
-    if ((uint64_t)i >= n) break;
-    const codag_stream_desc d = descs[i];
-    const uint64_t big = d.dst_cap;
-    if (big >= (2u << 20)) __builtin_amdgcn_s_setprio(3);
-    else if (big >= (1u << 20)) __builtin_amdgcn_s_setprio(2);
-    else if (big >= (512u << 10)) __builtin_amdgcn_s_setprio(1);
-    else __builtin_amdgcn_s_setprio(0);
-    if (wave == 0) {
-      SinkQueue out;
-      out.q = &S.q;
-      out.head = 0;
-      out.tail = 0;
-      out.ended = false;
-      out.stuck = false;
-      Result r = inflate_stream_t(d.src, d.src_bytes, d.dst, d.dst_cap, flags, S.dec, out);
-      if (!out.ended) {  // a header error before any output: release the writer
-        Result t;
-        const int32_t e = out.finish(lane, r.status, t);
-        if (r.status == kOk) r.status = e;
-      }
-      if (lane == 0) {
-        results[i].bytes_written = r.bytes;
-        results[i].status = status_code(r.status, flags);
-        results[i].adler32 = r.adler;
-      }
-    } else {
-      inflate_write(S.q, S.ring, d.dst, d.dst_cap, d.src);
-    }
-  }
-}
-
-// The chunk container decoded by two-wave workgroups, one chunk each.
-__global__ void __launch_bounds__(2 * kWave) __attribute__((amdgpu_waves_per_eu(kWavesPair)))
-inflate_chunks2_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
-                       const uint64_t *__restrict__ off, uint64_t n, uint64_t chunk_bytes,
-                       uint8_t *__restrict__ out, uint64_t *__restrict__ out_len,
-                       int32_t *__restrict__ status, uint32_t flags) {
-  __shared__ Lds2 S;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x) / kWave;
-  const uint32_t lane = lane_id();
-  const uint64_t c = blockIdx.x;
-  const uint64_t o0 = off[c], o1 = off[c + 1];
-  if (o1 < o0 || o1 > comp_bytes) {  // no stream: neither wave decodes
-    if (threadIdx.x == 0) {
-      if (status) status[c] = status_code(kCorrupt, flags);
-      if (out_len) out_len[c] = 0;
-    }
-    return;
-  }
-  if (threadIdx.x == 0) {
-    S.q.head = 0;
-    S.q.tail = 0;
-    S.q.wstat = kOk;
-    S.q.done = 0;
-  }
-  __syncthreads();
-  if (wave == 0) {
-    SinkQueue sink;
-    sink.q = &S.q;
-    sink.head = 0;
-    sink.tail = 0;
-    sink.ended = false;
-    sink.stuck = false;
-    Result r = inflate_stream_t(comp + o0, o1 - o0, out + c * chunk_bytes, chunk_bytes, flags, S.dec, sink);
-    if (!sink.ended) {
-      Result t;
-      const int32_t e = sink.finish(lane, r.status, t);
-      if (r.status == kOk) r.status = e;
-    }
-    if (lane == 0) {
-      if (status) status[c] = status_code(r.status, flags);
-      if (out_len) out_len[c] = r.bytes;
-    }
-  } else {
-    inflate_write(S.q, S.ring, out + c * chunk_bytes, chunk_bytes, comp + o0);
-  }
-}
-
-__global__ void zero_counter_kernel(uint32_t *c) { *c = 0; }
-
-// Device memory of the allocation-free batch entry point: word 0 is its
-// work-queue counter. Every GPU holds its own copy for the life of the
+// Device memory of the allocation-free batch entry point: its queue. Every GPU holds its own copy for the life of the
 // process; all calls on one GPU share it.
 constexpr uint32_t kScratchWords = 64;  // 256 bytes
 static __device__ __align__(256) uint32_t scratch[kScratchWords];
 constexpr int kScratchDevices = 64;
+static_assert(sizeof(BatchQueue) <= 256, "a queue fits a counter slot and the static array");
 
 }  // namespace inflate
 
@@ -1612,32 +1550,43 @@ hipError_t inflate_scratch_ptr(uint32_t **out) {
   return hipSuccess;
 }
 
+// Eight waves per chunk while there are at most five chunks per CU, else one
+// wave per chunk (128 KiB chunks, MI355X: 256 chunks 0.48 and 1.26 ms, 1024
+// 1.04 and 1.38 ms, 2048 2.02 and 1.51 ms, 4096 3.90 and 3.16 ms).
 hipError_t launch_inflate_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *off,
-                                 uint64_t n,
-                                 uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
-                                 int32_t *status, uint32_t flags, hipStream_t stream,
-                                 bool two_wave) {
+                                 uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
+                                 int32_t *status, uint32_t flags, hipStream_t stream, bool many) {
   if (n == 0) return hipSuccess;
-  if (two_wave)
-    hipLaunchKernelGGL(inflate::inflate_chunks2_kernel, dim3((uint32_t)n), dim3(2 * kWaveSize), 0,
-                       stream, comp, comp_bytes, off, n, chunk_bytes, out, out_len, status, flags);
+  if (many)
+    hipLaunchKernelGGL(inflate::inflate_chunks_many_kernel, dim3((uint32_t)n), dim3(inflate::Many::kThreads), 0,
+                       stream, comp, comp_bytes, off, chunk_bytes, out, out_len, status, flags);
   else
     hipLaunchKernelGGL(inflate::inflate_chunks_kernel, dim3((uint32_t)n), dim3(kWaveSize), 0,
-                       stream, comp, comp_bytes, off, n, chunk_bytes, out, out_len, status, flags);
+                       stream, comp, comp_bytes, off, chunk_bytes, out, out_len, status, flags);
   return hipGetLastError();
 }
 
+// Batches that all fit the GPU at once (two eight-wave groups per CU) go to
+// eight-wave groups; for larger ones the queue's plan picks one of two launches,
+// and the other's groups leave at once. !by_size: one wave per stream.
 hipError_t launch_inflate_batch(const codag_stream_desc *descs, uint64_t n,
                                 codag_stream_result *results, uint32_t flags, uint32_t *counter,
-                                uint32_t groups, hipStream_t stream, bool two_wave) {
-  hipLaunchKernelGGL(inflate::zero_counter_kernel, dim3(1), dim3(1), 0, stream, counter);
+                                uint32_t cus, uint32_t per_cu, hipStream_t stream, bool by_size) {
+  using namespace inflate;
+  auto *q = reinterpret_cast<BatchQueue *>(counter);
+  const uint32_t shape = !by_size ? 1u : (n <= 2ull * cus ? 2u : 0u);
+  hipLaunchKernelGGL(plan_batch_kernel, dim3(1), dim3(shape ? kWaveSize : kPlanThreads), 0, stream, descs, n, q, shape);
   if (n == 0) return hipGetLastError();
-  if (two_wave)
-    hipLaunchKernelGGL(inflate::inflate_batch2_kernel, dim3(groups), dim3(2 * kWaveSize), 0, stream,
-                       descs, n, results, flags, counter);
-  else
-    hipLaunchKernelGGL(inflate::inflate_batch_kernel, dim3(groups), dim3(kWaveSize), 0, stream,
-                       descs, n, results, flags, counter);
+  if (shape != 1) {
+    const uint64_t groups = std::min<uint64_t>(n, (uint64_t)cus * std::min(per_cu, 2u));
+    hipLaunchKernelGGL(inflate_batch_many_kernel, dim3((uint32_t)groups), dim3(Many::kThreads), 0, stream, descs, n,
+                       results, flags, q);
+  }
+  if (shape != 2) {
+    const uint64_t groups = std::min<uint64_t>(n, (uint64_t)cus * per_cu);
+    hipLaunchKernelGGL(inflate_batch_kernel, dim3((uint32_t)groups), dim3(kWaveSize), 0, stream, descs, n, results,
+                       flags, q);
+  }
   return hipGetLastError();
 }
 

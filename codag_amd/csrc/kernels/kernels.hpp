@@ -29,23 +29,22 @@ hipError_t launch_rlev2_wave(const uint8_t *comp, uint64_t comp_bytes, const uin
                              uint64_t chunk_bytes, uint8_t *out, int32_t *status, uint32_t win,
                              hipStream_t stream);
 
-// two_wave: a decoding and a writing wave per chunk; else one wave.
+// many: eight waves per chunk; else one wave.
 hipError_t launch_inflate_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *off,
-                                 uint64_t n,
-                                 uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
+                                 uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
                                  int32_t *status, uint32_t flags, hipStream_t stream,
-                                 bool two_wave = false);
+                                 bool many = false);
 
-// Persistent batch launch: `groups` resident workgroups pull streams from
-// *counter (zeroed by a kernel launched first on the same stream). two_wave:
-// workgroups of a decoding and a writing wave per stream; else one wave.
+// Persistent batch launch: up to per_cu resident workgroups on each of `cus` CUs
+// pull streams from the queue at `counter` (256 bytes, reset by a kernel launched
+// first on the same stream). by_size: eight waves or one wave per stream, by the
+// streams' number and sizes; else one wave per stream.
 hipError_t launch_inflate_batch(const codag_stream_desc *descs, uint64_t n,
                                 codag_stream_result *results, uint32_t flags, uint32_t *counter,
-                                uint32_t groups, hipStream_t stream, bool two_wave = false);
+                                uint32_t cus, uint32_t per_cu, hipStream_t stream, bool by_size);
 
 // Device address (on the current device) of the inflate kernels' static
-// 256-byte scratch array; its first word is the work-queue counter of the
-// allocation-free batch entry point.
+// 256-byte scratch array, the queue of the allocation-free batch entry point.
 hipError_t inflate_scratch_ptr(uint32_t **out);
 
 // RLE v1, one walker wave and nexp (1 or 3) expander waves per chunk.

@@ -133,7 +133,7 @@ codag_status codag_inflate_chunks(codag_ctx *ctx, const uint8_t *d_comp, uint64_
 
 /* Uneven batch of independent zlib streams (no reference counterpart: the
  * reference has fixed-size chunks only; shape follows cudf_deflate.cuh:236-250).
- * One persistent launch pulls streams from a device work queue in descriptor
+ * Persistent launches pull streams from a device work queue in descriptor
  * order (listing the largest streams first gives the best load balance).
  * The work queue's counter belongs to the HIP stream the batch is launched
  * on, so batches of one context on different streams may overlap; a context
@@ -163,7 +163,7 @@ codag_status codag_inflate_batch(codag_ctx *ctx, const codag_stream_desc *d_desc
  * inputs and outputs, the work-queue counter lives in a static 256-byte
  * device array of the library (one per GPU, held until the process ends), and
  * the call makes no hipMalloc/hipFree and builds no graph of its own (a
- * caller's stream capture records its two launches). The counter is reset by
+ * caller's stream capture records its launches). The counter is reset by
  * a kernel on `stream` (NULL = the device's null stream) before each launch.
  * All calls on one GPU in a process share that counter and it keeps the last
  * call's contents: calls that overlap on one GPU (different streams or host
@@ -396,7 +396,7 @@ typedef enum codag_codec { CODAG_RLEV1 = 1, CODAG_RLEV2 = 2, CODAG_DEFLATE = 3 }
  * (window 4096; 128, 192 (RLE v2 only) or 256 threads = 1, 2 or 3 expander
  * waves), 4 the RLE v1 pipeline (512 threads, window 2048). For Deflate's
  * batch launch (codag_inflate_batch), 64 threads = one wave per stream, 128
- * = a decoding and a writing wave per stream. codag_tune_set rejects shapes
+ * = eight waves or one wave per stream, by the streams' number and sizes. codag_tune_set rejects shapes
  * that are not compiled in. */
 typedef struct codag_tune_params {
   uint32_t threads_per_group; /* workgroup size (64..1024, multiple of 64) */
@@ -413,7 +413,7 @@ codag_status codag_tune_set(codag_ctx *ctx, codag_codec codec, const codag_tune_
  * candidate's; the shape in use stays if it is within 2% of that one (a tie
  * in run-to-run noise does not flip the choice). The kept shape becomes the
  * context's shape. best_ms (nullable) gets its time. DEFLATE candidates differ in
- * the batch launch's workgroup (one or two waves per stream) and workgroups
+ * the batch launch's workgroups (one wave per stream, or by size) and workgroups
  * per CU; the launch has min(CUs x groups_per_cu, n_chunks) workgroups, so
  * the sample needs more than CUs x 28 streams for all of them to differ. */
 codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_comp,
