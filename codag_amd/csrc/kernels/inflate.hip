@@ -1145,63 +1145,109 @@ struct X2nTable {
 };
 __constant__ X2nTable kX2n = X2nTable();
 
-// x^(8n) mod P.
-__device__ __forceinline__ uint32_t crc_x8n(uint32_t n) {
-  uint32_t p = 1u << 31;  // x^0
-  uint32_t k = 3;
-  while (n) {
-    if (n & 1) p = crc_mulmod(kX2n.t[k & 31], p);
-    n >>= 1;
-    k++;
+// b * a mod P for a wave-uniform a.
+__device__ __forceinline__ uint32_t crc_scale(uint32_t a, uint32_t b) {
+  uint32_t p = 0;
+#pragma unroll 4
+  for (uint32_t k = 0; k < 32; k++) {
+    p ^= (a >> 31) ? b : 0u;
+    a <<= 1;
+    b = (b >> 1) ^ ((b & 1) ? kCrcPoly : 0u);
   }
   return p;
 }
 
-// CRC-32 of n bytes at global address p, by the whole wave: four 256-entry
-// slice tables are built in `tab` (4 KiB of LDS), lane l takes the l-th of
-// 64 equal segments (slice-by-4), and the 64 segment CRCs are combined in
-// order. Every lane returns the same value.
-__device__ __forceinline__ uint32_t wave_crc32(const uint8_t *p, uint32_t n, uint32_t *tab) {
-  const uint32_t lane = lane_id();
-  // the bytes may have been stored by other lanes of this wave just before
-  wave_sync();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  for (uint32_t i = lane; i < 256; i += kWave) {
+// Builds the four 256-entry slice tables in `tab` (4 KiB of LDS) by T threads;
+// sync() orders the threads.
+template <class F> __device__ __forceinline__ void crc_tables(uint32_t *tab, uint32_t t, uint32_t T, F sync) {
+  for (uint32_t i = t; i < 256; i += T) {
     uint32_t c = i;
 #pragma unroll
     for (int k = 0; k < 8; k++) c = (c & 1) ? (c >> 1) ^ kCrcPoly : c >> 1;
     tab[i] = c;
   }
-  wave_sync();
+  sync();
 #pragma unroll
-  for (int t = 1; t < 4; t++) {
-    for (uint32_t i = lane; i < 256; i += kWave) {
-      const uint32_t c = tab[(t - 1) * 256 + i];
-      tab[t * 256 + i] = (c >> 8) ^ tab[c & 0xff];
+  for (int k = 1; k < 4; k++) {
+    for (uint32_t i = t; i < 256; i += T) {
+      const uint32_t c = tab[(k - 1) * 256 + i];
+      tab[k * 256 + i] = (c >> 8) ^ tab[c & 0xff];
     }
-    wave_sync();
+    sync();
   }
-  const uint32_t seg = ((n + kWave - 1) / kWave + 3) & ~3u;
-  const uint32_t lo = min(lane * seg, n), hi = min(lo + seg, n);
+}
+
+__device__ __forceinline__ uint32_t crc_dword(const uint32_t *tab, uint32_t c, uint32_t v) {
+  c ^= v;
+  return tab[768 + (c & 0xff)] ^ tab[512 + ((c >> 8) & 0xff)] ^ tab[256 + ((c >> 16) & 0xff)] ^ tab[c >> 24];
+}
+
+// The CRC register, begun at 0, after this wave's part of the n bytes at p:
+// thread t of T takes 2^lg bytes, the last thread the last ones, so that the
+// bytes missing to T * 2^lg stand at the front, where zeros leave the register
+// at 0. Neighbours are combined pairwise (crc(A B) = crc(A) * x^(8|B|) +
+// crc(B), all B of a step of one length), 6 products for 64 lanes; combined one
+// lane after the other, with a length of its own each, 64 lanes took about 80.
+__device__ __forceinline__ uint32_t crc_part(const uint8_t *p, uint32_t n, uint32_t lg, const uint32_t *tab,
+                                             uint32_t t, uint32_t T) {
+  const uint64_t behind = (uint64_t)(T - 1 - t) << lg;  // bytes after this thread's
+  uint32_t c = 0;
+  if (behind < n) {
+    const uint32_t hi = n - (uint32_t)behind, len = min(hi, 1u << lg);
+    uint32_t i = hi - len;
+    for (; i < hi && ((hi - i) & 15); i++) c = tab[(c ^ p[i]) & 0xff] ^ (c >> 8);
+    for (; i < hi; i += 16) {
+      uint4 v;
+      __builtin_memcpy(&v, p + i, 16);
+      c = crc_dword(tab, crc_dword(tab, crc_dword(tab, crc_dword(tab, c, v.x), v.y), v.z), v.w);
+    }
+  }
+#pragma unroll 1
+  for (uint32_t k = 0; k < 6; k++) c ^= crc_scale(kX2n.t[(3 + lg + k) & 31], __shfl_up(c, 1u << k, kWave));
+  return rdlane(c, kWave - 1);
+}
+
+// x^(8n) times the register's first value, all ones: what the bytes before the
+// first one contribute.
+__device__ __forceinline__ uint32_t crc_begin(uint32_t n) {
   uint32_t c = 0xFFFFFFFFu;
-  uint32_t i = lo;
-  for (; i + 4 <= hi; i += 4) {
-    c ^= (uint32_t)p[i] | ((uint32_t)p[i + 1] << 8) | ((uint32_t)p[i + 2] << 16) |
-         ((uint32_t)p[i + 3] << 24);
-    c = tab[768 + (c & 0xff)] ^ tab[512 + ((c >> 8) & 0xff)] ^ tab[256 + ((c >> 16) & 0xff)] ^
-        tab[c >> 24];
-  }
-  for (; i < hi; i++) c = tab[(c ^ p[i]) & 0xff] ^ (c >> 8);
-  const uint32_t mine = ~c;
-  // x^(8 * segment length) of this lane's segment, every lane at once
-  const uint32_t shift = crc_x8n(hi - lo);
-  uint32_t total = 0;  // CRC of the empty string
-  for (uint32_t l = 0; l < (uint32_t)kWave; l++) {
-    const uint32_t cl = rdlane(mine, l), xl = rdlane(shift, l);
-    total = crc_mulmod(xl, total) ^ cl;
-  }
+  for (uint32_t k = 3; n; n >>= 1, k++)
+    if (n & 1) c = crc_scale(kX2n.t[k & 31], c);
+  return c;
+}
+
+// Log2 of the bytes per thread, at least 16 (n < 2^31).
+__device__ __forceinline__ uint32_t crc_share(uint32_t n, uint32_t T) {
+  const uint32_t each = max((n + T - 1) / T, 16u);
+  return 32u - (uint32_t)__builtin_clz(each - 1);
+}
+
+// CRC-32 of n bytes at global address p by one wave; `tab`: 4 KiB of LDS.
+__device__ __forceinline__ uint32_t wave_crc32(const uint8_t *p, uint32_t n, uint32_t *tab) {
+  const uint32_t lane = lane_id();
   wave_sync();
-  return uni(total);
+  crc_tables(tab, lane, kWave, [] { wave_sync(); });
+  const uint32_t c = crc_part(p, n, crc_share(n, kWave), tab, lane, kWave);
+  wave_sync();
+  return uni(~(c ^ crc_begin(n)));
+}
+
+// The same by the whole group, which has written the bytes.
+template <class C>
+__device__ __forceinline__ uint32_t group_crc32(const uint8_t *p, uint32_t n, Sh<C> &S, uint32_t wave, uint32_t lane) {
+  uint32_t *tab = reinterpret_cast<uint32_t *>(S.win);
+  const uint32_t tid = wave * kWave + lane, lg = crc_share(n, C::kThreads);
+  group_sync<C>();
+  crc_tables(tab, tid, C::kThreads, [] { group_sync<C>(); });
+  uint32_t c = crc_part(p, n, lg, tab, tid, C::kThreads);
+  if constexpr (C::kNW > 1) {
+    if (lane == 0) S.part[0][wave] = c;
+    __syncthreads();
+    c = S.part[0][0];
+    for (uint32_t k = 1; k < (uint32_t)C::kNW; k++) c = crc_scale(kX2n.t[(9 + lg) & 31], c) ^ S.part[0][k];
+    __syncthreads();
+  }
+  return uni(~(c ^ crc_begin(n)));
 }
 
 // gzip member header (RFC 1952 2.3), checked as zlib's inflate() checks it:
@@ -1348,20 +1394,18 @@ __device__ __forceinline__ Result inflate_group(const uint8_t *src, uint64_t len
       group_sync<C>();  // the command is read by all
     }
   }
-  if (gzip) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // wave 0 reads the output back
-  const uint32_t adler = out_adler<C>(o, S, wave);
+  const uint32_t check = gzip ? group_crc32<C>(dst, o.pos, S, wave, lane) : out_adler<C>(o, S, wave);
   if (wave != 0) return res;
   if (!headed) {
     res.status = st;
     return res;
   }
-  res.adler = adler;
+  res.adler = check;
   res.bytes = o.pos;
   if (gzip) {
     // RFC 1952 trailer on the next byte boundary: CRC-32 and ISIZE, both
     // little-endian; zlib checks the CRC first ("incorrect data check"),
     // then the length ("incorrect length check")
-    res.adler = wave_crc32(dst, (uint32_t)res.bytes, crc_tab);
     if (st == kOk) {
       const uint64_t at = (P + 7) / 8 - lead;
       if (at + 8 > len) {
