@@ -645,8 +645,8 @@ struct Place {
   uint32_t at, w0, w1, w2;
 };
 
-__device__ __forceinline__ Place place_at(const uint32_t *stage, uint32_t q) {
-  const uint32_t *s = stage + (q >> 5);
+template <class Dwords> __device__ __forceinline__ Place place_at(Dwords stage, uint32_t q) {
+  const Dwords s = stage + (q >> 5);
   return Place{q, s[0], s[1], s[2]};
 }
 
@@ -654,7 +654,7 @@ __device__ __forceinline__ Place place_at(const uint32_t *stage, uint32_t q) {
 __device__ __forceinline__ uint32_t place_bits(const Place &p) { return __builtin_amdgcn_alignbit(p.w1, p.w0, p.at); }
 
 // Moves the place on by n <= 31 bits.
-__device__ __forceinline__ void place_move(Place &p, const uint32_t *stage, uint32_t n) {
+template <class Dwords> __device__ __forceinline__ void place_move(Place &p, Dwords stage, uint32_t n) {
   const uint32_t to = p.at + n;
   const bool cross = to > (p.at | 31);
   p.w0 = cross ? p.w1 : p.w0;
@@ -664,7 +664,7 @@ __device__ __forceinline__ void place_move(Place &p, const uint32_t *stage, uint
 }
 
 // The entry of bits x in the table of descriptor d.
-__device__ __forceinline__ uint32_t look(const uint32_t *tab, uint32_t x, uint32_t d) {
+template <class Dwords> __device__ __forceinline__ uint32_t look(Dwords tab, uint32_t x, uint32_t d) {
   return tab[(d >> 5) + __builtin_amdgcn_ubfe(x, 0, d)];  // the field's width is d's low five bits
 }
 
@@ -684,13 +684,14 @@ template <class C> __device__ __forceinline__ uint32_t next_table(uint32_t e) {
 // lookup a step in straight-line code: one LDS latency and about 30 vector
 // instructions; a branch per kind of entry doubled that in scalar mask
 // work.
-template <class C, bool Count>
-__device__ __forceinline__ bool run_tokens(const Sh<C> &S, uint32_t &q, uint32_t bound, uint32_t limit, uint32_t &n) {
+template <class C, bool Count, class Dwords>
+__device__ __forceinline__ bool run_tokens(Dwords stage, Dwords tab, uint32_t &q, uint32_t bound, uint32_t limit,
+                                           uint32_t &n) {
   uint32_t d = C::kLitDesc, pend = 1, end = bound;
-  Place p = place_at(S.stage, q);
+  Place p = place_at(stage, q);
   while (q < end) {
-    const uint32_t x = place_bits(p), e = look(S.tab, x, d);
-    place_move(p, S.stage, e & 31);
+    const uint32_t x = place_bits(p), e = look(tab, x, d);
+    place_move(p, stage, e & 31);
     const bool good = (e & 31) != 0 && p.at <= limit;
     const bool whole = good && e < kLenType;
     if (Count) {
@@ -871,7 +872,7 @@ __device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n
   const uint32_t end = x + n;  // this lane's bytes: [x, end) from o.pos on
   const bool check = o.pos < 32768u || o.pos + total > o.cap;
   uint32_t lastx = ~0u, lastm = 0;  // this lane's last token
-  Place p = place_at(S.stage, q);
+  Place p = place_at(&S.stage[0], q);
   uint32_t done = 0;
   int32_t st = kOk;
   while (done < total) {
@@ -886,9 +887,9 @@ __device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n
     const uint32_t stopx = min(end, done + wn);
     uint32_t d = C::kLitDesc, mlen = 0;
     while (x < stopx) {
-      const uint32_t bits = place_bits(p), e = look(S.tab, bits, d);
+      const uint32_t bits = place_bits(p), e = look(&S.tab[0], bits, d);
       if ((e & 31) == 0) break;  // not in a counted range
-      place_move(p, S.stage, e & 31);
+      place_move(p, &S.stage[0], e & 31);
       d = next_table<C>(e);
       const uint32_t v = entry_value(e, bits);
       mlen = (e >> 30) == 1 ? v : mlen;
@@ -933,18 +934,20 @@ constexpr uint32_t kHardYes = 3, kHardNo = 4;
 // length keep a wrong phase: 128 equally frequent bytes, say), lane j decodes its
 // part from each of the 16 bits at which the token before it may end, and a chain
 // through these exits gives every lane its entry. Returns the lanes that have
-// one; the first that stops, or whose successor begins further behind, is the
+// one, and this lane's entry in the low half; the first that stops, or whose successor begins further behind, is the
 // last. 128 KiB chunks of 7-bit literals, by passes (one or two lanes verified a
 // pass) and by candidates: 16 chunks 20.0 and 2.2 ms, 4096 chunks by one wave
 // each 30.8 and 17.5 ms.
 template <class C>
-__device__ __forceinline__ uint32_t chain_entries(Sh<C> &S, uint32_t lo, uint32_t bound, uint32_t limit, uint32_t wave,
-                                                  uint32_t lane, uint32_t &entry) {
+__device__ __noinline__ uint64_t chain_entries(lds<Sh<C>> *S, uint32_t lo, uint32_t bound, uint32_t limit,
+                                               uint32_t wave, uint32_t entry) {
+  const uint32_t lane = lane_id();
   uint32_t exits[4] = {0, 0, 0, 0};  // byte c: the exit behind `bound` of entry lo + c, 255 = stop
 #pragma unroll 1
   for (uint32_t c = 0; c < 16; c++) {
     uint32_t q = lo + c, n = 0;
-    const uint32_t x = run_tokens<C, false>(S, q, bound, limit, n) ? 255u : q - bound;
+    const uint32_t x =
+        run_tokens<C, false, const lds<uint32_t> *>(S->stage, S->tab, q, bound, limit, n) ? 255u : q - bound;
 #pragma unroll
     for (uint32_t k = 0; k < 4; k++) exits[k] |= c / 4 == k ? x << 8 * (c & 3) : 0u;
   }
@@ -960,17 +963,17 @@ __device__ __forceinline__ uint32_t chain_entries(Sh<C> &S, uint32_t lo, uint32_
     }
     if constexpr (C::kNW > 1) {
       if (w == wave && lane == 0) {
-        S.mis[w] = have;
-        S.stp[w] = off;
+        S->mis[w] = have;
+        S->stp[w] = off;
       }
       __syncthreads();
-      have = uni(S.mis[w]);
-      off = uni(S.stp[w]);
-      if (have < (uint32_t)kWave || off >= 16) return w * kWave + have;
+      have = uni(S->mis[w]);
+      off = uni(S->stp[w]);
+      if (have < (uint32_t)kWave || off >= 16) return (uint64_t)(w * kWave + have) << 32 | entry;
       have = 0;
     }
   }
-  return C::kNW > 1 ? C::kThreads : have;
+  return (uint64_t)(C::kNW > 1 ? C::kThreads : have) << 32 | entry;
 }
 
 // Decodes and writes the tokens of one span from stream bit P on; P becomes the
@@ -1000,7 +1003,7 @@ __device__ __forceinline__ int32_t span(const uint32_t *w, uint32_t nw, uint32_t
   uint32_t sq[C::kSub], sn[C::kSub];
 #pragma unroll
   for (int k = 0; k < C::kSub; k++) sq[k] = sn[k] = 0;
-  bool stop = run_tokens<C, false>(S, q, bound, limit, n);
+  bool stop = run_tokens<C, false>(&S.stage[0], &S.tab[0], q, bound, limit, n);
   uint32_t valid;  // lanes verified
   for (uint32_t pass = 2;; pass++) {
     const uint32_t mine = q | (stop ? 0x80000000u : 0u);
@@ -1037,7 +1040,9 @@ __device__ __forceinline__ int32_t span(const uint32_t *w, uint32_t nw, uint32_t
         if (hard < kHardYes && valid < max(C::kThreads / 8, 16u)) hard++;
         break;
       }
-      valid = chain_entries<C>(S, lo, bound, limit, wave, lane, entry);
+      const uint64_t r = chain_entries<C>((lds<Sh<C>> *)&S, lo, bound, limit, wave, entry);
+      valid = uni((uint32_t)(r >> 32));
+      entry = (uint32_t)r;
       if (valid < C::kThreads / 4) hard = kHardNo;
       q = entry;
       stop = false;
@@ -1045,7 +1050,7 @@ __device__ __forceinline__ int32_t span(const uint32_t *w, uint32_t nw, uint32_t
       for (int k = 0; k < C::kSub; k++) {
         sq[k] = q;
         n = 0;
-        if (!stop) stop = run_tokens<C, true>(S, q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
+        if (!stop) stop = run_tokens<C, true>(&S.stage[0], &S.tab[0], q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
         sn[k] = n;
       }
       break;
@@ -1064,7 +1069,7 @@ __device__ __forceinline__ int32_t span(const uint32_t *w, uint32_t nw, uint32_t
         if (!met) {
           sq[k] = q;
           n = 0;
-          if (!stop) stop = run_tokens<C, true>(S, q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
+          if (!stop) stop = run_tokens<C, true>(&S.stage[0], &S.tab[0], q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
           sn[k] = n;
         }
       }
@@ -1459,7 +1464,7 @@ inflate_chunks_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
   inflate_chunk<One>(comp, comp_bytes, off, chunk_bytes, out, out_len, status, flags, S);
 }
 
-__global__ void __launch_bounds__(Many::kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(Many::kThreads)
 inflate_chunks_many_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
                            const uint64_t *__restrict__ off, uint64_t chunk_bytes, uint8_t *out,
                            uint64_t *__restrict__ out_len, int32_t *__restrict__ status, uint32_t flags) {
@@ -1556,7 +1561,7 @@ inflate_batch_kernel(const codag_stream_desc *__restrict__ descs, uint64_t n,
   inflate_batch<One>(descs, n, results, flags, q, S);
 }
 
-__global__ void __launch_bounds__(Many::kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(Many::kThreads)
 inflate_batch_many_kernel(const codag_stream_desc *__restrict__ descs, uint64_t n,
                           codag_stream_result *__restrict__ results, uint32_t flags, BatchQueue *q) {
   __shared__ Sh<Many> S;
