@@ -60,6 +60,7 @@ struct codag_ctx {
   uint32_t cu_count = 0;
   char name[256] = {0};
   codag_tune_params tune[4];
+  bool tuned[4] = {};  // the shape was set or tuned by the caller
   uint32_t chunks_two_wave = 0;
   uint32_t poll_shift = 0;  // RLE v2 queue kernel: nonzero = waits without polls (tests)
 };
@@ -254,10 +255,17 @@ codag_status codag_rlev2_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t 
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "rlev2_decode: too many chunks");
   DeviceGuard g(ctx->device);
   const codag_tune_params &t = ctx->tune[CODAG_RLEV2];
+  // Expander waves per chunk, unless the caller chose a shape: a chunk's time is
+  // its expansion's while the CUs have wave slots left, so three up to 6 chunks
+  // per CU and two up to 12 (1, 2 and 3 expanders, us: 16-bit table column, 32
+  // chunks 1181, 648, 499, 1024 chunks 2276, 1276, 1051; 32-bit benchmark
+  // column, 1024 chunks 254, 249, 249, 2048 chunks 342, 317, 321).
+  uint32_t nexp = t.threads_per_group / 64 - 1;
+  if (!ctx->tuned[CODAG_RLEV2])
+    nexp = n_chunks <= 6ull * ctx->cu_count ? 3 : (n_chunks <= 12ull * ctx->cu_count ? 2 : 1);
   if (v2_pc_shape(t))  // walker wave + expander waves per chunk
     HIP_TRY(launch_rlev2_pc(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
-                            d_out, d_status, t.threads_per_group / 64 - 1, ctx->poll_shift,
-                            pick(ctx, stream)));
+                            d_out, d_status, nexp, ctx->poll_shift, pick(ctx, stream)));
   else if (t.threads_per_group == 64)  // one self-contained wave per chunk
     HIP_TRY(launch_rlev2_wave(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                               d_out, d_status, t.window_bytes, pick(ctx, stream)));
@@ -746,6 +754,7 @@ codag_status codag_tune_set(codag_ctx *ctx, codag_codec codec, const codag_tune_
   if (codec == CODAG_DEFLATE && p->threads_per_group != 64 && p->threads_per_group != 128)
     return fail(CODAG_ERR_INVALID, "tune_set: Deflate threads_per_group must be 64 or 128");
   ctx->tune[codec] = *p;
+  ctx->tuned[codec] = true;
   return CODAG_OK;
 }
 
@@ -775,6 +784,8 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
     for (auto &sh : shapes) cands.push_back({sh[0], sh[1], 0, 0});
   }
   const codag_tune_params saved = ctx->tune[codec];
+  const bool was_tuned = ctx->tuned[codec];
+  ctx->tuned[codec] = true;
   const uint64_t out_bytes = n_chunks * chunk_bytes;
   std::vector<uint8_t> ref, cur;
   float bestt = 1e30f, saved_ms = 0;
@@ -812,6 +823,7 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
     codag_status s = run();  // warm-up
     if (s) {
       ctx->tune[codec] = saved;
+      ctx->tuned[codec] = was_tuned;
       return s;
     }
     HIP_TRY(hipEventRecord(ctx->ev0, ctx->stream));
@@ -839,6 +851,7 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
     bestt = saved_ms;
   }
   ctx->tune[codec] = bestp;
+  ctx->tuned[codec] = true;
   if (best) *best = bestp;
   if (best_ms) *best_ms = bestt;
   return CODAG_OK;
