@@ -45,23 +45,6 @@ constexpr int32_t kTrunc = CODAG_CHUNK_TRUNCATED;
 constexpr int32_t kOverflow = CODAG_CHUNK_OVERFLOW;
 constexpr int32_t kCorrupt = CODAG_CHUNK_CORRUPT;
 
-// LDS input window: 64 lanes x 16 bytes from the 16-byte aligned address at
-// or below the first unconsumed stream byte (`lead` bytes before it).
-constexpr uint32_t kWin = 1024;
-// Header bytes the walk reads lie in window bytes [0, kHead): two VGPRs.
-constexpr uint32_t kHead = 512;
-// Output ring. LZSS needs the last 2047 bytes as history plus one batch.
-constexpr uint32_t kRing = 4096;
-constexpr uint32_t kRingMask = kRing - 1;
-// Batch output limits: BRLE has no history, LZSS keeps 2047 bytes of it.
-// Both leave the < 16 bytes a flush keeps back intact.
-constexpr uint32_t kBrleBatch = kRing - 32;
-static_assert(kHead + 130 <= kWin && kHead + 17 <= kWin, "items must end inside the window");
-
-// old with lane j's value replaced by the uniform v
-__device__ __forceinline__ uint32_t wrlane(uint32_t old, uint32_t v, uint32_t j) {
-  return lane_id() == j ? v : old;
-}
 // ------------------------------------------------------------------ input
 
 // Stream bytes [at, at + kWin - lead) as one 16-byte load per lane. A block
@@ -89,53 +72,6 @@ __device__ __forceinline__ Window window_load(const uint8_t *base, uint32_t len,
   return w;
 }
 
-// Header byte at window index q < kHead from the VGPR copies of window bytes
-// [0, 256) (h0) and [256, 512) (h1); q is wave-uniform.
-__device__ __forceinline__ uint32_t head_byte(uint32_t h0, uint32_t h1, uint32_t q) {
-  const uint32_t l = (q >> 2) & 63u;
-  const uint32_t d0 = rdlane(h0, l), d1 = rdlane(h1, l);
-  return ((q < 256u ? d0 : d1) >> ((q & 3u) * 8u)) & 0xffu;
-}
-
-// ------------------------------------------------------------------ output
-
-// Byte x of the chunk's output sits at ring[(x + mis) & kRingMask], mis =
-// dst & 15, so 16-byte aligned output addresses are 16-byte aligned in LDS.
-struct Out {
-  uint8_t *dst;
-  uint8_t *ring;
-  uint32_t cap;
-  uint32_t pos;      // bytes produced
-  uint32_t flushed;  // bytes [0, flushed) are in HBM
-  uint32_t mis;
-};
-
-__device__ __forceinline__ uint32_t ridx(const Out &o, uint32_t x) { return (x + o.mis) & kRingMask; }
-
-// Stores ring bytes [flushed, end) to HBM: single bytes up to a 16-byte
-// aligned address, then 16-byte vectors; `last` also writes the tail,
-// otherwise fewer than 16 bytes stay behind.
-__device__ __forceinline__ void out_store(Out &o, uint32_t lane, uint32_t end, bool last) {
-  uint32_t x = o.flushed;
-  uint32_t head = (16u - ((o.mis + x) & 15u)) & 15u;
-  if (head > end - x) head = end - x;
-  if (head) {
-    if (lane < head) o.dst[x + lane] = o.ring[ridx(o, x + lane)];
-    x += head;
-  }
-  const uint32_t nvec = (end - x) / 16u;
-  for (uint32_t k = lane; k < nvec; k += kWave) {
-    const uint32_t at = x + 16u * k;
-    *reinterpret_cast<uint4 *>(o.dst + at) = *reinterpret_cast<const uint4 *>(o.ring + ridx(o, at));
-  }
-  x += nvec * 16u;
-  if (last && x < end) {
-    if (lane < end - x) o.dst[x + lane] = o.ring[ridx(o, x + lane)];
-    x = end;
-  }
-  o.flushed = x;
-}
-
 __device__ __forceinline__ void chunk_bounds(const uint64_t lo, const uint64_t hi, uint64_t comp_bytes,
                                              uint64_t &len, int32_t &st) {
   st = kOk;
@@ -146,153 +82,305 @@ __device__ __forceinline__ void chunk_bounds(const uint64_t lo, const uint64_t h
 
 // ------------------------------------------------------------------ BRLE
 
-// Two waves per chunk, in lockstep (one workgroup barrier per batch): wave 0
-// walks batch i (window staging, header chain, item checks, output offsets)
-// while wave 1 writes batch i-1 into the ring and stores it to HBM. The walk
-// is scalar-bound and the writing vector/LDS-bound, so the two overlap, and a
-// 4096-chunk launch fills all 32 wave slots of a CU instead of 16. Batch i
-// uses window buffer i % 3 (the writer still reads i-1's literal bytes while
-// the walker stages i) and descriptor buffer i % 2.
-struct __align__(16) BrleLds2 {
-  uint8_t ring[kRing];
-  uint8_t win[3][kWin];
-  uint32_t item[2][kWave];  // header index | batch output offset << 16
-  uint32_t nk[2];           // items in the batch
-  uint32_t base[2];         // output position of the batch's first byte
-  uint32_t last;            // the walker's last batch (kNoLast while walking)
-};
-constexpr uint32_t kNoLast = 0xffffffffu;
+// Four waves per chunk. A step takes 253 blocks of 64 stream bytes, one per lane:
+//  * Item starts. Every lane walks its block from a guessed start (its first
+//    byte) and keeps the starts it passes in a 64-bit mask. Each lane's exit is
+//    then its successor's entry: a lane whose entry changed walks on from there
+//    until it meets a start of its mask, where its former path, and exit, hold
+//    again. Walks from a wrong start meet the right one soon (within two or three
+//    items in text with runs); where they never do, one block is put right per
+//    pass and the walk is the chain through the headers that it was before.
+//  * Each wave lists its items, with output offsets from a prefix sum, and makes
+//    its output in an LDS window: an item marks its first whole dword, a prefix
+//    maximum hands each dword its item and one load its bytes; the up to three
+//    bytes before and behind an item's whole dwords are then written by item.
+// One wave's walk by readlane took about 250 cycles an item, with a second wave
+// writing: 256 KiB chunks of runs and text, before and now: @@.
+// 16 bytes a lane and vector instructions bound it now, about half in the walk.
+constexpr int kBrWaves = 4;
+constexpr uint32_t kBrThreads = kBrWaves * kWave;
+constexpr uint32_t kBrBlock = 64, kBrLoads = 4;
+constexpr uint32_t kBrStage = kBrThreads * kBrLoads * 16;
+constexpr uint32_t kBrStep = kBrStage - 192;  // stream bytes in which a step's items begin
+constexpr uint32_t kBrList = 512;             // items listed at a time, per wave
+constexpr uint32_t kBrOut = 2048;             // a wave's output window
+static_assert(kBrThreads * kBrBlock >= kBrStep && 15 + kBrStep + 129 + 8 <= kBrStage,
+              "a lane per block; the last item lies in the stage");
 
-__global__ void __launch_bounds__(2 * kWave) brle_chunks2_kernel(const uint8_t *comp,
-                                                                 uint64_t comp_bytes,
+struct __align__(16) BrleLds {
+  uint8_t stage[kBrStage];
+  uint32_t list[kBrWaves][kBrList];  // literal << 31 | output offset in the wave << 12 | header
+  uint32_t out[kBrWaves][kBrOut / 4];
+  uint32_t exits[2][kBrWaves], entry[2][kBrWaves];
+  uint32_t part[kBrWaves];
+  uint32_t err;
+};
+constexpr uint32_t kBrSpan = kWave * kBrBlock;  // stream bytes of a wave
+static_assert(kBrSpan <= 4096 && kBrSpan / 2 * 130 < (1u << 19), "fields of a list entry");
+
+// Items [0, nb) of a wave's list, their headers counted from stage byte `first`.
+struct BrleItems {
+  const uint8_t *stage;
+  const uint32_t *list;
+  uint32_t first, nb;
+  struct Item {
+    uint32_t at, o, k;  // stage byte of the header, output offset, output bytes (0: none)
+    bool lit;
+  };
+  __device__ __forceinline__ Item get(uint32_t i) const {
+    const uint32_t x = list[min(i, nb - 1)];
+    Item t;
+    t.at = first + (x & 4095u);
+    t.lit = (int32_t)x < 0;
+    t.o = (x >> 12) & 0x7ffffu;
+    const uint32_t h = stage[t.at];
+    t.k = i < nb ? (t.lit ? h - 127u : h + 3u) : 0u;
+    return t;
+  }
+};
+
+// Writes the items, output offset 0 being byte o0 of dst, which is 16-byte
+// aligned, and their bytes [x0, x1).
+__device__ __forceinline__ void brle_write(uint8_t *dst, const BrleItems &it, uint32_t *ow, uint32_t o0, uint32_t x0,
+                                           uint32_t x1, uint32_t lane) {
+  uint8_t *ob = reinterpret_cast<uint8_t *>(ow);
+  const uint32_t *stage32 = reinterpret_cast<const uint32_t *>(it.stage);
+  uint32_t i0 = 0;  // the first item with bytes in the window
+  for (uint32_t w0 = x0 & ~15u; w0 < x1; w0 += kBrOut) {
+    const int32_t wn = (int32_t)min(kBrOut, x1 - w0);
+    const uint32_t ow0 = o0 - w0;
+#pragma unroll
+    for (uint32_t r = 0; r < kBrOut / 16; r += kWave) reinterpret_cast<uint4 *>(ow)[r + lane] = make_uint4(0, 0, 0, 0);
+    lds_order();
+    uint32_t i1 = i0;  // behind the window's items
+    for (;;) {
+      const BrleItems::Item t = it.get(i1 + lane);
+      const int32_t o = (int32_t)(ow0 + t.o), e = o + (int32_t)t.k;
+      const int32_t fd = max((o + 3) >> 2, 0), ed = min(e >> 2, (int32_t)(kBrOut / 4));
+      if (t.k && fd < ed) ow[fd] = i1 - i0 + lane + 1;
+      i1 += kWave;
+      if (i1 >= it.nb || (int32_t)rdlane((uint32_t)e, kWave - 1) >= wn) break;
+    }
+    lds_order();
+    // dwords: those not inside one item get bytes that the next loop replaces
+    uint32_t carry = 1;
+    for (int32_t r0 = 0; 4 * r0 < wn; r0 += 4 * kWave) {
+      uint32_t m[4], x[4], a[4], lo[4], hi[4];
+#pragma unroll
+      for (uint32_t r = 0; r < 4; r++) m[r] = ow[r0 + r * kWave + lane];
+#pragma unroll
+      for (uint32_t r = 0; r < 4; r++) {
+        m[r] = max(wave_max_dpp(m[r]), carry);
+        carry = rdlane(m[r], kWave - 1);
+      }
+#pragma unroll
+      for (uint32_t r = 0; r < 4; r++) x[r] = it.list[i0 + m[r] - 1];
+#pragma unroll
+      for (uint32_t r = 0; r < 4; r++) {
+        const uint32_t in_item = 4 * (r0 + r * kWave + lane) - ow0 - ((x[r] >> 12) & 0x7ffffu);
+        const int32_t b = (int32_t)(it.first + 1 + (x[r] & 4095u) + ((int32_t)x[r] < 0 ? in_item : 0u));
+        a[r] = (uint32_t)min(max(b, 0), (int32_t)kBrStage - 8);
+        lo[r] = stage32[a[r] >> 2];
+        hi[r] = stage32[(a[r] >> 2) + 1];
+      }
+#pragma unroll
+      for (uint32_t r = 0; r < 4; r++) {
+        const uint32_t v = __builtin_amdgcn_alignbyte(hi[r], lo[r], a[r] & 3u);
+        ow[r0 + r * kWave + lane] = (int32_t)x[r] < 0 ? v : __builtin_amdgcn_perm(0u, v, 0u);
+      }
+    }
+    lds_order();
+    for (uint32_t i = i0;; i += kWave) {
+      const BrleItems::Item t = it.get(i + lane);
+      const int32_t o = (int32_t)(ow0 + t.o), e = o + (int32_t)t.k;
+      const uint32_t step = t.lit ? 1u : 0u;
+      const int32_t hend = min((o + 3) & ~3, e), tbeg = max(e & ~3, hend);
+      if (o >= 0 && o < wn) {
+#pragma unroll
+        for (int32_t j = 0; j < 3; j++)
+          if (o + j < hend) ob[o + j] = it.stage[t.at + 1 + j * step];
+      }
+      if (tbeg >= 0 && tbeg < wn) {
+        const uint32_t s = t.at + 1 + (t.lit ? (uint32_t)(tbeg - o) : 0u);
+#pragma unroll
+        for (int32_t j = 0; j < 3; j++)
+          if (tbeg + j < e) ob[tbeg + j] = it.stage[s + j * step];
+      }
+      const uint64_t past = __ballot(t.k && e > (int32_t)kBrOut);
+      if (past || i + kWave >= i1) {
+        i0 = min(past ? i + (uint32_t)__builtin_ctzll(past) : i1, it.nb - 1);
+        break;
+      }
+    }
+    lds_order();
+    // whole vectors, then the bytes before and behind them
+#pragma unroll
+    for (uint32_t r = 0; r < kBrOut / 16; r += kWave) {
+      const uint32_t x = w0 + 16 * (r + lane);
+      if (x >= x0 && x + 16 <= x1) *reinterpret_cast<uint4 *>(dst + x) = reinterpret_cast<const uint4 *>(ow)[r + lane];
+    }
+    if (w0 < x0) {
+      const uint32_t x = w0 + lane;
+      if (lane < 16 && x >= x0 && x < x1) dst[x] = ob[lane];
+    }
+    const uint32_t xt = x1 & ~15u;
+    if (xt >= x0 && xt >= w0 && xt - w0 < kBrOut) {
+      const uint32_t x = xt + lane;
+      if (x < x1) dst[x] = ob[x - w0];
+    }
+    lds_order();
+  }
+}
+
+__global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
                                                                  const uint64_t *ptr, uint64_t n,
                                                                  uint64_t chunk_bytes, uint8_t *out,
                                                                  uint64_t *out_len, int32_t *status) {
-  __shared__ BrleLds2 S;
-  const uint32_t lane = lane_id();
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x) / kWave;
+  __shared__ BrleLds S;
+  const uint32_t lane = lane_id(), tid = threadIdx.x;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid) / kWave;
   const uint64_t ci = blockIdx.x;
   if (ci >= n) return;
   uint64_t len64;
   int32_t err;
   chunk_bounds(ptr[ci], ptr[ci + 1], comp_bytes, len64, err);
-  if (err != kOk) {  // both waves leave before any barrier
-    if (threadIdx.x == 0) {
+  if (err != kOk) {  // every wave leaves before any barrier
+    if (tid == 0) {
       if (out_len) out_len[ci] = 0;
       if (status) status[ci] = err;
     }
     return;
   }
   const uint8_t *src = comp + ptr[ci];
-  const uint32_t len = (uint32_t)len64;
+  const uint32_t len = (uint32_t)len64, cap = (uint32_t)chunk_bytes;
   uint8_t *dst = out + ci * chunk_bytes;
-  const uint32_t cap = (uint32_t)chunk_bytes;
-  if (threadIdx.x == 0) S.last = kNoLast;
-  __syncthreads();
-  // walker state
-  uint32_t at = 0, pos = 0;
-  Window w;
-  if (wave == 0) w = window_load(src, len, 0, lane);
-  // writer state
-  Out o;
-  o.dst = dst;
-  o.ring = S.ring;
-  o.cap = cap;
-  o.pos = 0;
-  o.flushed = 0;
-  o.mis = (uint32_t)(reinterpret_cast<uintptr_t>(dst) & 15u);
-  for (uint32_t i = 0;; i++) {
-    if (wave == 0 && uni(S.last) == kNoLast) {
-      uint8_t *win = S.win[i % 3];
-      reinterpret_cast<uint4 *>(win)[lane] = w.v;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-      const uint32_t lead = uni(w.lead);
-      const uint32_t h0 = reinterpret_cast<const uint32_t *>(win)[lane];
-      const uint32_t h1 = reinterpret_cast<const uint32_t *>(win)[kWave + lane];
-      const uint32_t qend = lead + (len - at);
-      const uint32_t qlim = min(qend, kHead);
-      uint32_t q = lead, nw = 0, iq = 0;
-      while (nw < (uint32_t)kWave && q < qlim) {
-        const uint32_t h = head_byte(h0, h1, q);
-        iq = wrlane(iq, q, nw);
-        nw++;
+  const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(dst) & 15u);
+  uint32_t at = 0, pos = 0, lead = 0;
+  uint4 v[kBrLoads];
+  auto load = [&](uint32_t from) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t k = 0; k < kBrLoads; k++) {
+      const Window w = window_load(src, len, from, k * kBrThreads + tid);
+      v[k] = w.v;
+      lead = uni(w.lead);
+    }
+  };
+  load(0);
+  while (at < len && err == kOk) {
+#pragma unroll
+    for (uint32_t k = 0; k < kBrLoads; k++) reinterpret_cast<uint4 *>(S.stage)[k * kBrThreads + tid] = v[k];
+    if (tid == 0) S.err = ~0u;
+    __syncthreads();
+    const uint32_t in0 = lead, left = len - at;
+    const uint8_t *in = S.stage + in0;  // stream byte `at`
+    const uint32_t lo = tid * kBrBlock, hi = min(lo + kBrBlock, min(left, kBrStep));
+    uint64_t mask = 0;  // the starts of the lane's items, from byte `from` on
+    uint32_t from = lo, exit = 0;
+    auto walk = [&]() __attribute__((always_inline)) {
+      uint64_t path = 0;
+      uint32_t q = from;
+      while (q < hi) {
+        const uint64_t bit = 1ull << (q - lo);
+        if (mask & bit) {
+          path |= mask & (0 - bit);
+          q = exit;
+          break;
+        }
+        path |= bit;
+        const uint32_t h = in[q];
         q += h > 127u ? h - 126u : 2u;
       }
-      const bool act = lane < nw;
-      const uint32_t hq = act ? (uint32_t)win[iq] : 0u;
-      const bool lit = hq > 127u;
-      const uint32_t k = act ? (lit ? hq - 127u : hq + 3u) : 0u;
-      const uint32_t inl = lit ? k + 1u : 2u;
-      const uint32_t incl = wave_scan_dpp(k);
-      const uint32_t bad = !act ? 0u : (iq + inl > qend ? 1u : (pos + incl > cap ? 2u : 0u));
-      const uint64_t stop = __ballot(bad != 0u || (act && incl > kBrleBatch));
-      uint32_t nk = nw;
-      if (stop) {
-        nk = (uint32_t)__builtin_ctzll(stop);
-        const uint32_t why = rdlane(bad, nk);
-        if (why) err = why == 1u ? kTrunc : kOverflow;
-        at += rdlane(iq, nk) - lead;
-      } else {
-        at += q - lead;
-      }
-      const uint32_t T = nk ? rdlane(incl, nk - 1u) : 0u;
-      S.item[i & 1][lane] = iq | ((incl - k) << 16);
-      if (lane == 0) {
-        S.nk[i & 1] = nk;
-        S.base[i & 1] = pos;
-        if (err != kOk || at >= len) S.last = i;
-      }
-      pos += T;
-      if (err == kOk && at < len) w = window_load(src, len, at, lane);
-    } else if (wave == 1 && i > 0) {
-      // write batch i-1
-      const uint32_t b = (i - 1) & 1;
-      const uint8_t *win = S.win[(i - 1) % 3];
-      const uint32_t nk = uni(S.nk[b]);
-      const uint32_t it = S.item[b][lane];
-      const uint32_t iq = it & 0xffffu, off = it >> 16;
-      const uint32_t kk0 = lane < nk ? (uint32_t)win[iq] : 0u;
-      const bool lit = kk0 > 127u;
-      const uint32_t kk = lane < nk ? (lit ? kk0 - 127u : kk0 + 3u) : 0u;
-      const uint32_t s0 = iq + 1u;
-      const uint32_t c = kk ? (uint32_t)win[s0] : 0u;
-      const uint32_t r0 = uni(S.base[b]) + off + o.mis;
-      const uint32_t hb = min((4u - (r0 & 3u)) & 3u, kk);
-#pragma unroll
-      for (uint32_t t = 0; t < 3u; t++)
-        if (t < hb) S.ring[(r0 + t) & kRingMask] = lit ? win[s0 + t] : (uint8_t)c;
-      const uint32_t nd = (kk - hb) >> 2;
-      const uint32_t c4 = c * 0x01010101u;
-      uint32_t *ring32 = reinterpret_cast<uint32_t *>(S.ring);
-      const uint32_t *win32 = reinterpret_cast<const uint32_t *>(win);
-      for (uint32_t d = 0; d < nd; d++) {
-        const uint32_t u = s0 + hb + 4u * d;
-        uint32_t v = c4;
-        if (lit) {
-          const uint32_t a = u >> 2;
-          v = __builtin_amdgcn_alignbit(win32[a + 1u], win32[a], (u & 3u) * 8u);
+      mask = path;
+      exit = q;
+    };
+    walk();
+    uint32_t entry = wave * kBrSpan, end;  // entry of the wave's first lane, exit of the step
+    for (uint32_t r = 0;; r ^= 1) {
+      for (;;) {
+        const uint32_t x0 = (uint32_t)__shfl_up((int)exit, 1, kWave);
+        const uint32_t x = lane == 0 ? entry : x0;
+        if (!__ballot(x != from)) break;
+        if (x != from) {
+          from = x;
+          walk();
         }
-        ring32[((r0 + hb + 4u * d) & kRingMask) >> 2] = v;
       }
-      const uint32_t tb = hb + 4u * nd;
+      if (lane == kWave - 1) {
+        S.exits[r][wave] = exit;
+        S.entry[r][wave] = entry;
+      }
+      __syncthreads();
+      bool all = true;
 #pragma unroll
-      for (uint32_t t = 0; t < 3u; t++)
-        if (tb + t < kk) S.ring[(r0 + tb + t) & kRingMask] = lit ? win[s0 + tb + t] : (uint8_t)c;
-      // the batch's last byte: the largest item end
-      uint32_t e = lane < nk ? off + kk : 0u;
+      for (int k = 1; k < kBrWaves; k++) {
+        const uint32_t x = uni(S.exits[r][k - 1]);
+        all = all && x == uni(S.entry[r][k]);
+        entry = k == (int)wave ? x : entry;
+      }
+      end = uni(S.exits[r][kBrWaves - 1]);
+      if (all) break;
+    }
+    if (end < left) load(at + end);
+    // output bytes and items, of the lane and before it
+    uint32_t n = 0;
+    for (uint64_t m = mask; m; m &= m - 1) {
+      const uint32_t h = in[lo + (uint32_t)__builtin_ctzll(m)];
+      n += h > 127u ? h - 127u : h + 3u;
+    }
+    uint32_t incl = wave_scan_dpp(n | (uint32_t)__builtin_popcountll(mask) << 20);
+    if (lane == kWave - 1) S.part[wave] = incl & 0xfffffu;
+    __syncthreads();
+    uint32_t base = 0, total = 0;
 #pragma unroll
-      for (uint32_t d = 32; d >= 1; d >>= 1) e = max(e, (uint32_t)__shfl_xor(e, (int)d, kWave));
-      o.pos = uni(S.base[b]) + uni(e);
-      out_store(o, lane, o.pos, false);
+    for (int k = 0; k < kBrWaves; k++) {
+      const uint32_t p = uni(S.part[k]);
+      base += k < (int)wave ? p : 0u;
+      total += p;
+    }
+    const uint32_t room = cap - pos;
+    if (end > left || total > room) {  // items from the first error on are left out
+      uint32_t o = base + (incl & 0xfffffu) - n;
+      n = 0;
+      for (uint64_t m = mask; m; m &= m - 1) {
+        const uint32_t q = lo + (uint32_t)__builtin_ctzll(m), h = in[q];
+        const uint32_t k = h > 127u ? h - 127u : h + 3u;
+        const uint32_t bad =
+            q + (h > 127u ? h - 126u : 2u) > left ? (uint32_t)kTrunc : (o + k > room ? (uint32_t)kOverflow : 0u);
+        if (bad) {
+          atomicMin(&S.err, o << 2 | bad);
+          mask &= (m & (0 - m)) - 1;
+          break;
+        }
+        o += k;
+        n += k;
+      }
+      incl = wave_scan_dpp(n | (uint32_t)__builtin_popcountll(mask) << 20);
+    }
+    const uint32_t items = rdlane(incl, kWave - 1) >> 20;
+    const uint32_t o0 = pos + base + mis;
+    BrleItems it{S.stage, S.list[wave], in0 + wave * kBrSpan, 0};
+    for (uint32_t b0 = 0; b0 < items; b0 += kBrList) {
+      uint32_t i = (incl >> 20) - (uint32_t)__builtin_popcountll(mask) - b0;
+      uint32_t o = (incl & 0xfffffu) - n;
+      for (uint64_t m = mask; m; m &= m - 1, i++) {
+        const uint32_t q = lo + (uint32_t)__builtin_ctzll(m), h = in[q];
+        if (i < kBrList) S.list[wave][i] = (h & 0x80u) << 24 | o << 12 | (q - wave * kBrSpan);
+        o += h > 127u ? h - 127u : h + 3u;
+      }
+      lds_order();
+      it.nb = min(items - b0, kBrList);
+      const uint32_t f = uni(it.get(0).o);
+      const BrleItems::Item l = it.get(it.nb - 1);
+      brle_write(dst - mis, it, S.out[wave], o0, o0 + f, o0 + uni(l.o + l.k), lane);
     }
     __syncthreads();
-    const uint32_t last = uni(S.last);
-    if (last != kNoLast && i >= last + 1u) break;
+    const uint32_t es = uni(S.err);
+    if (es != ~0u) err = (int32_t)(es & 3u);
+    pos += es != ~0u ? es >> 2 : total;
+    at += end;
+    __syncthreads();
   }
-  if (wave == 1) out_store(o, lane, o.pos, true);
-  if (wave == 0 && lane == 0) {
+  if (tid == 0) {
     if (out_len) out_len[ci] = pos;
     if (status) status[ci] = err;
   }
@@ -518,7 +606,7 @@ hipError_t launch_brle_chunks(const uint8_t *comp, uint64_t comp_bytes, const ui
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
                               int32_t *status, hipStream_t stream) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(bytecodec::brle_chunks2_kernel, dim3((uint32_t)n), dim3(2 * kWaveSize), 0,
+  hipLaunchKernelGGL(bytecodec::brle_chunks_kernel, dim3((uint32_t)n), dim3(bytecodec::kBrThreads), 0,
                      stream, comp, comp_bytes, ptr, n, chunk_bytes, out, out_len, status);
   return hipGetLastError();
 }
