@@ -82,7 +82,7 @@ __device__ __forceinline__ void chunk_bounds(const uint64_t lo, const uint64_t h
 
 // ------------------------------------------------------------------ BRLE
 
-// Four waves per chunk. A step takes 253 blocks of 64 stream bytes, one per lane:
+// Four waves per chunk. A step takes 256 blocks of 60 stream bytes, one per lane:
 //  * Item starts. Every lane walks its block from a guessed start (its first
 //    byte) and keeps the starts it passes in a 64-bit mask. Each lane's exit is
 //    then its successor's entry: a lane whose entry changed walks on from there
@@ -99,13 +99,15 @@ __device__ __forceinline__ void chunk_bounds(const uint64_t lo, const uint64_t h
 // 16 bytes a lane and vector instructions bound it now, about half in the walk.
 constexpr int kBrWaves = 4;
 constexpr uint32_t kBrThreads = kBrWaves * kWave;
-constexpr uint32_t kBrBlock = 64, kBrLoads = 4;
-constexpr uint32_t kBrStage = kBrThreads * kBrLoads * 16;
-constexpr uint32_t kBrStep = kBrStage - 192;  // stream bytes in which a step's items begin
+// 15 dwords: lanes at the same byte of their blocks read different LDS banks
+constexpr uint32_t kBrBlock = 60;
+typedef uint64_t blockmask_t;
+constexpr uint32_t kBrStep = kBrThreads * kBrBlock;  // stream bytes in which a step's items begin
+constexpr uint32_t kBrStage = (15 + kBrStep + 129 + 8 + 15) & ~15u;
+constexpr uint32_t kBrLoads = (kBrStage + kBrThreads * 16 - 1) / (kBrThreads * 16);
 constexpr uint32_t kBrList = 512;             // items listed at a time, per wave
 constexpr uint32_t kBrOut = 2048;             // a wave's output window
-static_assert(kBrThreads * kBrBlock >= kBrStep && 15 + kBrStep + 129 + 8 <= kBrStage,
-              "a lane per block; the last item lies in the stage");
+static_assert(kBrBlock <= 64, "the starts of a block in 64 bits");
 
 struct __align__(16) BrleLds {
   uint8_t stage[kBrStage];
@@ -153,13 +155,14 @@ __device__ __forceinline__ void brle_write(uint8_t *dst, const BrleItems &it, ui
     for (uint32_t r = 0; r < kBrOut / 16; r += kWave) reinterpret_cast<uint4 *>(ow)[r + lane] = make_uint4(0, 0, 0, 0);
     lds_order();
     uint32_t i1 = i0;  // behind the window's items
+    BrleItems::Item t = it.get(i0 + lane);  // kept for the loop after the next
     for (;;) {
-      const BrleItems::Item t = it.get(i1 + lane);
       const int32_t o = (int32_t)(ow0 + t.o), e = o + (int32_t)t.k;
       const int32_t fd = max((o + 3) >> 2, 0), ed = min(e >> 2, (int32_t)(kBrOut / 4));
       if (t.k && fd < ed) ow[fd] = i1 - i0 + lane + 1;
       i1 += kWave;
       if (i1 >= it.nb || (int32_t)rdlane((uint32_t)e, kWave - 1) >= wn) break;
+      t = it.get(i1 + lane);
     }
     lds_order();
     // dwords: those not inside one item get bytes that the next loop replaces
@@ -191,21 +194,23 @@ __device__ __forceinline__ void brle_write(uint8_t *dst, const BrleItems &it, ui
     }
     lds_order();
     for (uint32_t i = i0;; i += kWave) {
-      const BrleItems::Item t = it.get(i + lane);
+      if (i1 - i0 > kWave) t = it.get(i + lane);
       const int32_t o = (int32_t)(ow0 + t.o), e = o + (int32_t)t.k;
-      const uint32_t step = t.lit ? 1u : 0u;
       const int32_t hend = min((o + 3) & ~3, e), tbeg = max(e & ~3, hend);
-      if (o >= 0 && o < wn) {
+      // the bytes from the item's first one on, and from its byte tbeg on
+      const uint32_t ha = t.at + 1, ta = ha + (t.lit ? (uint32_t)(tbeg - o) : 0u);
+      const uint32_t h0 = stage32[ha >> 2], h1 = stage32[(ha >> 2) + 1];
+      const uint32_t t0 = stage32[ta >> 2], t1 = stage32[(ta >> 2) + 1];
+      uint32_t hv = __builtin_amdgcn_alignbyte(h1, h0, ha & 3u), tv = __builtin_amdgcn_alignbyte(t1, t0, ta & 3u);
+      hv = t.lit ? hv : __builtin_amdgcn_perm(0u, hv, 0u);
+      tv = t.lit ? tv : __builtin_amdgcn_perm(0u, tv, 0u);
+      const int32_t hn = o >= 0 && o < wn ? hend - o : 0, tn = tbeg >= 0 && tbeg < wn ? e - tbeg : 0;
 #pragma unroll
-        for (int32_t j = 0; j < 3; j++)
-          if (o + j < hend) ob[o + j] = it.stage[t.at + 1 + j * step];
-      }
-      if (tbeg >= 0 && tbeg < wn) {
-        const uint32_t s = t.at + 1 + (t.lit ? (uint32_t)(tbeg - o) : 0u);
+      for (int32_t j = 0; j < 3; j++)
+        if (j < hn) ob[o + j] = (uint8_t)(hv >> 8 * j);
 #pragma unroll
-        for (int32_t j = 0; j < 3; j++)
-          if (tbeg + j < e) ob[tbeg + j] = it.stage[s + j * step];
-      }
+      for (int32_t j = 0; j < 3; j++)
+        if (j < tn) ob[tbeg + j] = (uint8_t)(tv >> 8 * j);
       const uint64_t past = __ballot(t.k && e > (int32_t)kBrOut);
       if (past || i + kWave >= i1) {
         i0 = min(past ? i + (uint32_t)__builtin_ctzll(past) : i1, it.nb - 1);
@@ -258,43 +263,64 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
   uint32_t at = 0, pos = 0, lead = 0;
   uint4 v[kBrLoads];
   auto load = [&](uint32_t from) __attribute__((always_inline)) {
+    lead = (uint32_t)(reinterpret_cast<uintptr_t>(src) + from) & 15u;
 #pragma unroll
     for (uint32_t k = 0; k < kBrLoads; k++) {
-      const Window w = window_load(src, len, from, k * kBrThreads + tid);
-      v[k] = w.v;
-      lead = uni(w.lead);
+      const uint32_t i = k * kBrThreads + tid;
+      if (i < kBrStage / 16) v[k] = window_load(src, len, from, i).v;
     }
   };
   load(0);
   while (at < len && err == kOk) {
 #pragma unroll
-    for (uint32_t k = 0; k < kBrLoads; k++) reinterpret_cast<uint4 *>(S.stage)[k * kBrThreads + tid] = v[k];
+    for (uint32_t k = 0; k < kBrLoads; k++) {
+      const uint32_t i = k * kBrThreads + tid;
+      if (i < kBrStage / 16) reinterpret_cast<uint4 *>(S.stage)[i] = v[k];
+    }
     if (tid == 0) S.err = ~0u;
     __syncthreads();
-    const uint32_t in0 = lead, left = len - at;
-    const uint8_t *in = S.stage + in0;  // stream byte `at`
-    const uint32_t lo = tid * kBrBlock, hi = min(lo + kBrBlock, min(left, kBrStep));
-    uint64_t mask = 0;  // the starts of the lane's items, from byte `from` on
-    uint32_t from = lo, exit = 0;
+    // positions are stage bytes from here on; the stream's next byte is in0, and
+    // it ends at `limit`
+    const uint8_t *in = S.stage;
+    const uint32_t in0 = lead, limit = in0 + (len - at);
+    const uint32_t lo = tid * kBrBlock, hi = min(lo + kBrBlock, limit);
+    // the block's bytes above 128; every other header is two bytes before the next
+    blockmask_t jumps = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kBrBlock / 4; k++) {
+      const uint32_t d = reinterpret_cast<const uint32_t *>(in + lo)[k];
+      const uint32_t t = ((d & 0x7f7f7f7fu) + 0x7f7f7f7fu) & d & 0x80808080u;
+      jumps |= (blockmask_t)__builtin_amdgcn_udot4(t >> 7, 0x08040201u, 0u, false) << (4 * k);
+    }
+    blockmask_t mask = 0;  // the starts of the lane's items, from byte `from` on
+    uint32_t from = wave == 0 && lane == 0 ? in0 : lo, exit = 0;
     auto walk = [&]() __attribute__((always_inline)) {
-      uint64_t path = 0;
+      const blockmask_t old = mask, every2 = (blockmask_t)0x5555555555555555ull;
+      mask = 0;
       uint32_t q = from;
       while (q < hi) {
-        const uint64_t bit = 1ull << (q - lo);
-        if (mask & bit) {
-          path |= mask & (0 - bit);
+        // steps of two up to and with the next byte above 128, or the block's end
+        const blockmask_t path = (every2 << (q - lo)) & (((blockmask_t)1 << (hi - lo)) - 1), j = path & jumps;
+        const blockmask_t p = path & (j ^ (j - 1));
+        const blockmask_t met = p & old;
+        if (met) {
+          const blockmask_t bit = met & (0 - met);
+          mask |= (p & (bit - 1)) | (old & (0 - bit));
           q = exit;
           break;
         }
-        path |= bit;
-        const uint32_t h = in[q];
-        q += h > 127u ? h - 126u : 2u;
+        mask |= p;
+        if (!j) {
+          q = hi + ((q ^ hi) & 1u);
+        } else {
+          q = lo + (uint32_t)__builtin_ctzll(j);
+          q += in[q] - 126u;
+        }
       }
-      mask = path;
       exit = q;
     };
     walk();
-    uint32_t entry = wave * kBrSpan, end;  // entry of the wave's first lane, exit of the step
+    uint32_t entry = wave ? wave * kBrSpan : in0, end;  // entry of the wave's first lane, exit of the step
     for (uint32_t r = 0;; r ^= 1) {
       for (;;) {
         const uint32_t x0 = (uint32_t)__shfl_up((int)exit, 1, kWave);
@@ -320,10 +346,10 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
       end = uni(S.exits[r][kBrWaves - 1]);
       if (all) break;
     }
-    if (end < left) load(at + end);
+    if (end < limit) load(at + (end - in0));
     // output bytes and items, of the lane and before it
     uint32_t n = 0;
-    for (uint64_t m = mask; m; m &= m - 1) {
+    for (blockmask_t m = mask; m; m &= m - 1) {
       const uint32_t h = in[lo + (uint32_t)__builtin_ctzll(m)];
       n += h > 127u ? h - 127u : h + 3u;
     }
@@ -338,14 +364,14 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
       total += p;
     }
     const uint32_t room = cap - pos;
-    if (end > left || total > room) {  // items from the first error on are left out
+    if (end > limit || total > room) {  // items from the first error on are left out
       uint32_t o = base + (incl & 0xfffffu) - n;
       n = 0;
-      for (uint64_t m = mask; m; m &= m - 1) {
+      for (blockmask_t m = mask; m; m &= m - 1) {
         const uint32_t q = lo + (uint32_t)__builtin_ctzll(m), h = in[q];
         const uint32_t k = h > 127u ? h - 127u : h + 3u;
         const uint32_t bad =
-            q + (h > 127u ? h - 126u : 2u) > left ? (uint32_t)kTrunc : (o + k > room ? (uint32_t)kOverflow : 0u);
+            q + (h > 127u ? h - 126u : 2u) > limit ? (uint32_t)kTrunc : (o + k > room ? (uint32_t)kOverflow : 0u);
         if (bad) {
           atomicMin(&S.err, o << 2 | bad);
           mask &= (m & (0 - m)) - 1;
@@ -358,11 +384,11 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
     }
     const uint32_t items = rdlane(incl, kWave - 1) >> 20;
     const uint32_t o0 = pos + base + mis;
-    BrleItems it{S.stage, S.list[wave], in0 + wave * kBrSpan, 0};
+    BrleItems it{S.stage, S.list[wave], wave * kBrSpan, 0};
     for (uint32_t b0 = 0; b0 < items; b0 += kBrList) {
       uint32_t i = (incl >> 20) - (uint32_t)__builtin_popcountll(mask) - b0;
       uint32_t o = (incl & 0xfffffu) - n;
-      for (uint64_t m = mask; m; m &= m - 1, i++) {
+      for (blockmask_t m = mask; m; m &= m - 1, i++) {
         const uint32_t q = lo + (uint32_t)__builtin_ctzll(m), h = in[q];
         if (i < kBrList) S.list[wave][i] = (h & 0x80u) << 24 | o << 12 | (q - wave * kBrSpan);
         o += h > 127u ? h - 127u : h + 3u;
@@ -377,7 +403,7 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
     const uint32_t es = uni(S.err);
     if (es != ~0u) err = (int32_t)(es & 3u);
     pos += es != ~0u ? es >> 2 : total;
-    at += end;
+    at += end - in0;
     __syncthreads();
   }
   if (tid == 0) {
