@@ -15,14 +15,12 @@
 //         into out + i * chunk (128 KiB, lzss.h:21).
 //
 // Both formats are sequences of byte-aligned items whose sizes follow from
-// one header byte (BRLE) or one flag byte per eight items (LZSS). BRLE finds
-// a batch by a scalar walk over header bytes that sit in two VGPRs
-// (v_readlane, no memory round trip per step), each lane then takes one
-// item, and the batch's output is assembled in an LDS ring and stored to HBM
-// as 16-byte aligned vectors; two waves per chunk, the walking wave one batch
-// ahead of the writing wave. LZSS walks several parts of a chunk at once from
-// every byte a group may begin at and resolves its output in an LDS window of
-// marks; four waves per chunk. The next input window is loaded meanwhile.
+// one header byte (BRLE) or one flag byte per eight items (LZSS). Both decoders
+// take a chunk by four waves and find the item starts of many parts of the
+// stream at once: BRLE by walks from guessed starts that are put right until
+// they agree, LZSS from every byte a group may begin at. BRLE's output is made
+// from its items dword by dword, LZSS's resolved in an LDS window of marks. The
+// next part of the stream is loaded meanwhile.
 //
 // The reference checks nothing; these kernels report per chunk: TRUNCATED if
 // the stream ends inside an item, OVERFLOW if the output would pass the
@@ -83,25 +81,29 @@ __device__ __forceinline__ void chunk_bounds(const uint64_t lo, const uint64_t h
 // ------------------------------------------------------------------ BRLE
 
 // Four waves per chunk. A step takes 256 blocks of 60 stream bytes, one per lane:
-//  * Item starts. Every lane walks its block from a guessed start (its first
-//    byte) and keeps the starts it passes in a 64-bit mask. Each lane's exit is
-//    then its successor's entry: a lane whose entry changed walks on from there
-//    until it meets a start of its mask, where its former path, and exit, hold
-//    again. Walks from a wrong start meet the right one soon (within two or three
-//    items in text with runs); where they never do, one block is put right per
-//    pass and the walk is the chain through the headers that it was before.
+//  * Item starts. Only a header above 128 moves on by more than two bytes, so a
+//    walk visits every second byte up to the next such byte: one mask operation
+//    and one header read per long literal, not one per item. Every lane walks its
+//    block from a guessed start (its first byte) and keeps the starts it passes
+//    in a mask. Each lane's exit is then its successor's entry: a lane whose
+//    entry changed walks on from there until it meets a start of its mask, where
+//    its former path, and exit, hold again. In runs and text wrong starts have
+//    met the right one after 40 bytes in the median and 390 at the 99th
+//    percentile, nine passes a step; where they never do, a pass puts one block
+//    right, and the walk is the chain through the headers that it was before.
 //  * Each wave lists its items, with output offsets from a prefix sum, and makes
 //    its output in an LDS window: an item marks its first whole dword, a prefix
 //    maximum hands each dword its item and one load its bytes; the up to three
 //    bytes before and behind an item's whole dwords are then written by item.
 // One wave's walk by readlane took about 250 cycles an item, with a second wave
-// writing: 256 KiB chunks of runs and text, before and now: @@.
-// 16 bytes a lane and vector instructions bound it now, about half in the walk.
+// writing. 1024 chunks of 256 KiB, runs and text: 861 us before, 277 now (item by
+// item through the headers 449; eight waves and blocks of 44 bytes 305, as walks
+// then meet over more lanes). It is bound by latency: a step takes 54 K cycles,
+// 21 K of them in the walks and 20 K in the output, with one chunk per CU or four.
 constexpr int kBrWaves = 4;
 constexpr uint32_t kBrThreads = kBrWaves * kWave;
 // 15 dwords: lanes at the same byte of their blocks read different LDS banks
 constexpr uint32_t kBrBlock = 60;
-typedef uint64_t blockmask_t;
 constexpr uint32_t kBrStep = kBrThreads * kBrBlock;  // stream bytes in which a step's items begin
 constexpr uint32_t kBrStage = (15 + kBrStep + 129 + 8 + 15) & ~15u;
 constexpr uint32_t kBrLoads = (kBrStage + kBrThreads * 16 - 1) / (kBrThreads * 16);
@@ -113,7 +115,7 @@ struct __align__(16) BrleLds {
   uint8_t stage[kBrStage];
   uint32_t list[kBrWaves][kBrList];  // literal << 31 | output offset in the wave << 12 | header
   uint32_t out[kBrWaves][kBrOut / 4];
-  uint32_t exits[2][kBrWaves], entry[2][kBrWaves];
+  uint32_t exits[2][kBrWaves], entry[2][kBrWaves], early[kBrWaves];
   uint32_t part[kBrWaves];
   uint32_t err;
 };
@@ -237,7 +239,8 @@ __device__ __forceinline__ void brle_write(uint8_t *dst, const BrleItems &it, ui
   }
 }
 
-__global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
+__global__ void __launch_bounds__(kBrThreads) __attribute__((amdgpu_waves_per_eu(5)))
+brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
                                                                  const uint64_t *ptr, uint64_t n,
                                                                  uint64_t chunk_bytes, uint8_t *out,
                                                                  uint64_t *out_len, int32_t *status) {
@@ -278,6 +281,7 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
       if (i < kBrStage / 16) reinterpret_cast<uint4 *>(S.stage)[i] = v[k];
     }
     if (tid == 0) S.err = ~0u;
+    if (tid < kBrWaves) S.early[tid] = (tid + 1) * kBrSpan;
     __syncthreads();
     // positions are stage bytes from here on; the stream's next byte is in0, and
     // it ends at `limit`
@@ -285,26 +289,26 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
     const uint32_t in0 = lead, limit = in0 + (len - at);
     const uint32_t lo = tid * kBrBlock, hi = min(lo + kBrBlock, limit);
     // the block's bytes above 128; every other header is two bytes before the next
-    blockmask_t jumps = 0;
+    uint64_t jumps = 0;
 #pragma unroll
     for (uint32_t k = 0; k < kBrBlock / 4; k++) {
       const uint32_t d = reinterpret_cast<const uint32_t *>(in + lo)[k];
       const uint32_t t = ((d & 0x7f7f7f7fu) + 0x7f7f7f7fu) & d & 0x80808080u;
-      jumps |= (blockmask_t)__builtin_amdgcn_udot4(t >> 7, 0x08040201u, 0u, false) << (4 * k);
+      jumps |= (uint64_t)__builtin_amdgcn_udot4(t >> 7, 0x08040201u, 0u, false) << (4 * k);
     }
-    blockmask_t mask = 0;  // the starts of the lane's items, from byte `from` on
+    uint64_t mask = 0;  // the starts of the lane's items, from byte `from` on
     uint32_t from = wave == 0 && lane == 0 ? in0 : lo, exit = 0;
     auto walk = [&]() __attribute__((always_inline)) {
-      const blockmask_t old = mask, every2 = (blockmask_t)0x5555555555555555ull;
+      const uint64_t old = mask, every2 = (uint64_t)0x5555555555555555ull;
       mask = 0;
       uint32_t q = from;
       while (q < hi) {
         // steps of two up to and with the next byte above 128, or the block's end
-        const blockmask_t path = (every2 << (q - lo)) & (((blockmask_t)1 << (hi - lo)) - 1), j = path & jumps;
-        const blockmask_t p = path & (j ^ (j - 1));
-        const blockmask_t met = p & old;
+        const uint64_t path = (every2 << (q - lo)) & (((uint64_t)1 << (hi - lo)) - 1), j = path & jumps;
+        const uint64_t p = path & (j ^ (j - 1));
+        const uint64_t met = p & old;
         if (met) {
-          const blockmask_t bit = met & (0 - met);
+          const uint64_t bit = met & (0 - met);
           mask |= (p & (bit - 1)) | (old & (0 - bit));
           q = exit;
           break;
@@ -323,8 +327,10 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
     uint32_t entry = wave ? wave * kBrSpan : in0, end;  // entry of the wave's first lane, exit of the step
     for (uint32_t r = 0;; r ^= 1) {
       for (;;) {
-        const uint32_t x0 = (uint32_t)__shfl_up((int)exit, 1, kWave);
-        const uint32_t x = lane == 0 ? entry : x0;
+        // what the wave before has now; the check below is made on final exits
+        if (lane == kWave - 1) __hip_atomic_store(&S.early[wave], exit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (wave) entry = uni(__hip_atomic_load(&S.early[wave - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        const uint32_t x = (uint32_t)__builtin_amdgcn_update_dpp((int)entry, (int)exit, 0x138, 0xf, 0xf, false);  // wave_shr:1
         if (!__ballot(x != from)) break;
         if (x != from) {
           from = x;
@@ -349,7 +355,7 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
     if (end < limit) load(at + (end - in0));
     // output bytes and items, of the lane and before it
     uint32_t n = 0;
-    for (blockmask_t m = mask; m; m &= m - 1) {
+    for (uint64_t m = mask; m; m &= m - 1) {
       const uint32_t h = in[lo + (uint32_t)__builtin_ctzll(m)];
       n += h > 127u ? h - 127u : h + 3u;
     }
@@ -367,7 +373,7 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
     if (end > limit || total > room) {  // items from the first error on are left out
       uint32_t o = base + (incl & 0xfffffu) - n;
       n = 0;
-      for (blockmask_t m = mask; m; m &= m - 1) {
+      for (uint64_t m = mask; m; m &= m - 1) {
         const uint32_t q = lo + (uint32_t)__builtin_ctzll(m), h = in[q];
         const uint32_t k = h > 127u ? h - 127u : h + 3u;
         const uint32_t bad =
@@ -388,7 +394,7 @@ __global__ void __launch_bounds__(kBrThreads) brle_chunks_kernel(const uint8_t *
     for (uint32_t b0 = 0; b0 < items; b0 += kBrList) {
       uint32_t i = (incl >> 20) - (uint32_t)__builtin_popcountll(mask) - b0;
       uint32_t o = (incl & 0xfffffu) - n;
-      for (blockmask_t m = mask; m; m &= m - 1, i++) {
+      for (uint64_t m = mask; m; m &= m - 1, i++) {
         const uint32_t q = lo + (uint32_t)__builtin_ctzll(m), h = in[q];
         if (i < kBrList) S.list[wave][i] = (h & 0x80u) << 24 | o << 12 | (q - wave * kBrSpan);
         o += h > 127u ? h - 127u : h + 3u;

@@ -1,5 +1,5 @@
-"""BRLE chunks at the edges of the decoder's steps (16192 stream bytes in blocks
-of 64), lists (512 items) and output windows (2048 bytes), against the oracle:
+"""BRLE chunks at the edges of the decoder's steps (15360 stream bytes in blocks
+of 60), lists (512 items) and output windows (2048 bytes), against the oracle:
 streams in which a walk from a wrong byte never meets the right one, items of
 one size throughout, and steps that end inside an item or at the chunk's end."""
 import numpy as np
@@ -10,7 +10,7 @@ from tests.gpu_helpers import say
 from tests.test_gpu_bytecodec import brle_container, compare
 
 pytestmark = pytest.mark.gpu
-STEP = 16384 - 192
+STEP = 256 * 60
 
 
 @pytest.fixture(scope="module")
@@ -50,7 +50,7 @@ def stream(kind, n, rng):
 def test_streams(ctx, kind, shift):
     say(f"brle parts, {kind}, shift {shift}")
     rng = np.random.default_rng(5)
-    sizes = [1, 63, 64, 65, 4096, STEP - 1, STEP, STEP + 1, 2 * STEP + 77]
+    sizes = [1, 59, 60, 61, 3840, STEP - 1, STEP, STEP + 1, 2 * STEP + 77]
     data, ptr = brle_container([stream(kind, n, rng) for n in sizes])
     compare(ctx, False, data, ptr, 1 << 20, shift)  # the longest streams of runs overflow
 
