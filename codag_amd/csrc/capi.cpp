@@ -255,15 +255,21 @@ codag_status codag_rlev2_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t 
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "rlev2_decode: too many chunks");
   DeviceGuard g(ctx->device);
   const codag_tune_params &t = ctx->tune[CODAG_RLEV2];
-  // Expander waves per chunk, unless the caller chose a shape: a chunk's time is
-  // its expansion's while the CUs have wave slots left, so three up to 6 chunks
-  // per CU and two up to 12 (1, 2 and 3 expanders, us: 16-bit table column, 32
-  // chunks 1181, 648, 499, 1024 chunks 2276, 1276, 1051; 32-bit benchmark
-  // column, 1024 chunks 254, 249, 249, 2048 chunks 342, 317, 321).
+  // Unless the caller chose a shape: 16 waves per chunk that walk and expand by
+  // turns while two such groups per CU hold all chunks, as a lone walker's chain
+  // then bounds the launch (walker and three expanders, then 16 waves, us: 16-bit
+  // table column, 64 chunks 917, 376, 512 chunks 1063, 486, 1024 chunks 1054, 807;
+  // 64-bit benchmark column, 512 chunks 153, 127, 1024 chunks 152, 232). Above that,
+  // expanders by the chunk count: three up to 6 chunks per CU and two up to 12
+  // (1, 2 and 3 expanders, us: 16-bit table column, 1024 chunks 2276, 1276, 1051;
+  // 32-bit benchmark column, 1024 chunks 254, 249, 249, 2048 chunks 342, 317, 321).
+  const bool chosen = ctx->tuned[CODAG_RLEV2];
   uint32_t nexp = t.threads_per_group / 64 - 1;
-  if (!ctx->tuned[CODAG_RLEV2])
-    nexp = n_chunks <= 6ull * ctx->cu_count ? 3 : (n_chunks <= 12ull * ctx->cu_count ? 2 : 1);
-  if (v2_pc_shape(t))  // walker wave + expander waves per chunk
+  if (!chosen) nexp = n_chunks <= 6ull * ctx->cu_count ? 3 : (n_chunks <= 12ull * ctx->cu_count ? 2 : 1);
+  if (!chosen && !ctx->poll_shift && n_chunks <= 2ull * ctx->cu_count)
+    HIP_TRY(launch_rlev2_span(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
+                              d_out, d_status, pick(ctx, stream)));
+  else if (v2_pc_shape(t))  // walker wave + expander waves per chunk
     HIP_TRY(launch_rlev2_pc(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                             d_out, d_status, nexp, ctx->poll_shift, pick(ctx, stream)));
   else if (t.threads_per_group == 64)  // one self-contained wave per chunk
@@ -810,6 +816,8 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
   }
   for (size_t ci = 0; ci < cands.size(); ci++) {
     ctx->tune[codec] = cands[ci];
+    // the shape in use runs as it is in use: one that nobody chose by chunk count
+    ctx->tuned[codec] = was_tuned || std::memcmp(&cands[ci], &saved, sizeof saved) != 0;
     auto run = [&]() -> codag_status {
       if (codec == CODAG_RLEV1)
         return codag_rlev1_decode(ctx, d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w,
@@ -851,7 +859,7 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
     bestt = saved_ms;
   }
   ctx->tune[codec] = bestp;
-  ctx->tuned[codec] = true;
+  ctx->tuned[codec] = was_tuned || std::memcmp(&bestp, &saved, sizeof saved) != 0;
   if (best) *best = bestp;
   if (best_ms) *best_ms = bestt;
   return CODAG_OK;

@@ -68,7 +68,13 @@ hipError_t launch_rlev2_pc(const uint8_t *comp, uint64_t comp_bytes, const uint6
                            uint64_t chunk_bytes, uint8_t *out, int32_t *status, uint32_t nexp,
                            uint32_t poll_shift, hipStream_t stream);
 
-// BRLE / LZSS, one wave64 per chunk (chunk_bytes < 2^31).
+// RLE v2, 16 waves per chunk that walk and expand by turns.
+hipError_t launch_rlev2_span(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *blk_off,
+                             const uint64_t *col_len, uint64_t n_chunks, uint32_t w,
+                             uint64_t chunk_bytes, uint8_t *out, int32_t *status,
+                             hipStream_t stream);
+
+// BRLE / LZSS, four waves per chunk (chunk_bytes < 2^31).
 hipError_t launch_brle_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ptr,
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
                               int32_t *status, hipStream_t stream);

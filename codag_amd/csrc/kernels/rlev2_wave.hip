@@ -15,13 +15,15 @@
 //     patch gaps for PATCHED_BASE).
 // A block that does not fit in the window restarts the window at that block.
 //
-// Two kernels share the walk and the expansion:
+// Three kernels share the expansion, the first two the walk:
 //   * rlev2_wave_kernel: one wave per chunk walks and expands in turn, with no
 //     workgroup barriers; several chunks share each SIMD to hide latency.
 //   * rlev2_pc_kernel: one walker wave and kExp expander waves per chunk. The
 //     walker publishes batches of block descriptors through a four-deep LDS
 //     queue and walks ahead while the expanders write earlier batches, so a
 //     chunk's time approaches max(walk, expand) instead of their sum.
+//   * rlev2_span_kernel: sixteen waves per chunk find the headers of many spans
+//     at once and expand by turns, for launches of few chunks.
 //
 // Semantics: include/rlev2/decoder_new.h:909-1187 (decoder_warp_orig_rdw).
 #include "kernels.hpp"
@@ -612,6 +614,285 @@ rlev2_pc_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
   }
 }
 
+// ---------------------------------------------------------------- spans by all waves
+
+// Walk and expansion by turns, both by every wave of a group of kSpWaves: a
+// step looks at the headers that may start at kSpPos stream bytes.
+//  * Each wave sizes the blocks of its kSpSpans spans of 64 positions (span_block)
+//    and composes them: pointer doubling by ds_bpermute leaves every position the
+//    first one outside its span that its chain reaches, a pass from the wave's
+//    last span to its first the first one outside the wave's. A position that
+//    span_block does not take is its own successor and ends the chain.
+//  * One link per wave then gives each wave its entry, and each wave follows its
+//    own spans by v_readlane.
+//  * A prefix sum over the group places the blocks; block j is expanded by wave
+//    j mod kSpWaves.
+// The block that ended the chain is looked at alone (one_block), as in walk_batch.
+// It is bound by latency: of 36 K cycles a step with eight waves, at one chunk per
+// CU or two, 13 K were the expansion and 7 K the sizing, both halved by 16 (16-bit
+// table column, 64 chunks: one walker and three expanders 917 us, eight waves 495,
+// 16 waves 376). It sizes every position, the lone walker only spans it enters, and
+// so falls behind where chunks fill the GPU without it.
+constexpr uint32_t kSpWaves = 16, kSpSpans = 4;
+constexpr uint32_t kSpThreads = kSpWaves * kWave;
+constexpr uint32_t kSpWavePos = kSpSpans * kWave, kSpPos = kSpWaves * kSpWavePos;
+constexpr uint32_t kMaxBlock = 2304;  // PATCHED_BASE: 12 header, 2040 value and 248 patch bytes
+constexpr uint32_t kNoPos = ~0u;
+constexpr uint32_t kSpWin = 16 + kSpPos + kMaxBlock + 16;
+static_assert(kSpWin <= 8192 && kSpWin / 16 <= kSpThreads, "packed descriptors, a 16-byte load per thread");
+
+struct SpanLds {
+  uint8_t sbuf[kSpWin + 288];
+  union {
+    uint16_t to[kSpPos];        // the first position outside its wave's that a position's chain reaches
+    uint32_t desc[kSpPos / 2];  // packed descriptors (put_desc); a block has two bytes at least
+  };
+  uint32_t values[kSpWaves], blocks[kSpWaves];
+  uint32_t ovf;  // the first block past the chunk's values
+  uint32_t bad;  // a patch outside its block
+};
+
+// The block at LDS offset p that span_block did not take: its size and value
+// count, or how the walk goes on without it. Same order of checks as walk_batch.
+enum : uint32_t { kOneBlock, kOneDone, kOneRestage, kOneError };
+__device__ __forceinline__ uint32_t one_block(const uint8_t *sbuf, uint32_t p, uint32_t P, bool at_end, uint32_t o,
+                                              uint32_t cap, uint32_t &size, uint32_t &cnt, int32_t &err) {
+  if (at_end && p >= P) return kOneDone;
+  if (!at_end && p > P - 32) return kOneRestage;
+  const uint32_t first = uni(sbuf[p]), second = uni(sbuf[p + 1]);
+  const uint32_t kind = first >> 6, code = (first >> 1) & 0x1f, fbw = decode_width(code);
+  const uint32_t len8 = (second + 1) & 0xff;
+  if (kind == 0) {
+    size = 2 + ((first >> 3) & 7);
+    cnt = (first & 7) + 3;
+  } else if (kind == 1) {
+    size = 2 + (len8 * fbw + 7) / 8;
+    cnt = len8;
+  } else if (kind == 3) {
+    const uint32_t nd8 = (len8 - 2) & 0xff;
+    auto varint = [&](uint32_t q) {
+      uint32_t n = 0;
+      while (q + n < P && uni(sbuf[q + n]) >= 0x80) n++;
+      return n + 1;
+    };
+    uint32_t q = p + 2;
+    const uint32_t l1 = varint(q), l2 = q + l1 < P ? varint(q + l1) : 1u;
+    if (q + l1 + l2 <= P && (l1 > 10 || l2 > 10)) {
+      err = kCorrupt;
+      return kOneError;
+    }
+    q += l1 + l2;
+    size = (q - p) + (code ? (nd8 * fbw + 7) / 8 : 0u);
+    cnt = 2 + nd8;
+  } else {
+    const uint32_t third = uni(sbuf[p + 2]), fourth = uni(sbuf[p + 3]);
+    const uint32_t pw = decode_width(third & 0x1f), pgw = (fourth >> 5) + 1;
+    if (pw + pgw > 64) {
+      err = kCorrupt;
+      return kOneError;
+    }
+    size = 4 + (third >> 5) + 1 + (len8 * fbw + 7) / 8 + ((fourth & 0x1f) * closest_fixed(pw + pgw) + 7) / 8;
+    cnt = len8;
+  }
+  if (p + size > P) {
+    err = kTrunc;
+    return at_end ? kOneError : kOneRestage;
+  }
+  if (o + cnt > cap) {
+    err = kOverflow;
+    return kOneError;
+  }
+  return kOneBlock;
+}
+
+// 64 registers: two groups per CU.
+template <uint32_t W>
+__global__ void __launch_bounds__(kSpThreads) __attribute__((amdgpu_waves_per_eu(8)))
+rlev2_span_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes, const uint64_t *__restrict__ blk_off,
+                  const uint64_t *__restrict__ col_len, uint64_t n_chunks, uint64_t chunk_bytes,
+                  uint8_t *__restrict__ out, int32_t *__restrict__ status) {
+  __shared__ __align__(16) SpanLds L;
+  const uint64_t chunk = blockIdx.x;
+  const uint32_t lane = lane_id(), tid = threadIdx.x;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const uint64_t boff = blk_off[chunk], len64 = col_len[chunk];
+  if (!chunk_ok(boff, len64, comp_bytes)) {  // uniform over the workgroup
+    if (tid == 0 && status) status[chunk] = kCorrupt;
+    return;
+  }
+  const uint8_t *src = comp + boff;
+  const uint32_t len = (uint32_t)len64, cap = (uint32_t)(chunk_bytes / W);
+  uint8_t *dst = out + chunk * chunk_bytes;
+  if (tid == 0) L.bad = 0;
+  uint32_t pos = 0, o = 0, bad = 0;  // stream position of the window, values produced
+  int32_t st = kOk;
+  uint4 pre = make_uint4(0, 0, 0, 0);
+  // only 16-byte blocks with a byte of [from, from + kSpWin - 16) of the stream are read
+  auto load = [&](uint32_t from) __attribute__((always_inline)) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(src + from), a0 = a & ~uintptr_t(15);
+    const uint32_t n = min(len - from, kSpWin - 16), blocks = ((uint32_t)(a - a0) + n + 15) / 16;
+    if (tid < blocks) pre = *reinterpret_cast<const uint4 *>(a0 + 16u * tid);
+  };
+  bool done = len == 0;
+  if (!done) load(0);
+  while (!done) {
+    if (tid < kSpWin / 16) reinterpret_cast<uint4 *>(L.sbuf)[tid] = pre;
+    if (tid == 0) L.ovf = ~0u;
+    __syncthreads();
+    const uint32_t p0 = uni((uint32_t)(reinterpret_cast<uintptr_t>(src + pos) & 15));
+    const uint32_t n = min(len - pos, kSpWin - 16), P = p0 + n;
+    const bool at_end = pos + n == len;
+    // positions count from p0 on; wave w's are [w0, w1)
+    const uint32_t w0 = wave * kSpWavePos, w1 = w0 + kSpWavePos;
+    uint32_t nx[kSpSpans], cn[kSpSpans], ex[kSpSpans];
+#pragma unroll
+    for (uint32_t k = 0; k < kSpSpans; k++) {
+      uint32_t sz, c;
+      bool ok;
+      span_block(L.sbuf, p0 + w0 + k * kWave, lane, P, sz, c, ok);
+      nx[k] = ok ? lane + sz : lane;
+      cn[k] = c;
+      ex[k] = nx[k];
+    }
+    // a chain in a span has 32 links at most
+#pragma unroll
+    for (uint32_t d = 0; d < 5; d++) {
+#pragma unroll
+      for (uint32_t k = 0; k < kSpSpans; k++) {
+        const uint32_t x = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(ex[k] * 4), (int)ex[k]);
+        ex[k] = ex[k] < (uint32_t)kWave ? x : ex[k];
+      }
+    }
+#pragma unroll
+    for (uint32_t k = kSpSpans; k-- > 0;) {
+      const uint32_t b = w0 + k * kWave;
+      uint32_t x = b + ex[k];
+      if (k + 1 < kSpSpans) {
+        const uint32_t y = L.to[min(x, w1 - 1)];
+        x = x >= b + kWave && x < w1 ? y : x;
+      }
+      L.to[b + lane] = (uint16_t)x;
+      asm volatile("" ::: "memory");  // other lanes read it; one wave's LDS operations keep their order
+    }
+    __syncthreads();
+    // the chain over the waves: this wave's entry, and where the step ends
+    uint32_t p = 0, entry = kNoPos;
+    bool trap = false;
+#pragma unroll
+    for (uint32_t w = 0; w < kSpWaves; w++) {
+      if (!trap && p < (w + 1) * kSpWavePos) {
+        entry = w == wave ? p : entry;
+        p = uni((uint32_t)L.to[p]);
+        trap = p < (w + 1) * kSpWavePos;
+      }
+    }
+    // this wave's blocks, span by span
+    uint64_t mk[kSpSpans];
+    uint32_t values = 0, blocks = 0, incl[kSpSpans];
+    {
+      uint32_t q = entry;
+      bool go = entry != kNoPos;
+#pragma unroll
+      for (uint32_t k = 0; k < kSpSpans; k++) {
+        const uint32_t b = w0 + k * kWave;
+        uint64_t m = 0;
+        if (go && q < b + kWave) {
+          uint32_t r = q - b;
+          for (;;) {
+            const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)nx[k], (int)r);
+            if (t == r) {
+              go = false;
+              break;
+            }
+            m |= 1ull << r;
+            r = t;
+            if (r >= (uint32_t)kWave) break;
+          }
+          q = b + r;
+        }
+        mk[k] = m;
+        const uint32_t c = (m >> lane) & 1 ? cn[k] : 0u;
+        incl[k] = wave_scan_dpp(c);
+        cn[k] = c;
+        values += (uint32_t)__builtin_amdgcn_readlane((int)incl[k], kWave - 1);
+        blocks += (uint32_t)__builtin_popcountll(m);
+      }
+    }
+    if (lane == 0) {
+      L.values[wave] = values;
+      L.blocks[wave] = blocks;
+    }
+    const uint32_t next = pos + p;  // the step's end in the stream
+    if (!trap && next < len) load(next);
+    __syncthreads();  // L.to is done with: descriptors take its place
+    uint32_t at_o = o, at_n = 0, total = 0, nblk = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kSpWaves; w++) {
+      const uint32_t v = uni(L.values[w]), b = uni(L.blocks[w]);
+      at_o += w < wave ? v : 0u;
+      at_n += w < wave ? b : 0u;
+      total += v;
+      nblk += b;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kSpSpans; k++) {
+      if ((mk[k] >> lane) & 1) {
+        const uint32_t j = at_n + lanes_below(mk[k]), end = at_o + incl[k];
+        if (end > cap) atomicMin(&L.ovf, j);
+        else put_desc<true>(L.desc, nullptr, j, p0 + w0 + k * kWave + lane, end - cn[k]);
+      }
+      at_o += (uint32_t)__builtin_amdgcn_readlane((int)incl[k], kWave - 1);
+      at_n += (uint32_t)__builtin_popcountll(mk[k]);
+    }
+    __syncthreads();
+    const uint32_t ovf = uni(L.ovf);
+    if (ovf != ~0u) {
+      nblk = ovf;
+      st = kOverflow;
+      done = true;
+    }
+    for (uint32_t j0 = 0; j0 < nblk; j0 += kSpThreads) {
+      const uint32_t j = j0 + kSpWaves * lane + wave, have = min(nblk - j0, kSpThreads);
+      const uint32_t nd = have > wave ? (have - wave + kSpWaves - 1) / kSpWaves : 0u;
+      const uint32_t d = lane < nd ? L.desc[j] : 0u;
+      if (nd) expand_batch<W>(L.sbuf, nd, ~0ull, d & 0x1fff, d >> 13, dst, lane, &bad);
+    }
+    if (!done) {
+      o += total;
+      pos = next;
+      if (trap) {
+        uint32_t size = 0, cnt = 0;
+        const uint32_t how = one_block(L.sbuf, p0 + p, P, at_end, o, cap, size, cnt, st);
+        if (how == kOneDone) {
+          done = true;
+        } else if (how == kOneRestage) {
+          st = kOk;
+          if (p == 0) st = kCorrupt;  // a fresh window holds any block
+        } else if (how == kOneBlock) {
+          const uint32_t first = uni(L.sbuf[p0 + p]);
+          if (wave == 0) {
+            if (first < 64) expand_sr<W>(L.sbuf, 1, 1, p0 + p, o, dst, lane);
+            else expand_big<W>(L.sbuf, p0 + p, o, dst, lane, &bad);
+          }
+          pos += size;
+          o += cnt;
+        }
+        if (st != kOk) done = true;
+      }
+      if (pos >= len) done = true;
+      if (!done && trap) load(pos);
+    }
+    __syncthreads();  // every wave is done with the window
+  }
+  if (__ballot(bad) && lane == 0) L.bad = 1;
+  __syncthreads();
+  if (st == kOk && uni(L.bad)) st = kCorrupt;
+  // positions the stream did not produce are zero (decoder_trans.h:81)
+  if (st == kOk)
+    for (uint32_t i = o + tid; i < cap; i += kSpThreads) store_w<W>(dst, i, 0);
+  if (tid == 0 && status) status[chunk] = st;
+}
+
 }  // namespace rle2
 
 namespace {
@@ -637,6 +918,13 @@ void pc_launch(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *blk_off
     hipLaunchKernelGGL((rle2::rlev2_pc_kernel<4096, kExp, W, false>), dim3((uint32_t)n_chunks),
                        dim3((1 + kExp) * kWaveSize), 0, stream, comp, comp_bytes, blk_off, col_len,
                        n_chunks, chunk_bytes, out, status);
+}
+
+template <uint32_t W>
+void span_launch(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *blk_off, const uint64_t *col_len,
+                 uint64_t n_chunks, uint64_t chunk_bytes, uint8_t *out, int32_t *status, hipStream_t stream) {
+  hipLaunchKernelGGL((rle2::rlev2_span_kernel<W>), dim3((uint32_t)n_chunks), dim3(rle2::kSpThreads), 0, stream, comp,
+                     comp_bytes, blk_off, col_len, n_chunks, chunk_bytes, out, status);
 }
 
 // Instantiates F<..., W> for the element width w (1, 2, 4 or 8).
@@ -684,6 +972,15 @@ hipError_t launch_rlev2_pc(const uint8_t *comp, uint64_t comp_bytes, const uint6
     return hipErrorInvalidValue;
   }
 #undef ARGS
+  return hipGetLastError();
+}
+
+hipError_t launch_rlev2_span(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *blk_off,
+                             const uint64_t *col_len, uint64_t n_chunks, uint32_t w, uint64_t chunk_bytes,
+                             uint8_t *out, int32_t *status, hipStream_t stream) {
+  if (n_chunks == 0) return hipSuccess;
+  auto *launch = w == 1 ? span_launch<1> : w == 2 ? span_launch<2> : w == 4 ? span_launch<4> : span_launch<8>;
+  launch(comp, comp_bytes, blk_off, col_len, n_chunks, chunk_bytes, out, status, stream);
   return hipGetLastError();
 }
 
