@@ -228,7 +228,14 @@ codag_status codag_rlev1_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t 
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "rlev1_decode: too many chunks");
   DeviceGuard g(ctx->device);
   const codag_tune_params &t = ctx->tune[CODAG_RLEV1];
-  if (pipe_shape(t) && chunk_bytes / w <= (1u << 17))  // pipelined walker + helpers
+  // Unless the caller chose a shape: all waves by turns up to one chunk per CU
+  // (us, pipeline and turns: 256 chunks of an 8-bit table column 2448, 430, of the
+  // 64-bit benchmark column 76, 67; above it dense columns still gain, 512 chunks
+  // 2467, 543, but the benchmark column loses, 84, 95).
+  if (!ctx->tuned[CODAG_RLEV1] && n_chunks <= ctx->cu_count)
+    HIP_TRY(launch_rlev1_span(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
+                              d_out, d_status, pick(ctx, stream)));
+  else if (pipe_shape(t) && chunk_bytes / w <= (1u << 17))  // pipelined walker + helpers
     HIP_TRY(launch_rlev1_pipe(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                               d_out, d_status, pick(ctx, stream)));
   else if (pipe_shape(t))  // values per chunk beyond the pipeline's descriptor field

@@ -481,6 +481,374 @@ rlev1_pipe_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
   }
 }
 
+// ---------------------------------------------------------------- spans by all waves
+
+// Walk and expansion by turns, both by every wave of a group of kSpWaves. A step
+// stages 8 KiB of the stream from a segment's header on and numbers the
+// terminators in it, 0 being the byte before the header.
+//  * Lane i of a span of 64 terminators sizes the segment after its terminator.
+//    Pointer doubling by ds_bpermute leaves every terminator the first one
+//    outside its span that its chain reaches, a pass from the wave's last span to
+//    its first the first one outside the wave's. A terminator whose segment is
+//    not whole in the window is its own successor and ends the chain.
+//  * One link per wave then gives each wave its entry, and each wave follows its
+//    own spans by v_readlane.
+//  * A prefix sum over the group places the segments, and the values are dealt
+//    out in passes of 64, one lane per value.
+// A segment that is not whole at the stream's end, or in a window of its own, is
+// read value by value (one_segment), which finds its error.
+// The pipeline's walker takes about 115 cycles a segment, so a column of short
+// runs (3 bytes of stream each) is bound by it alone; here the chain costs the
+// same whatever the segments. Latency bounds it: a step of dense segments takes
+// 42 K cycles, 10 K each in the doubling, the placing and the values. 128 KiB
+// chunks, pipeline and spans: 32 chunks of an 8-bit table column 2105 and 378 us,
+// 64 chunks of a 64-bit one 545 and 125, benchmark columns of 64 chunks, 8 bits
+// 438 and 312, 64 bits 73 and 64. With two groups per CU the benchmark columns
+// are slower (512 chunks, 64 bits, 84 and 95).
+constexpr uint32_t kSpBytes = 8192, kSpWaves = 16;
+constexpr uint32_t kSpThreads = kSpWaves * kWave;
+constexpr uint32_t kSpans = kSpBytes / kSpThreads;  // spans of a wave, at most
+
+constexpr uint32_t kMaxSpanCap = (1u << 19) - 1;  // values per chunk (descriptor field; later ones are not read)
+
+__device__ __forceinline__ uint32_t rdlast(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, kWave - 1);
+}
+// of an inclusive prefix sum over the waves, the sum of those before this wave
+__device__ __forceinline__ uint32_t before(uint32_t sums, uint32_t wave) {
+  return wave ? (uint32_t)__builtin_amdgcn_readlane((int)sums, (int)wave - 1) : 0u;
+}
+
+struct SpanLds {
+  uint8_t sbuf[kSpBytes + 32];
+  uint16_t sel[kSpBytes];  // window byte of each terminator
+  union {
+    uint16_t to[kSpBytes];        // the first terminator outside its wave's that a chain reaches
+    uint32_t desc[kSpBytes / 2];  // segment: terminator before it (13 bits) | first value of the step << 13
+  };
+  uint32_t count[kSpWaves], values[kSpWaves], segs[kSpWaves];
+  uint8_t mark[kSpWaves][kWave];
+  uint32_t key;   // first error: value of the step << 2 | priority
+  uint32_t over;  // 1: a segment reaches past the chunk; 2: a terminator follows an overlong varint
+  uint32_t pos, o, pending;  // one_segment's results
+  int32_t st;
+};
+
+// Reads the segment at stream byte pos and writes its values from element o on, as
+// the oracle does. Returns the status; `pending`: a varint longer than 10 bytes
+// begins before pos, whose status hangs on whether any terminator follows.
+template <uint32_t W>
+__device__ __forceinline__ int32_t one_segment(const uint8_t *src, uint32_t len, uint32_t cap, uint8_t *dst,
+                                            uint32_t &pos, uint32_t &o, uint32_t &pending) {
+  pending = 0;
+  if (pos >= len) return kTrunc;
+  const uint32_t h = src[pos++];
+  const uint32_t cnt = h < 0x80 ? h + 3 : 256 - h;
+  int64_t delta = 0;
+  if (h < 0x80) {
+    if (pos >= len) return kTrunc;
+    delta = (int8_t)src[pos++];
+  }
+  uint64_t v = 0;
+  for (uint32_t i = 0; i < cnt; i++) {
+    if (i == 0 || h >= 0x80) {
+      v = 0;
+      for (uint32_t n = 0;; n++) {
+        if (pos >= len) return kTrunc;
+        if (n == 10) {
+          pending = 1;
+          return kCorrupt;
+        }
+        const uint32_t b = src[pos++];
+        v |= (uint64_t)(b & 0x7f) << (7 * n);
+        if (b < 0x80) break;
+      }
+    }
+    if (o >= cap) return kOverflow;
+    store_val<W>(dst, o++, v + (uint64_t)((int64_t)i * delta));
+  }
+  return kOk;
+}
+
+// 64 registers: two groups per CU.
+template <uint32_t W>
+__global__ void __launch_bounds__(kSpThreads) __attribute__((amdgpu_waves_per_eu(8)))
+rlev1_span_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes, const uint64_t *__restrict__ blk_off,
+                  const uint64_t *__restrict__ col_len, uint64_t chunk_bytes, uint8_t *__restrict__ out,
+                  int32_t *__restrict__ status) {
+  constexpr uint32_t kDw = kSpBytes / 4 / kSpThreads;  // window dwords a thread indexes
+  __shared__ __align__(16) SpanLds L;
+  const uint64_t chunk = blockIdx.x;
+  const uint32_t lane = lane_id(), tid = threadIdx.x;
+  const uint32_t wave = uni(tid / kWave);
+  const uint64_t boff = blk_off[chunk], len64 = col_len[chunk];
+  if (boff > comp_bytes || len64 > comp_bytes - boff || len64 >= (1ull << 30)) {
+    if (tid == 0 && status) status[chunk] = kCorrupt;  // uniform over the workgroup
+    return;
+  }
+  const uint32_t len = (uint32_t)len64, cap = (uint32_t)(chunk_bytes / W);
+  const uint8_t *src = comp + boff;
+  uint8_t *dst = out + chunk * chunk_bytes;
+  const uintptr_t s_addr = reinterpret_cast<uintptr_t>(src), e_addr = s_addr + len;
+  uint32_t pos = 0, o = 0;  // stream position and value index of the step's first header
+  int32_t st = kOk;
+  uint4 pre = make_uint4(0, 0, 0, 0);
+  // the window begins at the 16-byte block of the byte before `from`; only blocks
+  // with stream bytes are read
+  auto load = [&](uint32_t from) __attribute__((always_inline)) {
+    const uintptr_t a = ((s_addr + from - 1) & ~uintptr_t(15)) + 16u * tid;
+    pre = make_uint4(0, 0, 0, 0);
+    if (tid < kSpBytes / 16 && a + 16 > s_addr && a < e_addr) pre = *reinterpret_cast<const uint4 *>(a);
+  };
+  load(0);
+  for (;;) {
+    if (tid < kSpBytes / 16) reinterpret_cast<uint4 *>(L.sbuf)[tid] = pre;
+    if (tid == 0) {
+      L.key = ~0u;
+      L.over = 0;
+    }
+    __syncthreads();
+    const uint32_t lead = uni((uint32_t)((s_addr + pos - 1) & 15) + 1);  // window byte of stream byte pos
+    const uint32_t P = min(lead + (len - pos), kSpBytes);
+    const bool at_end = lead + (len - pos) <= kSpBytes;
+    // ---- number the terminators
+    uint32_t tm = 0;  // bit 4 i + j: byte j of the thread's dword i ends a varint
+#pragma unroll
+    for (uint32_t i = 0; i < kDw; i++) {
+      const uint32_t at = 4 * (tid * kDw + i);
+      const uint32_t t = ~reinterpret_cast<const uint32_t *>(L.sbuf)[tid * kDw + i] & 0x80808080u;
+      uint32_t m = __builtin_amdgcn_udot4(t >> 7, 0x08040201u, 0u, false);
+      const int32_t a = (int32_t)(lead - at), z = (int32_t)(P - at);  // stream bytes of the dword
+      m &= z >= 4 ? 0xfu : (z > 0 ? (1u << z) - 1 : 0u);
+      m &= a <= 0 ? 0xfu : (a < 4 ? 0xfu << a : 0u);
+      m |= a >= 1 && a <= 4 ? 1u << (a - 1) : 0u;  // terminator 0
+      tm |= m << (4 * i);
+    }
+    const uint32_t mine = (uint32_t)__popc(tm), incl0 = wave_scan_dpp(mine);
+    if (lane == kWave - 1) L.count[wave] = incl0;
+    __syncthreads();
+    const uint32_t counts = wave_scan_dpp(lane < kSpWaves ? L.count[lane] : 0u);  // lane w: of waves 0 to w
+    const uint32_t terms = rdlast(counts);
+    uint32_t rank = incl0 - mine + before(counts, wave);
+#pragma unroll
+    for (uint32_t b = 0; b < 4 * kDw; b++) {
+      if ((tm >> b) & 1) L.sel[rank++] = (uint16_t)(4 * tid * kDw + b);
+    }
+    __syncthreads();
+    // ---- the segments after this wave's terminators
+    const uint32_t spans = (terms + kSpThreads - 1) / kSpThreads, own = spans * kWave;  // of a wave
+    const uint32_t w0 = wave * own, w1 = w0 + own;
+    // per terminator: values << 8 | next, as a lane of its span; later the span's
+    // values up to and with this segment << 8 | its own
+    uint32_t sg[kSpans], ex[kSpans];
+#pragma unroll
+    for (uint32_t k = 0; k < kSpans; k++) {
+      if (k >= spans) continue;
+      const uint32_t r = w0 + k * kWave + lane;
+      const uint32_t s = r < terms ? L.sel[r] : 0u;
+      const uint32_t h = L.sbuf[s + 1], d = L.sbuf[s + 2];
+      const bool run = h < 0x80;
+      const uint32_t adv = run ? 2 + (d < 0x80) : 256 - h;
+      const bool ok = r + adv < terms && s + (run ? 2u : 1u) < P;
+      ex[k] = ok ? lane + adv : lane;
+      sg[k] = (run ? h + 3 : adv) << 8 | ex[k];
+    }
+    // a chain in a span has 64 links at most
+#pragma unroll
+    for (uint32_t d = 0; d < 6; d++) {
+#pragma unroll
+      for (uint32_t k = 0; k < kSpans; k++) {
+        if (k >= spans) continue;
+        const uint32_t x = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(ex[k] * 4), (int)ex[k]);
+        ex[k] = ex[k] < (uint32_t)kWave ? x : ex[k];
+      }
+    }
+#pragma unroll
+    for (uint32_t k = kSpans; k-- > 0;) {
+      if (k >= spans) continue;
+      const uint32_t b = w0 + k * kWave;
+      uint32_t x = b + ex[k];
+      if (k + 1 < spans) {
+        const uint32_t y = L.to[min(x, w1 - 1)];
+        x = x >= b + kWave && x < w1 ? y : x;
+      }
+      L.to[b + lane] = (uint16_t)x;
+      asm volatile("" ::: "memory");  // other lanes read it; one wave's LDS operations keep their order
+    }
+    __syncthreads();
+    // the chain over the waves; it ends at a terminator without a whole segment
+    uint32_t p = 0, entry = kNone;
+    bool end = false;
+#pragma unroll
+    for (uint32_t w = 0; w < kSpWaves; w++) {
+      if (!end && p < (w + 1) * own) {
+        entry = w == wave ? p : entry;
+        p = uni((uint32_t)L.to[p]);
+        end = p < (w + 1) * own;
+      }
+    }
+    // this wave's segments, span by span
+    uint64_t mk[kSpans];
+    uint32_t values = 0, segs = 0;
+    {
+      uint32_t q = entry;
+      bool go = entry != kNone;
+#pragma unroll
+      for (uint32_t k = 0; k < kSpans; k++) {
+        mk[k] = 0;
+        if (k >= spans) continue;
+        const uint32_t b = w0 + k * kWave;
+        uint64_t m = 0;
+        if (go && q < b + kWave) {
+          uint32_t r = q - b;
+          for (;;) {
+            const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)sg[k], (int)r) & 0xff;
+            if (t == r) {
+              go = false;
+              break;
+            }
+            m |= 1ull << r;
+            r = t;
+            if (r >= (uint32_t)kWave) break;
+          }
+          q = b + r;
+        }
+        mk[k] = m;
+        const uint32_t c = (m >> lane) & 1 ? sg[k] >> 8 : 0u, incl = wave_scan_dpp(c);
+        sg[k] = incl << 8 | c;
+        values += rdlast(incl);
+        segs += (uint32_t)__builtin_popcountll(m);
+      }
+    }
+    if (lane == 0) {
+      L.values[wave] = values;
+      L.segs[wave] = segs;
+    }
+    const uint32_t next = pos + (uni((uint32_t)L.sel[p]) + 1 - lead);
+    const bool alone = at_end || p == 0;  // what follows is no whole segment
+    if (!alone) load(next);
+    __syncthreads();  // L.to is done with: descriptors take its place
+    const uint32_t vs = wave_scan_dpp(lane < kSpWaves ? L.values[lane] : 0u);
+    const uint32_t ss = wave_scan_dpp(lane < kSpWaves ? L.segs[lane] : 0u);
+    const uint32_t total = rdlast(vs), nd = rdlast(ss);
+    uint32_t at_o = before(vs, wave), at_n = before(ss, wave);
+    const uint32_t room = cap - o;
+#pragma unroll
+    for (uint32_t k = 0; k < kSpans; k++) {
+      if (k >= spans) continue;
+      if ((mk[k] >> lane) & 1) {
+        const uint32_t to = at_o + (sg[k] >> 8), os = to - (sg[k] & 0xff);
+        L.desc[at_n + lanes_below(mk[k])] = (w0 + k * kWave + lane) | min(os, kMaxSpanCap) << 13;
+        if (os < room && to > room) L.over = 1;
+      }
+      at_o += rdlast(sg[k]) >> 8;
+      at_n += (uint32_t)__builtin_popcountll(mk[k]);
+    }
+    __syncthreads();
+    // ---- values; the one at index cap is read as well, as its varint's error comes first
+    const uint32_t over = uni(L.over), vend = over ? room + 1 : min(total, room);
+    const uint32_t npass = (vend + kWave - 1) / kWave, per = (npass + kSpWaves - 1) / kSpWaves;
+    const uint32_t pa = wave * per, pb = min(pa + per, npass);
+    uint32_t cur = 0;  // the last segment that starts at or before the pass's first value
+    if (pa < pb) {
+      uint32_t lo = 0, hi = nd;  // by 64 probes at a time
+      while (hi - lo > 1) {
+        const uint32_t step = (hi - lo + kWave - 1) / kWave, i = lo + lane * step;
+        const uint64_t le = __ballot(i < hi && (L.desc[min(i, nd - 1)] >> 13) <= pa * kWave);
+        const uint32_t c = (uint32_t)__builtin_popcountll(le);  // lane 0 always is one
+        lo += (c - 1) * step;
+        hi = min(lo + step, hi);
+      }
+      cur = lo;
+    }
+    uint8_t *mkb = L.mark[wave];
+#pragma clang loop unroll(disable)
+    for (uint32_t t = pa; t < pb; t++) {
+      const uint32_t ob = t * kWave;
+      uint32_t di, oi;
+      bool iv;
+      for (;;) {
+        const uint32_t i = cur + lane;
+        iv = i < nd;
+        di = iv ? L.desc[i] : 0u;
+        oi = di >> 13;
+        const uint32_t c = (uint32_t)__popcll(__ballot(iv && lane >= 1 && oi <= ob));
+        if (c == 0) break;
+        cur += c;
+      }
+      // segment of value ob + lane = cur + (segments starting in (ob, ob + lane])
+      mkb[lane] = 0;
+      if (lane >= 1 && iv && oi - ob < (uint32_t)kWave) mkb[oi - ob] = 1;
+      asm volatile("" ::: "memory");
+      const uint64_t starts = __ballot(mkb[lane] != 0);
+      const uint32_t j = lanes_below(starts) + (uint32_t)((starts >> lane) & 1);
+      const uint32_t dsc = (uint32_t)__shfl((int)di, (int)j, kWave);
+      const uint32_t v = ob + lane;
+      const bool act = v < vend;
+      const uint32_t rl = dsc & 0x1fff, os = dsc >> 13;
+      const uint32_t ii = act ? v - os : 0u;
+      const uint32_t s0 = L.sel[rl];
+      const uint32_t hb = L.sbuf[s0 + 1], db = L.sbuf[s0 + 2];
+      const bool run = hb < 0x80;
+      // the varint ends on terminator qb and follows qa, or the header (and delta
+      // byte) after it
+      const uint32_t qb = min(run ? rl + 2 + (db < 0x80) : rl + 1 + ii, terms - 1);
+      const bool front = run || ii == 0;
+      const uint32_t start = (front ? s0 : (uint32_t)L.sel[qb - 1]) + 1 + (front ? (run ? 2u : 1u) : 0u);
+      const uint32_t n = L.sel[qb] + 1u - start;
+      if (act && n <= 10) {
+        if (v < room) {
+          uint64_t val = ring_varint<W>(L.sbuf, start, n);
+          if (run) val += (uint64_t)((int64_t)ii * (int32_t)(int8_t)db);
+          store_val<W>(dst, o + v, val);
+        }
+      } else if (act) {  // longer than any 64-bit varint
+        atomicMin(&L.key, (run ? os : v) << 2 | kPrCorrupt);
+      }
+    }
+    if (over && tid == 0) atomicMin(&L.key, room << 2 | kPrOverflow);
+    __syncthreads();
+    const uint32_t key = uni(L.key);
+    if (key != ~0u) {
+      st = (key & 3) == kPrCorrupt ? kCorrupt : kOverflow;
+      break;
+    }
+    o += min(total, room);
+    pos = next;
+    if (o >= cap) break;
+    if (alone) {
+      if (tid == 0) {
+        uint32_t pending;
+        L.st = one_segment<W>(src, len, cap, dst, pos, o, pending);
+        L.pos = pos;
+        L.o = o;
+        L.pending = pending;
+      }
+      __syncthreads();
+      st = (int32_t)uni((uint32_t)L.st);
+      pos = uni(L.pos);
+      o = uni(L.o);
+      if (uni(L.pending)) {  // no terminator after it: the stream ends in it
+        uint32_t found = 0;
+        const uintptr_t from = (s_addr + pos) & ~uintptr_t(15);
+        for (uintptr_t a = from + 16u * tid; a < e_addr; a += 16u * kSpThreads) {
+          uint32_t m = term_mask16(*reinterpret_cast<const uint4 *>(a));
+          if (a < s_addr + pos) m &= 0xffffu << (s_addr + pos - a);
+          if (e_addr - a < 16) m &= (1u << (e_addr - a)) - 1;
+          found |= m & 0xffffu;
+        }
+        if (__ballot(found != 0) && lane == 0) L.over = 2;
+        __syncthreads();
+        st = uni(L.over) == 2 ? kCorrupt : kTrunc;
+      }
+      if (st != kOk || o >= cap) break;
+      load(pos);
+      __syncthreads();  // every wave has read L.st
+    }
+  }
+  if (tid == 0 && status) status[chunk] = st;
+}
+
 }  // namespace rle1p
 
 hipError_t launch_rlev1_pipe(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *blk_off,
@@ -501,6 +869,26 @@ hipError_t launch_rlev1_pipe(const uint8_t *comp, uint64_t comp_bytes, const uin
   default: return hipErrorInvalidValue;
   }
 #undef CODAG_V1P
+  return hipGetLastError();
+}
+
+hipError_t launch_rlev1_span(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *blk_off,
+                             const uint64_t *col_len, uint64_t n_chunks, uint32_t w, uint64_t chunk_bytes,
+                             uint8_t *out, int32_t *status, hipStream_t stream) {
+  if (n_chunks == 0) return hipSuccess;
+  if (chunk_bytes / w > rle1p::kMaxSpanCap) return hipErrorInvalidValue;
+  const dim3 grid((uint32_t)n_chunks), block(rle1p::kSpThreads);
+#define CODAG_V1S(W)                                                                         \
+  hipLaunchKernelGGL((rle1p::rlev1_span_kernel<W>), grid, block, 0, stream, comp, comp_bytes, \
+                     blk_off, col_len, chunk_bytes, out, status)
+  switch (w) {
+  case 1: CODAG_V1S(1); break;
+  case 2: CODAG_V1S(2); break;
+  case 4: CODAG_V1S(4); break;
+  case 8: CODAG_V1S(8); break;
+  default: return hipErrorInvalidValue;
+  }
+#undef CODAG_V1S
   return hipGetLastError();
 }
 
