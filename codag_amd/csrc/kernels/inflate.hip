@@ -124,7 +124,7 @@ using Many = Cfg<8, 9, 1, 2560, 10, 8, 308, 144>;
 template <class C> struct Sh {
   alignas(16) uint32_t stage[C::kStage];  // the span's stream dwords
   alignas(16) uint32_t tab[C::kTab];      // literal/length root, its sub-tables, distance root, its sub-tables
-  alignas(16) uint16_t win[C::kWin];      // marks of the window being written; CRC-32 slice tables
+  alignas(16) uint16_t win[C::kWin + 2];  // marks of the window being written, and one for none; CRC-32 slice tables
   Huff<288> hl;
   Huff<32> hd;
   alignas(4) uint8_t lens[320];
@@ -720,32 +720,37 @@ __device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n
     if (tid == 0 && wn < C::kWin) S.win[wn] = 0x8000u;
     if (x > done && lastx < done) S.win[0] = (uint16_t)lastm;  // a token that began before this window
     const uint32_t stopx = min(end, done + wn);
-    uint32_t d = C::kLitDesc, mlen = 0;
-    while (x < stopx) {
+    // One lookup a step without branches: a lookup that completes no token writes
+    // its mark behind the window (a branch for each kind of entry took 30 scalar
+    // instructions a step).
+    uint32_t d = C::kLitDesc, mlen = 0, bad = ~0u;
+    uint32_t goal = stopx;
+    while (x < goal) {
       const uint32_t bits = place_bits(p), e = look(&S.tab[0], bits, d);
-      if ((e & 31) == 0) break;  // not in a counted range
       place_move(p, &S.stage[0], e & 31);
       d = next_table<C>(e);
       const uint32_t v = entry_value(e, bits);
-      mlen = (e >> 30) == 1 ? v : mlen;
-      if (e >= kLenType) continue;
-      const bool lit = e & kLitFlag;
+      const bool whole = e < kLenType, lit = e & kLitFlag;
+      mlen = (int32_t)e >= (int32_t)kLenType ? v : mlen;
       const uint32_t tl = lit ? 1u : mlen;
       const uint32_t m = lit ? 0x8000u | v : v - 1;
       if (check) {
         const uint32_t at = o.pos + x;
-        if (at + tl > o.cap) atomicMin(&S.err, x << 2 | (uint32_t)kOverflow);
-        else if (!lit && v > at) atomicMin(&S.err, x << 2 | (uint32_t)kCorrupt);  // "invalid distance too far back"
+        const uint32_t why =
+            at + tl > o.cap ? (uint32_t)kOverflow : (!lit && v > at ? (uint32_t)kCorrupt : 0u);  // distance too far back
+        bad = whole && why ? min(bad, x << 2 | why) : bad;
       }
-      S.win[x - done] = (uint16_t)m;
+      S.win[whole ? x - done : C::kWin] = (uint16_t)m;
       if constexpr (C::kNW > 1) {  // a mark for the next segment's wave, too
         const uint32_t b = (x - done + tl - 1) / C::kSeg * C::kSeg;
-        if (b > x - done && b < C::kWin) S.win[b] = (uint16_t)m;
+        if (whole && b > x - done && b < C::kWin) S.win[b] = (uint16_t)m;
       }
-      lastx = x;
-      lastm = m;
-      x += tl;
+      lastx = whole ? x : lastx;
+      lastm = whole ? m : lastm;
+      x += whole ? tl : 0u;
+      goal = (e & 31) ? goal : 0u;  // no stop in a counted range
     }
+    if (check && bad != ~0u) atomicMin(&S.err, bad);
     group_sync<C>();
     if (check) {
       const uint32_t e = uni(S.err);
