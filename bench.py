@@ -378,7 +378,7 @@ def bench_bytecodec(ctx, args, kind):
     d_len = ctx.alloc(8 * n)
     d_st = ctx.alloc(4 * n)
     fn = ctx.lzss_decode if lz else ctx.brle_decode
-    kname = "lzss_chunks_kernel" if lz else "brle_chunks2_kernel"
+    kname = "lzss_chunks_kernel" if lz else "brle_chunks_kernel"
 
     def launch():
         fn(d_comp, len(data), d_idx, n, chunk, d_out, d_len, d_st)
@@ -500,7 +500,7 @@ def bench_batch(ctx, args):
         log(f"[bench] c4: autotuner on {tuned['sample']}: {tbest.threads_per_group} threads x "
             f"{tbest.groups_per_cu} workgroups per CU ({tms:.1f} ms)")
     best = ctx.tune_get(ca.DEFLATE)
-    kname = "inflate_batch2_kernel" if best.threads_per_group == 128 else "inflate_batch_kernel"
+    kname = "inflate_batch_many_kernel" if best.threads_per_group == 128 else "inflate_batch_kernel"
     log(f"[bench] c4: persistent launch, {best.threads_per_group} threads x "
         f"{best.groups_per_cu} workgroups per CU")
 
