@@ -433,7 +433,7 @@ brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
 // One wave per chunk, eight groups at a time and serial where matches overlap,
 // was bound by its scalar chain and the latency of two waves a SIMD: 128 KiB
 // chunks of text, before and now: 2 chunks 1.59 and 0.41 ms, 512 chunks 1.65 and
-// 0.47 ms, 2048 chunks 1.95 and 1.01 ms (bound by vector issue, mostly the
+// 0.47 ms, 2048 chunks 1.95 and 0.94 ms (bound by vector issue, mostly the
 // window's resolving).
 constexpr int kLzWaves = 4;
 constexpr uint32_t kLzThreads = kLzWaves * kWave;
@@ -597,7 +597,7 @@ __device__ __forceinline__ int32_t lzss_stream(const uint8_t *src, uint32_t len,
           wn = (es >> 2) - done;
           err = (int32_t)(es & 3);
         }
-        resolve_window<kLzWaves, kLzSeg, false>(dst, S.win, pos + done, wn, wave, lane, none, none);
+        resolve_window<kLzWaves, kLzSeg, false, true>(dst, S.win, pos + done, wn, wave, lane, none, none);
         __syncthreads();
         done += wn;
         if (err != kOk) break;

@@ -16,17 +16,17 @@
 //  * Output. The verified lanes know their byte counts; a prefix sum gives each
 //    its output position. They decode once more and write a 16-bit mark at each
 //    token's first byte into an LDS window (literal byte, or distance). The
-//    window is then resolved in rows of 64 bytes, one byte a lane: a DPP max
-//    scan hands every byte its token's mark, sources before the window are
-//    gathered from HBM (four rows in flight), sources inside it are followed by
-//    pointer doubling; the bytes are stored and summed for the Adler-32.
+//    window is then resolved 256 bytes at a time, four a lane: a DPP max scan
+//    hands every byte its token's mark, sources before the window are gathered
+//    from HBM a step ahead, sources inside it are followed by pointer doubling;
+//    the bytes are stored and summed for the Adler-32.
 //  * The scalar symbol loop decodes the symbol a span stopped at (end of block,
 //    or the error), so statuses are exactly the serial decoder's.
 // What bounds it: vector issue and its latency, not memory (without the far
 // gathers and the stores the launches take the same time). 128 KiB zlib level-6
 // chunks, before (one token chain per stream: 64 bit positions decoded to keep
-// about seven tokens, the chain scalar) and now: 4096 chunks 9.1 and 3.2 ms, 256
-// chunks 4.0 and 0.46 ms, 3 chunks 3.7 and 0.43 ms; 300 mixed streams of 4 KiB
+// about seven tokens, the chain scalar) and now: 4096 chunks 9.1 and 3.0 ms, 256
+// chunks 4.0 and 0.45 ms, 3 chunks 3.7 and 0.42 ms; 300 mixed streams of 4 KiB
 // to 4 MiB 119 and 15 ms. A chunk takes 0.27 M vector instructions (0.69 M
 // before): half of them passes, headers and tables, a fifth marks, a third the
 // resolving. Data that compress below 5% are slower than the copy loop of the
@@ -721,8 +721,9 @@ __device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n
     if (x > done && lastx < done) S.win[0] = (uint16_t)lastm;  // a token that began before this window
     const uint32_t stopx = min(end, done + wn);
     // One lookup a step without branches: a lookup that completes no token writes
-    // its mark behind the window (a branch for each kind of entry took 30 scalar
-    // instructions a step).
+    // its mark behind the window (with a branch for each kind of entry, 25 scalar
+    // instructions more a step, 4096 chunks took 3.20 ms and 3 chunks 445 us, now
+    // 3.09 and 419).
     uint32_t d = C::kLitDesc, mlen = 0, bad = ~0u;
     uint32_t goal = stopx;
     while (x < goal) {
@@ -759,7 +760,7 @@ __device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n
         st = (int32_t)(e & 3);
       }
     }
-    resolve_window<C::kNW, C::kSeg, true>(o.dst, S.win, o.pos + done, wn, wave, lane, o.s1, o.s2);
+    resolve_window<C::kNW, C::kSeg, true, C::kNW == 1>(o.dst, S.win, o.pos + done, wn, wave, lane, o.s1, o.s2);
     group_sync<C>();
     done += wn;
     if (st != kOk) break;
@@ -1441,7 +1442,7 @@ hipError_t inflate_scratch_ptr(uint32_t **out) {
 
 // Eight waves per chunk while there are at most five chunks per CU, else one
 // wave per chunk (128 KiB chunks, MI355X: 256 chunks 0.48 and 1.26 ms, 1024
-// 1.04 and 1.38 ms, 2048 2.02 and 1.51 ms, 4096 3.90 and 3.16 ms).
+// 1.04 and 1.38 ms, 2048 2.02 and 1.51 ms, 4096 3.90 and 2.96 ms).
 hipError_t launch_inflate_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *off,
                                  uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
                                  int32_t *status, uint32_t flags, hipStream_t stream, bool many) {

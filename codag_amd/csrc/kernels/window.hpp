@@ -44,14 +44,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, uint3
 // before it (a literal then repeats); a token also has a mark where it crosses
 // into another wave's segment of SEG bytes. The window is initialised up to the
 // next multiple of 512 bytes and has a literal mark behind its last byte.
-// Each wave resolves its segment in groups of four rows of 64 bytes; the far
-// sources of the next group are loaded while this one's near sources are
-// followed. Nothing is stored before the segment is done: a wait for loads
-// would also wait for the stores before them.
+// Each wave resolves its segment in groups of 256 bytes; the far sources of the
+// next group are loaded while this one's near sources are followed. Nothing is
+// stored before the segment is done: a wait for loads would also wait for the
+// stores before them.
+// A lane has one byte of each of the group's four rows of 64, or, with QUADS, four
+// consecutive bytes: one prefix maximum a group instead of four and half the LDS
+// instructions, but LDS gathers of a lane stride and far loads over four times
+// the cache lines. Rows and quads, us: LZSS, 2048 chunks, 1000 and 932; one-wave Deflate,
+// 4096 chunks, 3092 and 2963; eight-wave groups, 3000 gzip members, 912 and 962.
 // A group's bytes first get 0x8000 | byte where the byte is known (literals,
 // far sources) and else the window index of their source; a byte then takes
 // what its source holds, byte or index, until it is a byte (pointer doubling).
-template <int NW, uint32_t SEG, bool SUM>
+template <int NW, uint32_t SEG, bool SUM, bool QUADS>
 __device__ __forceinline__ void resolve_window(uint8_t *dst, uint16_t *win, uint32_t w0, uint32_t wn, uint32_t wave,
                                                uint32_t lane, uint32_t &adler1, uint32_t &adler2) {
   static_assert(SEG % 512 == 0 && SEG <= 4096, "a segment is whole pairs of row groups, tracked in one 64-bit mask");
@@ -61,23 +66,46 @@ __device__ __forceinline__ void resolve_window(uint8_t *dst, uint16_t *win, uint
   uint32_t carry = 0x8000u;
   uint64_t late = 0;  // groups with bytes whose source lies in another wave's segment
   const __amdgpu_buffer_rsrc_t rsrc = buffer_of(dst, 0x80000000u);
+  auto at = [&](uint32_t g, uint32_t r) { return QUADS ? g + R * lane + r : g + r * kWave + lane; };
+  auto read4 = [&](uint32_t g, uint32_t *v) __attribute__((always_inline)) {
+    const uint2 m = *reinterpret_cast<const uint2 *>(win + g + R * lane);
+    v[0] = m.x & 0xffff, v[1] = m.x >> 16, v[2] = m.y & 0xffff, v[3] = m.y >> 16;
+  };
+  auto write4 = [&](uint32_t g, const uint32_t *v) __attribute__((always_inline)) {
+    *reinterpret_cast<uint2 *>(win + g + R * lane) =
+        make_uint2(__builtin_amdgcn_perm(v[1], v[0], 0x05040100u), __builtin_amdgcn_perm(v[3], v[2], 0x05040100u));
+  };
   // reads the marks of a group and loads its far sources
   auto open = [&](uint32_t row, uint32_t *c, uint32_t *f) __attribute__((always_inline)) {
-    uint32_t k[R];
+    if constexpr (QUADS) {
+      uint32_t m[R];
+      read4(row, m);
+      uint32_t last = m[0];
 #pragma unroll
-    for (uint32_t r = 0; r < R; r++) {
-      const uint32_t m = win[row + r * kWave + lane];
-      k[r] = m == 0xffffu ? 0u : ((lane + 1) << 16) | m;
+      for (uint32_t r = 1; r < R; r++) last = m[r] != 0xffffu ? m[r] : last;
+      const uint32_t key = wave_max_dpp(last != 0xffffu ? ((lane + 1) << 16) | last : 0u);
+      const uint32_t up = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key, 0x138, 0xf, 0xf, false);  // wave_shr:1
+      uint32_t t = up ? up & 0xffff : carry;
+#pragma unroll
+      for (uint32_t r = 0; r < R; r++) t = c[r] = m[r] != 0xffffu ? m[r] : t;
+      carry = rdlane(t, kWave - 1);
+    } else {
+      uint32_t k[R];
+#pragma unroll
+      for (uint32_t r = 0; r < R; r++) {
+        const uint32_t m = win[at(row, r)];
+        k[r] = m == 0xffffu ? 0u : ((lane + 1) << 16) | m;
+      }
+#pragma unroll
+      for (uint32_t r = 0; r < R; r++) {
+        k[r] = wave_max_dpp(k[r]);
+        c[r] = k[r] ? k[r] & 0xffff : carry;
+        carry = rdlane(c[r], kWave - 1);
+      }
     }
 #pragma unroll
     for (uint32_t r = 0; r < R; r++) {
-      k[r] = wave_max_dpp(k[r]);
-      c[r] = k[r] ? k[r] & 0xffff : carry;
-      carry = rdlane(c[r], kWave - 1);
-    }
-#pragma unroll
-    for (uint32_t r = 0; r < R; r++) {
-      const uint32_t i = row + r * kWave + lane;
+      const uint32_t i = at(row, r);
       // a distance beyond the window; past the stored bytes it may be anything,
       // and an offset below 0 lies outside the buffer
       const bool isfar = c[r] >= i && c[r] < 0x8000u;
@@ -88,10 +116,11 @@ __device__ __forceinline__ void resolve_window(uint8_t *dst, uint16_t *win, uint
     uint32_t v[R];
 #pragma unroll
     for (uint32_t r = 0; r < R; r++) {
-      const uint32_t i = row + r * kWave + lane;
+      const uint32_t i = at(row, r);
       v[r] = c[r] < i ? i - 1 - c[r] : (c[r] >= 0x8000u ? c[r] : 0x8000u | f[r]);
-      win[i] = (uint16_t)v[r];
+      if constexpr (!QUADS) win[i] = (uint16_t)v[r];
     }
+    if constexpr (QUADS) write4(row, v);
     // an index in another wave's segment waits for the second pass
     for (;;) {
       bool go[R], more = false;
@@ -108,8 +137,9 @@ __device__ __forceinline__ void resolve_window(uint8_t *dst, uint16_t *win, uint
 #pragma unroll
       for (uint32_t r = 0; r < R; r++) {
         v[r] = go[r] ? t[r] : v[r];
-        win[row + r * kWave + lane] = (uint16_t)v[r];
+        if constexpr (!QUADS) win[at(row, r)] = (uint16_t)v[r];
       }
+      if constexpr (QUADS) write4(row, v);
     }
     if constexpr (NW > 1) {
       uint32_t low = v[0];
@@ -136,8 +166,12 @@ __device__ __forceinline__ void resolve_window(uint8_t *dst, uint16_t *win, uint
       const uint32_t row = s0 + (uint32_t)__builtin_ctzll(late) * G;
       late &= late - 1;
       uint32_t v[R];
+      if constexpr (QUADS) {
+        read4(row, v);
+      } else {
 #pragma unroll
-      for (uint32_t r = 0; r < R; r++) v[r] = win[row + r * kWave + lane];
+        for (uint32_t r = 0; r < R; r++) v[r] = win[at(row, r)];
+      }
       for (;;) {
         uint32_t low = v[0];
 #pragma unroll
@@ -150,8 +184,9 @@ __device__ __forceinline__ void resolve_window(uint8_t *dst, uint16_t *win, uint
 #pragma unroll
         for (uint32_t r = 0; r < R; r++) {
           v[r] = v[r] < 0x8000u ? t[r] : v[r];
-          win[row + r * kWave + lane] = (uint16_t)v[r];
+          if constexpr (!QUADS) win[at(row, r)] = (uint16_t)v[r];
         }
+        if constexpr (QUADS) write4(row, v);
       }
     }
   }
