@@ -453,7 +453,7 @@ def _parallel(fn, items):
 
 def bench_batch(ctx, args):
     """Uneven batch: n zlib streams, sizes log-uniform 4 KiB..4 MiB, blocks mixed
-    fixed/dynamic/stored 20/75/5, decoded by one persistent graph-replayed launch."""
+    fixed/dynamic/stored 20/75/5, decoded by one persistent launch."""
     rng = np.random.default_rng(0xC0DA6 + 4)
     n = args.streams
     sizes = np.exp(rng.uniform(np.log(4096), np.log(4 << 20), n)).astype(np.int64)
@@ -574,7 +574,7 @@ def bench_batch(ctx, args):
                       f"system zlib {oracle.zlib_version()} inflate, one stream per task")
     return {
         "workload": f"batched uneven deflate, {n} zlib streams log-uniform 4 KiB-4 MiB, "
-                    "block mix fixed/dynamic/stored 20/75/5, one persistent graph-replayed launch",
+                    "block mix fixed/dynamic/stored 20/75/5, one persistent launch",
         "value": round(total / (ms / 1e3) / 1e9, 2), "unit": "GB/s", "ms_per_step": round(ms, 4),
         "dtype": "u8", "bit_exact": True, "streams": n,
         "decompressed_bytes": total, "compressed_bytes": int(slen.sum()),
