@@ -433,15 +433,19 @@ __device__ __forceinline__ int32_t read_dynamic(lds<Sh<C>> *S, uint32_t *qp, uin
   uint32_t q = *qp;
   const uint32_t h = uni(stage_bits(S->stage, q));
   const uint32_t nlen = (h & 31) + 257, ndist = ((h >> 5) & 31) + 1, ncode = ((h >> 10) & 15) + 4;
-  if (nlen > 286 || ndist > 30) return kCorrupt;  // zlib: "too many length or distance symbols"
   q += 14;
+  if (q > limit) return kTrunc;
+  if (nlen > 286 || ndist > 30) return kCorrupt;  // zlib: "too many length or distance symbols"
   if (lane < 19)  // code-length code lengths, 3 bits each, in permuted order
     S->lens[kClOrder[lane]] = lane < ncode ? (uint8_t)(stage_bits(S->stage, q + 3 * lane) & 7) : (uint8_t)0;
   q += 3 * ncode;
+  if (q > limit) return kTrunc;
   lds_order();
+  const uint32_t total = nlen + ndist;
+  // without any code zlib reads a length 0 from every bit, and no end-of-block in the end
+  if (!__ballot(lane < 19 && S->lens[lane])) return q + total > limit ? kTrunc : kCorrupt;
   int32_t st = (int32_t)uni((uint32_t)build_table(S->lens, 19, kTabCodes, &S->hl, S->tab, 0, kCodeBits, 0));
   if (st != kOk) return st;
-  const uint32_t total = nlen + ndist;
   for (uint32_t k = lane; k < sizeof(S->lens) / 4; k += kWave) reinterpret_cast<lds<uint32_t> *>(S->lens)[k] = 0;
   lds_order();
   uint32_t i = 0, prev = 0;
@@ -476,8 +480,9 @@ __device__ __forceinline__ int32_t read_dynamic(lds<Sh<C>> *S, uint32_t *qp, uin
     const uint32_t incl = wave_scan_dpp(start ? rep : 0u);
     const uint32_t off = i + incl - rep;
     const bool take = start && off < total;
-    // a repeat with no length before it, or past the last length
-    if (__ballot(take && ((sym == 16 && off == 0) || off + rep > total))) return kCorrupt;
+    // a repeat with no length before it, or past the last length: an error once it is read whole
+    const uint64_t bad = __ballot(take && ((sym == 16 && off == 0) || off + rep > total));
+    if (bad) return q + (uint32_t)__builtin_ctzll(bad) + rdlane(tl, (uint32_t)__builtin_ctzll(bad)) > limit ? kTrunc : kCorrupt;
     const uint32_t key = wave_max_dpp(start && sym != 16 ? ((lane + 1) << 8) | (sym < 16 ? sym : 0u) : 0u);
     const uint32_t val = key ? key & 0xff : prev;
     if (take && val)  // at most six copies of a length that is not 0
@@ -522,7 +527,7 @@ __device__ __forceinline__ int32_t one_symbol(const lds<Sh<C>> *S, uint32_t *q, 
                                               uint32_t *dist) {
   uint32_t L = 0;
   const int32_t sym = slow_decode(&S->hl, uni(stage_bits(S->stage, *q)), &L);
-  if (sym < 0) return *q > limit ? kTrunc : kCorrupt;
+  if (sym < 0) return *q >= limit ? kTrunc : kCorrupt;  // a set with such bits has one code, of one bit, or none
   *q += L;
   if (sym == 256) return kEob;
   if (sym > 285) return kCorrupt;
@@ -533,9 +538,9 @@ __device__ __forceinline__ int32_t one_symbol(const lds<Sh<C>> *S, uint32_t *q, 
   *len = len_base(c, lx) + __builtin_amdgcn_ubfe(uni(stage_bits(S->stage, *q)), 0, lx);
   *q += lx;
   const int32_t ds = slow_decode(&S->hd, uni(stage_bits(S->stage, *q)), &L);
-  if (ds < 0) return *q > limit ? kTrunc : kCorrupt;
-  if (ds >= 30) return kCorrupt;
+  if (ds < 0) return *q >= limit ? kTrunc : kCorrupt;
   *q += L;
+  if (ds >= 30) return kCorrupt;
   const uint32_t dx = dist_extra((uint32_t)ds);
   *dist = dist_base((uint32_t)ds, dx) + __builtin_amdgcn_ubfe(uni(stage_bits(S->stage, *q)), 0, dx);
   *q += dx;
