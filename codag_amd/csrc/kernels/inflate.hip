@@ -788,6 +788,7 @@ template <class C>
 __device__ __noinline__ uint64_t chain_entries(lds<Sh<C>> *S, uint32_t lo, uint32_t bound, uint32_t limit,
                                                uint32_t wave, uint32_t entry) {
   const uint32_t lane = lane_id();
+  if constexpr (C::kNW > 1) __syncthreads();  // every wave has read the pass's mis and stp
   uint32_t exits[4] = {0, 0, 0, 0};  // byte c: the exit behind `bound` of entry lo + c, 255 = stop
 #pragma unroll 1
   for (uint32_t c = 0; c < 16; c++) {
