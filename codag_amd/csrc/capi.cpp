@@ -30,11 +30,15 @@ void clear_error() { g_last_error.clear(); }
 
 using namespace codag;
 
+// A failed call's error is reported here and must not be found again by the check
+// after the next launch (hipGetLastError keeps it until it is read).
 #define HIP_TRY(expr)                                                                   \
   do {                                                                                  \
     hipError_t e_ = (expr);                                                             \
-    if (e_ != hipSuccess)                                                               \
+    if (e_ != hipSuccess) {                                                             \
+      (void)hipGetLastError();                                                          \
       return fail(CODAG_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));    \
+    }                                                                                   \
   } while (0)
 
 namespace {
@@ -896,7 +900,10 @@ codag_status codag_dev_alloc(codag_ctx *ctx, uint64_t bytes, void **d_ptr) {
   if (!ctx || !d_ptr) return fail(CODAG_ERR_INVALID, "dev_alloc: null argument");
   DeviceGuard g(ctx->device);
   hipError_t e = hipMalloc(d_ptr, bytes ? bytes : 1);
-  if (e == hipErrorOutOfMemory) return fail(CODAG_ERR_NOMEM, "hipMalloc: out of memory");
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return fail(CODAG_ERR_NOMEM, "hipMalloc: out of memory");
+  }
   HIP_TRY(e);
   return CODAG_OK;
 }
