@@ -66,7 +66,6 @@ struct codag_ctx {
   uint32_t cu_count = 0;
   char name[256] = {0};
   codag_tune_params tune[4];
-  bool tuned[4] = {};  // the shape was set or tuned by the caller
   uint32_t chunks_two_wave = 0;
   uint32_t poll_shift = 0;  // RLE v2 queue kernel: nonzero = waits without polls (tests)
 };
@@ -114,16 +113,68 @@ bool pipe_shape(const codag_tune_params &t) {
   return t.threads_per_group == 512 && t.window_bytes == 2048 && t.queue_depth == 4;
 }
 
-void default_tune(codag_ctx *c) {
-  // defaults: the fastest shapes on the benchmark columns (MI355X); the
-  // autotuner can pick per column
-  c->tune[CODAG_RLEV1] = {512, 2048, 0, 4};
-  c->tune[CODAG_RLEV2] = {128, 4096, 0, 2};
-  // batches by eight waves or one wave per stream, as their sizes have it, up
-  // to 12 workgroups per CU
-  c->tune[CODAG_DEFLATE] = {128, 0, 12, 1};
-  c->tune[0] = {0, 0, 0, 0};
+// The shapes of a new context. For RLE v1 and v2 they leave the kernel to the
+// launch's chunk count (rlev1_route, rlev2_route); another shape is launched as it
+// is. The shape alone says so, so that setting what tune_get returned changes
+// nothing. Deflate batches go by eight waves or one wave per stream, as their
+// sizes have it, up to 12 workgroups per CU.
+constexpr codag_tune_params kDefaultTune[4] = {{0, 0, 0, 0}, {512, 2048, 0, 4}, {128, 4096, 0, 2}, {128, 0, 12, 1}};
+
+bool same_shape(const codag_tune_params &a, const codag_tune_params &b) {
+  return std::memcmp(&a, &b, sizeof a) == 0;
 }
+
+enum Route : uint32_t {
+  kRouteGroup = 0,  // the per-chunk kernels
+  kRouteWave = 1,   // RLE v2, one wave per chunk
+  kRoutePc = 2,     // walker + expander waves: kRoutePc + expanders
+  kRoutePipe = 8,   // RLE v1 pipeline
+  kRouteSpan = 9,   // sixteen waves that walk and expand by turns
+};
+
+// With the default shape, all waves by turns up to one chunk per CU (us, pipeline
+// and turns: 256 chunks of an 8-bit table column 2448, 430, of the 64-bit benchmark
+// column 76, 67; above it dense columns still gain, 512 chunks 2467, 543, but the
+// benchmark column loses, 84, 95).
+uint32_t rlev1_route(const codag_tune_params &t, uint64_t n, uint32_t w, uint64_t chunk_bytes, uint32_t cus) {
+  if (same_shape(t, kDefaultTune[CODAG_RLEV1]) && n <= cus) return kRouteSpan;
+  if (pipe_shape(t)) return chunk_bytes / w <= (1u << 17) ? kRoutePipe : kRouteGroup;  // its descriptors' value field
+  if (pc_shape(t)) return kRoutePc + t.threads_per_group / 64 - 1;
+  return kRouteGroup;
+}
+
+// With the default shape, 16 waves per chunk that walk and expand by turns while
+// two such groups per CU hold all chunks, as a lone walker's chain then bounds the
+// launch (walker and three expanders, then 16 waves, us: 16-bit table column, 64
+// chunks 917, 376, 512 chunks 1063, 486, 1024 chunks 1054, 807; 64-bit benchmark
+// column, 512 chunks 153, 127, 1024 chunks 152, 232). Above that, expanders by the
+// chunk count: three up to 6 chunks per CU and two up to 12 (1, 2 and 3 expanders,
+// us: 16-bit table column, 1024 chunks 2276, 1276, 1051; 32-bit benchmark column,
+// 1024 chunks 254, 249, 249, 2048 chunks 342, 317, 321). `polls`: the walker's
+// waits are as usual (a test takes their polls away).
+uint32_t rlev2_route(const codag_tune_params &t, uint64_t n, uint32_t cus, bool polls) {
+  if (same_shape(t, kDefaultTune[CODAG_RLEV2])) {
+    if (n <= 2ull * cus && polls) return kRouteSpan;
+    return kRoutePc + (n <= 6ull * cus ? 3 : (n <= 12ull * cus ? 2 : 1));
+  }
+  if (v2_pc_shape(t)) return kRoutePc + t.threads_per_group / 64 - 1;
+  return t.threads_per_group == 64 ? kRouteWave : kRouteGroup;
+}
+
+void default_tune(codag_ctx *c) {
+  for (int k = 0; k < 4; k++) c->tune[k] = kDefaultTune[k];
+}
+
+// Gives a codec its shape back, however the scope ends, unless `keep` is set.
+struct TuneGuard {
+  codag_tune_params &shape;
+  const codag_tune_params saved;
+  bool keep = false;
+  explicit TuneGuard(codag_tune_params &s) : shape(s), saved(s) {}
+  ~TuneGuard() {
+    if (!keep) shape = saved;
+  }
+};
 
 // RAII device buffer used by the synchronous host wrappers.
 struct DevBuf {
@@ -261,26 +312,20 @@ codag_status codag_rlev1_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t 
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "rlev1_decode: too many chunks");
   DeviceGuard g(ctx->device);
   const codag_tune_params &t = ctx->tune[CODAG_RLEV1];
-  // Unless the caller chose a shape: all waves by turns up to one chunk per CU
-  // (us, pipeline and turns: 256 chunks of an 8-bit table column 2448, 430, of the
-  // 64-bit benchmark column 76, 67; above it dense columns still gain, 512 chunks
-  // 2467, 543, but the benchmark column loses, 84, 95).
-  if (!ctx->tuned[CODAG_RLEV1] && n_chunks <= ctx->cu_count)
+  const uint32_t route = rlev1_route(t, n_chunks, w, chunk_bytes, ctx->cu_count);
+  if (route == kRouteSpan)
     HIP_TRY(launch_rlev1_span(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                               d_out, d_status, pick(ctx, stream)));
-  else if (pipe_shape(t) && chunk_bytes / w <= (1u << 17))  // pipelined walker + helpers
+  else if (route == kRoutePipe)  // pipelined walker + helpers
     HIP_TRY(launch_rlev1_pipe(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                               d_out, d_status, pick(ctx, stream)));
-  else if (pipe_shape(t))  // values per chunk beyond the pipeline's descriptor field
-    HIP_TRY(launch_rlev1_decode(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w,
-                                chunk_bytes, d_out, d_status, 512, 4096, pick(ctx, stream)));
-  else if (pc_shape(t))  // walker wave + expander waves per chunk
+  else if (route > kRoutePc)  // walker wave + expander waves per chunk
     HIP_TRY(launch_rlev1_pc(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
-                            d_out, d_status, t.threads_per_group / 64 - 1, pick(ctx, stream)));
+                            d_out, d_status, route - kRoutePc, pick(ctx, stream)));
   else
     HIP_TRY(launch_rlev1_decode(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w,
-                                chunk_bytes, d_out, d_status, t.threads_per_group, t.window_bytes,
-                                pick(ctx, stream)));
+                                chunk_bytes, d_out, d_status, t.threads_per_group,
+                                pipe_shape(t) ? 4096 : t.window_bytes, pick(ctx, stream)));
   return CODAG_OK;
 }
 
@@ -295,24 +340,14 @@ codag_status codag_rlev2_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t 
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "rlev2_decode: too many chunks");
   DeviceGuard g(ctx->device);
   const codag_tune_params &t = ctx->tune[CODAG_RLEV2];
-  // Unless the caller chose a shape: 16 waves per chunk that walk and expand by
-  // turns while two such groups per CU hold all chunks, as a lone walker's chain
-  // then bounds the launch (walker and three expanders, then 16 waves, us: 16-bit
-  // table column, 64 chunks 917, 376, 512 chunks 1063, 486, 1024 chunks 1054, 807;
-  // 64-bit benchmark column, 512 chunks 153, 127, 1024 chunks 152, 232). Above that,
-  // expanders by the chunk count: three up to 6 chunks per CU and two up to 12
-  // (1, 2 and 3 expanders, us: 16-bit table column, 1024 chunks 2276, 1276, 1051;
-  // 32-bit benchmark column, 1024 chunks 254, 249, 249, 2048 chunks 342, 317, 321).
-  const bool chosen = ctx->tuned[CODAG_RLEV2];
-  uint32_t nexp = t.threads_per_group / 64 - 1;
-  if (!chosen) nexp = n_chunks <= 6ull * ctx->cu_count ? 3 : (n_chunks <= 12ull * ctx->cu_count ? 2 : 1);
-  if (!chosen && !ctx->poll_shift && n_chunks <= 2ull * ctx->cu_count)
+  const uint32_t route = rlev2_route(t, n_chunks, ctx->cu_count, ctx->poll_shift == 0);
+  if (route == kRouteSpan)
     HIP_TRY(launch_rlev2_span(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                               d_out, d_status, pick(ctx, stream)));
-  else if (v2_pc_shape(t))  // walker wave + expander waves per chunk
+  else if (route > kRoutePc)  // walker wave + expander waves per chunk
     HIP_TRY(launch_rlev2_pc(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
-                            d_out, d_status, nexp, ctx->poll_shift, pick(ctx, stream)));
-  else if (t.threads_per_group == 64)  // one self-contained wave per chunk
+                            d_out, d_status, route - kRoutePc, ctx->poll_shift, pick(ctx, stream)));
+  else if (route == kRouteWave)  // one self-contained wave per chunk
     HIP_TRY(launch_rlev2_wave(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                               d_out, d_status, t.window_bytes, pick(ctx, stream)));
   else
@@ -755,6 +790,15 @@ codag_status codag_test_chunks_two_wave(codag_ctx *ctx, uint32_t on) {
   return CODAG_OK;
 }
 
+// Test hook, not in the public header: the kernel (a Route) that a decode of n
+// chunks is launched with.
+uint32_t codag_test_route(codag_ctx *ctx, codag_codec codec, uint64_t n, uint32_t w, uint64_t chunk_bytes) {
+  if (!ctx || (codec != CODAG_RLEV1 && codec != CODAG_RLEV2)) return ~0u;
+  const codag_tune_params &t = ctx->tune[codec];
+  return codec == CODAG_RLEV1 ? rlev1_route(t, n, w, chunk_bytes, ctx->cu_count)
+                              : rlev2_route(t, n, ctx->cu_count, ctx->poll_shift == 0);
+}
+
 // Test hook, not in the public header (no counterpart in the reference):
 // `shift` nonzero switches the RLE v2 walker + expander kernel to its
 // variant without polls in its bounded waits (0 restores the normal one), so
@@ -789,7 +833,6 @@ codag_status codag_tune_set(codag_ctx *ctx, codag_codec codec, const codag_tune_
   if (codec == CODAG_DEFLATE && p->threads_per_group != 64 && p->threads_per_group != 128)
     return fail(CODAG_ERR_INVALID, "tune_set: Deflate threads_per_group must be 64 or 128");
   ctx->tune[codec] = *p;
-  ctx->tuned[codec] = true;
   return CODAG_OK;
 }
 
@@ -818,9 +861,8 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
     const uint32_t shapes[][2] = {{256, 4096}, {128, 4096}, {512, 4096}, {256, 8192}, {512, 8192}};
     for (auto &sh : shapes) cands.push_back({sh[0], sh[1], 0, 0});
   }
-  const codag_tune_params saved = ctx->tune[codec];
-  const bool was_tuned = ctx->tuned[codec];
-  ctx->tuned[codec] = true;
+  TuneGuard guard(ctx->tune[codec]);
+  const codag_tune_params saved = guard.saved;
   const uint64_t out_bytes = n_chunks * chunk_bytes;
   std::vector<uint8_t> ref, cur;
   float bestt = 1e30f, saved_ms = 0;
@@ -845,8 +887,6 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
   }
   for (size_t ci = 0; ci < cands.size(); ci++) {
     ctx->tune[codec] = cands[ci];
-    // the shape in use runs as it is in use: one that nobody chose by chunk count
-    ctx->tuned[codec] = was_tuned || std::memcmp(&cands[ci], &saved, sizeof saved) != 0;
     auto run = [&]() -> codag_status {
       if (codec == CODAG_RLEV1)
         return codag_rlev1_decode(ctx, d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w,
@@ -858,11 +898,7 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
                                  d_res.as<codag_stream_result>(), 0, ctx->stream);
     };
     codag_status s = run();  // warm-up
-    if (s) {
-      ctx->tune[codec] = saved;
-      ctx->tuned[codec] = was_tuned;
-      return s;
-    }
+    if (s) return s;
     HIP_TRY(hipEventRecord(ctx->ev0, ctx->stream));
     for (int r = 0; r < reps; r++) run();
     HIP_TRY(hipEventRecord(ctx->ev1, ctx->stream));
@@ -879,7 +915,7 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
       bestt = ms;
       bestp = cands[ci];
     }
-    if (same && std::memcmp(&cands[ci], &saved, sizeof saved) == 0) saved_ms = ms;
+    if (same && same_shape(cands[ci], saved)) saved_ms = ms;
   }
   // the shape in use stays unless a candidate beats it by more than 2%
   // (run-to-run noise must not flip the choice)
@@ -888,7 +924,7 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
     bestt = saved_ms;
   }
   ctx->tune[codec] = bestp;
-  ctx->tuned[codec] = was_tuned || std::memcmp(&bestp, &saved, sizeof saved) != 0;
+  guard.keep = true;
   if (best) *best = bestp;
   if (best_ms) *best_ms = bestt;
   return CODAG_OK;

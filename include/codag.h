@@ -396,8 +396,12 @@ typedef enum codag_codec { CODAG_RLEV1 = 1, CODAG_RLEV2 = 2, CODAG_DEFLATE = 3 }
  * (window 4096; 128, 192 (RLE v2 only) or 256 threads = 1, 2 or 3 expander
  * waves), 4 the RLE v1 pipeline (512 threads, window 2048). For Deflate's
  * batch launch (codag_inflate_batch), 64 threads = one wave per stream, 128
- * = eight waves or one wave per stream, by the streams' number and sizes. codag_tune_set rejects shapes
- * that are not compiled in. */
+ * = eight waves or one wave per stream, by the streams' number and sizes.
+ * A new context's RLE shapes (RLE v1: 512, 2048, 0, 4; RLE v2: 128, 4096, 0, 2)
+ * leave the kernel to each launch's chunk count: sixteen waves per chunk up to
+ * one (RLE v1) or two (RLE v2) chunks per CU, then the pipeline, or the walker
+ * with three, two or one expander. Any other shape is launched as it is.
+ * codag_tune_set rejects shapes that are not compiled in. */
 typedef struct codag_tune_params {
   uint32_t threads_per_group; /* workgroup size (64..1024, multiple of 64) */
   uint32_t window_bytes;      /* compressed bytes staged in LDS per window */
@@ -412,7 +416,7 @@ codag_status codag_tune_set(codag_ctx *ctx, codag_codec codec, const codag_tune_
  * d_col_len is ignored) and keep the fastest whose output equals the first
  * candidate's; the shape in use stays if it is within 2% of that one (a tie
  * in run-to-run noise does not flip the choice). The kept shape becomes the
- * context's shape. best_ms (nullable) gets its time. DEFLATE candidates differ in
+ * context's shape; on an error the context's shape stays. best_ms (nullable) gets its time. DEFLATE candidates differ in
  * the batch launch's workgroups (one wave per stream, or by size) and workgroups
  * per CU; the launch has min(CUs x groups_per_cu, n_chunks) workgroups, so
  * the sample needs more than CUs x 28 streams for all of them to differ. */

@@ -1,0 +1,104 @@
+"""Which kernel an RLE launch takes: the default shape leaves it to the chunk
+count, and does so again after it was read, replaced and put back, and after an
+autotuner call that failed. The kernels of larger launches (RLE v1: the
+pipeline; RLE v2: walker and expanders) give the statuses and values that those
+of small launches give, and the oracle's: streams are repeated until there are
+more chunks than the small launches take."""
+import numpy as np
+import pytest
+
+import codag_amd as ca
+import oracle
+from tests.gpu_helpers import rle_decode, say
+from tests import test_gpu_rlev1_spans as v1
+from tests import test_gpu_rlev2_spans as v2
+
+pytestmark = pytest.mark.gpu
+
+PC, PIPE, SPAN = 2, 8, 9  # capi.cpp, enum Route
+
+
+@pytest.fixture(scope="module")
+def ctx(gpu_required):
+    c = ca.Context(0)
+    yield c
+    c.close()
+
+
+def routes(ctx, codec):
+    cus = ctx.info()[1]
+    return [ca.lib().codag_test_route(ctx.h, codec, n, 4, 131072)
+            for n in (1, cus, cus + 1, 2 * cus, 2 * cus + 1, 6 * cus + 1, 12 * cus + 1)]
+
+
+DEFAULT = {ca.RLEV1: [SPAN, SPAN] + [PIPE] * 5, ca.RLEV2: [SPAN] * 4 + [PC + 3, PC + 2, PC + 1]}
+
+
+@pytest.mark.parametrize("codec,other,routed", [(ca.RLEV1, (256, 4096, 2), PC + 3), (ca.RLEV2, (192, 4096, 2), PC + 2)])
+def test_shape_put_back(ctx, codec, other, routed):
+    say(f"rle routes, codec {codec}")
+    assert routes(ctx, codec) == DEFAULT[codec]
+    saved = ctx.tune_get(codec)
+    ctx.tune_set(codec, ctx.tune_get(codec))
+    assert routes(ctx, codec) == DEFAULT[codec]
+    ctx.tune_set(codec, ca.TuneParams(other[0], other[1], 0, other[2]))
+    assert routes(ctx, codec) == [routed] * 7
+    ctx.tune_set(codec, saved)
+    assert routes(ctx, codec) == DEFAULT[codec]
+
+
+@pytest.mark.parametrize("codec", [ca.RLEV1, ca.RLEV2])
+def test_failed_tune_run_keeps_the_shape(ctx, codec):
+    say(f"rle routes after an autotuner call with a bad width, codec {codec}")
+    d = ctx.alloc(64)
+    with pytest.raises(ca.CodagError):
+        ctx.tune_run(codec, d, 8, d, d, 1, 3, 12, d, reps=1)  # 3-byte elements
+    assert routes(ctx, codec) == DEFAULT[codec]
+    with pytest.raises(ca.CodagError):
+        ctx.tune_run(codec, d, 8, d, d, 1 << 60, 1, 16, d, reps=1)  # no room for the statuses
+    assert routes(ctx, codec) == DEFAULT[codec]
+
+
+def repeated(ctx, codec, streams, w, chunk, per_cu):
+    """The streams by a small launch, and repeated by one of more than per_cu chunks per CU."""
+    n = len(streams)
+    off = np.cumsum([0] + [(len(s) + 15) // 16 * 16 + 1 + i % 7 for i, s in enumerate(streams)]).astype(np.uint64)
+    comp = np.zeros(int(off[-1]) + 16, np.uint8)
+    for a, s in zip(off, streams):
+        comp[int(a):int(a) + len(s)] = np.frombuffer(s, np.uint8)
+    cl = np.array([len(s) for s in streams], np.uint64)
+    k = np.arange(per_cu * ctx.info()[1] + 1) % n
+    want = rle_decode(ctx, codec, comp, off[:-1], cl, w, chunk)
+    st, out = rle_decode(ctx, codec, comp, off[:-1][k], cl[k], w, chunk)
+    assert st.tolist() == want[0][k].tolist()
+    out, ref = out.reshape(len(k), chunk), want[1].reshape(n, chunk)
+    for i, j in enumerate(k):
+        if want[0][j] == 0:
+            assert np.array_equal(out[i], ref[j]), (i, j)
+    return comp, off, cl, want[0]
+
+
+@pytest.mark.parametrize("w", [1, 2, 4, 8])
+@pytest.mark.parametrize("kind", ["runs", "wide_runs", "ones", "long", "huge", "mixed"])
+def test_v1_pipeline_segments(ctx, kind, w):
+    say(f"rlev1 pipeline, {kind}, width {w}")
+    rng = np.random.default_rng(160 + w)
+    streams = [v1.stream(rng, n, kind) for n in (1, 2000, 2048, 8191, 8192, 16384)]
+    streams += [b"", bytes([0]), bytes([0, 1]), bytes([255])]
+    for cap in (1, 65, 4099):
+        comp, off, cl, st = repeated(ctx, ca.RLEV1, streams, w, cap * w, 1)
+        assert st.tolist() == oracle.rlev1_decode_chunks(comp, off[:-1], cl, w, cap * w, threads=8)[0].tolist()
+
+
+@pytest.mark.parametrize("w", [1, 2, 4, 8])
+def test_v2_walker_blocks(ctx, w):
+    say(f"rlev2 walker and expanders, width {w}")
+    rng = np.random.default_rng(180 + w)
+    streams = v2.streams_of(rng, 9000, 24) + [b"", b"\x00", b"\x01\x02"]
+    for i in range(24):
+        s = bytearray(streams[i])
+        for _ in range(1 + i % 3):
+            s[int(rng.integers(0, len(s)))] = int(rng.integers(0, 256))
+        streams.append(bytes(s[:len(s) if i % 2 else int(rng.integers(1, len(s)))]))
+    for cap in (700, 60000):
+        repeated(ctx, ca.RLEV2, streams, w, cap * w, 2)
