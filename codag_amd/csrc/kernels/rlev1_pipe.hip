@@ -477,7 +477,8 @@ rlev1_pipe_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes,
       if (rem < 16) m &= (1u << rem) - 1;
       found |= m;
     }
-    if (lane == 0 && status) status[chunk] = __ballot(found != 0) ? kCorrupt : kTrunc;
+    const uint64_t any = __ballot(found != 0);  // of all lanes: not inside lane 0's branch
+    if (lane == 0 && status) status[chunk] = any ? kCorrupt : kTrunc;
   }
 }
 

@@ -90,6 +90,30 @@ def test_v1_pipeline_segments(ctx, kind, w):
         assert st.tolist() == oracle.rlev1_decode_chunks(comp, off[:-1], cl, w, cap * w, threads=8)[0].tolist()
 
 
+@pytest.mark.parametrize("w", [1, 8])
+def test_v1_pipeline_damaged(ctx, w):
+    """Damaged streams, overlong varints up to many windows long among them."""
+    say(f"rlev1 pipeline, damaged, width {w}")
+    rng = np.random.default_rng(170 + w)
+    streams = []
+    for i in range(40):
+        s = bytearray(v1.stream(rng, 9000, "mixed"))
+        k = int(rng.integers(0, len(s)))
+        if i % 4 == 0:
+            s[k:k + int(rng.choice([9, 10, 11, 3000, 9000]))] = b"\xff" * min(9000, len(s) - k)
+        elif i % 4 == 1:
+            s = s[:k]
+        for _ in range(i % 3):
+            s[int(rng.integers(0, len(s)))] = int(rng.integers(0, 256))
+        streams.append(bytes(s))
+    for k in (9, 10, 11, 2040, 4090, 4100, 6000, 8170, 9000, 20000):
+        for end in (b"\x01", b"\x01" + bytes(40), b""):
+            streams += [b"\xff" + b"\x80" * k + end, b"\x05\x81" + b"\x90" * k + end, b"\x05\x02" + b"\x90" * k + end]
+    comp, off, cl, st = repeated(ctx, ca.RLEV1, streams, w, 3000 * w, 1)
+    assert st.tolist() == oracle.rlev1_decode_chunks(comp, off[:-1], cl, w, 3000 * w, threads=8)[0].tolist()
+    assert {1, 3} <= set(st.tolist())
+
+
 @pytest.mark.parametrize("w", [1, 2, 4, 8])
 def test_v2_walker_blocks(ctx, w):
     say(f"rlev2 walker and expanders, width {w}")
