@@ -135,9 +135,13 @@ enum Route : uint32_t {
 // With the default shape, all waves by turns up to one chunk per CU (us, pipeline
 // and turns: 256 chunks of an 8-bit table column 2448, 430, of the 64-bit benchmark
 // column 76, 67; above it dense columns still gain, 512 chunks 2467, 543, but the
-// benchmark column loses, 84, 95).
-uint32_t rlev1_route(const codag_tune_params &t, uint64_t n, uint32_t w, uint64_t chunk_bytes, uint32_t cus) {
-  if (same_shape(t, kDefaultTune[CODAG_RLEV1]) && n <= cus) return kRouteSpan;
+// benchmark column loses, 84, 95). Narrow columns of random values, literal groups
+// of varints longer than the values, stay with the pipeline (256 chunks of random
+// 16-bit values 192, 202; of 8-bit ones 317, 316).
+uint32_t rlev1_route(const codag_tune_params &t, uint64_t n, uint32_t w, uint64_t chunk_bytes, uint64_t comp_bytes,
+                     uint32_t cus) {
+  const bool random = w <= 2 && comp_bytes / 5 > n * chunk_bytes / 4;
+  if (same_shape(t, kDefaultTune[CODAG_RLEV1]) && n <= cus && !random) return kRouteSpan;
   if (pipe_shape(t)) return chunk_bytes / w <= (1u << 17) ? kRoutePipe : kRouteGroup;  // its descriptors' value field
   if (pc_shape(t)) return kRoutePc + t.threads_per_group / 64 - 1;
   return kRouteGroup;
@@ -150,10 +154,24 @@ uint32_t rlev1_route(const codag_tune_params &t, uint64_t n, uint32_t w, uint64_
 // column, 512 chunks 153, 127, 1024 chunks 152, 232). Above that, expanders by the
 // chunk count: three up to 6 chunks per CU and two up to 12 (1, 2 and 3 expanders,
 // us: 16-bit table column, 1024 chunks 2276, 1276, 1051; 32-bit benchmark column,
-// 1024 chunks 254, 249, 249, 2048 chunks 342, 317, 321). `polls`: the walker's
-// waits are as usual (a test takes their polls away).
-uint32_t rlev2_route(const codag_tune_params &t, uint64_t n, uint32_t cus, bool polls) {
+// 1024 chunks 254, 249, 249, 2048 chunks 342, 317, 321).
+// One walker and one expander where that work is not there: streams of up to 128
+// bytes a chunk (16 chunks of 1024 equal values: 7.8 by one, 9.1 by 16 waves), and
+// columns of wide DIRECT blocks, a few of which fill a step that 16 waves size
+// byte by byte (random 64-bit values, one expander, three, and 16 waves: 256 chunks
+// 180, 187, 235, 512 chunks 184, 191, 352; 40 bits, 256 chunks 137, 142, 147; 32
+// bits, 16 chunks 119, 122, 124, 256 chunks 131, 135, 127; 20 bits, 256 chunks
+// 118, 120, 99, 512 chunks 124, 126, 148; 16 bits, 512 chunks 114, 116, 110): from
+// 3.5 stream bytes a value at one chunk per CU, from 2.25 above. comp_bytes may
+// hold more than the chunks, which makes a column look wide: that is the kernel of
+// one walker, not an error. `polls`: the walker's waits are as usual (a test takes
+// their polls away).
+uint32_t rlev2_route(const codag_tune_params &t, uint64_t n, uint32_t w, uint64_t chunk_bytes, uint64_t comp_bytes,
+                     uint32_t cus, bool polls) {
   if (same_shape(t, kDefaultTune[CODAG_RLEV2])) {
+    const uint64_t values = n * (chunk_bytes / w);
+    const uint64_t quarters = n <= cus ? 14 : 9;  // of a stream byte, per value
+    if (comp_bytes <= 128 * n || comp_bytes / quarters > values / 4) return kRoutePc + 1;
     if (n <= 2ull * cus && polls) return kRouteSpan;
     return kRoutePc + (n <= 6ull * cus ? 3 : (n <= 12ull * cus ? 2 : 1));
   }
@@ -312,7 +330,7 @@ codag_status codag_rlev1_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t 
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "rlev1_decode: too many chunks");
   DeviceGuard g(ctx->device);
   const codag_tune_params &t = ctx->tune[CODAG_RLEV1];
-  const uint32_t route = rlev1_route(t, n_chunks, w, chunk_bytes, ctx->cu_count);
+  const uint32_t route = rlev1_route(t, n_chunks, w, chunk_bytes, comp_bytes, ctx->cu_count);
   if (route == kRouteSpan)
     HIP_TRY(launch_rlev1_span(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                               d_out, d_status, pick(ctx, stream)));
@@ -340,7 +358,8 @@ codag_status codag_rlev2_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t 
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "rlev2_decode: too many chunks");
   DeviceGuard g(ctx->device);
   const codag_tune_params &t = ctx->tune[CODAG_RLEV2];
-  const uint32_t route = rlev2_route(t, n_chunks, ctx->cu_count, ctx->poll_shift == 0);
+  const uint32_t route =
+      rlev2_route(t, n_chunks, w, chunk_bytes, comp_bytes, ctx->cu_count, ctx->poll_shift == 0);
   if (route == kRouteSpan)
     HIP_TRY(launch_rlev2_span(d_comp, comp_bytes, d_blk_off, d_col_len, n_chunks, w, chunk_bytes,
                               d_out, d_status, pick(ctx, stream)));
@@ -792,11 +811,12 @@ codag_status codag_test_chunks_two_wave(codag_ctx *ctx, uint32_t on) {
 
 // Test hook, not in the public header: the kernel (a Route) that a decode of n
 // chunks is launched with.
-uint32_t codag_test_route(codag_ctx *ctx, codag_codec codec, uint64_t n, uint32_t w, uint64_t chunk_bytes) {
+uint32_t codag_test_route(codag_ctx *ctx, codag_codec codec, uint64_t comp_bytes, uint64_t n, uint32_t w,
+                          uint64_t chunk_bytes) {
   if (!ctx || (codec != CODAG_RLEV1 && codec != CODAG_RLEV2)) return ~0u;
   const codag_tune_params &t = ctx->tune[codec];
-  return codec == CODAG_RLEV1 ? rlev1_route(t, n, w, chunk_bytes, ctx->cu_count)
-                              : rlev2_route(t, n, ctx->cu_count, ctx->poll_shift == 0);
+  return codec == CODAG_RLEV1 ? rlev1_route(t, n, w, chunk_bytes, comp_bytes, ctx->cu_count)
+                              : rlev2_route(t, n, w, chunk_bytes, comp_bytes, ctx->cu_count, ctx->poll_shift == 0);
 }
 
 // Test hook, not in the public header (no counterpart in the reference):

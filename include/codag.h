@@ -398,9 +398,10 @@ typedef enum codag_codec { CODAG_RLEV1 = 1, CODAG_RLEV2 = 2, CODAG_DEFLATE = 3 }
  * batch launch (codag_inflate_batch), 64 threads = one wave per stream, 128
  * = eight waves or one wave per stream, by the streams' number and sizes.
  * A new context's RLE shapes (RLE v1: 512, 2048, 0, 4; RLE v2: 128, 4096, 0, 2)
- * leave the kernel to each launch's chunk count: sixteen waves per chunk up to
- * one (RLE v1) or two (RLE v2) chunks per CU, then the pipeline, or the walker
- * with three, two or one expander. Any other shape is launched as it is.
+ * leave the kernel to each launch's chunk count and stream bytes: sixteen waves
+ * per chunk up to one (RLE v1) or two (RLE v2) chunks per CU, unless the column
+ * is one of wide or random narrow values; then the pipeline, or the walker with
+ * three, two or one expander. Any other shape is launched as it is.
  * codag_tune_set rejects shapes that are not compiled in. */
 typedef struct codag_tune_params {
   uint32_t threads_per_group; /* workgroup size (64..1024, multiple of 64) */

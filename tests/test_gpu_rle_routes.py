@@ -27,7 +27,7 @@ def ctx(gpu_required):
 
 def routes(ctx, codec):
     cus = ctx.info()[1]
-    return [ca.lib().codag_test_route(ctx.h, codec, n, 4, 131072)
+    return [ca.lib().codag_test_route(ctx.h, codec, n * 30000, n, 4, 131072)
             for n in (1, cus, cus + 1, 2 * cus, 2 * cus + 1, 6 * cus + 1, 12 * cus + 1)]
 
 
@@ -85,12 +85,12 @@ def test_v1_pipeline_segments(ctx, kind, w):
     rng = np.random.default_rng(160 + w)
     streams = [v1.stream(rng, n, kind) for n in (1, 2000, 2048, 8191, 8192, 16384)]
     streams += [b"", bytes([0]), bytes([0, 1]), bytes([255])]
-    for cap in (1, 65, 4099):
+    for cap in (1, 65, 4099, 30000):
         comp, off, cl, st = repeated(ctx, ca.RLEV1, streams, w, cap * w, 1)
         assert st.tolist() == oracle.rlev1_decode_chunks(comp, off[:-1], cl, w, cap * w, threads=8)[0].tolist()
 
 
-@pytest.mark.parametrize("w", [1, 8])
+@pytest.mark.parametrize("w", [1, 2, 8])
 def test_v1_pipeline_damaged(ctx, w):
     """Damaged streams, overlong varints up to many windows long among them."""
     say(f"rlev1 pipeline, damaged, width {w}")
@@ -109,9 +109,10 @@ def test_v1_pipeline_damaged(ctx, w):
     for k in (9, 10, 11, 2040, 4090, 4100, 6000, 8170, 9000, 20000):
         for end in (b"\x01", b"\x01" + bytes(40), b""):
             streams += [b"\xff" + b"\x80" * k + end, b"\x05\x81" + b"\x90" * k + end, b"\x05\x02" + b"\x90" * k + end]
-    comp, off, cl, st = repeated(ctx, ca.RLEV1, streams, w, 3000 * w, 1)
-    assert st.tolist() == oracle.rlev1_decode_chunks(comp, off[:-1], cl, w, 3000 * w, threads=8)[0].tolist()
-    assert {1, 3} <= set(st.tolist())
+    for cap in (3000, 30000):  # shorter than most streams; room for all
+        comp, off, cl, st = repeated(ctx, ca.RLEV1, streams, w, cap * w, 1)
+        assert st.tolist() == oracle.rlev1_decode_chunks(comp, off[:-1], cl, w, cap * w, threads=8)[0].tolist()
+        assert {1, 3} <= set(st.tolist())
 
 
 @pytest.mark.parametrize("w", [1, 2, 4, 8])
@@ -126,3 +127,55 @@ def test_v2_walker_blocks(ctx, w):
         streams.append(bytes(s[:len(s) if i % 2 else int(rng.integers(1, len(s)))]))
     for cap in (700, 60000):
         repeated(ctx, ca.RLEV2, streams, w, cap * w, 2)
+
+
+def test_v2_routes_by_bytes(ctx):
+    """Streams of up to 128 bytes, and from 3.5 (2.25 above one chunk per CU) stream bytes a value on."""
+    say("rlev2 routes by bytes")
+    cus = ctx.info()[1]
+
+    def route(comp_bytes, n):
+        return ca.lib().codag_test_route(ctx.h, ca.RLEV2, comp_bytes, n, 8, 8192)  # 1024 values a chunk
+
+    for n in (1, cus, cus + 1, 2 * cus):
+        line = n * (3584 if n <= cus else 2304)
+        assert route(128 * n + 1, n) == SPAN and route(128 * n, n) == PC + 1
+        assert route(line, n) == SPAN and route(line + 16, n) == PC + 1
+    assert route(2304 * 3 * cus, 3 * cus) == PC + 3 and route(2304 * 3 * cus + 16, 3 * cus) == PC + 1
+    assert route((1 << 64) - 1, 2 * cus) == PC + 1 and route(0, 1) == PC + 1
+
+
+def test_v1_routes_by_bytes(ctx):
+    say("rlev1 routes by bytes")
+    for w, above in ((1, PIPE), (2, PIPE), (4, SPAN), (8, SPAN)):
+        for n in (1, ctx.info()[1]):
+            line = n * 8192 * 5 // 4
+            got = [ca.lib().codag_test_route(ctx.h, ca.RLEV1, b, n, w, 8192) for b in (line, line + 5)]
+            assert got == [SPAN, above]
+
+
+def test_v1_random_narrow_columns(ctx):
+    """Columns at both sides of that line, by one launch each."""
+    say("rlev1 random narrow columns")
+    rng = np.random.default_rng(9)
+    for w, top in ((1, 100), (1, 256), (2, 16000), (2, 65536)):
+        raw = rng.integers(0, top, 20 * 4096 // w).astype("u%d" % w)
+        cont, off, ln, nc = ca.rlev1_encode(raw, w, 4096)
+        n = 20  # the container's last chunks are padding
+        st, out = rle_decode(ctx, ca.RLEV1, cont[8:8 + int(off[n - 1] + ln[n - 1])], off[:n], ln[:n], w, 4096)
+        assert not st.any() and out.tobytes() == raw.tobytes()
+
+
+@pytest.mark.parametrize("bits,w", [(64, 8), (40, 8), (32, 4), (20, 4), (0, 8)])
+def test_v2_wide_and_tiny_columns(ctx, bits, w):
+    """Random values of so many bits, or equal ones, around the chunk counts where the kernel changes."""
+    say(f"rlev2 wide columns, {bits} bits, width {w}")
+    rng = np.random.default_rng(bits + w)
+    cus, chunk = ctx.info()[1], 2048
+    m = (2 * cus + 1) * (chunk // w)
+    raw = (rng.integers(0, 1 << 63, m, dtype=np.uint64) << np.uint64(1) >> np.uint64(64 - bits) if bits else
+           np.full(m, 5)).astype("u%d" % w)
+    comp, off, ln, nc = ca.rlev2_encode(raw, w, chunk)
+    for n in (1, cus, cus + 1, 2 * cus, 2 * cus + 1):
+        st, out = rle_decode(ctx, ca.RLEV2, comp[:int(off[n - 1] + ln[n - 1])], off[:n], ln[:n], w, chunk)
+        assert not st.any() and out.tobytes() == raw[:n * (chunk // w)].tobytes()
