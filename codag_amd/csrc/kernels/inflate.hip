@@ -508,15 +508,34 @@ __device__ __forceinline__ int32_t read_dynamic(lds<Sh<C>> *S, uint32_t *qp, uin
   return (int32_t)uni((uint32_t)build_table(S->lens + nlen, ndist, kTabDist, &S->hd, S->tab, C::kDistAt, C::kDB, C::kDS));
 }
 
+// The tables of the fixed codes (RFC 1951 3.2.6), entry by entry from their closed
+// form: literals and lengths 256..279 have the 7-bit codes from 0 on, 0..143 the
+// 8-bit codes from 48, 280..287 from 192, 144..255 the 9-bit codes from 400; the
+// distances 5 bits. (Built from their lengths, as a dynamic block's, they were most
+// of the time of a stream of 64 bytes.)
 template <class C> __device__ __forceinline__ void load_fixed(lds<Sh<C>> *S) {
   const uint32_t lane = lane_id();
-  for (uint32_t s = lane; s < 288; s += kWave)
-    S->lens[s] = (uint8_t)(s < 144 ? 8 : (s < 256 ? 9 : (s < 280 ? 7 : 8)));
+  static_assert(C::kLB >= 9 && C::kDB >= 5, "no sub-tables");
+  for (uint32_t k = lane; k < (1u << C::kLB); k += kWave) {
+    const uint32_t v = __builtin_bitreverse32(k) >> 23, c = v >> 1;
+    const uint32_t L = v < 96 ? 7u : (v < 400 ? 8u : 9u);
+    const uint32_t sym = v < 96 ? 256 + (v >> 2) : (v < 400 ? (c < 192 ? c - 48 : c + 88) : v - 256);
+    S->tab[k] = make_entry(kTabLit, sym, L);
+  }
+  for (uint32_t k = lane; k < (1u << C::kDB); k += kWave)
+    S->tab[C::kDistAt + k] = make_entry(kTabDist, __builtin_bitreverse32(k) >> 27, 5);
+  for (uint32_t i = lane; i < 288; i += kWave)
+    S->hl.sym[i] = (uint16_t)(i < 24 ? 256 + i : (i < 168 ? i - 24 : (i < 176 ? i + 112 : i - 32)));
+  if (lane < 32) S->hd.sym[lane] = (uint16_t)lane;
+  if (lane < 16) {
+    S->hl.count[lane] = (uint16_t)(lane == 7 ? 24 : (lane == 8 ? 152 : (lane == 9 ? 112 : 0)));
+    S->hl.first[lane] = (uint16_t)(lane == 8 ? 48 : (lane == 9 ? 400 : 0));
+    S->hl.index[lane] = (uint16_t)(lane == 8 ? 24 : (lane == 9 ? 176 : 0));
+    S->hd.count[lane] = (uint16_t)(lane == 5 ? 32 : 0);
+    S->hd.first[lane] = 0;
+    S->hd.index[lane] = 0;
+  }
   lds_order();
-  build_table(S->lens, 288, kTabLit, &S->hl, S->tab, 0, C::kLB, C::kLS);
-  for (uint32_t s = lane; s < 32; s += kWave) S->lens[s] = 5;
-  lds_order();
-  build_table(S->lens, 32, kTabDist, &S->hd, S->tab, C::kDistAt, C::kDB, C::kDS);
 }
 
 // Decodes the one symbol at stage bit *q with zlib's rules: kMore and the token
