@@ -793,38 +793,62 @@ __device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n
   return st;
 }
 
-constexpr uint32_t kHardYes = 3, kHardNo = 4;
+// Eight passes that verify fewer lanes than these cost more than the chain, per lane
+// (literals of 4096 chunks of text, no matches, 64 lanes: below 16 of them 11.7 ms,
+// below 32 11.0 ms; base64 text 7.9 and 8.0 ms).
+template <class C> constexpr uint32_t kFewLanes = C::kNW > 1 ? C::kThreads / 4 : C::kThreads / 2;
+constexpr uint32_t kHard = 3;  // spans of few verified lanes before a block goes on with chain_entries
 
 // Where a span's lanes do not find each other's token starts (codes of nearly one
 // length keep a wrong phase: 128 equally frequent bytes, say), lane j decodes its
 // part from each of the 16 bits at which the token before it may end, and a chain
-// through these exits gives every lane its entry. Returns the lanes that have
-// one, and this lane's entry in the low half; the first that stops, or whose successor begins further behind, is the
-// last. 128 KiB chunks of 7-bit literals, by passes (one or two lanes verified a
-// pass) and by candidates: 16 chunks 20.0 and 2.2 ms, 4096 chunks by one wave
-// each 30.8 and 17.5 ms.
+// through these exits gives every lane its entry. A candidate whose first token ends
+// at another one has its exit (of 7-bit literals, 7 or 8 of the 16 are decoded). A
+// part that begins further behind, after a match, is decoded from there when the
+// chain comes to it. Returns the lanes that have an entry, all up to the first that
+// stops, and this lane's entry in the low half. 128 KiB chunks of 7-bit literals, by
+// passes where the chain broke at a match, all 16 decoded, and now: 4096 chunks by
+// one wave each 24.3 and 11.1 ms, 512 by eight waves 11.9 and 2.3 ms; base64 text,
+// 512 chunks 4.9 and 3.1 ms.
 template <class C>
-__device__ __noinline__ uint64_t chain_entries(lds<Sh<C>> *S, uint32_t lo, uint32_t bound, uint32_t limit,
-                                               uint32_t wave, uint32_t entry) {
+__device__ __noinline__ uint64_t chain_entries(lds<Sh<C>> *S, uint32_t lo, uint32_t bound, uint32_t limit, uint32_t wave) {
   const uint32_t lane = lane_id();
-  if constexpr (C::kNW > 1) __syncthreads();  // every wave has read the pass's mis and stp
-  uint32_t exits[4] = {0, 0, 0, 0};  // byte c: the exit behind `bound` of entry lo + c, 255 = stop
+  const lds<uint32_t> *stage = S->stage, *tab = S->tab;
+  if constexpr (C::kNW > 1) __syncthreads();  // mis and stp are free
+  // the exit behind `bound` of entry q, 255 = stop
+  auto exit_of = [&](uint32_t q) __attribute__((always_inline)) {
+    uint32_t n = 0;
+    const bool stop = run_tokens<C, false, const lds<uint32_t> *>(stage, tab, q, bound, limit, n);
+    return stop ? 255u : q - bound;
+  };
+  uint32_t exits[4] = {0, 0, 0, 0};  // byte c: of entry lo + c
 #pragma unroll 1
-  for (uint32_t c = 0; c < 16; c++) {
-    uint32_t q = lo + c, n = 0;
-    const uint32_t x =
-        run_tokens<C, false, const lds<uint32_t> *>(S->stage, S->tab, q, bound, limit, n) ? 255u : q - bound;
+  for (uint32_t c = 16; c-- > 0;) {
+    // a literal that the root table holds leads to candidate `to`
+    const uint32_t e = look(tab, stage_bits(stage, lo + c), C::kLitDesc), to = c + (e & 31);
+    const bool known = (e & 31) && e < kLenType && to < 16 && lo + to <= limit;
+    const uint32_t m = to < 4 ? exits[0] : to < 8 ? exits[1] : to < 12 ? exits[2] : exits[3];
+    uint32_t x = (m >> 8 * (to & 3)) & 255;
+    if (__ballot(!known)) {
+      const uint32_t y = exit_of(lo + c);
+      x = known ? x : y;
+    }
 #pragma unroll
     for (uint32_t k = 0; k < 4; k++) exits[k] |= c / 4 == k ? x << 8 * (c & 3) : 0u;
   }
-  uint32_t off = 0, have = 0;
+  uint32_t entry = lo, off = 0, have = 0;
   for (uint32_t w = 0; w < (uint32_t)C::kNW; w++) {
     if (w == wave) {
-      for (; have < (uint32_t)kWave && off < 16; have++) {
+      for (; have < (uint32_t)kWave && off != 255; have++) {
         if (lane == have) entry = lo + off;
-        const uint32_t k = off / 4;
-        const uint32_t m = k == 0 ? exits[0] : k == 1 ? exits[1] : k == 2 ? exits[2] : exits[3];
-        off = (rdlane(m, have) >> 8 * (off & 3)) & 255;
+        uint32_t m;
+        if (off < 16) {
+          const uint32_t k = off / 4;
+          m = (k == 0 ? exits[0] : k == 1 ? exits[1] : k == 2 ? exits[2] : exits[3]) >> 8 * (off & 3);
+        } else {
+          m = exit_of(lo + off);
+        }
+        off = rdlane(m, have) & 255;
       }
     }
     if constexpr (C::kNW > 1) {
@@ -835,7 +859,7 @@ __device__ __noinline__ uint64_t chain_entries(lds<Sh<C>> *S, uint32_t lo, uint3
       __syncthreads();
       have = uni(S->mis[w]);
       off = uni(S->stp[w]);
-      if (have < (uint32_t)kWave || off >= 16) return (uint64_t)(w * kWave + have) << 32 | entry;
+      if (off == 255) return (uint64_t)(w * kWave + have) << 32 | entry;
       have = 0;
     }
   }
@@ -848,7 +872,7 @@ __device__ __noinline__ uint64_t chain_entries(lds<Sh<C>> *S, uint32_t lo, uint3
 template <class C>
 __device__ __forceinline__ int32_t span(const uint32_t *w, uint32_t nw, uint32_t limit_bits, uint32_t &P, bool &stopped,
                                         uint32_t &hard, Out &o, Sh<C> &S, uint32_t wave, uint32_t lane) {
-  const uint32_t max_pass = hard == kHardYes ? 2 : 8;  // pass k verifies at least k lanes
+  constexpr uint32_t max_pass = 8;  // pass k verifies at least k lanes
   const uint32_t tid = wave * kWave + lane;
   const uint32_t d0 = P >> 5, off0 = P & 31;
   {
@@ -869,79 +893,75 @@ __device__ __forceinline__ int32_t span(const uint32_t *w, uint32_t nw, uint32_t
   uint32_t sq[C::kSub], sn[C::kSub];
 #pragma unroll
   for (int k = 0; k < C::kSub; k++) sq[k] = sn[k] = 0;
-  bool stop = run_tokens<C, false>(&S.stage[0], &S.tab[0], q, bound, limit, n);
+  bool stop = false;
   uint32_t valid;  // lanes verified
-  for (uint32_t pass = 2;; pass++) {
-    const uint32_t mine = q | (stop ? 0x80000000u : 0u);
-    uint32_t up = __shfl_up(mine, 1, kWave);
-    if constexpr (C::kNW > 1) {
-      if (lane == kWave - 1) S.ex[wave] = mine;
-      __syncthreads();
-      if (lane == 0 && wave) up = S.ex[wave - 1];
-    }
-    const uint32_t next = tid == 0 ? off0 : (up >> 31 ? entry : up);
-    const uint64_t mm = __ballot(next != entry), sm = __ballot(stop);
-    uint32_t fm = mm ? wave * kWave + (uint32_t)__builtin_ctzll(mm) : C::kThreads;
-    uint32_t fs = sm ? wave * kWave + (uint32_t)__builtin_ctzll(sm) : C::kThreads;
-    if constexpr (C::kNW > 1) {
-      if (lane == 0) {
-        S.mis[wave] = fm;
-        S.stp[wave] = fs;
-      }
-      __syncthreads();
-      for (uint32_t k = 0; k < (uint32_t)C::kNW; k++) {
-        fm = min(fm, uni(S.mis[k]));
-        fs = min(fs, uni(S.stp[k]));
-      }
-    }
-    if (pass > 2 && (fm > fs || fm == C::kThreads)) {
-      valid = min(fs + 1, C::kThreads);
-      break;
-    }
-    if (pass > max_pass) {
-      // the verified lanes make the span; a block in which they are few three
-      // times goes on with chain_entries, unless that finds few as well
-      valid = fm;
-      if (hard != kHardYes) {
-        if (hard < kHardYes && valid < max(C::kThreads / 8, 16u)) hard++;
-        break;
-      }
-      const uint64_t r = chain_entries<C>((lds<Sh<C>> *)&S, lo, bound, limit, wave, entry);
-      valid = uni((uint32_t)(r >> 32));
-      entry = (uint32_t)r;
-      if (valid < C::kThreads / 4) hard = kHardNo;
-      q = entry;
-      stop = false;
+  if (hard == kHard) {
+    const uint64_t r = chain_entries<C>((lds<Sh<C>> *)&S, lo, bound, limit, wave);
+    valid = uni((uint32_t)(r >> 32));
+    q = (uint32_t)r;
 #pragma unroll
-      for (int k = 0; k < C::kSub; k++) {
-        sq[k] = q;
-        n = 0;
-        if (!stop) stop = run_tokens<C, true>(&S.stage[0], &S.tab[0], q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
-        sn[k] = n;
-      }
-      break;
+    for (int k = 0; k < C::kSub; k++) {
+      sq[k] = q;
+      n = 0;
+      if (!stop) stop = run_tokens<C, true>(&S.stage[0], &S.tab[0], q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
+      sn[k] = n;
     }
-    // every lane counts its bytes in pass 2; later only lanes with a new entry
-    // (those behind a stop, too: most stops before the last pass are not real)
-    if (pass == 2 || next != entry) {
-      const uint32_t q0 = q;
-      const bool stop0 = stop;
-      bool met = false;  // back on the tokens of the pass before
-      entry = q = next;
-      stop = false;
-#pragma unroll
-      for (int k = 0; k < C::kSub; k++) {
-        if (k && pass > 2 && q == sq[k]) met = true;
-        if (!met) {
-          sq[k] = q;
-          n = 0;
-          if (!stop) stop = run_tokens<C, true>(&S.stage[0], &S.tab[0], q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
-          sn[k] = n;
+  } else {
+    stop = run_tokens<C, false>(&S.stage[0], &S.tab[0], q, bound, limit, n);
+    for (uint32_t pass = 2;; pass++) {
+      const uint32_t mine = q | (stop ? 0x80000000u : 0u);
+      uint32_t up = __shfl_up(mine, 1, kWave);
+      if constexpr (C::kNW > 1) {
+        if (lane == kWave - 1) S.ex[wave] = mine;
+        __syncthreads();
+        if (lane == 0 && wave) up = S.ex[wave - 1];
+      }
+      const uint32_t next = tid == 0 ? off0 : (up >> 31 ? entry : up);
+      const uint64_t mm = __ballot(next != entry), sm = __ballot(stop);
+      uint32_t fm = mm ? wave * kWave + (uint32_t)__builtin_ctzll(mm) : C::kThreads;
+      uint32_t fs = sm ? wave * kWave + (uint32_t)__builtin_ctzll(sm) : C::kThreads;
+      if constexpr (C::kNW > 1) {
+        if (lane == 0) {
+          S.mis[wave] = fm;
+          S.stp[wave] = fs;
+        }
+        __syncthreads();
+        for (uint32_t k = 0; k < (uint32_t)C::kNW; k++) {
+          fm = min(fm, uni(S.mis[k]));
+          fs = min(fs, uni(S.stp[k]));
         }
       }
-      if (met) {
-        q = q0;
-        stop = stop0;
+      if (pass > 2 && (fm > fs || fm == C::kThreads)) {
+        valid = min(fs + 1, C::kThreads);
+        break;
+      }
+      if (pass > max_pass) {
+        valid = fm;  // the verified lanes make the span
+        if (valid < kFewLanes<C>) hard++;
+        break;
+      }
+      // every lane counts its bytes in pass 2; later only lanes with a new entry
+      // (those behind a stop, too: most stops before the last pass are not real)
+      if (pass == 2 || next != entry) {
+        const uint32_t q0 = q;
+        const bool stop0 = stop;
+        bool met = false;  // back on the tokens of the pass before
+        entry = q = next;
+        stop = false;
+#pragma unroll
+        for (int k = 0; k < C::kSub; k++) {
+          if (k && pass > 2 && q == sq[k]) met = true;
+          if (!met) {
+            sq[k] = q;
+            n = 0;
+            if (!stop) stop = run_tokens<C, true>(&S.stage[0], &S.tab[0], q, lo + (k + 1) * C::kSpanBits / C::kSub, limit, n);
+            sn[k] = n;
+          }
+        }
+        if (met) {
+          q = q0;
+          stop = stop0;
+        }
       }
     }
   }
@@ -1221,7 +1241,7 @@ __device__ __forceinline__ Result inflate_group(const uint8_t *src, uint64_t len
   const bool headed = st == kOk;  // the stream's header is accepted
   uint32_t P = (uint32_t)((lead + start) * 8);
   bool last = false, inside = false, stopped = false;
-  uint32_t hard = 0;  // the block's spans that were cut short, or kHardYes / kHardNo
+  uint32_t hard = 0;  // the block's spans in which few lanes were verified
   for (;;) {
     uint32_t op = kOpEnd;
     if (wave == 0 && st == kOk) {
@@ -1255,7 +1275,8 @@ __device__ __forceinline__ Result inflate_group(const uint8_t *src, uint64_t len
     if (op == kOpEnd) break;
     if (op == kOpSpan) {
       const int32_t e = span<C>(w, nw, limit, P, stopped, hard, o, S, wave, lane);
-      hard = stopped ? 0u : hard;
+      // a block after one of equal code lengths is expected to be another
+      hard = stopped ? (hard == kHard ? kHard - 1 : 0u) : hard;
       if (wave == 0) st = e;
     } else {
       const uint32_t ln = uni(S.ln);
