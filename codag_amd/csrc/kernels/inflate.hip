@@ -141,9 +141,16 @@ template <class C> struct Sh {
   uint32_t stream;                            // the group's current stream
 };
 
-// LDS seen through a pointer of its own address space: functions that are not
-// inlined would else reach it by flat accesses.
+// LDS and global memory seen through pointers of their own address spaces:
+// functions that are not inlined would else reach them by flat accesses.
 template <class T> using lds = __attribute__((address_space(3))) T;
+template <class T> using glob = __attribute__((address_space(1))) T;
+
+// A wave-uniform pointer as such.
+template <class T> __device__ __forceinline__ glob<T> *uni_ptr(T *p) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  return (glob<T> *)((uint64_t)uni((uint32_t)(a >> 32)) << 32 | uni((uint32_t)a));
+}
 
 // Orders this wave's LDS accesses around a point where its lanes exchange data
 // through LDS.
@@ -170,6 +177,12 @@ struct Out {
   uint32_t pos;  // bytes produced; all of them are stored
   uint32_t s1, s2;
 };
+
+// Eight passes that verify fewer lanes than these cost more than the chain, per lane
+// (literals of 4096 chunks of text, no matches, 64 lanes: below 16 of them 11.7 ms,
+// below 32 11.0 ms; base64 text 7.9 and 8.0 ms).
+template <class C> constexpr uint32_t kFewLanes = C::kNW > 1 ? C::kThreads / 4 : C::kThreads / 2;
+constexpr uint32_t kHard = 3;  // spans of few verified lanes before a block goes on with chain_entries
 
 __device__ __forceinline__ void adler_add(Out &o, uint32_t at, uint32_t b) {
   o.s1 += b;
@@ -420,6 +433,30 @@ __device__ __forceinline__ uint32_t stage_bits(const lds<uint32_t> *stage, uint3
   return __builtin_amdgcn_alignbit(stage[(q >> 5) + 1], stage[q >> 5], q);
 }
 
+// The chain of lengths from lane 0 on: lane j's n bits lead to lane j + n, and a
+// length of 128 stops. Returns the lanes it visits; *next gets the bit behind the
+// 64 that it leads to, or 128 + the lane that stops. Eight links written out with a
+// fall-through test each: j is kept as j - 64, so the add's carry is the test.
+__device__ __forceinline__ uint64_t chain_links(uint32_t n, uint32_t *next) {
+  uint64_t M = 0;
+  uint32_t j = 0u - (uint32_t)kWave;
+  uint32_t t;
+  asm("1:\n"
+      ".rept 8\n"
+      "s_bitset1_b64 %[M], %[j]\n"
+      "v_readlane_b32 %[t], %[n], %[j]\n"
+      "s_add_u32 %[j], %[j], %[t]\n"
+      "s_cbranch_scc1 2f\n"
+      ".endr\n"
+      "s_branch 1b\n"
+      "2:"
+      : [j] "+s"(j), [M] "+s"(M), [t] "=&s"(t)
+      : [n] "v"(n)
+      : "scc");
+  *next = j + (uint32_t)kWave;
+  return M;
+}
+
 // Reads a dynamic block's code lengths (RFC 1951 3.2.7) from stage bit *q on
 // and builds its tables; `limit` is the stage bit after the stream's last.
 // The run-length coded lengths are decoded 64 bits at a time: lane j decodes
@@ -456,26 +493,8 @@ __device__ __forceinline__ int32_t read_dynamic(lds<Sh<C>> *S, uint32_t *qp, uin
     const uint32_t xb = sym < 16 ? 0u : (sym == 16 ? 2u : (sym == 17 ? 3u : 7u));
     const uint32_t rep = (sym < 16 ? 1u : (sym == 18 ? 11u : 3u)) + __builtin_amdgcn_ubfe(x, L, xb);
     const uint32_t tl = L ? L + xb : 128u;  // no such code: stops the chain
-    // M gets the starts. Eight links written out with a fall-through test each:
-    // j is kept as j - 64, so the add's carry is the test.
-    uint64_t M = 0;
-    uint32_t j = 0u - (uint32_t)kWave;
-    {
-      uint32_t t;
-      asm("1:\n"
-          ".rept 8\n"
-          "s_bitset1_b64 %[M], %[j]\n"
-          "v_readlane_b32 %[t], %[tl], %[j]\n"
-          "s_add_u32 %[j], %[j], %[t]\n"
-          "s_cbranch_scc1 2f\n"
-          ".endr\n"
-          "s_branch 1b\n"
-          "2:"
-          : [j] "+s"(j), [M] "+s"(M), [t] "=&s"(t)
-          : [tl] "v"(tl)
-          : "scc");
-    }
-    j += (uint32_t)kWave;
+    uint32_t j;
+    const uint64_t M = chain_links(tl, &j);  // the starts
     const bool start = (M >> lane) & 1 && L;
     const uint32_t incl = wave_scan_dpp(start ? rep : 0u);
     const uint32_t off = i + incl - rep;
@@ -793,11 +812,218 @@ __device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n
   return st;
 }
 
-// Eight passes that verify fewer lanes than these cost more than the chain, per lane
-// (literals of 4096 chunks of text, no matches, 64 lanes: below 16 of them 11.7 ms,
-// below 32 11.0 ms; base64 text 7.9 and 8.0 ms).
-template <class C> constexpr uint32_t kFewLanes = C::kNW > 1 ? C::kThreads / 4 : C::kThreads / 2;
-constexpr uint32_t kHard = 3;  // spans of few verified lanes before a block goes on with chain_entries
+// ------------------------------------------------------------- narrow decode
+
+typedef uint32_t __attribute__((aligned(1))) unaligned_dword;
+
+// What the narrow decoder leaves: the next stream bit, the output position and
+// this lane's Adler-32 sums; whether a symbol at P needs the symbol loop.
+struct Narrow {
+  uint32_t P, pos, s1, s2, stopped;
+  int32_t st;
+};
+
+// Output bytes per stream byte from which the narrow decoder is the faster. In a
+// group of eight waves it leaves seven idle, so spans hold on longer there (128 KiB
+// chunks of zeros with a one every 200 bytes, 78 output bytes per stream byte, spans
+// and narrow, us: 512 chunks by eight waves 321, 577 (an earlier copy loop), 4096
+// chunks by one wave 1998, 958).
+template <class C> constexpr uint32_t kNarrowRatio = C::kNW > 1 ? 200 : 32;
+
+// Decodes tokens from stream bit P on by one wave, 64 bits at a time: lane j looks
+// up the token that would start at bit j, a scalar chain through their lengths
+// marks those that do, and each is written at once: literals by their lanes,
+// matches one after the other by all lanes, into the window's LDS as a ring of the
+// last H bytes, which is stored in blocks of 1024 bytes. It is for long matches: a
+// span costs about 200 instructions per 256 output bytes, whatever the tokens, and
+// keeps two or three lanes busy with all of them, several times over; here a match
+// of 258 bytes is five reads and writes. It is bound by latency, about 1.2 K cycles
+// a match and 1.5 K per 64 bits. 128 KiB chunks of zeros, spans and this, us: 4096
+// chunks 2593, 738, 512 chunks 540, 325, one 449, 303; of a repeated 300 bytes, 4096
+// chunks 1656, 670; 600 streams of 4 MiB of zeros 23.8 and 10.0 ms.
+// It goes on while the output is kNarrowRatio times the stream's bytes, or still
+// promises to be by the room that is left, for 3072 bits at most. At most kTake
+// bytes are produced from one set of 64 bits, so the ring's last H - kTake bytes are
+// there for matches; sources before them, or before the first byte that is produced
+// here, come from HBM, where all but the last 1024 bytes are.
+template <class C>
+__device__ __noinline__ Narrow narrow_span(const uint32_t *w_, uint32_t nw, uint32_t limit_bits, uint32_t P,
+                                           uint8_t *dst_, uint32_t pos, uint32_t cap, uint32_t s1, uint32_t s2,
+                                           lds<Sh<C>> *S) {
+  constexpr uint32_t H = C::kNW == 1 ? 8192 : 32768, kTake = 2048, kStaged = 256;
+  static_assert(H < sizeof(S->win) && kStaged <= C::kStage, "the ring fits the window, the dwords the stage");
+  const uint32_t lane = lane_id();
+  lds<uint8_t> *ring = reinterpret_cast<lds<uint8_t> *>(S->win);
+  const glob<const uint32_t> *w = uni_ptr(w_);
+  glob<uint8_t> *dst = uni_ptr(dst_);
+  P = uni(P);
+  pos = uni(pos);
+  nw = uni(nw);
+  limit_bits = uni(limit_bits);
+  cap = uni(cap);
+  const uint32_t enter = pos;
+  uint32_t fl = pos;                   // bytes stored
+  uint32_t d0 = 0, staged = 0;         // the stage holds dwords [d0, d0 + staged)
+  uint32_t P1 = P, pos1 = pos;         // where the ratio is measured from
+  uint32_t stopped = 0;
+  int32_t st = kOk;
+  auto store = [&](uint32_t to) __attribute__((always_inline)) {  // bytes [fl, to), to - fl <= 1024 + 3
+    lds_order();
+    const uint32_t head = min((0u - fl) & 3, to - fl);
+    if (head) {
+      if (lane < head) {
+        const uint32_t b = ring[(fl + lane) & (H - 1)];
+        dst[fl + lane] = (uint8_t)b;
+        s1 += b;
+        s2 = (s2 + ((fl + lane) % 65521u) * b) % 65521u;
+      }
+      fl += head;
+    }
+    uint32_t a1 = 0, a2 = 0;
+    for (uint32_t k = 4 * lane; k < to - fl; k += 4 * kWave) {
+      uint32_t b = *reinterpret_cast<lds<uint32_t> *>(ring + ((fl + k) & (H - 1)));
+      glob<uint8_t> *d = dst + (fl + k);
+      if (k + 4 <= to - fl) {
+        *reinterpret_cast<glob<unaligned_dword> *>(d) = b;
+      } else {
+        b &= (1u << 8 * (to - fl - k)) - 1;
+        for (uint32_t j = 0; j < to - fl - k; j++) d[j] = (uint8_t)(b >> 8 * j);
+      }
+      const uint32_t sum = __builtin_amdgcn_udot4(b, 0x01010101u, 0u, false);
+      a1 += sum;
+      a2 += k * sum + __builtin_amdgcn_udot4(b, 0x03020100u, 0u, false);
+    }
+    s1 = (s1 + a1) % 65521u;
+    s2 = (s2 + (fl % 65521u) * a1 + a2) % 65521u;
+    fl = to;
+    lds_order();
+  };
+  for (;;) {
+    if ((P >> 5) + 8 > d0 + staged) {  // 64 positions, a token of 48 bits and the dword behind it
+      d0 = P >> 5;
+      staged = kStaged;
+      lds_order();
+#pragma unroll
+      for (uint32_t k = 0; k < kStaged; k += kWave) S->stage[k + lane] = d0 + k + lane < nw ? w[d0 + k + lane] : 0u;
+      lds_order();
+    }
+    const uint32_t a = P - d0 * 32 + lane, limit = limit_bits - d0 * 32;
+    // the token at bit a: `at` its end, len and val or dist. It has 48 bits at most,
+    // and its last lookup begins at its 28th: all from the 64 bits at a
+    const lds<uint32_t> *bits = S->stage + (a >> 5);
+    const uint32_t b0 = bits[0], b1 = bits[1], b2 = bits[2];
+    const uint32_t x0 = __builtin_amdgcn_alignbit(b1, b0, a), x1 = __builtin_amdgcn_alignbit(b2, b1, a);
+    auto from_bit = [&](uint32_t q) __attribute__((always_inline)) { return __builtin_amdgcn_alignbit(x1, x0, q - a); };
+    uint32_t x = x0, e = look((const lds<uint32_t> *)S->tab, x, C::kLitDesc), at = a + (e & 31);
+    bool ok = (e & 31) != 0;
+    const bool sub = ok && e >= kSubType;
+    if (__ballot(sub)) {
+      const uint32_t x2 = from_bit(at);
+      const uint32_t e2 = look((const lds<uint32_t> *)S->tab, x2, sub ? __builtin_amdgcn_ubfe(e, 14, 16) : C::kLitDesc);
+      x = sub ? x2 : x;
+      e = sub ? e2 : e;
+      at += sub ? e2 & 31 : 0u;
+      ok = ok && (e & 31) != 0;
+    }
+    const bool lit = e & kLitFlag, match = ok && !lit;
+    const uint32_t val = entry_value(e, x), len = lit ? 1u : val;
+    uint32_t dist = 0;
+    if (__ballot(match)) {
+      uint32_t y = from_bit(at), f = look((const lds<uint32_t> *)S->tab, y, C::kDistDesc);
+      uint32_t to = at + (f & 31);
+      bool fine = (f & 31) != 0;
+      const bool dsub = match && fine && f >= kSubType;
+      if (__ballot(dsub)) {
+        const uint32_t y2 = from_bit(to);
+        const uint32_t f2 = look((const lds<uint32_t> *)S->tab, y2, dsub ? __builtin_amdgcn_ubfe(f, 14, 16) : C::kDistDesc);
+        y = dsub ? y2 : y;
+        f = dsub ? f2 : f;
+        to += dsub ? f2 & 31 : 0u;
+        fine = fine && (f & 31) != 0;
+      }
+      dist = match ? entry_value(f, y) : 0u;
+      at = match ? to : at;
+      ok = match ? fine : ok;
+    }
+    ok = ok && at <= limit;
+    uint32_t next;
+    const uint64_t M = chain_links(ok ? at - a : 128u, &next);
+    const bool start = (M >> lane) & 1 && ok;
+    const uint32_t incl = wave_scan_dpp(start ? len : 0u), off = incl - (start ? len : 0u);
+    bool take = start && incl <= kTake;
+    const uint64_t left = __ballot(start && !take);
+    const uint32_t last = left ? (uint32_t)__builtin_ctzll(left) : 64u;  // the first token left for the next turn
+    const bool over = take && pos + incl > cap, wrong = take && dist > pos + off;  // distance too far back
+    const uint64_t bad = __ballot(over || wrong);
+    uint64_t taken = __ballot(take);
+    if (bad) {  // the tokens before the first error are written
+      const uint32_t f = (uint32_t)__builtin_ctzll(bad);
+      st = rdlane(over, f) ? kOverflow : kCorrupt;
+      taken &= (1ull << f) - 1;
+      take = take && lane < f;
+    }
+    const uint32_t total = taken ? rdlane(incl, 63u - (uint32_t)__builtin_clzll(taken)) : 0u;
+    if (take && lit) ring[(pos + off) & (H - 1)] = (uint8_t)val;
+    const uint32_t lo = max(enter, pos + kTake > H ? pos + kTake - H : 0u);  // the ring's first byte
+    for (uint64_t mm = __ballot(take && !lit); mm; mm &= mm - 1) {
+      const uint32_t l = (uint32_t)__builtin_ctzll(mm);
+      const uint32_t n = rdlane(len, l), d = rdlane(dist, l), t = pos + rdlane(off, l), from = t - d;
+      // ROWS rows of 64 bytes; the lanes behind the match write behind the ring
+      auto copy = [&]<uint32_t ROWS>() __attribute__((always_inline)) {
+        uint32_t src[ROWS], b[ROWS];
+#pragma unroll
+        for (uint32_t r = 0; r < ROWS; r++) src[r] = from + r * kWave + lane;
+        if (d < n) {
+          // a match longer than its distance repeats its first d bytes; i + 0.5 is at
+          // least 0.5 away from a multiple of d < 258, so the quotient is exact
+          const float rc = __builtin_amdgcn_rcpf((float)d);
+#pragma unroll
+          for (uint32_t r = 0; r < ROWS; r++)
+            src[r] -= __umul24((uint32_t)(((float)(r * kWave + lane) + 0.5f) * rc), d);
+        }
+        lds_order();
+#pragma unroll
+        for (uint32_t r = 0; r < ROWS; r++) b[r] = ring[src[r] & (H - 1)];
+        if (from < lo) {
+#pragma unroll
+          for (uint32_t r = 0; r < ROWS; r++)
+            if (r * kWave + lane < n && src[r] < lo) b[r] = dst[src[r]];
+          // waits here, and not on the other path, where it would wait for the stores
+#pragma unroll
+          for (uint32_t r = 0; r < ROWS; r++) asm volatile("" : "+v"(b[r]));
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < ROWS; r++)
+          ring[r * kWave + lane < n ? (t + r * kWave + lane) & (H - 1) : H] = (uint8_t)b[r];
+      };
+      if (n <= kWave) copy.template operator()<1>();
+      else if (n <= 3 * kWave) copy.template operator()<3>();
+      else copy.template operator()<5>();
+    }
+    pos += total;
+    if (bad) break;
+    while (pos - fl >= 1024) store(fl + 1024 - (fl & 3));
+    if (left) {
+      P += last;
+    } else {
+      P += next >= 128 ? next - 128 : next;
+      if (next >= 128) {
+        stopped = 1;
+        break;
+      }
+    }
+    if (P - P1 >= 1024) {
+      if ((pos - pos1) * 8 >= kNarrowRatio<C> * (P - P1)) {
+        P1 = P;
+        pos1 = pos;
+      } else if (P - P1 >= 3072 || (uint64_t)(cap - pos) * 8 < (uint64_t)kNarrowRatio<C> * (limit_bits - P)) {
+        break;
+      }
+    }
+  }
+  while (fl < pos) store(min(pos, fl + 1024 - (fl & 3)));
+  return Narrow{P, pos, s1, s2, stopped, st};
+}
 
 // Where a span's lanes do not find each other's token starts (codes of nearly one
 // length keep a wrong phase: 128 equally frequent bytes, say), lane j decodes its
@@ -1241,25 +1467,50 @@ __device__ __forceinline__ Result inflate_group(const uint8_t *src, uint64_t len
   const bool headed = st == kOk;  // the stream's header is accepted
   uint32_t P = (uint32_t)((lead + start) * 8);
   bool last = false, inside = false, stopped = false;
-  uint32_t hard = 0;  // the block's spans in which few lanes were verified
+  uint32_t hard = 0;     // the block's spans in which few lanes were verified
+  // the block goes on by narrow_span; the output's room has nothing to do with its bytes (wave 0)
+  bool narrow = false, roomy = false;
   for (;;) {
     uint32_t op = kOpEnd;
-    if (wave == 0 && st == kOk) {
-      if (inside && !stopped) {
-        op = kOpSpan;
-      } else if (inside || !last) {
-        serial_step<C>(w, nw, limit, P, inside, last, (lds<Sh<C>> *)&S);
-        op = uni(S.op);
-        P = uni(S.P);
-        st = (int32_t)uni((uint32_t)S.st);
-        last = uni(S.last);
-        if (op == kOpToken) {
-          const uint32_t val = uni(S.val), dist = uni(S.dist);
-          st = out_token(o, lane, dist == 0, val, dist);
-          op = st == kOk ? kOpSpan : kOpEnd;
+    if (wave == 0) {
+      while (st == kOk) {
+        if (inside && !stopped) {
+          if (!narrow) {
+            op = kOpSpan;
+            break;
+          }
+          const Narrow r = narrow_span<C>(w, nw, limit, P, o.dst, o.pos, o.cap, o.s1, o.s2, (lds<Sh<C>> *)&S);
+          P = uni(r.P);
+          o.pos = uni(r.pos);
+          o.s1 = r.s1;
+          o.s2 = r.s2;
+          st = (int32_t)uni((uint32_t)r.st);
+          stopped = uni(r.stopped);
+          narrow = stopped;  // else it left for want of long matches: the sizes promised too much
+          roomy = roomy || !stopped;
+        } else if (inside || !last) {
+          const bool symbol = inside;
+          serial_step<C>(w, nw, limit, P, symbol, last, (lds<Sh<C>> *)&S);
+          op = uni(S.op);
+          P = uni(S.P);
+          st = (int32_t)uni((uint32_t)S.st);
+          last = uni(S.last);
+          inside = op == kOpSpan || op == kOpToken;
+          stopped = false;
+          if (op == kOpToken) {
+            const uint32_t val = uni(S.val), dist = uni(S.dist);
+            st = out_token(o, lane, dist == 0, val, dist);
+          }
+          if (op == kOpStored || op == kOpEnd) break;
+          if (op == kOpSpan) {  // a new block: by the bytes that the stream's rest has to give
+            narrow = !roomy && (uint64_t)(o.cap - o.pos) * 8 >= (uint64_t)kNarrowRatio<C> * (limit - P);
+          }
+        } else {
+          op = kOpEnd;
+          break;
         }
-        inside = op == kOpSpan;
       }
+      if (st != kOk) op = kOpEnd;
     }
     if constexpr (C::kNW > 1) {
       if (threadIdx.x == 0) {
@@ -1274,10 +1525,12 @@ __device__ __forceinline__ Result inflate_group(const uint8_t *src, uint64_t len
     }
     if (op == kOpEnd) break;
     if (op == kOpSpan) {
+      const uint32_t P0 = P, pos0 = o.pos;
       const int32_t e = span<C>(w, nw, limit, P, stopped, hard, o, S, wave, lane);
+      if (wave == 0) st = e;
       // a block after one of equal code lengths is expected to be another
       hard = stopped ? (hard == kHard ? kHard - 1 : 0u) : hard;
-      if (wave == 0) st = e;
+      narrow = (uint64_t)(o.pos - pos0) * 8 >= (uint64_t)kNarrowRatio<C> * (P - P0);
     } else {
       const uint32_t ln = uni(S.ln);
       const int32_t e = store_copy(o, reinterpret_cast<const uint8_t *>(w) + P / 8, ln, wave * kWave + lane, C::kThreads);
@@ -1369,6 +1622,8 @@ inflate_chunks_many_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes
 //    to 64 KiB 0.86 / 0.90, of up to 1 MiB 11.2 / 4.5, 6000 of up to 16 KiB
 //    0.49 / 1.08, of up to 256 KiB 3.19 / 3.39. (The large streams by eight
 //    waves and then the small ones by one wave each was never the faster.)
+//  * Streams that the narrow decoder takes keep one wave busy in either group: one
+//    (600 streams of 128 KiB of zeros 0.33 / 0.63).
 struct BatchQueue {
   uint32_t next;
   uint32_t many;
@@ -1380,35 +1635,40 @@ constexpr uint32_t kPlanThreads = 1024, kPlanSample = 1u << 16;
 // here, 1 one wave, 2 eight waves.
 __global__ void __launch_bounds__(kPlanThreads)
 plan_batch_kernel(const codag_stream_desc *__restrict__ descs, uint64_t n, BatchQueue *q, uint32_t shape) {
-  __shared__ uint64_t sums[kPlanThreads / kWave], tops[kPlanThreads / kWave];
+  __shared__ uint64_t sums[kPlanThreads / kWave], tops[kPlanThreads / kWave], rooms[kPlanThreads / kWave];
   const uint64_t m = min(n, (uint64_t)kPlanSample);
-  uint64_t sum = 0, top = 0;
+  uint64_t sum = 0, top = 0, room = 0;
   if (shape == 0)
     for (uint64_t k = threadIdx.x; k < m; k += blockDim.x) {
       const uint64_t b = min(descs[k * n / m].src_bytes, (uint64_t)1 << 28);
       sum += b;
+      room += min(descs[k * n / m].dst_cap, (uint64_t)1 << 31);
       top = max(top, b);
     }
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) {
     sum += __shfl_xor(sum, d, kWave);
+    room += __shfl_xor(room, d, kWave);
     top = max(top, __shfl_xor(top, d, kWave));
   }
   if (lane_id() == 0) {
     sums[threadIdx.x / kWave] = sum;
     tops[threadIdx.x / kWave] = top;
+    rooms[threadIdx.x / kWave] = room;
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
-  sum = top = 0;
+  sum = top = room = 0;
   for (uint32_t i = 0; i < blockDim.x / kWave; i++) {
     sum += sums[i];
     top = max(top, tops[i]);
+    room += rooms[i];
   }
+  const bool small = room < kNarrowRatio<One> * sum;  // outputs below so many times their streams
   if (m) sum = sum / m * n;
   const uint64_t one = max(200000 + 20 * top, sum / 85), many = 150 * n + sum / 78;  // ns
   q->next = 0;
-  q->many = shape == 0 ? many <= one : shape == 2;
+  q->many = shape == 0 ? small && many <= one : shape == 2;
 }
 
 // Persistent loop over a batch: each group takes the next stream from the queue
