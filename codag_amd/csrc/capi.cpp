@@ -179,6 +179,28 @@ uint32_t rlev2_route(const codag_tune_params &t, uint64_t n, uint32_t w, uint64_
   return t.threads_per_group == 64 ? kRouteWave : kRouteGroup;
 }
 
+// Whether a Deflate container of n chunks goes by eight waves per chunk (two such
+// groups fit a CU) or one (nine fit). Eight and one wave, us, unless said otherwise
+// on 128 KiB chunks of text (half its size when compressed):
+//  * Up to two chunks per CU eight: 256 chunks 437, 1169, 512 chunks 547, 1266. Of
+//    chunks of up to 4 KiB of very compressible or hardly compressible bytes the
+//    headers and the first token are all there is to spread: one (512 chunks of 4
+//    KiB: base64 text 366, 310, zeros 31, 26; text 142, 137, numbers 80, 89).
+//  * Up to five, eight as well: 1280 chunks 1355, 1397 (64 KiB 822, 770; of 32-bit
+//    counters 812, 1011). But one where the chunks are small (768 of 4 KiB 267,
+//    141), where the output is 32 times the stream, as narrow_span then works by
+//    one wave anyway (1280 chunks of zeros 958, 358), and where the stream is
+//    nearly as long as the output but not stored, mostly literals that cost eight
+//    waves the most (1280 chunks of base64 text 7483, 3693; stored 207, 286).
+//  * Above that one: 2048 chunks 2.02 and 1.40 ms, 4096 3.90 and 3.04 ms.
+// comp_bytes may hold more than the chunks; that only moves the choice.
+bool inflate_many(uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes, uint32_t cus) {
+  if (n > 5ull * cus) return false;
+  const double ratio = (double)comp_bytes / ((double)n * (double)chunk_bytes);  // stream bytes per output byte
+  if (n <= 2ull * cus) return chunk_bytes > 4096 || (ratio >= 0.125 && ratio <= 0.65);
+  return chunk_bytes > 8192 && ratio > 1.0 / 32 && (ratio <= 0.65 || ratio > 0.99);
+}
+
 void default_tune(codag_ctx *c) {
   for (int k = 0; k < 4; k++) c->tune[k] = kDefaultTune[k];
 }
@@ -386,9 +408,7 @@ codag_status codag_inflate_chunks(codag_ctx *ctx, const uint8_t *d_comp, uint64_
   if (chunk_bytes == 0) return fail(CODAG_ERR_INVALID, "inflate_chunks: chunk_bytes is 0");
   if (n_chunks > 0x7fffffffull) return fail(CODAG_ERR_INVALID, "inflate_chunks: too many chunks");
   DeviceGuard g(ctx->device);
-  // Eight waves per chunk while there are few chunks, else one wave per chunk
-  // (the line is drawn where launch_inflate_chunks gives both sides' times).
-  bool many = n_chunks <= (uint64_t)ctx->cu_count * 5;
+  bool many = inflate_many(comp_bytes, n_chunks, chunk_bytes, ctx->cu_count);
   if (ctx->chunks_two_wave) many = ctx->chunks_two_wave == 1;
   HIP_TRY(launch_inflate_chunks(d_comp, comp_bytes, d_offsets, n_chunks, chunk_bytes, d_out,
                                 d_out_len, d_status, flags, pick(ctx, stream), many));
@@ -817,6 +837,11 @@ uint32_t codag_test_route(codag_ctx *ctx, codag_codec codec, uint64_t comp_bytes
   const codag_tune_params &t = ctx->tune[codec];
   return codec == CODAG_RLEV1 ? rlev1_route(t, n, w, chunk_bytes, comp_bytes, ctx->cu_count)
                               : rlev2_route(t, n, w, chunk_bytes, comp_bytes, ctx->cu_count, ctx->poll_shift == 0);
+}
+
+// Test hook, not in the public header: whether codag_inflate_chunks takes eight waves.
+uint32_t codag_test_inflate_many(codag_ctx *ctx, uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes) {
+  return ctx ? inflate_many(comp_bytes, n, chunk_bytes, ctx->cu_count) : ~0u;
 }
 
 // Test hook, not in the public header (no counterpart in the reference):

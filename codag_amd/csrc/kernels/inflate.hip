@@ -1746,9 +1746,7 @@ hipError_t inflate_scratch_ptr(uint32_t **out) {
   return hipSuccess;
 }
 
-// Eight waves per chunk while there are at most five chunks per CU, else one
-// wave per chunk (128 KiB chunks, MI355X: 256 chunks 0.48 and 1.26 ms, 1024
-// 1.04 and 1.38 ms, 2048 2.02 and 1.51 ms, 4096 3.90 and 2.96 ms).
+// many: eight waves per chunk, else one (inflate_many).
 hipError_t launch_inflate_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *off,
                                  uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
                                  int32_t *status, uint32_t flags, hipStream_t stream, bool many) {
