@@ -67,6 +67,7 @@ struct codag_ctx {
   char name[256] = {0};
   codag_tune_params tune[4];
   uint32_t chunks_two_wave = 0;
+  uint32_t byte_waves = 0;  // BRLE kernel: 0 chosen by the streams, 1 or 4 waves per chunk (tests)
   uint32_t poll_shift = 0;  // RLE v2 queue kernel: nonzero = waits without polls (tests)
 };
 
@@ -199,6 +200,19 @@ bool inflate_many(uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes, uint32_
   const double ratio = (double)comp_bytes / ((double)n * (double)chunk_bytes);  // stream bytes per output byte
   if (n <= 2ull * cus) return chunk_bytes > 4096 || (ratio >= 0.125 && ratio <= 0.65);
   return chunk_bytes > 8192 && ratio > 1.0 / 32 && (ratio <= 0.65 || ratio > 0.99);
+}
+
+// Whether a BRLE container goes by one wave per chunk (19 such groups fit a CU) or
+// four (five fit). Four and one wave, us: a chunk whose stream fits one wave's step
+// leaves the others little (256 KiB of zeros, 4034 stream bytes, 512 chunks 183, 187,
+// 2048 chunks 408, 220; 4 KiB of the benchmark column, 1024 chunks 17, 14, 16384
+// chunks 231, 66), and where five groups per CU are filled several times over one
+// wave's slower chunks overtake (16 KiB of it, 2048 chunks 47, 47, 4096 chunks 87,
+// 63; 256 KiB, 1024 chunks 260, 580, 2048 chunks 500, 645, 4096 chunks 956, 861).
+bool brle_few(uint64_t comp_bytes, uint64_t n, uint32_t cus) {
+  const uint64_t each = comp_bytes / n;  // stream bytes of a chunk
+  if (each <= 4200) return true;
+  return n > (each <= 24576 ? 7ull : 15ull) * cus;
 }
 
 void default_tune(codag_ctx *c) {
@@ -434,8 +448,10 @@ codag_status codag_brle_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t c
   if (codag_status s = byte_codec_args("brle_decode", ctx, d_comp, d_ptr, n_chunks, chunk_bytes, d_out))
     return s;
   DeviceGuard g(ctx->device);
+  bool few = n_chunks && brle_few(comp_bytes, n_chunks, ctx->cu_count);
+  if (ctx->byte_waves) few = ctx->byte_waves == 1;
   HIP_TRY(launch_brle_chunks(d_comp, comp_bytes, d_ptr, n_chunks, chunk_bytes, d_out, d_out_len,
-                             d_status, pick(ctx, stream)));
+                             d_status, pick(ctx, stream), few));
   return CODAG_OK;
 }
 
@@ -837,6 +853,21 @@ uint32_t codag_test_route(codag_ctx *ctx, codag_codec codec, uint64_t comp_bytes
   const codag_tune_params &t = ctx->tune[codec];
   return codec == CODAG_RLEV1 ? rlev1_route(t, n, w, chunk_bytes, comp_bytes, ctx->cu_count)
                               : rlev2_route(t, n, w, chunk_bytes, comp_bytes, ctx->cu_count, ctx->poll_shift == 0);
+}
+
+// Test hook, not in the public header: the waves per chunk of the BRLE kernel, 1 or
+// 4, or 0 for the choice by the streams.
+codag_status codag_test_byte_waves(codag_ctx *ctx, uint32_t waves) {
+  if (!ctx) return fail(CODAG_ERR_INVALID, "test_byte_waves: null ctx");
+  ctx->byte_waves = waves;
+  return CODAG_OK;
+}
+
+// Test hook, not in the public header: whether codag_brle_decode of n > 0 chunks
+// takes the kernel of one wave per chunk.
+uint32_t codag_test_byte_one(codag_ctx *ctx, uint32_t lzss, uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes) {
+  (void)chunk_bytes;
+  return !ctx || !n || lzss ? ~0u : brle_few(comp_bytes, n, ctx->cu_count);
 }
 
 // Test hook, not in the public header: whether codag_inflate_chunks takes eight waves.

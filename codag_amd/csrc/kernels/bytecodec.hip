@@ -16,11 +16,11 @@
 //
 // Both formats are sequences of byte-aligned items whose sizes follow from
 // one header byte (BRLE) or one flag byte per eight items (LZSS). Both decoders
-// take a chunk by four waves and find the item starts of many parts of the
-// stream at once: BRLE by walks from guessed starts that are put right until
-// they agree, LZSS from every byte a group may begin at. BRLE's output is made
-// from its items dword by dword, LZSS's resolved in an LDS window of marks. The
-// next part of the stream is loaded meanwhile.
+// find the item starts of many parts of the stream at once: BRLE by walks from
+// guessed starts that are put right until they agree, LZSS from every byte a group
+// may begin at. BRLE's output is made from its items dword by dword, LZSS's
+// resolved in an LDS window of marks. The next part of the stream is loaded
+// meanwhile.
 //
 // The reference checks nothing; these kernels report per chunk: TRUNCATED if
 // the stream ends inside an item, OVERFLOW if the output would pass the
@@ -80,43 +80,49 @@ __device__ __forceinline__ void chunk_bounds(const uint64_t lo, const uint64_t h
 
 // ------------------------------------------------------------------ BRLE
 
-// Four waves per chunk. A step takes 256 blocks of 60 stream bytes, one per lane:
+// Four waves per chunk, or one (brle_few in capi.cpp has both sides' times). A step
+// takes 64 blocks of 60 stream bytes per wave, one per lane:
 //  * Item starts. Only a header above 128 moves on by more than two bytes, so a
 //    walk visits every second byte up to the next such byte: one mask operation
 //    and one header read per long literal, not one per item. Every lane walks its
 //    block from a guessed start (its first byte) and keeps the starts it passes
-//    in a mask. Each lane's exit is then its successor's entry: a lane whose
+//    in a mask. A block is entered at the greatest exit before it: a lane whose
 //    entry changed walks on from there until it meets a start of its mask, where
 //    its former path, and exit, hold again. In runs and text wrong starts have
 //    met the right one after 40 bytes in the median and 390 at the 99th
-//    percentile, nine passes a step; where they never do, a pass puts one block
-//    right, and the walk is the chain through the headers that it was before.
+//    percentile, nine passes a step. Where they do not (long literals of any
+//    bytes), each wave in turn follows its chain block by block.
 //  * Each wave lists its items, with output offsets from a prefix sum, and makes
 //    its output in an LDS window: an item marks its first whole dword, a prefix
 //    maximum hands each dword its item and one load its bytes; the up to three
 //    bytes before and behind an item's whole dwords are then written by item.
 // One wave's walk by readlane took about 250 cycles an item, with a second wave
-// writing. 1024 chunks of 256 KiB, runs and text: 861 us before, 277 now (item by
-// item through the headers 449; eight waves and blocks of 44 bytes 305, as walks
-// then meet over more lanes). It is bound by latency: a step takes 54 K cycles,
-// 21 K of them in the walks and 20 K in the output, with one chunk per CU or four.
-constexpr int kBrWaves = 4;
-constexpr uint32_t kBrThreads = kBrWaves * kWave;
+// writing. 1024 chunks of 256 KiB, that way and now, us: runs and text 873 and 264
+// (item by item through the headers 449), random bytes 1598 and 740 (by walks alone
+// 1837), 16384 chunks of 4 KiB of the former 143 and 70 (by four waves and with
+// entries handed on from lane to lane 799). It is bound by latency: of a step's
+// cycles about two fifths are the walks and as many the output, with one chunk per
+// CU or four.
 // 15 dwords: lanes at the same byte of their blocks read different LDS banks
 constexpr uint32_t kBrBlock = 60;
-constexpr uint32_t kBrStep = kBrThreads * kBrBlock;  // stream bytes in which a step's items begin
-constexpr uint32_t kBrStage = (15 + kBrStep + 129 + 8 + 15) & ~15u;
-constexpr uint32_t kBrLoads = (kBrStage + kBrThreads * 16 - 1) / (kBrThreads * 16);
 constexpr uint32_t kBrList = 512;             // items listed at a time, per wave
 constexpr uint32_t kBrOut = 2048;             // a wave's output window
+constexpr uint32_t kBrPasses = 24, kBrFew = 2;  // walks before a wave follows its chain block by block; see there
 static_assert(kBrBlock <= 64, "the starts of a block in 64 bits");
 
-struct __align__(16) BrleLds {
-  uint8_t stage[kBrStage];
-  uint32_t list[kBrWaves][kBrList];  // literal << 31 | output offset in the wave << 12 | header
-  uint32_t out[kBrWaves][kBrOut / 4];
-  uint32_t exits[2][kBrWaves], entry[2][kBrWaves], early[kBrWaves];
-  uint32_t part[kBrWaves];
+template <int NW> struct BrCfg {
+  static constexpr uint32_t kThreads = NW * kWave;
+  static constexpr uint32_t kStep = kThreads * kBrBlock;  // stream bytes in which a step's items begin
+  static constexpr uint32_t kStage = (15 + kStep + 129 + 8 + 15) & ~15u;
+  static constexpr uint32_t kLoads = (kStage + kThreads * 16 - 1) / (kThreads * 16);
+};
+
+template <int NW> struct __align__(16) BrleLds {
+  uint8_t stage[BrCfg<NW>::kStage];
+  uint32_t list[NW][kBrList];  // literal << 31 | output offset in the wave << 12 | header
+  uint32_t out[NW][kBrOut / 4];
+  uint32_t exits[2][NW], entry[2][NW], early[NW];
+  uint32_t part[NW];
   uint32_t err;
 };
 constexpr uint32_t kBrSpan = kWave * kBrBlock;  // stream bytes of a wave
@@ -145,6 +151,7 @@ struct BrleItems {
 
 // Writes the items, output offset 0 being byte o0 of dst, which is 16-byte
 // aligned, and their bytes [x0, x1).
+template <uint32_t STAGE>
 __device__ __forceinline__ void brle_write(uint8_t *dst, const BrleItems &it, uint32_t *ow, uint32_t o0, uint32_t x0,
                                            uint32_t x1, uint32_t lane) {
   uint8_t *ob = reinterpret_cast<uint8_t *>(ow);
@@ -184,7 +191,7 @@ __device__ __forceinline__ void brle_write(uint8_t *dst, const BrleItems &it, ui
       for (uint32_t r = 0; r < 4; r++) {
         const uint32_t in_item = 4 * (r0 + r * kWave + lane) - ow0 - ((x[r] >> 12) & 0x7ffffu);
         const int32_t b = (int32_t)(it.first + 1 + (x[r] & 4095u) + ((int32_t)x[r] < 0 ? in_item : 0u));
-        a[r] = (uint32_t)min(max(b, 0), (int32_t)kBrStage - 8);
+        a[r] = (uint32_t)min(max(b, 0), (int32_t)STAGE - 8);
         lo[r] = stage32[a[r] >> 2];
         hi[r] = stage32[(a[r] >> 2) + 1];
       }
@@ -239,12 +246,13 @@ __device__ __forceinline__ void brle_write(uint8_t *dst, const BrleItems &it, ui
   }
 }
 
-__global__ void __launch_bounds__(kBrThreads) __attribute__((amdgpu_waves_per_eu(5)))
-brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
-                                                                 const uint64_t *ptr, uint64_t n,
-                                                                 uint64_t chunk_bytes, uint8_t *out,
-                                                                 uint64_t *out_len, int32_t *status) {
-  __shared__ BrleLds S;
+template <int NW>
+__global__ void __launch_bounds__(NW *kWave) __attribute__((amdgpu_waves_per_eu(5)))
+brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ptr, uint64_t n, uint64_t chunk_bytes,
+                   uint8_t *out, uint64_t *out_len, int32_t *status) {
+  constexpr int kBrWaves = NW;
+  constexpr uint32_t kBrThreads = BrCfg<NW>::kThreads, kBrStage = BrCfg<NW>::kStage, kBrLoads = BrCfg<NW>::kLoads;
+  __shared__ BrleLds<NW> S;
   const uint32_t lane = lane_id(), tid = threadIdx.x;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid) / kWave;
   const uint64_t ci = blockIdx.x;
@@ -263,7 +271,7 @@ brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
   const uint32_t len = (uint32_t)len64, cap = (uint32_t)chunk_bytes;
   uint8_t *dst = out + ci * chunk_bytes;
   const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(dst) & 15u);
-  uint32_t at = 0, pos = 0, lead = 0;
+  uint32_t at = 0, pos = 0, lead = 0, passes = kBrPasses;
   uint4 v[kBrLoads];
   auto load = [&](uint32_t from) __attribute__((always_inline)) {
     lead = (uint32_t)(reinterpret_cast<uintptr_t>(src) + from) & 15u;
@@ -323,23 +331,76 @@ brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
       }
       exit = q;
     };
-    walk();
-    uint32_t entry = wave ? wave * kBrSpan : in0, end;  // entry of the wave's first lane, exit of the step
-    for (uint32_t r = 0;; r ^= 1) {
-      for (;;) {
-        // what the wave before has now; the check below is made on final exits
-        if (lane == kWave - 1) __hip_atomic_store(&S.early[wave], exit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (wave) entry = uni(__hip_atomic_load(&S.early[wave - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-        const uint32_t x = (uint32_t)__builtin_amdgcn_update_dpp((int)entry, (int)exit, 0x138, 0xf, 0xf, false);  // wave_shr:1
-        if (!__ballot(x != from)) break;
-        if (x != from) {
-          from = x;
-          walk();
+    // The wave's chain from byte q on, block by block in scalars, where its lanes do
+    // not find each other: the starts that count lie far apart then (long literals),
+    // and many blocks are passed over.
+    bool chained = false;
+    auto chain = [&](uint32_t q) __attribute__((always_inline)) {
+      const uint32_t base = wave * kBrSpan, stop = min(base + kBrSpan, limit), entry = q;
+      mask = 0;
+      from = exit = 0;
+      while (q < stop) {
+        const uint32_t l = (q - base) / kBrBlock, l0 = base + l * kBrBlock, l1 = min(l0 + kBrBlock, limit);
+        const uint64_t js = (uint64_t)rdlane((uint32_t)(jumps >> 32), l) << 32 | rdlane((uint32_t)jumps, l);
+        const uint32_t q0 = q;
+        uint64_t m = 0;
+        while (q < l1) {
+          const uint64_t path = ((uint64_t)0x5555555555555555ull << (q - l0)) & (((uint64_t)1 << (l1 - l0)) - 1), j = path & js;
+          m |= path & (j ^ (j - 1));
+          if (!j) {
+            q = l1 + ((q ^ l1) & 1u);
+          } else {
+            q = l0 + (uint32_t)__builtin_ctzll(j);
+            q += uni(in[q]) - 126u;
+          }
+        }
+        if (lane == l) {
+          mask = m;
+          from = q0;
+          exit = q;
         }
       }
-      if (lane == kWave - 1) {
-        S.exits[r][wave] = exit;
-        S.entry[r][wave] = entry;
+      chained = true;
+      // the blocks passed over
+      const uint32_t incl = wave_max_dpp(exit);
+      const uint32_t x = max((uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x138, 0xf, 0xf, false), entry);
+      if (lo < limit && !exit) from = exit = x;
+    };
+    walk();
+    // a block behind the stream's end has no part in what follows
+    const bool mine = lo < limit;
+    const uint32_t blocks = (uint32_t)__builtin_popcountll(__ballot(mine));
+    exit = mine ? exit : 0u;
+    uint32_t entry = wave ? wave * kBrSpan : in0, end;  // entry of the wave's first lane, exit of the step
+    for (uint32_t round = 0;; round++) {
+      const uint32_t r = round & 1;
+      uint32_t top = 0;  // the wave's exit
+      // where chains are followed one by one, a wave waits for the one before it
+      const bool ready = passes == kBrPasses || wave <= round;
+      for (uint32_t pass = 0; ready; pass++) {
+        // Right exits grow from lane to lane, so a block is entered at the greatest exit
+        // before it: an item that passes whole blocks reaches the one it ends in at once.
+        const uint32_t incl = wave_max_dpp(exit);
+        // what the wave before has now; the check below is made on final exits
+        if (wave) entry = uni(__hip_atomic_load(&S.early[wave - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        top = max(rdlane(incl, kWave - 1), entry);
+        if (lane == 0) __hip_atomic_store(&S.early[wave], top, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint32_t x = max((uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x138, 0xf, 0xf, false), entry);  // wave_shr:1
+        const uint64_t wrong = __ballot(mine && x != from);
+        if (!wrong) break;
+        // where walks meet, few blocks are left after three
+        if (pass < passes && (pass < 3 || 8 * (uint32_t)__builtin_popcountll(wrong) <= 3 * blocks)) {
+          if (mine && x != from) {
+            from = x;
+            walk();
+          }
+        } else {
+          chain(entry);
+        }
+      }
+      if (lane == 0) {
+        S.exits[r][wave] = top;
+        S.entry[r][wave] = ready ? entry : ~0u;  // no exit: another round
       }
       __syncthreads();
       bool all = true;
@@ -353,11 +414,17 @@ brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
       if (all) break;
     }
     if (end < limit) load(at + (end - in0));
-    // output bytes and items, of the lane and before it
-    uint32_t n = 0;
-    for (uint64_t m = mask; m; m &= m - 1) {
-      const uint32_t h = in[lo + (uint32_t)__builtin_ctzll(m)];
-      n += h > 127u ? h - 127u : h + 3u;
+    // while a third of the blocks and more are passed over, the next steps come to the
+    // chain after kBrFew walks
+    if (chained) passes = __builtin_popcountll(__ballot(mask != 0)) <= 42 ? kBrFew : kBrPasses;
+    // output bytes and items, of the lane and before it: a header h is 3 + h bytes, one
+    // above 127 is 130 fewer
+    uint32_t n = 3 * (uint32_t)__builtin_popcountll(mask);
+#pragma unroll
+    for (uint32_t k = 0; k < kBrBlock / 4; k++) {
+      const uint32_t d = reinterpret_cast<const uint32_t *>(in + lo)[k];
+      const uint32_t ones = (((uint32_t)(mask >> (4 * k)) & 15u) * 0x204081u) & 0x01010101u;  // bytes with a start
+      n = __builtin_amdgcn_udot4(d, ones, n, false) - 130u * (uint32_t)__popc(d & ones << 7);
     }
     uint32_t incl = wave_scan_dpp(n | (uint32_t)__builtin_popcountll(mask) << 20);
     if (lane == kWave - 1) S.part[wave] = incl & 0xfffffu;
@@ -394,16 +461,25 @@ brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes,
     for (uint32_t b0 = 0; b0 < items; b0 += kBrList) {
       uint32_t i = (incl >> 20) - (uint32_t)__builtin_popcountll(mask) - b0;
       uint32_t o = (incl & 0xfffffu) - n;
-      for (uint64_t m = mask; m; m &= m - 1, i++) {
-        const uint32_t q = lo + (uint32_t)__builtin_ctzll(m), h = in[q];
-        if (i < kBrList) S.list[wave][i] = (h & 0x80u) << 24 | o << 12 | (q - wave * kBrSpan);
-        o += h > 127u ? h - 127u : h + 3u;
+      for (uint64_t m = mask; m;) {  // the headers of four items are read together
+        uint32_t q[4], h[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          q[k] = m ? lo + (uint32_t)__builtin_ctzll(m) : ~0u;
+          m &= m - 1;
+          h[k] = in[min(q[k], kBrStage - 1)];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++, i++) {
+          if (q[k] != ~0u && i < kBrList) S.list[wave][i] = (h[k] & 0x80u) << 24 | o << 12 | (q[k] - wave * kBrSpan);
+          o += h[k] > 127u ? h[k] - 127u : h[k] + 3u;
+        }
       }
       lds_order();
       it.nb = min(items - b0, kBrList);
       const uint32_t f = uni(it.get(0).o);
       const BrleItems::Item l = it.get(it.nb - 1);
-      brle_write(dst - mis, it, S.out[wave], o0, o0 + f, o0 + uni(l.o + l.k), lane);
+      brle_write<kBrStage>(dst - mis, it, S.out[wave], o0, o0 + f, o0 + uni(l.o + l.k), lane);
     }
     __syncthreads();
     const uint32_t es = uni(S.err);
@@ -636,10 +712,14 @@ lzss_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *end
 
 hipError_t launch_brle_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ptr,
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
-                              int32_t *status, hipStream_t stream) {
+                              int32_t *status, hipStream_t stream, bool few) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(bytecodec::brle_chunks_kernel, dim3((uint32_t)n), dim3(bytecodec::kBrThreads), 0,
-                     stream, comp, comp_bytes, ptr, n, chunk_bytes, out, out_len, status);
+  if (few)
+    hipLaunchKernelGGL(bytecodec::brle_chunks_kernel<1>, dim3((uint32_t)n), dim3(kWaveSize), 0, stream, comp, comp_bytes,
+                       ptr, n, chunk_bytes, out, out_len, status);
+  else
+    hipLaunchKernelGGL(bytecodec::brle_chunks_kernel<4>, dim3((uint32_t)n), dim3(4 * kWaveSize), 0, stream, comp,
+                       comp_bytes, ptr, n, chunk_bytes, out, out_len, status);
   return hipGetLastError();
 }
 
