@@ -67,7 +67,7 @@ struct codag_ctx {
   char name[256] = {0};
   codag_tune_params tune[4];
   uint32_t chunks_two_wave = 0;
-  uint32_t byte_waves = 0;  // BRLE kernel: 0 chosen by the streams, 1 or 4 waves per chunk (tests)
+  uint32_t byte_waves = 0;  // BRLE and LZSS kernels: 0 chosen by the streams, 1 or 4 waves per chunk (tests)
   uint32_t poll_shift = 0;  // RLE v2 queue kernel: nonzero = waits without polls (tests)
 };
 
@@ -213,6 +213,22 @@ bool brle_few(uint64_t comp_bytes, uint64_t n, uint32_t cus) {
   const uint64_t each = comp_bytes / n;  // stream bytes of a chunk
   if (each <= 4200) return true;
   return n > (each <= 24576 ? 7ull : 15ull) * cus;
+}
+
+// Whether an LZSS container goes by lzss_serial_kernel, one wave per chunk with its
+// matches copied one after the other, or by four waves through a window of marks,
+// where every output byte costs the same. Four waves and one, us: text never one (512
+// chunks of 128 KiB 631, 2474, 2048 chunks 1326, 3061); zeros and the like, 16 output
+// bytes per stream byte, 512 chunks 157, 166, 1024 chunks 195, 170, 2048 chunks 338,
+// 191, of 1 KiB 16384 chunks 97, 22; a log, 4 to 7 output bytes per stream byte,
+// chunks of 1 KiB (253 stream bytes) 1024 chunks 12, 10, of 4 KiB (697) 1024 chunks
+// 17, 23, 2048 chunks 28, 27, of 16 KiB (2476) 2048 chunks 65, 80, 4096 chunks 111,
+// 102, of 128 KiB 2048 chunks 473, 579.
+bool lzss_serial(uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes, uint32_t cus) {
+  const uint64_t each = comp_bytes / n;  // stream bytes of a chunk
+  if (each <= chunk_bytes / 10) return n > 2ull * cus || each <= 128;
+  if (each > chunk_bytes / 7 * 2) return false;
+  return each <= 300 || n > (each <= 1000 ? 7ull : 15ull) * cus;
 }
 
 void default_tune(codag_ctx *c) {
@@ -462,8 +478,10 @@ codag_status codag_lzss_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t c
   if (codag_status s = byte_codec_args("lzss_decode", ctx, d_comp, d_ends, n_chunks, chunk_bytes, d_out))
     return s;
   DeviceGuard g(ctx->device);
+  bool serial = n_chunks && lzss_serial(comp_bytes, n_chunks, chunk_bytes, ctx->cu_count);
+  if (ctx->byte_waves) serial = ctx->byte_waves == 1;
   HIP_TRY(launch_lzss_chunks(d_comp, comp_bytes, d_ends, n_chunks, chunk_bytes, d_out, d_out_len,
-                             d_status, pick(ctx, stream)));
+                             d_status, pick(ctx, stream), serial));
   return CODAG_OK;
 }
 
@@ -855,19 +873,19 @@ uint32_t codag_test_route(codag_ctx *ctx, codag_codec codec, uint64_t comp_bytes
                               : rlev2_route(t, n, w, chunk_bytes, comp_bytes, ctx->cu_count, ctx->poll_shift == 0);
 }
 
-// Test hook, not in the public header: the waves per chunk of the BRLE kernel, 1 or
-// 4, or 0 for the choice by the streams.
+// Test hook, not in the public header: the waves per chunk of the BRLE and LZSS
+// kernels, 1 or 4, or 0 for the choice by the streams.
 codag_status codag_test_byte_waves(codag_ctx *ctx, uint32_t waves) {
   if (!ctx) return fail(CODAG_ERR_INVALID, "test_byte_waves: null ctx");
   ctx->byte_waves = waves;
   return CODAG_OK;
 }
 
-// Test hook, not in the public header: whether codag_brle_decode of n > 0 chunks
-// takes the kernel of one wave per chunk.
+// Test hook, not in the public header: whether codag_brle_decode (codag_lzss_decode)
+// of n > 0 chunks takes the kernel of one wave per chunk.
 uint32_t codag_test_byte_one(codag_ctx *ctx, uint32_t lzss, uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes) {
-  (void)chunk_bytes;
-  return !ctx || !n || lzss ? ~0u : brle_few(comp_bytes, n, ctx->cu_count);
+  if (!ctx || !n) return ~0u;
+  return lzss ? lzss_serial(comp_bytes, n, chunk_bytes, ctx->cu_count) : brle_few(comp_bytes, n, ctx->cu_count);
 }
 
 // Test hook, not in the public header: whether codag_inflate_chunks takes eight waves.

@@ -20,7 +20,8 @@
 // guessed starts that are put right until they agree, LZSS from every byte a group
 // may begin at. BRLE's output is made from its items dword by dword, LZSS's
 // resolved in an LDS window of marks. The next part of the stream is loaded
-// meanwhile.
+// meanwhile. A second LZSS kernel, one wave per chunk, copies match by match: for
+// very compressible streams and many small chunks.
 //
 // The reference checks nothing; these kernels report per chunk: TRUNCATED if
 // the stream ends inside an item, OVERFLOW if the output would pass the
@@ -708,6 +709,145 @@ lzss_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *end
   }
 }
 
+// One wave per chunk, eight groups at a time, lane 8g + k holding item k of group g;
+// the output goes through a ring of LDS. Literals and matches with sources before
+// the eight groups are written by all lanes at once, other matches one after the
+// other, a match a step. A byte costs next to nothing in a long match, and a chunk
+// next to nothing in setup, so this is the kernel for very compressible streams and
+// for many small chunks (see lzss_serial in capi.cpp for both kernels' times).
+constexpr uint32_t kLsWin = 1024;   // staged stream bytes, 16 a lane
+constexpr uint32_t kLsHead = 512;   // flag bytes the walk reads lie in these: two registers
+constexpr uint32_t kLsRing = 4096;  // 2047 bytes of history, a batch, and the < 16 bytes a store keeps back
+constexpr uint32_t kLsBatch = kLsRing - 2048 - 16;
+static_assert(kLsHead + 17 <= kLsWin && 7 * 8 * 34 <= kLsBatch, "items end in the window; seven groups fit a batch");
+
+struct __align__(16) LzssSerialLds {
+  uint8_t ring[kLsRing];
+  uint8_t win[kLsWin];
+};
+
+__global__ void __launch_bounds__(kWave)
+lzss_serial_kernel(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ends, uint64_t n, uint64_t chunk_bytes,
+                   uint8_t *out, uint64_t *out_len, int32_t *status) {
+  __shared__ LzssSerialLds S;
+  const uint32_t lane = lane_id(), g = lane >> 3, k = lane & 7u;
+  const uint64_t ci = blockIdx.x;
+  if (ci >= n) return;
+  const uint64_t begin = ci ? ends[ci - 1] : 0;  // lzss.h:237-238
+  uint64_t len64;
+  int32_t err;
+  chunk_bounds(begin, ends[ci], comp_bytes, len64, err);
+  const uint8_t *src = comp + begin;
+  const uint32_t len = (uint32_t)len64, cap = (uint32_t)chunk_bytes;
+  uint8_t *dst = out + ci * chunk_bytes;
+  // output byte x is ring byte (x + mis) mod kLsRing, so 16-byte aligned addresses stay so
+  const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(dst) & 15u);
+  auto at_ring = [&](uint32_t x) -> uint8_t & { return S.ring[(x + mis) & (kLsRing - 1)]; };
+  uint32_t pos = 0, flushed = 0, at = 0;
+  // bytes up to a 16-byte boundary, then vectors; the last call also writes the tail
+  auto store = [&](bool last) {
+    uint32_t x = flushed;
+    const uint32_t head = min((0u - (mis + x)) & 15u, pos - x);
+    if (lane < head) dst[x + lane] = at_ring(x + lane);
+    x += head;
+    const uint32_t nvec = (pos - x) / 16u;
+    for (uint32_t i = lane; i < nvec; i += kWave)
+      *reinterpret_cast<uint4 *>(dst + x + 16 * i) = *reinterpret_cast<const uint4 *>(&at_ring(x + 16 * i));
+    x += nvec * 16u;
+    if (last) {
+      if (lane < pos - x) dst[x + lane] = at_ring(x + lane);
+      x = pos;
+    }
+    flushed = x;
+  };
+  Window w = window_load(src, len, 0, lane);
+  while (at < len && err == kOk) {
+    lds_order();
+    reinterpret_cast<uint4 *>(S.win)[lane] = w.v;
+    lds_order();
+    const uint32_t lead = uni(w.lead), qend = lead + (len - at);
+    const uint32_t h0 = reinterpret_cast<const uint32_t *>(S.win)[lane];
+    const uint32_t h1 = reinterpret_cast<const uint32_t *>(S.win)[kWave + lane];
+    // walk over the flag bytes: group j's start -> lane j of gq
+    uint32_t q = lead, ng = 0, gq = 0;
+    while (ng < 8u && q < kLsHead && q < qend) {
+      const uint32_t l = (q >> 2) & 63u, d0 = rdlane(h0, l), d1 = rdlane(h1, l);
+      const uint32_t f = ((q < 256u ? d0 : d1) >> 8 * (q & 3u)) & 255u;
+      gq = lane == ng ? q : gq;
+      ng++;
+      q += 17u - (uint32_t)__builtin_popcount(f);
+    }
+    // items (lzss.h:268-303)
+    const uint32_t gs = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(g << 2), (int)gq), f = S.win[gs];
+    const uint32_t ip = gs + 1u + 2u * k - (uint32_t)__builtin_popcount(f & ((1u << k) - 1u));
+    const bool exists = g < ng && ip < qend;
+    const bool lit = exists && ((f >> k) & 1u), mat = exists && !lit;
+    const uint32_t b0 = S.win[ip], v = b0 | (uint32_t)S.win[ip + 1u] << 8;
+    const uint32_t mlen = (v & 31u) + 3u, off = v >> 5;
+    const uint32_t tl = lit ? 1u : (mat ? mlen : 0u);
+    const uint32_t incl = wave_scan_dpp(tl);
+    // an eighth group that would take the batch past kLsBatch waits
+    const uint32_t keep_g = rdlane(incl, kWave - 1) > kLsBatch ? 7u : ng;
+    const uint32_t x = pos + incl - tl;
+    uint32_t e = 0;
+    if (g < keep_g && exists) {
+      if (mat && ip + 2u > qend) e = (uint32_t)kTrunc;
+      else if (mat && (off == 0u || off > x)) e = (uint32_t)kCorrupt;
+      else if (x + tl > cap) e = (uint32_t)kOverflow;
+    }
+    const uint64_t em = __ballot(e != 0u);
+    uint32_t nk = keep_g * 8u;  // lanes kept (items past the stream end have tl 0)
+    if (em) {
+      nk = (uint32_t)__builtin_ctzll(em);
+      err = (int32_t)rdlane(e, nk);
+    }
+    const bool keep = lane < nk;
+    const uint32_t pend = pos + (nk ? rdlane(incl, nk - 1u) : 0u);
+    // the kept groups are consumed (the last may end at the stream's end)
+    at += (keep_g < ng ? rdlane(gq, keep_g) : min(q, qend)) - lead;
+    if (err == kOk && at < len) w = window_load(src, len, at, lane);
+    if (keep && lit) at_ring(x) = (uint8_t)b0;
+    // matches whose source ends before the batch: all lanes at once, 4 bytes a
+    // step (bytes past a match's end repeat its last byte's copy)
+    const bool km = keep && mat, ind = km && (x - off) + mlen <= pos;
+    if (__ballot(ind)) {
+      const uint32_t sp = x - off, last = mlen - 1u;
+      for (uint32_t i = 0; i < 34u; i += 4u) {
+        if (!__ballot(ind && i < mlen)) break;
+        if (ind && i < mlen) {
+          const uint32_t k1 = min(i + 1u, last), k2 = min(i + 2u, last), k3 = min(i + 3u, last);
+          const uint8_t c0 = at_ring(sp + i), c1 = at_ring(sp + k1), c2 = at_ring(sp + k2), c3 = at_ring(sp + k3);
+          at_ring(x + i) = c0;
+          at_ring(x + k1) = c1;
+          at_ring(x + k2) = c2;
+          at_ring(x + k3) = c3;
+        }
+      }
+    }
+    // the others read bytes of this batch: in stream order, one per step; byte i is
+    // source byte i, or i mod oj where the match overlaps itself (lzss.h:285-288)
+    for (uint64_t dm = __ballot(km && !ind); dm; dm &= dm - 1) {
+      const uint32_t j = (uint32_t)__builtin_ctzll(dm);
+      const uint32_t xj = rdlane(x, j), oj = rdlane(off, j), lj = rdlane(mlen, j);
+      lds_order();
+      if (lane < lj) {
+        uint32_t m = lane;  // lane + 0.5 is at least 0.5 away from a multiple of oj: the quotient is exact
+        if (oj < lj) m -= __umul24((uint32_t)(((float)lane + 0.5f) * __builtin_amdgcn_rcpf((float)oj)), oj);
+        at_ring(xj + lane) = at_ring(xj - oj + m);
+      }
+    }
+    lds_order();
+    pos = pend;
+    store(false);
+  }
+  lds_order();
+  store(true);
+  if (lane == 0) {
+    if (out_len) out_len[ci] = pos;
+    if (status) status[ci] = err;
+  }
+}
+
 }  // namespace bytecodec
 
 hipError_t launch_brle_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ptr,
@@ -725,10 +865,14 @@ hipError_t launch_brle_chunks(const uint8_t *comp, uint64_t comp_bytes, const ui
 
 hipError_t launch_lzss_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ends,
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
-                              int32_t *status, hipStream_t stream) {
+                              int32_t *status, hipStream_t stream, bool serial) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(bytecodec::lzss_chunks_kernel, dim3((uint32_t)n), dim3(bytecodec::kLzThreads), 0, stream,
-                     comp, comp_bytes, ends, n, chunk_bytes, out, out_len, status);
+  if (serial)
+    hipLaunchKernelGGL(bytecodec::lzss_serial_kernel, dim3((uint32_t)n), dim3(kWaveSize), 0, stream, comp, comp_bytes,
+                       ends, n, chunk_bytes, out, out_len, status);
+  else
+    hipLaunchKernelGGL(bytecodec::lzss_chunks_kernel, dim3((uint32_t)n), dim3(bytecodec::kLzThreads), 0, stream,
+                       comp, comp_bytes, ends, n, chunk_bytes, out, out_len, status);
   return hipGetLastError();
 }
 

@@ -81,13 +81,14 @@ hipError_t launch_rlev2_span(const uint8_t *comp, uint64_t comp_bytes, const uin
                              uint64_t chunk_bytes, uint8_t *out, int32_t *status,
                              hipStream_t stream);
 
-// BRLE / LZSS, four waves per chunk (chunk_bytes < 2^31); few: one wave (BRLE).
+// BRLE / LZSS, four waves per chunk (chunk_bytes < 2^31); few (BRLE), serial
+// (LZSS): one wave.
 hipError_t launch_brle_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ptr,
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
                               int32_t *status, hipStream_t stream, bool few);
 hipError_t launch_lzss_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ends,
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
-                              int32_t *status, hipStream_t stream);
+                              int32_t *status, hipStream_t stream, bool serial);
 
 // Plain device copy (16-byte loads/stores): the reference point for HBM
 // traffic counters.

@@ -27,7 +27,7 @@ def ctx(gpu_required, request):
     c.close()
 
 
-@pytest.mark.parametrize("lzss", [False])
+@pytest.mark.parametrize("lzss", [False, True])
 def test_kats(ctx, lzss):
     say(f"byte codecs by waves: KATs, lzss {lzss}")
     for s, chunk in LZSS_KATS if lzss else BRLE_KATS:
@@ -84,6 +84,51 @@ def test_brle_random_and_damaged(ctx):
         compare(ctx, False, data, ptr, cap, 7)
 
 
+@pytest.mark.parametrize("kind", ["noise", "runs", "period", "text"])
+def test_lzss_payloads(ctx, kind):
+    say(f"lzss by waves, {kind}")
+    streams = []
+    for n in (1, 17, 1535, 1536, 6145, 50000):
+        data, ends, _, _ = ca.lzss_container(ca.lzss_encode(lparts.payload(kind, n), max(n, 1)))
+        streams.append(np.array(data)[:int(ends[0])].tobytes())
+    streams += [streams[-1][:k] for k in (*range(0, 40), 400, 512, 520, 1000, 1023, 1024, 3119, 3120, 3121) if k < len(streams[-1])]
+    data, ends = lzss_container(streams)
+    for cap in (1, 100, 4096, 49999, 50000):
+        compare(ctx, True, data, ends, cap, 9)
+
+
+def test_lzss_random_and_damaged(ctx):
+    say("lzss by waves, random and damaged")
+    rng = np.random.default_rng(23)
+    streams = []
+    for near in (0.0, 0.3, 0.8, 1.0):
+        s, _ = random_lzss_stream(rng, 60000, near)
+        streams.append(s)
+        for _ in range(5):
+            d = bytearray(s)
+            for _ in range(3):
+                d[int(rng.integers(0, len(d)))] = int(rng.integers(0, 256))
+            streams.append(bytes(d[:int(rng.integers(1, len(d) + 1))]))
+    streams += [rng.integers(0, 256, n, dtype=np.uint8).tobytes() for n in (5, 700, 5000)] + [b""]
+    # matches that repeat 1 to 40 bytes, one after the other
+    for d in (1, 2, 3, 7, 33, 34, 35, 40):
+        s = bytearray()
+        made = 0
+        for item in range(4000):
+            if item % 8 == 0:
+                s.append(0xFF if item < (d + 7) // 8 * 8 else 0)
+            if item < (d + 7) // 8 * 8:
+                s.append(int(rng.integers(0, 256)))
+                made += 1
+            else:
+                v = (d << 5) | int(rng.integers(0, 32))
+                s += bytes([v & 255, v >> 8])
+        streams.append(bytes(s))
+    data, ends = lzss_container(streams)
+    for cap in (30000, 80000):
+        compare(ctx, True, data, ends, cap, 11)
+
+
 def test_choice(ctx):
     say("byte codecs: the choice by the streams")
     cus = ctx.info()[1]
@@ -95,4 +140,8 @@ def test_choice(ctx):
         assert one(0, 4200, n, 262144) == 1
     assert [one(0, 20000, n, 262144) for n in (1, 7 * cus, 7 * cus + 1)] == [0, 0, 1]
     assert [one(0, 100000, n, 262144) for n in (1, 15 * cus, 15 * cus + 1)] == [0, 0, 1]
-    assert one(0, 0, 1, 1) == 1
+    assert [one(1, 8000, n, 131072) for n in (1, 2 * cus, 2 * cus + 1)] == [0, 0, 1]
+    assert one(1, 100, 1, 1024) == 1 and one(1, 250, 1, 1024) == 1 and one(1, 900, 10 ** 6, 1024) == 0
+    assert [one(1, 700, n, 4096) for n in (7 * cus, 7 * cus + 1)] == [0, 1]
+    assert [one(1, 20000, n, 131072) for n in (15 * cus, 15 * cus + 1)] == [0, 1]
+    assert one(0, 0, 1, 1) == 1 and one(1, 0, 1, 1) == 1
