@@ -256,9 +256,9 @@ struct DevBuf {
   template <typename T> T *as() const { return static_cast<T *>(p); }
 };
 
-// The device buffers of one call, 256-byte aligned parts of one allocation: a
-// hipMalloc and a hipFree take 19 us, which five buffers paid five times (host call
-// of a 4 MiB RLE v1 column: 885 us, now 855).
+// The device buffers of one call, 256-byte aligned parts of one allocation instead
+// of five: a hipMalloc and its hipFree take up to 19 us, though the host call of a
+// 4 MiB RLE v1 column gained less than four of them (885 us, with one 855).
 struct DevPart {
   void *p = nullptr;
   template <typename T> T *as() const { return static_cast<T *>(p); }
@@ -856,7 +856,7 @@ codag_status codag_lzss_decode_host(codag_ctx *ctx, const uint8_t *c, uint64_t c
 // ------------------------------------------------------------------ tuning
 
 // Test hook, not in the public header: codag_inflate_chunks' workgroups --
-// 0 chosen by chunk count, 1 eight waves per chunk, 2 one wave per chunk.
+// 0 chosen by inflate_many, 1 eight waves per chunk, 2 one wave per chunk.
 codag_status codag_test_chunks_two_wave(codag_ctx *ctx, uint32_t on) {
   if (!ctx) return fail(CODAG_ERR_INVALID, "test_chunks_two_wave: null ctx");
   ctx->chunks_two_wave = on;
@@ -964,8 +964,8 @@ codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_
   DevBuf d_st, d_descs, d_res;
   HIP_TRY(d_st.alloc(n_chunks * 8 + 8));
   if (codec == CODAG_DEFLATE) {
-    // Deflate candidates differ in the persistent batch launch (waves per CU
-    // pulling from the work queue): time that launch on the sample's chunks.
+    // Deflate candidates differ in the persistent batch launch (one wave a stream or
+    // the plan's choice, and groups per CU): time that launch on the sample's chunks.
     std::vector<uint64_t> off(n_chunks + 1);
     HIP_TRY(hipMemcpy(off.data(), d_blk_off, 8 * (n_chunks + 1), hipMemcpyDeviceToHost));
     std::vector<codag_stream_desc> descs(n_chunks);

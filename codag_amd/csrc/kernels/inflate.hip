@@ -20,18 +20,21 @@
 //    hands every byte its token's mark, sources before the window are gathered
 //    from HBM a step ahead, sources inside it are followed by pointer doubling;
 //    the bytes are stored and summed for the Adler-32.
+//  * Codes of nearly one length do not synchronise: chain_entries finds the lanes'
+//    entries from all bits at which the token before may end.
+//  * Long matches: narrow_span decodes by one wave, 64 stream bits at a time.
 //  * The scalar symbol loop decodes the symbol a span stopped at (end of block,
 //    or the error), so statuses are exactly the serial decoder's.
 // What bounds it: vector issue and its latency, not memory (without the far
 // gathers and the stores the launches take the same time). 128 KiB zlib level-6
 // chunks, before (one token chain per stream: 64 bit positions decoded to keep
-// about seven tokens, the chain scalar) and now: 4096 chunks 9.1 and 3.0 ms, 256
-// chunks 4.0 and 0.45 ms, 3 chunks 3.7 and 0.42 ms; 300 mixed streams of 4 KiB
-// to 4 MiB 119 and 15 ms. A chunk takes 0.27 M vector instructions (0.69 M
+// about seven tokens, the chain scalar) and now: 4096 chunks 9.1 and 2.96 ms, 256
+// chunks 4.0 and 0.44 ms, 3 chunks 3.7 and 0.42 ms; 300 mixed streams of 4 KiB
+// to 4 MiB 119 and 14.6 ms. A chunk takes 0.27 M vector instructions (0.69 M
 // before): half of them passes, headers and tables, a fifth marks, a third the
-// resolving. Data that compress below 5% are slower than the copy loop of the
-// serial decoder where there are many chunks (4096 chunks of zeros 1.1 and 2.7
-// ms): a window byte costs the same whatever token it is in.
+// resolving. A window byte costs the same whatever token it is in, so data that
+// compress to less than a thirtieth go by narrow_span (4096 chunks of zeros 1.1
+// before, 0.74 ms now; with a one every 200 bytes 0.88 and 0.96).
 //
 // Reference counterpart: include/zlib/zlib.h:807-866 (full_warp_shared_lut),
 // 531-707 (dynamic header / table build), 712-805 (symbol loop), 188-347
@@ -765,8 +768,8 @@ __device__ __forceinline__ int32_t emit(Out &o, Sh<C> &S, uint32_t q, uint32_t n
     const uint32_t stopx = min(end, done + wn);
     // One lookup a step without branches: a lookup that completes no token writes
     // its mark behind the window (with a branch for each kind of entry, 25 scalar
-    // instructions more a step, 4096 chunks took 3.20 ms and 3 chunks 445 us, now
-    // 3.09 and 419).
+    // instructions more a step, 4096 chunks took 3.20 ms and 3 chunks 445 us, without
+    // 3.09 and 419; both before the window was resolved four bytes a lane).
     uint32_t d = C::kLitDesc, mlen = 0, bad = ~0u;
     uint32_t goal = stopx;
     while (x < goal) {
@@ -1614,9 +1617,12 @@ inflate_chunks_many_kernel(const uint8_t *__restrict__ comp, uint64_t comp_bytes
 
 // The queue of a batch, in device memory: its next stream and whether groups of
 // eight waves or of one decode it.
-//  * One wave takes about 20 ns per compressed byte of its stream and the GPU's
-//    one-wave groups together 1/85 ns; eight-wave groups take about 150 ns per
-//    stream and 1/78 ns per compressed byte over all. So eight waves win until
+//  * The plan's constants are fits to zlib streams of text and numbers on 256 CUs:
+//    one wave takes about 20 ns per compressed byte of its stream and the GPU's
+//    one-wave groups together 1/85 ns; its eight-wave groups together take about
+//    150 ns per stream and 1/78 ns per compressed byte. (gzip members also pay
+//    their CRC-32: 3000 small ones go by eight waves, 0.93 ms, and would take 0.78
+//    by one.) So eight waves win until
 //    there are many streams of about one size. Mixed zlib streams from 4 KiB on
 //    (one wave / eight waves, ms): 700 of up to 64 KiB 0.77 / 0.37, 3000 of up
 //    to 64 KiB 0.86 / 0.90, of up to 1 MiB 11.2 / 4.5, 6000 of up to 16 KiB

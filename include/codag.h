@@ -168,8 +168,9 @@ codag_status codag_inflate_batch(codag_ctx *ctx, const codag_stream_desc *d_desc
  * All calls on one GPU in a process share that counter and it keeps the last
  * call's contents: calls that overlap on one GPU (different streams or host
  * threads) race and must be serialized by the caller. Limits: n <= 2^32-2 streams per call
- * (larger n is rejected with CODAG_ERR_INVALID); groups_per_cu 0..64 resident
- * waves per CU (0 = 28). */
+ * (larger n is rejected with CODAG_ERR_INVALID); groups_per_cu 0..64 workgroups
+ * per CU (0 = 28) at most, of eight waves or one as in codag_inflate_batch: of
+ * eight waves never more than two are launched, of one about nine fit a CU. */
 codag_status codag_inflate_batch_noalloc(const codag_stream_desc *d_descs, uint64_t n,
                                          codag_stream_result *d_results, uint32_t flags,
                                          uint32_t groups_per_cu, codag_stream_t stream);
@@ -417,10 +418,11 @@ codag_status codag_tune_set(codag_ctx *ctx, codag_codec codec, const codag_tune_
  * d_col_len is ignored) and keep the fastest whose output equals the first
  * candidate's; the shape in use stays if it is within 2% of that one (a tie
  * in run-to-run noise does not flip the choice). The kept shape becomes the
- * context's shape; on an error the context's shape stays. best_ms (nullable) gets its time. DEFLATE candidates differ in
- * the batch launch's workgroups (one wave per stream, or by size) and workgroups
- * per CU; the launch has min(CUs x groups_per_cu, n_chunks) workgroups, so
- * the sample needs more than CUs x 28 streams for all of them to differ. */
+ * context's shape; on an error the context's shape stays. best_ms (nullable) gets
+ * its time. DEFLATE candidates differ in the batch launch's workgroups (one wave
+ * per stream, or by size) and in the most workgroups per CU, which only matters
+ * for groups of one wave and more than CUs x groups_per_cu streams: eight-wave
+ * groups are at most two per CU, and of one-wave groups about nine fit. */
 codag_status codag_tune_run(codag_ctx *ctx, codag_codec codec, const uint8_t *d_comp,
                             uint64_t comp_bytes, const uint64_t *d_blk_off, const uint64_t *d_col_len,
                             uint64_t n_chunks, uint32_t elem_bytes, uint64_t chunk_bytes,
