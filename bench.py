@@ -485,9 +485,9 @@ def bench_batch(ctx, args):
         tpg, per = (int(x) for x in args.c4_shape.split(","))
         ctx.tune_set(ca.DEFLATE, ca.TuneParams(tpg, 0, per, 1))
     elif not args.no_autotune:
-        # the autotuner times its launch shapes (one or two waves per stream,
-        # workgroups per CU) on the largest streams, which set the batch's
-        # finish time; it keeps the fastest shape whose output matches
+        # the autotuner times its launch shapes (one wave per stream, or eight or
+        # one by the streams' sizes; workgroups per CU) on the largest streams, which
+        # set the batch's finish time; it keeps the fastest shape whose output matches
         k = min(n, 512)
         ch = int(cap[0])
         d_soff = ctx.upload(soff[: k + 1].astype(np.uint64))
@@ -500,9 +500,11 @@ def bench_batch(ctx, args):
         log(f"[bench] c4: autotuner on {tuned['sample']}: {tbest.threads_per_group} threads x "
             f"{tbest.groups_per_cu} workgroups per CU ({tms:.1f} ms)")
     best = ctx.tune_get(ca.DEFLATE)
+    # with the shape that goes by size, this workload's streams (large and uneven) are
+    # decoded by eight waves each: profiles/byte_codecs_and_deflate.md
     kname = "inflate_batch_many_kernel" if best.threads_per_group == 128 else "inflate_batch_kernel"
-    log(f"[bench] c4: persistent launch, {best.threads_per_group} threads x "
-        f"{best.groups_per_cu} workgroups per CU")
+    how = "one wave per stream" if best.threads_per_group == 64 else "eight waves or one by size"
+    log(f"[bench] c4: persistent launch, {how}, up to {best.groups_per_cu} workgroups per CU")
 
     def check():
         rr = np.frombuffer(d_res.download(n * rsz).tobytes(), dtype=np.dtype(
@@ -584,7 +586,7 @@ def bench_batch(ctx, args):
         "wall_s": round(wall, 3),
         "per_file_launch_gbs": round(pf_gbs, 3),
         "per_file_sample": f"{len(samp)} streams, one inflate launch each",
-        "roofline": roofline(kname, ms, alg, f"{kname}:c4:{ctx.info()[1] * best.groups_per_cu}"),
+        "roofline": roofline(kname, ms, alg, f"{kname}:c4:{n}"),
         "cpu_baseline": cpu,
     }
 
@@ -747,11 +749,11 @@ def main():
     ap.add_argument("--no-autotune", action="store_true",
                     help="c1/c2: keep the default launch shape instead of tuning per column")
     ap.add_argument("--c4-shape", default=None, metavar="THREADS,PER_CU",
-                    help="c4: batch launch shape (64 = one wave per stream, 128 = a decoding "
-                         "and a writing wave), workgroups per CU; default: the library's")
+                    help="c4: batch launch shape (64 = one wave per stream, 128 = eight waves "
+                         "or one by size), workgroups per CU; default: the library's")
     ap.add_argument("--c3-waves", type=int, default=0, choices=[0, 1, 2],
-                    help="c3: waves per chunk (2 = a decoding and a writing wave; "
-                         "0 = the library's choice by chunk count)")
+                    help="c3: workgroups (1 = one wave per chunk, 2 = eight waves; "
+                         "0 = the library's choice by chunk count and sizes)")
     ap.add_argument("--copy-ref", type=int, default=0, metavar="MIB",
                     help="first run the plain copy kernel over MIB MiB (traffic calibration)")
     args = ap.parse_args()
