@@ -134,6 +134,7 @@ def lib():
         _sig(L, "codag_test_inflate_many", _u32, [_vp, _u64, _u64, _u64])
         _sig(L, "codag_test_byte_one", _u32, [_vp, _u32, _u64, _u64, _u64])
         _sig(L, "codag_test_byte_waves", st, [_vp, _u32])
+        _sig(L, "codag_test_lzss_waves", _u32, [_vp, _u64, _u64, _u64])
         _sig(L, "codag_test_route", _u32, [_vp, ctypes.c_int, _u64, _u64, _u32, _u64])
         _sig(L, "codag_brle_decode", st, [_vp, _vp, _u64, _vp, _u64, _u64, _vp, _vp, _vp, _vp])
         _sig(L, "codag_lzss_decode", st, [_vp, _vp, _u64, _vp, _u64, _u64, _vp, _vp, _vp, _vp])

@@ -67,7 +67,7 @@ struct codag_ctx {
   char name[256] = {0};
   codag_tune_params tune[4];
   uint32_t chunks_two_wave = 0;
-  uint32_t byte_waves = 0;  // BRLE and LZSS kernels: 0 chosen by the streams, 1 or 4 waves per chunk (tests)
+  uint32_t byte_waves = 0;  // BRLE and LZSS kernels: 0 chosen by the streams, 1 or 4 waves per chunk, 2 LZSS one wave with a window (tests)
   uint32_t poll_shift = 0;  // RLE v2 queue kernel: nonzero = waits without polls (tests)
 };
 
@@ -216,19 +216,31 @@ bool brle_few(uint64_t comp_bytes, uint64_t n, uint32_t cus) {
 }
 
 // Whether an LZSS container goes by lzss_serial_kernel, one wave per chunk with its
-// matches copied one after the other, or by four waves through a window of marks,
-// where every output byte costs the same. Four waves and one, us: text never one (512
+// matches copied one after the other, or through a window of marks (lzss_waves),
+// where every output byte costs the same. Window by four waves and this, us: text never one (512
 // chunks of 128 KiB 631, 2474, 2048 chunks 1326, 3061); zeros and the like, 16 output
 // bytes per stream byte, 512 chunks 157, 166, 1024 chunks 195, 170, 2048 chunks 338,
-// 191, of 1 KiB 16384 chunks 97, 22; a log, 4 to 7 output bytes per stream byte,
+// 191, of 1 KiB 16384 chunks 97, 22; 37 bytes repeated in 4 KiB (298 stream bytes) 512
+// chunks 13, 10; a log, 4 to 7 output bytes per stream byte,
 // chunks of 1 KiB (253 stream bytes) 1024 chunks 12, 10, of 4 KiB (697) 1024 chunks
 // 17, 23, 2048 chunks 28, 27, of 16 KiB (2476) 2048 chunks 65, 80, 4096 chunks 111,
 // 102, of 128 KiB 2048 chunks 473, 579.
 bool lzss_serial(uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes, uint32_t cus) {
   const uint64_t each = comp_bytes / n;  // stream bytes of a chunk
-  if (each <= chunk_bytes / 10) return n > 2ull * cus || each <= 128;
+  if (each <= chunk_bytes / 10) return n > 2ull * cus || each <= 300;
   if (each > chunk_bytes / 7 * 2) return false;
   return each <= 300 || n > (each <= 1000 ? 7ull : 15ull) * cus;
+}
+
+// The kernel of an LZSS container: 0 lzss_serial_kernel, 4 waves with a window, or 1
+// where there are many small chunks, whose streams are a step of one wave or two and
+// leave most lanes of four idle (four waves and one, us, 1 KiB chunks of a table: 1024
+// chunks 12, 14, 2048 chunks 20, 15, 4096 chunks 33, 20, 16384 chunks 114, 56; of
+// random bytes 11, 15, 18, 17, 30, 22, 106, 62; 4 KiB chunks of a log 2048 chunks 28,
+// 25, of random bytes 48, 68).
+uint32_t lzss_waves(uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes, uint32_t cus) {
+  if (lzss_serial(comp_bytes, n, chunk_bytes, cus)) return 0;
+  return n > 7ull * cus && chunk_bytes <= 4096 && comp_bytes / n <= 1500 ? 1 : 4;
 }
 
 void default_tune(codag_ctx *c) {
@@ -478,10 +490,10 @@ codag_status codag_lzss_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t c
   if (codag_status s = byte_codec_args("lzss_decode", ctx, d_comp, d_ends, n_chunks, chunk_bytes, d_out))
     return s;
   DeviceGuard g(ctx->device);
-  bool serial = n_chunks && lzss_serial(comp_bytes, n_chunks, chunk_bytes, ctx->cu_count);
-  if (ctx->byte_waves) serial = ctx->byte_waves == 1;
+  uint32_t waves = n_chunks ? lzss_waves(comp_bytes, n_chunks, chunk_bytes, ctx->cu_count) : 0;
+  if (ctx->byte_waves) waves = ctx->byte_waves == 1 ? 0 : (ctx->byte_waves == 2 ? 1 : 4);
   HIP_TRY(launch_lzss_chunks(d_comp, comp_bytes, d_ends, n_chunks, chunk_bytes, d_out, d_out_len,
-                             d_status, pick(ctx, stream), serial));
+                             d_status, pick(ctx, stream), waves));
   return CODAG_OK;
 }
 
@@ -886,6 +898,11 @@ codag_status codag_test_byte_waves(codag_ctx *ctx, uint32_t waves) {
 uint32_t codag_test_byte_one(codag_ctx *ctx, uint32_t lzss, uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes) {
   if (!ctx || !n) return ~0u;
   return lzss ? lzss_serial(comp_bytes, n, chunk_bytes, ctx->cu_count) : brle_few(comp_bytes, n, ctx->cu_count);
+}
+
+// Test hook, not in the public header: the kernel that LZSS chunks go by (lzss_waves).
+uint32_t codag_test_lzss_waves(codag_ctx *ctx, uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes) {
+  return ctx && n ? lzss_waves(comp_bytes, n, chunk_bytes, ctx->cu_count) : ~0u;
 }
 
 // Test hook, not in the public header: whether codag_inflate_chunks takes eight waves.

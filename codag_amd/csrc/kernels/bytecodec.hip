@@ -497,7 +497,8 @@ brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ptr
 
 // ------------------------------------------------------------------ LZSS
 
-// Four waves per chunk. A step takes kParts parts of kPart stream bytes:
+// Four waves per chunk, or one (lzss_waves in capi.cpp has both sides' times). A
+// step takes kParts parts of kPart stream bytes (of four waves 15, of one 3):
 //  * Group starts. A group is a flag byte and 8 items, 9 to 17 bytes by the
 //    flag's zeros, so the first group of a part starts in its first 17 bytes.
 //    Lane (part, entry) walks one part from one of these 17 bytes and notes the
@@ -512,28 +513,31 @@ brle_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ptr
 // chunks of text, before and now: 2 chunks 1.59 and 0.41 ms, 512 chunks 1.65 and
 // 0.47 ms, 2048 chunks 1.95 and 0.94 ms (bound by vector issue, mostly the
 // window's resolving).
-constexpr int kLzWaves = 4;
-constexpr uint32_t kLzThreads = kLzWaves * kWave;
-constexpr uint32_t kParts = 15, kPart = 208, kEntries = 17;
+constexpr uint32_t kPart = 208, kEntries = 17;
 constexpr uint32_t kSteps = (kPart + 8) / 9;  // groups that can start in a part
-constexpr uint32_t kLzSeg = 1536, kLzWin = kLzWaves * kLzSeg;
-constexpr uint32_t kLzStage = kLzThreads * 16;  // 16 bytes a thread
-static_assert(kParts * kEntries <= kLzThreads && kPart < 256, "a lane per part and entry, a byte per start");
-static_assert(15 + kParts * kPart + 16 + 17 + 16 <= kLzStage, "the last group of a step lies in the stage");
+constexpr uint32_t kLzSeg = 1536;
 
-struct __align__(16) LzssLds {
-  uint8_t stage[kLzStage];
-  uint16_t win[kLzWin];
+template <int NW> struct __align__(16) LzssLds {
+  static constexpr uint32_t kThreads = NW * kWave;
+  static constexpr uint32_t kParts = kThreads / kEntries;
+  static constexpr uint32_t kWin = NW * kLzSeg;
+  static constexpr uint32_t kStage = kThreads * 16;  // 16 bytes a thread
+  static_assert(kPart < 256, "a byte per start");
+  static_assert(15 + kParts * kPart + 16 + 17 + 16 <= kStage, "the last group of a step lies in the stage");
+  uint8_t stage[kStage];
+  uint16_t win[kWin];
   uint8_t start[kSteps * kParts * kEntries];  // [step][part][entry]: a group's start in its part
-  uint32_t exits[kLzThreads];                 // [part][entry]: groups << 8 | exit behind the part
-  uint32_t part[kLzWaves];
+  uint32_t exits[kThreads];                   // [part][entry]: groups << 8 | exit behind the part
+  uint32_t part[NW];
   uint32_t err;
 };
 
-// Decodes one LZSS stream of `len` bytes into dst (at most cap bytes) by four
+// Decodes one LZSS stream of `len` bytes into dst (at most cap bytes) by NW
 // waves. Every thread returns the same status and byte count.
+template <int NW>
 __device__ __forceinline__ int32_t lzss_stream(const uint8_t *src, uint32_t len, uint8_t *dst, uint32_t cap,
-                                               LzssLds &S, uint32_t *produced) {
+                                               LzssLds<NW> &S, uint32_t *produced) {
+  constexpr uint32_t kLzThreads = LzssLds<NW>::kThreads, kParts = LzssLds<NW>::kParts, kLzWin = LzssLds<NW>::kWin;
   const uint32_t lane = lane_id(), tid = threadIdx.x;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid) / kWave;
   uint32_t at = 0, pos = 0, none = 0;
@@ -558,9 +562,9 @@ __device__ __forceinline__ int32_t lzss_stream(const uint8_t *src, uint32_t len,
     }
     __syncthreads();
     // chain the parts: entry of part k and groups before it
-    uint32_t x4[kLzWaves];
+    uint32_t x4[NW];
 #pragma unroll
-    for (int k = 0; k < kLzWaves; k++) x4[k] = S.exits[k * kWave + lane];
+    for (int k = 0; k < NW; k++) x4[k] = S.exits[k * kWave + lane];
     uint32_t before[kParts], e = 0, groups = 0;
     uint32_t parts = 0;  // lane k: part k's entry, and the groups before it << 8
 #pragma unroll
@@ -569,14 +573,14 @@ __device__ __forceinline__ int32_t lzss_stream(const uint8_t *src, uint32_t len,
       parts = lane == k ? groups << 8 | e : parts;
       const uint32_t i = k * kEntries + e;
       const uint32_t a = rdlane(x4[k * kEntries / kWave], i & 63);
-      const uint32_t b = rdlane(x4[min((k * kEntries + 16) / (uint32_t)kWave, (uint32_t)kLzWaves - 1)], i & 63);
+      const uint32_t b = rdlane(x4[min((k * kEntries + 16) / (uint32_t)kWave, (uint32_t)NW - 1)], i & 63);
       const uint32_t x = i / kWave == k * kEntries / kWave ? a : b;
       e = x & 255;
       groups += x >> 8;
     }
     const uint32_t next = kParts * kPart + e;  // stream bytes this step takes
     if (next < left) w = window_load(src, len, at + next, tid);
-    // the groups, 256 at a time
+    // the groups, one a thread at a time
     for (uint32_t g0 = 0; g0 < groups && err == kOk; g0 += kLzThreads) {
       const uint32_t g = g0 + tid;
       const bool have = g < groups;
@@ -610,7 +614,7 @@ __device__ __forceinline__ int32_t lzss_stream(const uint8_t *src, uint32_t len,
       __syncthreads();
       uint32_t base = incl - n, total = 0;
 #pragma unroll
-      for (int k = 0; k < kLzWaves; k++) {
+      for (int k = 0; k < NW; k++) {
         const uint32_t p = uni(S.part[k]);
         base += k < (int)wave ? p : 0u;
         total += p;
@@ -674,7 +678,7 @@ __device__ __forceinline__ int32_t lzss_stream(const uint8_t *src, uint32_t len,
           wn = (es >> 2) - done;
           err = (int32_t)(es & 3);
         }
-        resolve_window<kLzWaves, kLzSeg, false, true>(dst, S.win, pos + done, wn, wave, lane, none, none);
+        resolve_window<NW, kLzSeg, false, true>(dst, S.win, pos + done, wn, wave, lane, none, none);
         __syncthreads();
         done += wn;
         if (err != kOk) break;
@@ -688,12 +692,13 @@ __device__ __forceinline__ int32_t lzss_stream(const uint8_t *src, uint32_t len,
   return err;
 }
 
-// 80 registers: six groups per CU (2048 chunks 1.05 -> 1.01 ms against the 96 of
+// 80 registers: six waves per SIMD (2048 chunks 1.05 -> 1.01 ms against the 96 of
 // five).
-__global__ void __launch_bounds__(kLzThreads) __attribute__((amdgpu_waves_per_eu(6)))
+template <int NW>
+__global__ void __launch_bounds__(LzssLds<NW>::kThreads) __attribute__((amdgpu_waves_per_eu(6)))
 lzss_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ends, uint64_t n, uint64_t chunk_bytes,
                    uint8_t *out, uint64_t *out_len, int32_t *status) {
-  __shared__ LzssLds S;
+  __shared__ LzssLds<NW> S;
   const uint64_t i = blockIdx.x;
   if (i >= n) return;
   const uint64_t lo = i ? ends[i - 1] : 0;  // lzss.h:237-238
@@ -702,7 +707,7 @@ lzss_chunks_kernel(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *end
   chunk_bounds(lo, ends[i], comp_bytes, len, st);
   uint32_t produced = 0;
   if (st == kOk)
-    st = lzss_stream(comp + lo, (uint32_t)len, out + i * chunk_bytes, (uint32_t)chunk_bytes, S, &produced);
+    st = lzss_stream<NW>(comp + lo, (uint32_t)len, out + i * chunk_bytes, (uint32_t)chunk_bytes, S, &produced);
   if (threadIdx.x == 0) {
     if (out_len) out_len[i] = produced;
     if (status) status[i] = st;
@@ -865,14 +870,17 @@ hipError_t launch_brle_chunks(const uint8_t *comp, uint64_t comp_bytes, const ui
 
 hipError_t launch_lzss_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ends,
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
-                              int32_t *status, hipStream_t stream, bool serial) {
+                              int32_t *status, hipStream_t stream, uint32_t waves) {
   if (n == 0) return hipSuccess;
-  if (serial)
+  if (waves == 0)
     hipLaunchKernelGGL(bytecodec::lzss_serial_kernel, dim3((uint32_t)n), dim3(kWaveSize), 0, stream, comp, comp_bytes,
                        ends, n, chunk_bytes, out, out_len, status);
+  else if (waves == 1)
+    hipLaunchKernelGGL(bytecodec::lzss_chunks_kernel<1>, dim3((uint32_t)n), dim3(kWaveSize), 0, stream, comp,
+                       comp_bytes, ends, n, chunk_bytes, out, out_len, status);
   else
-    hipLaunchKernelGGL(bytecodec::lzss_chunks_kernel, dim3((uint32_t)n), dim3(bytecodec::kLzThreads), 0, stream,
-                       comp, comp_bytes, ends, n, chunk_bytes, out, out_len, status);
+    hipLaunchKernelGGL(bytecodec::lzss_chunks_kernel<4>, dim3((uint32_t)n), dim3(4 * kWaveSize), 0, stream, comp,
+                       comp_bytes, ends, n, chunk_bytes, out, out_len, status);
   return hipGetLastError();
 }
 

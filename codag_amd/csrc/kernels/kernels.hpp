@@ -81,14 +81,14 @@ hipError_t launch_rlev2_span(const uint8_t *comp, uint64_t comp_bytes, const uin
                              uint64_t chunk_bytes, uint8_t *out, int32_t *status,
                              hipStream_t stream);
 
-// BRLE / LZSS, four waves per chunk (chunk_bytes < 2^31); few (BRLE), serial
-// (LZSS): one wave.
+// BRLE / LZSS, four waves per chunk (chunk_bytes < 2^31); few (BRLE): one wave.
+// LZSS by waves 4 or 1 with a window, 0 lzss_serial_kernel.
 hipError_t launch_brle_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ptr,
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
                               int32_t *status, hipStream_t stream, bool few);
 hipError_t launch_lzss_chunks(const uint8_t *comp, uint64_t comp_bytes, const uint64_t *ends,
                               uint64_t n, uint64_t chunk_bytes, uint8_t *out, uint64_t *out_len,
-                              int32_t *status, hipStream_t stream, bool serial);
+                              int32_t *status, hipStream_t stream, uint32_t waves);
 
 // Plain device copy (16-byte loads/stores): the reference point for HBM
 // traffic counters.
