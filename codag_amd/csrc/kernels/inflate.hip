@@ -30,7 +30,7 @@
 // chunks, before (one token chain per stream: 64 bit positions decoded to keep
 // about seven tokens, the chain scalar) and now: 4096 chunks 9.1 and 2.96 ms, 256
 // chunks 4.0 and 0.44 ms, 3 chunks 3.7 and 0.42 ms; 300 mixed streams of 4 KiB
-// to 4 MiB 119 and 14.6 ms. A chunk takes 0.27 M vector instructions (0.69 M
+// to 4 MiB 119 and 14.6 ms. A chunk takes 0.25 M vector instructions (0.69 M
 // before): half of them passes, headers and tables, a fifth marks, a third the
 // resolving. A window byte costs the same whatever token it is in, so data that
 // compress to less than a thirtieth go by narrow_span (4096 chunks of zeros 1.1
