@@ -209,10 +209,13 @@ bool inflate_many(uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes, uint32_
 // chunks 231, 66), and where five groups per CU are filled several times over one
 // wave's slower chunks overtake (16 KiB of it, 2048 chunks 47, 47, 4096 chunks 87,
 // 63; 256 KiB, 1024 chunks 260, 580, 2048 chunks 500, 645, 4096 chunks 956, 861).
-bool brle_few(uint64_t comp_bytes, uint64_t n, uint32_t cus) {
+// Streams longer than their chunks are long literals, whose starts often never meet;
+// then most of a step is one wave's chain (64 KiB, 1024 chunks: random bytes 220, 222,
+// counters 238, 237, text 59, 113; 2048 chunks: 424, 257, 470, 272, 111, 134).
+bool brle_few(uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes, uint32_t cus) {
   const uint64_t each = comp_bytes / n;  // stream bytes of a chunk
   if (each <= 4200) return true;
-  return n > (each <= 24576 ? 7ull : 15ull) * cus;
+  return n > (each <= 24576 || (each >= chunk_bytes && each <= 98304) ? 7ull : 15ull) * cus;
 }
 
 // Whether an LZSS container goes by lzss_serial_kernel, one wave per chunk with its
@@ -476,7 +479,7 @@ codag_status codag_brle_decode(codag_ctx *ctx, const uint8_t *d_comp, uint64_t c
   if (codag_status s = byte_codec_args("brle_decode", ctx, d_comp, d_ptr, n_chunks, chunk_bytes, d_out))
     return s;
   DeviceGuard g(ctx->device);
-  bool few = n_chunks && brle_few(comp_bytes, n_chunks, ctx->cu_count);
+  bool few = n_chunks && brle_few(comp_bytes, n_chunks, chunk_bytes, ctx->cu_count);
   if (ctx->byte_waves) few = ctx->byte_waves == 1;
   HIP_TRY(launch_brle_chunks(d_comp, comp_bytes, d_ptr, n_chunks, chunk_bytes, d_out, d_out_len,
                              d_status, pick(ctx, stream), few));
@@ -897,7 +900,7 @@ codag_status codag_test_byte_waves(codag_ctx *ctx, uint32_t waves) {
 // of n > 0 chunks takes the kernel of one wave per chunk.
 uint32_t codag_test_byte_one(codag_ctx *ctx, uint32_t lzss, uint64_t comp_bytes, uint64_t n, uint64_t chunk_bytes) {
   if (!ctx || !n) return ~0u;
-  return lzss ? lzss_serial(comp_bytes, n, chunk_bytes, ctx->cu_count) : brle_few(comp_bytes, n, ctx->cu_count);
+  return lzss ? lzss_serial(comp_bytes, n, chunk_bytes, ctx->cu_count) : brle_few(comp_bytes, n, chunk_bytes, ctx->cu_count);
 }
 
 // Test hook, not in the public header: the kernel that LZSS chunks go by (lzss_waves).
